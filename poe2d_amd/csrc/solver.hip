@@ -44,6 +44,7 @@ namespace {
 const float kRefPiF = 3.1415926535897932f;  // the reference's float PI (seismic_CPML_2d_poroelastic.cpp:9)
 const double kStabilityThreshold = 1.0e25;  // STABILITY_THRESHOLD of the reference (declared, unused there)
 const int kGraphSteps = 32;                 // steps per captured graph
+const long long kShortTilesMax = 1280;      // launches of up to this many short tiles use them (five per CU)
 
 #define HIP_TRY(expr)                                                                              \
     do {                                                                                           \
@@ -128,28 +129,29 @@ struct Model {
 // the per-model arguments it points to are rewritten before every run.
 struct StepList {
     void *models = nullptr;      // StepArgs<T>[nmodels]
-    WorkItem *work = nullptr;    // [nwork]
+    void *work = nullptr;        // WorkItem[nwork], or TileItem[nwork] (tile kernel)
     int *rec_ptr = nullptr;      // receiver offsets per (row, tile column), all models
-    int2 *rec_ent = nullptr;     // receiver entries, all models
+    void *rec_ent = nullptr;     // receiver entries, all models: int2, or int4 (tile kernel)
     long long *base = nullptr;   // step of launch 0 of the current chunk
     long long *h_base = nullptr; // pinned host staging of base
     size_t cap_models = 0, cap_work = 0, cap_ptr = 0, cap_ent = 0;
     int nmodels = 0, nwork = 0, per_xcd = 0, bw = 0;
     bool palette = false;
     bool avg = false;  // POE2D_MATERIAL_AVERAGED (all members alike)
-    bool two = false;  // two-step kernel: each launch advances two steps
+    bool two = false;  // two-step or tile kernel: each launch advances two steps
+    bool tiles = false;  // tile kernel
     int nint = 0;      // two-step kernel: interior tiles in the list
     int precision = POE2D_F32;
     // graph of kGraphSteps launches plus the base advance, and the launch it was captured for
     hipGraphExec_t exec = nullptr;
     struct Sig {
         void *models, *work, *base;
-        int nwork, nint, per_xcd, bw, palette, avg, two, precision;
+        int nwork, nint, per_xcd, bw, palette, avg, two, tiles, precision;
         bool operator==(const Sig &o) const
         {
             return models == o.models && work == o.work && base == o.base && nwork == o.nwork && nint == o.nint &&
                    per_xcd == o.per_xcd && bw == o.bw && palette == o.palette && avg == o.avg && two == o.two &&
-                   precision == o.precision;
+                   tiles == o.tiles && precision == o.precision;
         }
     } sig{};
 
@@ -158,6 +160,7 @@ struct StepList {
         Sig g{};
         g.models = models; g.work = work; g.base = base;
         g.nwork = nwork; g.nint = nint; g.per_xcd = per_xcd; g.bw = bw; g.palette = palette; g.avg = avg; g.two = two;
+        g.tiles = tiles;
         g.precision = precision;
         return g;
     }
@@ -167,9 +170,9 @@ struct StepList {
         if (exec) (void)hipGraphExecDestroy(exec);
         exec = nullptr;
         dev_free(models);
-        void *q = work; dev_free(q); work = nullptr;
-        q = rec_ptr; dev_free(q); rec_ptr = nullptr;
-        q = rec_ent; dev_free(q); rec_ent = nullptr;
+        dev_free(work);
+        void *q = rec_ptr; dev_free(q); rec_ptr = nullptr;
+        dev_free(rec_ent);
         q = base; dev_free(q); base = nullptr;
         if (h_base) (void)hipHostFree(h_base);
         h_base = nullptr;
@@ -210,8 +213,9 @@ struct poe2d_solver {
     long long src_n0 = 0;
     int src_len = 0;
     // schedule
-    int schedule = SCHED_FUSED;
+    int schedule = SCHED_FUSED2;
     int block_w = 256, tile_rows = 14;
+    bool auto_shape = true;  // until a schedule or a tile shape is chosen: see tile_shape
     bool graphs = true;
     // source
     bool have_src = false;
@@ -223,6 +227,7 @@ struct poe2d_solver {
     int nrec = 0, dec = 1, nsamp = 0, ncomp = 0;
     unsigned mask = 0;
     int *rix = nullptr, *riz = nullptr;
+    std::vector<int> hrx, hrz;  // their host copies
     void *traces = nullptr;  // [slot][comp][rec]
     int step = 0;
     double last_ms = 0;
@@ -251,6 +256,7 @@ struct poe2d_batch {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int block_w = 256, tile_rows = 14;
+    bool auto_shape = true;
     bool graphs = true;
     double last_ms = 0;
     int last_steps = 0;
@@ -508,7 +514,7 @@ StepArgs<T> step_args(const poe2d_solver *s, int in, int out, int bw, int th, bo
     A.par = (int)(((long long)s->cur - s->step) & 1);
     A.th = th;
     const int W = two ? fused2_tile_width(bw) : fused_tile_width(bw);
-    A.ntx = (g.nx + 1 + W - 1) / W;
+    A.ntx = (g.nx + 1 + W - 1) / W;  // (the tile kernel's items carry their own columns and rows)
     A.psi_mid = (T *)s->psi_mid;
     A.pair0 = s->step;
     A.pcur = s->cur;
@@ -535,6 +541,36 @@ poe2d_status upload_source(poe2d_solver *s, long long n0, int k)
     HIP_TRY(hipMemcpy(s->src_dev, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
     s->src_n0 = n0;
     s->src_len = k;
+    return POE2D_OK;
+}
+
+// Device copies of a list's arrays: work items, receiver offsets and entries, and the members'
+// arguments once `fix` has pointed each at its receivers.  Waits for `stream` first.
+template <class T, class F>
+poe2d_status upload_list(StepList &L, std::vector<StepArgs<T>> &args, const void *work, size_t work_bytes,
+                         const std::vector<int> &ptr, const void *ent, size_t nent, size_t ent_size, hipStream_t stream,
+                         F fix)
+{
+    poe2d_status st;
+    HIP_TRY(hipStreamSynchronize(stream));
+    if ((st = grow(&L.models, &L.cap_models, args.size() * sizeof(StepArgs<T>)))) return st;
+    if ((st = grow(&L.work, &L.cap_work, work_bytes))) return st;
+    void *pp = L.rec_ptr;
+    st = grow(&pp, &L.cap_ptr, std::max<size_t>(ptr.size(), 1) * sizeof(int));
+    L.rec_ptr = (int *)pp;
+    if (st) return st;
+    if ((st = grow(&L.rec_ent, &L.cap_ent, std::max<size_t>(nent, 1) * ent_size))) return st;
+    for (size_t i = 0; i < args.size(); ++i) fix(args[i], (int)i);
+    if (!L.base) {
+        void *q = nullptr;
+        if ((st = dev_alloc(&q, sizeof(long long)))) return st;
+        L.base = (long long *)q;
+    }
+    if (!L.h_base) HIP_TRY(hipHostMalloc((void **)&L.h_base, sizeof(long long), hipHostMallocDefault));
+    HIP_TRY(hipMemcpy(L.models, args.data(), args.size() * sizeof(StepArgs<T>), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(L.work, work, work_bytes, hipMemcpyHostToDevice));
+    if (!ptr.empty()) HIP_TRY(hipMemcpy(L.rec_ptr, ptr.data(), ptr.size() * sizeof(int), hipMemcpyHostToDevice));
+    if (nent) HIP_TRY(hipMemcpy(L.rec_ent, ent, nent * ent_size, hipMemcpyHostToDevice));
     return POE2D_OK;
 }
 
@@ -576,11 +612,7 @@ poe2d_status build_list(StepList &L, const std::vector<poe2d_solver *> &members,
         const int ntx = args[i].ntx, nrow = s->grid.nz + 1;
         std::vector<int> order(s->nrec);
         for (int r = 0; r < s->nrec; ++r) order[r] = r;
-        std::vector<int> hx(s->nrec), hz(s->nrec);
-        if (s->nrec > 0) {
-            HIP_TRY(hipMemcpy(hx.data(), s->rix, s->nrec * sizeof(int), hipMemcpyDeviceToHost));
-            HIP_TRY(hipMemcpy(hz.data(), s->riz, s->nrec * sizeof(int), hipMemcpyDeviceToHost));
-        }
+        const std::vector<int> &hx = s->hrx, &hz = s->hrz;
         std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
             if (hx[a] / W != hx[b] / W) return hx[a] / W < hx[b] / W;
             return hz[a] != hz[b] ? hz[a] < hz[b] : hx[a] < hx[b];
@@ -636,35 +668,12 @@ poe2d_status build_list(StepList &L, const std::vector<poe2d_solver *> &members,
             for (size_t q = (size_t)x * ni; q < std::min(inter.size(), (size_t)(x + 1) * ni); ++q) work[o++] = inter[q];
         }
     }
-    poe2d_status st;
-    if ((st = grow(&L.models, &L.cap_models, args.size() * sizeof(StepArgs<T>)))) return st;
-    void *w = L.work;
-    st = grow(&w, &L.cap_work, work.size() * sizeof(WorkItem));
-    L.work = (WorkItem *)w;
+    const poe2d_status st = upload_list<T>(L, args, work.data(), work.size() * sizeof(WorkItem), ptr, ent.data(),
+                                           ent.size(), sizeof(int2), stream, [&](StepArgs<T> &A, int i) {
+                                               A.rec_tile_ptr = L.rec_ptr + ptr_off[i];
+                                               A.rec_entries = (const int2 *)L.rec_ent + ent_off[i];
+                                           });
     if (st) return st;
-    void *pp = L.rec_ptr;
-    st = grow(&pp, &L.cap_ptr, ptr.size() * sizeof(int));
-    L.rec_ptr = (int *)pp;
-    if (st) return st;
-    void *pe = L.rec_ent;
-    st = grow(&pe, &L.cap_ent, std::max<size_t>(ent.size(), 1) * sizeof(int2));
-    L.rec_ent = (int2 *)pe;
-    if (st) return st;
-    for (int i = 0; i < nm; ++i) {
-        args[i].rec_tile_ptr = L.rec_ptr + ptr_off[i];
-        args[i].rec_entries = L.rec_ent + ent_off[i];
-    }
-    if (!L.base) {
-        void *q = nullptr;
-        if ((st = dev_alloc(&q, sizeof(long long)))) return st;
-        L.base = (long long *)q;
-    }
-    if (!L.h_base) HIP_TRY(hipHostMalloc((void **)&L.h_base, sizeof(long long), hipHostMallocDefault));
-    HIP_TRY(hipStreamSynchronize(stream));
-    HIP_TRY(hipMemcpy(L.models, args.data(), args.size() * sizeof(StepArgs<T>), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(L.work, work.data(), work.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(L.rec_ptr, ptr.data(), ptr.size() * sizeof(int), hipMemcpyHostToDevice));
-    if (!ent.empty()) HIP_TRY(hipMemcpy(L.rec_ent, ent.data(), ent.size() * sizeof(int2), hipMemcpyHostToDevice));
     L.nmodels = nm;
     L.nint = two ? nint : (int)work.size();
     L.nwork = (int)work.size();
@@ -673,6 +682,96 @@ poe2d_status build_list(StepList &L, const std::vector<poe2d_solver *> &members,
     L.palette = palette;
     L.avg = material == POE2D_MATERIAL_AVERAGED;
     L.two = two;
+    L.tiles = false;
+    L.precision = sizeof(T) == 4 ? POE2D_F32 : POE2D_F64;
+    return POE2D_OK;
+}
+
+// As build_list, for the tile kernel: each member's grid cut into tiles of kTileCols columns, their
+// rows in tiles of kTileShort rows where the region reaches a C-PML strip or the border (edge tiles)
+// and of kTileTall rows elsewhere (`tall`; else kTileShort), each with its receivers.
+template <class T>
+poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members, bool tall, bool palette,
+                         hipStream_t stream)
+{
+    const int nm = (int)members.size();
+    const int material = members[0]->grid.staggered_material;
+    tall = tall && sizeof(T) == 4;
+    std::vector<StepArgs<T>> args(nm);
+    std::vector<TileItem> edge, inter;
+    std::vector<int4> ent;
+    for (int i = 0; i < nm; ++i) {
+        const poe2d_solver *s = members[i];
+        const Model *md = s->m;
+        if (palette && (md->npal < 1 || !md->mid || !md->pal))
+            return fail(POE2D_E_INVALID, "run: a palette launch over a grid without a palette");
+        if (s->grid.staggered_material != material)
+            return fail(POE2D_E_INVALID, "run: batch members differ in staggered material");
+        args[i] = step_args<T>(s, 0, 1, 64, kTileShort, true);
+        args[i].rec_n = s->nrec;
+        args[i].rec_ncomp = s->ncomp;
+        args[i].rec_dec = s->dec;
+        args[i].rec_nsamp = s->nsamp;
+        args[i].rec_mask = s->mask;
+        args[i].traces = (T *)s->traces;
+        const int nx = s->grid.nx, nz = s->grid.nz;
+        // receivers by tile column and row
+        std::vector<int> order(s->nrec);
+        for (int r = 0; r < s->nrec; ++r) order[r] = r;
+        std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+            const int ta = s->hrx[a] / kTileCols, tb = s->hrx[b] / kTileCols;
+            return ta != tb ? ta < tb : s->hrz[a] < s->hrz[b];
+        });
+        size_t next = 0;
+        for (int x0 = 0; x0 <= nx; x0 += kTileCols) {
+            const int c0 = x0 - kTileHalo, c1 = c0 + 63;  // the region's columns
+            const bool xs = c0 < std::max(md->xlo, 2) || c1 >= std::min(md->xhi, nx - 1);
+            const int zlo = std::max(md->ztop, 2), zhi = std::min(md->zbot, nz - 1);
+            for (int z0 = 0; z0 <= nz;) {
+                // rows [z0 - halo, z0 + rows + halo) of the region within [zlo, zhi)
+                auto inside = [&](int rows) { return !xs && z0 - kTileHalo >= zlo && z0 + rows + kTileHalo <= zhi; };
+                TileItem it{};
+                it.model = i;
+                it.x0 = x0;
+                it.z0 = z0;
+                it.kind = tall && inside(kTileTall) ? TILE_TALL : inside(kTileShort) ? TILE_SHORT : TILE_EDGE;
+                it.z1 = std::min(z0 + (it.kind == TILE_TALL ? kTileTall : kTileShort), nz + 1);
+                it.rec_lo = (int)ent.size();
+                while (next < order.size() && s->hrx[order[next]] < x0 + kTileCols && s->hrz[order[next]] < it.z1) {
+                    const int r = order[next++];
+                    ent.push_back(int4{s->hrx[r], s->hrz[r], r, 0});
+                }
+                it.rec_hi = (int)ent.size();
+                (it.kind == TILE_EDGE ? edge : inter).push_back(it);
+                z0 = it.z1;
+            }
+            if (edge.size() + inter.size() > (1u << 28)) return fail(POE2D_E_INVALID, "run: too many tiles in one launch");
+        }
+    }
+    // as the two-step kernel's list: every XCD gets an eighth of the edge tiles first, then a run of
+    // consecutive interior tiles; shares padded to equal length with empty items
+    const int ne = (int)((edge.size() + 7) / 8), ni = (int)((inter.size() + 7) / 8);
+    TileItem none{};
+    none.model = -1;
+    std::vector<TileItem> work((size_t)8 * (ne + ni), none);
+    for (int x = 0; x < 8; ++x) {
+        size_t o = (size_t)x * (ne + ni);
+        for (size_t e = x; e < edge.size(); e += 8) work[o++] = edge[e];
+        for (size_t q = (size_t)x * ni; q < std::min(inter.size(), (size_t)(x + 1) * ni); ++q) work[o++] = inter[q];
+    }
+    const poe2d_status st = upload_list<T>(L, args, work.data(), work.size() * sizeof(TileItem), {}, ent.data(), ent.size(),
+                                           sizeof(int4), stream,
+                                           [&](StepArgs<T> &A, int) { A.rec_points = (const int4 *)L.rec_ent; });
+    if (st) return st;
+    L.nmodels = nm;
+    L.nint = (int)inter.size();
+    L.nwork = (int)work.size();
+    L.per_xcd = ne + ni;
+    L.bw = 64;
+    L.palette = palette;
+    L.avg = material == POE2D_MATERIAL_AVERAGED;
+    L.two = true;
+    L.tiles = true;
     L.precision = sizeof(T) == 4 ? POE2D_F32 : POE2D_F64;
     return POE2D_OK;
 }
@@ -682,10 +781,18 @@ poe2d_status build_list(StepList &L, const std::vector<poe2d_solver *> &members,
 template <class T>
 hipError_t launch_list_chunk(const StepList &L, int count, hipStream_t stream)
 {
+    if (L.tiles) {
+        for (int k = 0; k < count; ++k) {
+            const hipError_t e = launch_tiles<T>((const StepArgs<T> *)L.models, (const TileItem *)L.work, L.nwork, L.per_xcd,
+                                                 L.palette, L.avg, L.base, 2 * k, 2, stream);
+            if (e != hipSuccess) return e;
+        }
+        return launch_base_advance(L.base, 2 * count, stream);
+    }
     if (L.two) {
         if constexpr (sizeof(T) == 4) {
             for (int k = 0; k < count; ++k) {
-                const hipError_t e = launch_fused2<T>((const StepArgs<T> *)L.models, L.work, L.nwork, L.per_xcd, L.bw,
+                const hipError_t e = launch_fused2<T>((const StepArgs<T> *)L.models, (const WorkItem *)L.work, L.nwork, L.per_xcd, L.bw,
                                                       L.palette, L.avg, L.base, 2 * k, stream);
                 if (e != hipSuccess) return e;
             }
@@ -694,7 +801,7 @@ hipError_t launch_list_chunk(const StepList &L, int count, hipStream_t stream)
         return hipErrorInvalidValue;
     }
     for (int k = 0; k < count; ++k) {
-        hipError_t e = launch_fused<T>((const StepArgs<T> *)L.models, L.work, L.nwork, L.per_xcd, L.bw, L.palette,
+        hipError_t e = launch_fused<T>((const StepArgs<T> *)L.models, (const WorkItem *)L.work, L.nwork, L.per_xcd, L.bw, L.palette,
                                        L.avg, L.base, k, stream);
         if (e != hipSuccess) return e;
     }
@@ -738,6 +845,19 @@ poe2d_status run_list(StepList &L, long long n0, int k, bool graphs, hipStream_t
     return POE2D_OK;
 }
 
+// nsteps steps of the members (all at step n0) on the tile kernel: step pairs, and a launch of one
+// step for an odd last one.
+template <class T>
+poe2d_status run_tiles(StepList &L, long long n0, int nsteps, bool graphs, hipStream_t stream)
+{
+    poe2d_status st;
+    if ((st = run_list<T>(L, n0, nsteps / 2, graphs, stream))) return st;
+    if (nsteps & 1)
+        HIP_TRY(launch_tiles<T>((const StepArgs<T> *)L.models, (const TileItem *)L.work, L.nwork, L.per_xcd, L.palette, L.avg,
+                                L.base, 0, 1, stream));
+    return POE2D_OK;
+}
+
 // Largest |v| of the handle's current state; POE2D_E_UNSTABLE above the reference's threshold.
 template <class T>
 poe2d_status stability_check(poe2d_solver *s)
@@ -753,18 +873,58 @@ poe2d_status stability_check(poe2d_solver *s)
     return POE2D_OK;
 }
 
-// The kernel a handle's steps run on: schedule 3 takes the two-step kernel on FP32 grids (through
-// the palette where the grid's fits that kernel's LDS copy, else through the coefficient groups),
-// and the single-step kernel (as schedule 0, 64-thread blocks widened to 128) on FP64 grids.
+// The kernel a handle's steps run on: schedule 3 takes the tile kernel (block width 64) or, on FP32
+// grids, the two-step kernel (through the palette where the grid's fits that kernel's LDS copy, else
+// through the coefficient groups); FP64 grids take the single-step kernel at the other widths.
 bool two_step_kernel(const poe2d_solver *s)
 {
     return s->schedule == SCHED_FUSED2 && s->precision == POE2D_F32;
 }
 // Whether the two-step kernel reads handle s through its palette.
 bool two_step_palette(const poe2d_solver *s) { return s->m->npal > 0 && s->m->npal <= kMaxPalette2; }
-int effective_schedule(const poe2d_solver *s)
+struct TileShape {
+    bool tiles;  // the tile kernel
+    int bw, th;
+};
+
+// The tile shape the members advance with: the chosen one, or (auto_shape) the tile kernel, whose
+// short tiles (twice the blocks, half the rows per thread) serve launches that tall ones would not
+// spread over the chip: us per step, short / tall, 401^2 continuous 7.4 / 9.3, 1001 x 777 14.9 /
+// 15.1 (1300 short tiles), 1201^2 22.3 / 20.1 (2400), 4001^2 190.6 / 137.1.  FP64 has short tiles only.
+TileShape tile_shape(const std::vector<poe2d_solver *> &members, bool auto_shape, int bw, int th)
 {
-    return s->schedule == SCHED_FUSED2 && !two_step_kernel(s) ? SCHED_FUSED : s->schedule;
+    for (const poe2d_solver *s : members)
+        if (s->schedule != SCHED_FUSED2) return {false, bw, th};
+    if (!auto_shape) return {bw == 64, bw, th};
+    long long tiles = 0;
+    for (const poe2d_solver *s : members)
+        tiles += (long long)(s->grid.nx / kTileCols + 1) * (s->grid.nz / kTileShort + 1);
+    return {true, 64, tiles > kShortTilesMax ? kTileTall : kTileShort};
+}
+
+// Shapes an autotuner times: of the two-step schedule (the tile kernel's two and the marching
+// kernel's), of the single-step kernel, and for FP64 handles on schedule 3 the tile kernel's too.
+std::vector<std::pair<int, int>> tune_shapes(const std::vector<poe2d_solver *> &members)
+{
+    bool two = true, tiles = true;
+    int nz = 0;
+    for (const poe2d_solver *s : members) {
+        two = two && two_step_kernel(s);
+        tiles = tiles && s->schedule == SCHED_FUSED2;
+        nz = std::max(nz, s->grid.nz);
+    }
+    std::vector<std::pair<int, int>> out;
+    if (tiles) out.push_back({64, kTileShort});
+    if (two) out.push_back({64, kTileTall});
+    // Tile heights of 6k + 2 rows (6k for the two-step kernel) make whole groups of the kernels'
+    // 6-step row loops.
+    const std::vector<int> widths = two ? std::vector<int>{128, 256} : std::vector<int>{128, 256, 512};
+    const std::vector<int> heights = two ? std::vector<int>{6, 12, 18, 24, 30, 42, 60}
+                                         : std::vector<int>{8, 14, 20, 26, 32, 44, 62, 98};
+    for (int w : widths)
+        for (int h : heights)
+            if (h <= nz + 1 || h == heights[0]) out.push_back({w, h});
+    return out;
 }
 
 template <class T>
@@ -787,18 +947,24 @@ poe2d_status run_steps(poe2d_solver *s, int nsteps)
         }
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipEventRecord(s->ev1, s->stream));
+    } else if (const TileShape shape = tile_shape({s}, s->auto_shape, s->block_w, s->tile_rows); shape.tiles) {
+        if ((st = upload_source<T>(s, s->step, nsteps))) return st;
+        if ((st = build_tiles<T>(s->list2, {s}, shape.th >= kTileTall, s->m->npal > 0, s->stream))) return st;
+        HIP_TRY(hipEventRecord(s->ev0, s->stream));
+        if ((st = run_tiles<T>(s->list2, s->step, nsteps, s->graphs, s->stream))) return st;
+        HIP_TRY(hipEventRecord(s->ev1, s->stream));
+        s->cur = (s->cur + nsteps / 2 + (nsteps & 1)) & 1;
     } else if (sizeof(T) == 4 && two_step_kernel(s)) {
         // step pairs on the two-step kernel, an odd last step on the single-step kernel
         const int pairs = nsteps / 2, rem = nsteps & 1;
         if (!s->psi_mid && (st = dev_alloc(&s->psi_mid, std::max<size_t>(s->m->psi_half_elems(), 1) * s->rs)))
             return st;
         if ((st = upload_source<T>(s, s->step, nsteps))) return st;
-        if (pairs && (st = build_list<T>(s->list2, {s}, s->block_w, s->tile_rows, two_step_palette(s), s->stream, true)))
+        if (pairs && (st = build_list<T>(s->list2, {s}, shape.bw, shape.th, two_step_palette(s), s->stream, true)))
             return st;
-        // (the single-step kernel has no 64-thread blocks; it reads the palette whenever the grid
-        // has one, which may be larger than the two-step kernel's)
-        if (rem && (st = build_list<T>(s->list, {s}, std::max(s->block_w, 128), s->tile_rows, s->m->npal > 0,
-                                       s->stream, false, pairs)))
+        // (the single-step kernel reads the palette whenever the grid has one, which may be larger
+        // than the two-step kernel's)
+        if (rem && (st = build_list<T>(s->list, {s}, shape.bw, shape.th, s->m->npal > 0, s->stream, false, pairs)))
             return st;
         HIP_TRY(hipEventRecord(s->ev0, s->stream));
         if (pairs && (st = run_list<T>(s->list2, s->step, pairs, s->graphs, s->stream))) return st;
@@ -808,8 +974,7 @@ poe2d_status run_steps(poe2d_solver *s, int nsteps)
     } else {
         if ((st = upload_source<T>(s, s->step, nsteps))) return st;
         const bool palette = (s->schedule == SCHED_FUSED || s->schedule == SCHED_FUSED2) && s->m->npal > 0;
-        const int bw = s->schedule == SCHED_FUSED2 ? std::max(s->block_w, 128) : s->block_w;
-        if ((st = build_list<T>(s->list, {s}, bw, s->tile_rows, palette, s->stream))) return st;
+        if ((st = build_list<T>(s->list, {s}, shape.bw, shape.th, palette, s->stream))) return st;
         HIP_TRY(hipEventRecord(s->ev0, s->stream));
         if ((st = run_list<T>(s->list, s->step, nsteps, s->graphs, s->stream))) return st;
         HIP_TRY(hipEventRecord(s->ev1, s->stream));
@@ -886,12 +1051,6 @@ poe2d_solver *new_handle(Model *md, poe2d_status *st)
     s->precision = md->precision;
     s->rs = md->rs;
     s->grid = md->grid;
-    if (s->precision == POE2D_F32) {
-        // FP32 handles start on schedule 3: the two-step kernel where the grid's palette fits it,
-        // the single-step kernel elsewhere, the same results either way
-        s->schedule = SCHED_FUSED2;
-        s->tile_rows = 24;
-    }
     auto bail = [&](poe2d_status e) -> poe2d_solver * {
         *st = e;
         free_handle(s);
@@ -923,31 +1082,40 @@ template <class T>
 poe2d_status batch_run_steps(poe2d_batch *b, int nsteps)
 {
     const long long n0 = b->members[0]->step;
-    bool palette = true, two = sizeof(T) == 4, palette2 = true;
+    bool palette = true, two = sizeof(T) == 4, palette2 = true, tile_palette = true;
     for (poe2d_solver *s : b->members) {
         poe2d_status st = upload_source<T>(s, n0, nsteps);
         if (st) return st;
         palette = palette && (s->schedule == SCHED_FUSED || s->schedule == SCHED_FUSED2) && s->m->npal > 0;
         two = two && two_step_kernel(s);
         palette2 = palette2 && two_step_palette(s);
+        tile_palette = tile_palette && s->m->npal > 0;
     }
+    const TileShape shape = tile_shape(b->members, b->auto_shape, b->block_w, b->tile_rows);
     // (the single-step kernel widens 64-thread blocks to 128, below)
-    if (two && b->block_w == 512)
+    if ((two || shape.tiles) && shape.bw == 512)
         return fail(POE2D_E_INVALID, "batch_run: the two-step kernel takes block widths 64, 128 or 256");
+    two = two || shape.tiles;
     const int pairs = two ? nsteps / 2 : 0, rem = two ? nsteps & 1 : nsteps;
     poe2d_status st;
-    if (pairs) {
+    if (shape.tiles) {
+        if ((st = build_tiles<T>(b->list2, b->members, shape.th >= kTileTall, tile_palette, b->stream))) return st;
+    } else if (pairs) {
         for (poe2d_solver *s : b->members)
             if (!s->psi_mid && (st = dev_alloc(&s->psi_mid, std::max<size_t>(s->m->psi_half_elems(), 1) * s->rs)))
                 return st;
-        if ((st = build_list<T>(b->list2, b->members, b->block_w, b->tile_rows, palette2, b->stream, true))) return st;
+        if ((st = build_list<T>(b->list2, b->members, shape.bw, shape.th, palette2, b->stream, true))) return st;
     }
-    if (rem && (st = build_list<T>(b->list, b->members, std::max(b->block_w, 128), b->tile_rows, palette, b->stream,
-                                   false, pairs)))
+    if (rem && !shape.tiles &&
+        (st = build_list<T>(b->list, b->members, std::max(shape.bw, 128), shape.th, palette, b->stream, false, pairs)))
         return st;
     HIP_TRY(hipEventRecord(b->ev0, b->stream));
-    if (pairs && (st = run_list<T>(b->list2, n0, pairs, b->graphs, b->stream))) return st;
-    if (rem && (st = run_list<T>(b->list, n0 + 2LL * pairs, rem, b->graphs, b->stream))) return st;
+    if (shape.tiles) {
+        if ((st = run_tiles<T>(b->list2, n0, nsteps, b->graphs, b->stream))) return st;
+    } else {
+        if (pairs && (st = run_list<T>(b->list2, n0, pairs, b->graphs, b->stream))) return st;
+        if (rem && (st = run_list<T>(b->list, n0 + 2LL * pairs, rem, b->graphs, b->stream))) return st;
+    }
     HIP_TRY(hipEventRecord(b->ev1, b->stream));
     HIP_TRY(hipEventSynchronize(b->ev1));
     float ms = 0.f;
@@ -1066,6 +1234,7 @@ poe2d_status poe2d_clone(poe2d_solver *s, poe2d_solver **out)
     c->schedule = s->schedule;
     c->block_w = s->block_w;
     c->tile_rows = s->tile_rows;
+    c->auto_shape = s->auto_shape;
     c->graphs = s->graphs;
     *out = c;
     return POE2D_OK;
@@ -1126,6 +1295,7 @@ poe2d_status poe2d_set_schedule(poe2d_solver *s, int schedule, int block_w, int 
     s->schedule = schedule;
     s->block_w = block_w;
     s->tile_rows = tile_rows;
+    s->auto_shape = false;
     return POE2D_OK;
 }
 
@@ -1205,6 +1375,8 @@ poe2d_status poe2d_set_receivers(poe2d_solver *s, const poe2d_receivers *r)
     s->riz = (int *)q;
     if ((st = dev_alloc_zero(&s->traces, s->trace_bytes(), s->stream))) return st;
     HIP_TRY(hipStreamSynchronize(s->stream));
+    s->hrx.assign(r->ix, r->ix + r->n);
+    s->hrz.assign(r->iz, r->iz + r->n);
     HIP_TRY(hipMemcpy(s->rix, r->ix, (size_t)r->n * sizeof(int), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(s->riz, r->iz, (size_t)r->n * sizeof(int), hipMemcpyHostToDevice));
     return POE2D_OK;
@@ -1411,36 +1583,30 @@ poe2d_status poe2d_autotune(poe2d_solver *s, int nsteps, int *block_w, int *tile
     if (st) return st;
     if (s->schedule == SCHED_TWOPASS) return fail(POE2D_E_INVALID, "autotune: the two-pass schedule has no tile shape");
     if (s->step != 0) return fail(POE2D_E_STATE, "autotune: needs a handle at step 0 (call poe2d_reset first)");
-    const std::string key = tune_key({s}, effective_schedule(s));
+    const std::string key = tune_key({s}, s->schedule);
     if (nsteps >= 0) {
         int w, h;
         if (tune_lookup(key, &w, &h)) {
             s->block_w = w;
             s->tile_rows = h;
+            s->auto_shape = false;
             if (block_w) *block_w = w;
             if (tile_rows) *tile_rows = h;
             return POE2D_OK;
         }
     }
     nsteps = nsteps == 0 ? 10 : std::abs(nsteps);
-    // Tile heights of 6k + 2 rows (6k for the two-step kernel) make whole groups of the kernels'
-    // 6-step row loops.
-    const bool two = two_step_kernel(s);
-    const std::vector<int> widths = two ? std::vector<int>{64, 128, 256} : std::vector<int>{128, 256, 512};
-    const std::vector<int> heights = two ? std::vector<int>{6, 12, 18, 24, 30, 42, 60}
-                                         : std::vector<int>{8, 14, 20, 26, 32, 44, 62, 98};
     // One timed run per shape, then the three fastest timed again over three times the steps, twice
     // each, the best of those kept: shapes within a few per cent of each other are told apart by
     // more than one sample.
     std::vector<std::pair<double, std::pair<int, int>>> cand;
-    for (int w : widths)
-        for (int h : heights) {
-            if (h > s->grid.nz + 1 && h != heights[0]) continue;
-            s->block_w = w;
-            s->tile_rows = h;
-            if ((st = poe2d_run(s, 1)) || (st = poe2d_run(s, nsteps))) break;
-            cand.push_back({s->last_ms, {w, h}});
-        }
+    s->auto_shape = false;
+    for (const auto &shape : tune_shapes({s})) {
+        s->block_w = shape.first;
+        s->tile_rows = shape.second;
+        if ((st = poe2d_run(s, 1)) || (st = poe2d_run(s, nsteps))) break;
+        cand.push_back({s->last_ms, shape});
+    }
     int best_w = s->block_w, best_h = s->tile_rows;
     if (!st && !cand.empty()) {
         std::sort(cand.begin(), cand.end());
@@ -1502,6 +1668,7 @@ poe2d_status poe2d_batch_create(int n, poe2d_solver *const *members, poe2d_batch
     b->precision = members[0]->precision;
     b->block_w = members[0]->block_w;
     b->tile_rows = members[0]->tile_rows;
+    for (int i = 0; i < n; ++i) b->auto_shape = b->auto_shape && members[i]->auto_shape;
     if (hipSetDevice(b->device) != hipSuccess || hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&b->ev0) != hipSuccess || hipEventCreate(&b->ev1) != hipSuccess) {
         poe2d_batch_destroy(b);
@@ -1521,6 +1688,7 @@ poe2d_status poe2d_batch_set_schedule(poe2d_batch *b, int block_w, int tile_rows
     if (tile_rows < 4 || tile_rows > 1 << 20) return fail(POE2D_E_INVALID, "batch_set_schedule: tile rows out of range");
     b->block_w = block_w;
     b->tile_rows = tile_rows;
+    b->auto_shape = false;
     return POE2D_OK;
 }
 
@@ -1562,36 +1730,29 @@ poe2d_status poe2d_batch_autotune(poe2d_batch *b, int nsteps, int *block_w, int 
     for (poe2d_solver *s : b->members)
         if (s->step != 0) return fail(POE2D_E_STATE, "batch_autotune: needs every member at step 0");
     int kinds = 0;
-    for (poe2d_solver *s : b->members) kinds |= 1 << effective_schedule(s);
+    for (poe2d_solver *s : b->members) kinds |= 1 << s->schedule;
     const std::string key = "batch/" + tune_key(b->members, kinds);
     if (nsteps >= 0) {
         int w, h;
         if (tune_lookup(key, &w, &h)) {
             b->block_w = w;
             b->tile_rows = h;
+            b->auto_shape = false;
             if (block_w) *block_w = w;
             if (tile_rows) *tile_rows = h;
             return POE2D_OK;
         }
     }
     nsteps = nsteps == 0 ? 10 : std::abs(nsteps);
-    bool two = b->precision == POE2D_F32;
-    for (poe2d_solver *s : b->members) two = two && two_step_kernel(s);
-    const std::vector<int> widths = two ? std::vector<int>{64, 128, 256} : std::vector<int>{128, 256, 512};
-    const std::vector<int> heights = two ? std::vector<int>{6, 12, 18, 24, 30, 42, 60}
-                                         : std::vector<int>{8, 14, 20, 26, 32, 44, 62, 98};
-    int nzmax = 0;
-    for (poe2d_solver *s : b->members) nzmax = std::max(nzmax, s->grid.nz);
     // as poe2d_autotune: one timed run per shape, the three fastest timed again
     std::vector<std::pair<double, std::pair<int, int>>> cand;
-    for (int w : widths)
-        for (int h : heights) {
-            if (h > nzmax + 1 && h != heights[0]) continue;
-            b->block_w = w;
-            b->tile_rows = h;
-            if ((st = poe2d_batch_run(b, 1)) || (st = poe2d_batch_run(b, nsteps))) break;
-            cand.push_back({b->last_ms, {w, h}});
-        }
+    b->auto_shape = false;
+    for (const auto &shape : tune_shapes(b->members)) {
+        b->block_w = shape.first;
+        b->tile_rows = shape.second;
+        if ((st = poe2d_batch_run(b, 1)) || (st = poe2d_batch_run(b, nsteps))) break;
+        cand.push_back({b->last_ms, shape});
+    }
     int best_w = b->block_w, best_h = b->tile_rows;
     if (!st && !cand.empty()) {
         std::sort(cand.begin(), cand.end());

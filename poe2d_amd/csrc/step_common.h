@@ -122,6 +122,7 @@ struct StepArgs {
     // n / rec_dec of traces ([slot][comp][receiver], components of rec_mask).
     const int *rec_tile_ptr;
     const int2 *rec_entries;
+    const int4 *rec_points;  // the tile kernel's: (x, z, receiver index, -), the tiles' runs one after the other
     T *traces;
     int rec_n, rec_ncomp, rec_dec, rec_nsamp;
     unsigned rec_mask;
@@ -189,6 +190,15 @@ __device__ __forceinline__ T cpml_from(T d, T psi_old, PN psi_n, bool store, T a
 {
     const T s = b * psi_old + a * d;
     if (store) *psi_n = s;
+    return d * rk + s;
+}
+
+// The same on a memory variable held in a register.
+template <class T>
+__device__ __forceinline__ T cpml_held(T d, T &psi, T a, T b, T rk)
+{
+    const T s = b * psi + a * d;
+    psi = s;
     return d * rk + s;
 }
 
@@ -329,5 +339,20 @@ hipError_t launch_fused2(const StepArgs<T> *models, const WorkItem *work, int nw
 // the over-run of its row loop): a tile with a C-PML strip point, or a point of the grid's two
 // outer rows or columns on either side, in this range is an edge tile.
 constexpr int kFused2RowsBefore = 10, kFused2RowsAfter = 12, kFused2ColsBefore = 6;
+
+// The tile kernel (kernels_tile.hip): one or two steps of a region of 64 columns held on chip.  A
+// work item owns columns [x0, x0 + kTileCols) and rows [z0, z1), at most kTileShort rows (TILE_EDGE,
+// TILE_SHORT) or kTileTall (TILE_TALL).  TILE_EDGE items are those whose region (the owned points and
+// kTileHalo on every side) reaches a C-PML strip or the grid's two outer rows or columns; the others
+// run without that code.  Receivers rec_points[rec_lo .. rec_hi) are the item's.
+enum { TILE_EDGE = 0, TILE_SHORT = 1, TILE_TALL = 2 };
+constexpr int kTileHalo = 6, kTileCols = 64 - 2 * kTileHalo, kTileShort = 24 - 2 * kTileHalo, kTileTall = 48 - 2 * kTileHalo;
+struct TileItem {
+    int model, x0, z0, z1, kind, rec_lo, rec_hi, unused;
+};
+// nst (1 or 2) steps from step n = *base + k; buffers as the two-step kernel's launches use them.
+template <class T>
+hipError_t launch_tiles(const StepArgs<T> *models, const TileItem *work, int nwork, int per_xcd, bool palette, bool avg,
+                        const long long *base, int k, int nst, hipStream_t stream);
 
 }  // namespace poe2d

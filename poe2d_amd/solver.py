@@ -216,7 +216,8 @@ class Solver(HandleSolver):
         """0: single fused launch per step (tiles of block_w-8 columns x tile_rows rows), reading
         the coefficients through the material palette when the grid has one;
         1: separate stress and velocity launches;
-        2: as 0, always reading the per-point coefficient arrays."""
+        2: as 0, always reading the per-point coefficient arrays;
+        3: two steps per launch (block_w 64: the tile kernel, what a handle runs until this call)."""
         self._check(self._lib.poe2d_set_schedule(self._h, schedule, block_w, tile_rows), "set_schedule")
 
     def set_graphs(self, on=True):

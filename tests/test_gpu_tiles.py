@@ -1,0 +1,85 @@
+"""The tile kernel (schedule 3, block width 64, and what a handle runs until a shape is chosen)
+against the single-step kernel it must reproduce bit for bit: from a random state, on grids at the
+remainders of its 52-column tiles and 12- and 36-row tiles, with a material palette, one beyond the
+marching kernel's limit and none, in both precisions, over odd and even step counts."""
+import numpy as np
+import pytest
+
+from poe2d_amd import _abi
+from poe2d_amd.configs import BRINE, biot_fields
+from poe2d_amd.material import material_biot
+from poe2d_amd.solver import Batch, Problem, ReceiverSpec, Solver, SourceSpec
+
+pytestmark = pytest.mark.gpu
+
+STATE = ("vx", "vy", "wx", "wy", "exx", "eyy", "zeta", "sxy")
+
+
+def _problem(nx, nz, npml, entries, seed=3, **opts):
+    rng = np.random.default_rng(seed)
+    p = biot_fields(nx, nz)
+    if entries:  # `entries` materials in random places; 0: every point its own
+        p["phi"] = 0.2 + 0.1 * rng.integers(0, entries, p["phi"].shape) / entries
+    else:
+        p["phi"] = rng.uniform(0.2, 0.3, p["phi"].shape)
+        p["mu_fr"] = BRINE["mu_fr"] * rng.uniform(0.9, 1.1, p["phi"].shape)
+    ix = np.unique(np.clip([0, 5, 51, 52, 53, nx // 2, nx - 1, nx], 0, nx)).astype(np.int32)
+    iz = np.unique(np.clip([0, 11, 12, 35, 36, nz // 2, nz], 0, nz)).astype(np.int32)
+    gx, gz = (a.ravel() for a in np.meshgrid(ix, iz))
+    return Problem(nx=nx, nz=nz, dx=0.5, dz=0.5, dt=5e-5, nt=9, coeffs=material_biot(**p),
+                   source=SourceSpec(kind=_abi.SRC_PRESSURE_DGAUSS, ix=nx // 2, iz=nz // 2, amp=1e6),
+                   receivers=ReceiverSpec(ix=gx, iz=gz, decimate=2), npml=npml, f0=80.0, **opts)
+
+
+def _run(prob, precision, shape, steps):
+    with Solver(prob, precision=precision) as s:
+        rng = np.random.default_rng(11)
+        if shape:
+            s.set_schedule(*shape)
+        for f in STATE:
+            s.set_field(f, rng.standard_normal((prob.nz + 1, prob.nx + 1)) * (1e-9 if f[0] in "ez" else 1e-6))
+        for n in steps:
+            s.run(n)
+        return s.seismograms(), {f: s.snapshot(f) for f in STATE + ("p",)}, s.checkpoint()
+
+
+def _same(a, b, label):
+    assert np.isfinite(a[0]).all() and np.abs(a[0]).max() > 0
+    assert np.array_equal(a[0], b[0]), f"{label}: traces differ"
+    for f in a[1]:
+        assert np.array_equal(a[1][f], b[1][f]), f"{label}: field {f} differs"
+    assert np.array_equal(a[2], b[2]), f"{label}: checkpoint differs"
+
+
+@pytest.mark.parametrize("nx,nz,npml", [(10, 10, 1), (51, 47, 4), (103, 107, 20), (104, 131, 10), (230, 171, 20)])
+@pytest.mark.parametrize("entries", [2, 40, 0])
+@pytest.mark.parametrize("precision", [32, 64])
+def test_tiles_equal_the_single_step_kernel(nx, nz, npml, entries, precision):
+    prob = _problem(nx, nz, npml, entries)
+    ref = _run(prob, precision, (0, 256, 14), [9])
+    for shape, steps in (((3, 64, 12), [4, 5]), ((3, 64, 36), [9]), (None, [1, 2, 6])):
+        _same(_run(prob, precision, shape, steps), ref, f"{nx}x{nz} npml {npml} {entries} entries shape {shape}")
+
+
+@pytest.mark.parametrize("opts", [dict(stress_law=1), dict(staggered_material=1)])
+@pytest.mark.parametrize("entries", [2, 0])
+@pytest.mark.parametrize("precision", [32, 64])
+def test_tiles_physics_variants(opts, entries, precision):
+    prob = _problem(230, 171, 20, entries, **opts)
+    _same(_run(prob, precision, (3, 64, 36), [9]), _run(prob, precision, (0, 256, 14), [9]), f"{opts} {entries}")
+
+
+def test_ragged_fp64_batch_on_tiles():
+    probs = [_problem(130, 90, 10, 2, seed=1), _problem(61, 200, 10, 2, seed=2)]
+    alone = [_run(p, 64, (0, 256, 14), [9])[0] for p in probs]
+    solvers = [Solver(p, precision=64) for p in probs]
+    rng = [np.random.default_rng(11) for _ in probs]
+    for s, g in zip(solvers, rng):
+        for f in STATE:
+            s.set_field(f, g.standard_normal((s.problem.nz + 1, s.problem.nx + 1)) * (1e-9 if f[0] in "ez" else 1e-6))
+    with Batch(solvers) as b:
+        b.run(9)
+        for s, ref in zip(solvers, alone):
+            assert np.array_equal(s.seismograms(), ref)
+    for s in solvers:
+        s.close()
