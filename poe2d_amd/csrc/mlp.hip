@@ -74,6 +74,24 @@ poe2d_status dmalloc(P **p, size_t count)
     return POE2D_OK;
 }
 
+// *p with room for at least `count` elements (contents lost when it grows).
+template <class P>
+poe2d_status grow(P **p, size_t *cap, size_t count)
+{
+    if (count <= *cap) return POE2D_OK;
+    if (*p) (void)hipFree((void *)*p);
+    *p = nullptr;
+    *cap = 0;
+    void *q = nullptr;
+    const hipError_t e = hipMalloc(&q, count * sizeof(P));
+    if (e != hipSuccess)
+        return fail(e == hipErrorOutOfMemory ? POE2D_E_NOMEM : POE2D_E_HIP,
+                    std::string("hipMalloc: ") + hipGetErrorString(e));
+    *p = (P *)q;
+    *cap = count;
+    return POE2D_OK;
+}
+
 template <class P>
 void dfree(P *&p)
 {
@@ -104,8 +122,17 @@ struct poe2d_mlp {
     size_t work_floats = 0;
     float *partial = nullptr;      // loss partial sums
     int nred = 512;
-    // prediction accumulators
-    float *acc_mean = nullptr, *acc_m2 = nullptr;
+    // prediction: hidden activations of every member (per layer boundary l = 1..L-1, [members]
+    // [max_batch][pad(sizes[l])]), the members' weight and bias pointers (per layer, [members]), the
+    // row sums behind the spread, a batch's mean on its way to host memory, and the inputs and spreads
+    // of a whole call (grown to the largest call)
+    std::vector<uint16_t *> hens;
+    std::vector<const uint16_t **> ens_w;
+    std::vector<const float **> ens_b;
+    double *ens_part = nullptr;
+    float *acc_mean = nullptr;
+    float *x_all = nullptr, *spread_all = nullptr;
+    size_t x_all_cap = 0, spread_all_cap = 0;
     float *oscale = nullptr;  // per-output factor of the predicted mean (null: none)
     // resident dataset
     float *data_x = nullptr, *data_t = nullptr;
@@ -150,7 +177,11 @@ void free_mlp(poe2d_mlp *m)
     for (auto &p : m->g16) dfree(p);
     for (auto &p : m->g16t) dfree(p);
     dfree(m->dh); dfree(m->y); dfree(m->tgt); dfree(m->xin); dfree(m->work); dfree(m->partial);
-    dfree(m->acc_mean); dfree(m->acc_m2); dfree(m->oscale); dfree(m->data_x); dfree(m->data_t); dfree(m->idx); dfree(m->dloss);
+    for (auto &p : m->hens) dfree(p);
+    for (auto &p : m->ens_w) dfree(p);
+    for (auto &p : m->ens_b) dfree(p);
+    dfree(m->ens_part); dfree(m->x_all); dfree(m->spread_all);
+    dfree(m->acc_mean); dfree(m->oscale); dfree(m->data_x); dfree(m->data_t); dfree(m->idx); dfree(m->dloss);
     dfree(m->idx_all); dfree(m->loss_all);
     for (hipEvent_t ev : m->step_done) (void)hipEventDestroy(ev);
     m->step_done.clear();
@@ -186,59 +217,6 @@ __global__ void gather_rows(const float *__restrict__ src, int ld_src, const int
     if (i >= (size_t)n * cols) return;
     const int r = (int)(i / cols), c = (int)(i % cols);
     dst[(size_t)r * ld_dst + c] = src[(size_t)idx[r] * ld_src + c];
-}
-
-// Running mean / sum of squared deviations over members (Welford), k = member index.
-__global__ void welford(const float *__restrict__ y, int ldy, int n, int cols, int k, float *__restrict__ mean,
-                        float *__restrict__ m2)
-{
-    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (i >= (size_t)n * cols) return;
-    const int r = (int)(i / cols), c = (int)(i % cols);
-    const float v = y[(size_t)r * ldy + c];
-    const size_t j = (size_t)r * cols + c;
-    if (k == 0) {
-        mean[j] = v;
-        m2[j] = 0.f;
-        return;
-    }
-    const float d = v - mean[j];
-    const float mu = mean[j] + d / (float)(k + 1);
-    m2[j] += d * (v - mu);
-    mean[j] = mu;
-}
-
-// spread[r] = ||std over members|| / ||mean|| over the outputs of row r (one block per row).
-__global__ void row_spread(const float *__restrict__ mean, const float *__restrict__ m2, int cols, int members,
-                           float *__restrict__ spread)
-{
-    __shared__ double sv[256], sn[256];
-    const int r = blockIdx.x;
-    double var = 0, nrm = 0;
-    for (int c = threadIdx.x; c < cols; c += blockDim.x) {
-        const float mu = mean[(size_t)r * cols + c];
-        var += m2[(size_t)r * cols + c];
-        nrm += (double)mu * mu;
-    }
-    sv[threadIdx.x] = var;
-    sn[threadIdx.x] = nrm;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            sv[threadIdx.x] += sv[threadIdx.x + s];
-            sn[threadIdx.x] += sn[threadIdx.x + s];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) spread[r] = (float)(sqrt(sv[0] / (members > 1 ? members - 1 : 1)) / fmax(sqrt(sn[0]), 1e-30));
-}
-
-// mean[r][c] *= scale[c] for n rows of `cols` values.
-__global__ void scale_cols(float *__restrict__ mean, int n, int cols, const float *__restrict__ scale)
-{
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < (size_t)n * cols;
-         i += (size_t)gridDim.x * blockDim.x)
-        mean[i] *= scale[i % cols];
 }
 
 int blocks(size_t n) { return (int)std::min<size_t>((n + 255) / 256, 1u << 20); }
@@ -335,6 +313,46 @@ poe2d_status forward(poe2d_mlp *m, Member &e, int n)
     return POE2D_OK;
 }
 
+
+// The ensemble on the nb rows in h16[0]: the hidden layers of every member, layer by layer (as many
+// members to a launch as the partials buffer holds), then their output layers and statistics in one
+// pass.  mean [nb][outputs] (scaled) and spread [nb] are device memory; either may be null.
+poe2d_status ensemble_batch(poe2d_mlp *m, int nb, float *mean, float *spread)
+{
+    const int E = (int)m->members.size(), B = m->max_batch;
+    const uint16_t *h = m->h16[0];
+    size_t stride = 0;  // (the first layer's input is every member's)
+    for (int li = 0; li < m->L; ++li) {
+        const Layer &l = m->members[0].layers[li];
+        if (li == m->L - 1) {
+            HIP_TRY(ensemble_output(h, l.inp, stride, m->ens_w[li], l.inp, m->ens_b[li], E, nb, l.out, l.inp, mean, l.out,
+                                    m->oscale, m->ens_part, spread, m->stream));
+            break;
+        }
+        uint16_t *const next = m->hens[li + 1];
+        const size_t next_stride = (size_t)B * l.outp;
+        const int ksplit = product_splits(m, nb, l.out, l.inp);
+        const int group = std::max<int>(1, (int)std::min<size_t>(E, m->work_floats / ((size_t)ksplit * nb * l.out)));
+        for (int k = 0; k < E; k += group)
+            HIP_TRY(gemm_bf16_members(h + k * stride, l.inp, stride, m->ens_w[li] + k, l.inp, m->ens_b[li] + k,
+                                      std::min(group, E - k), nb, l.out, l.inp, next + k * next_stride, l.outp, next_stride,
+                                      m->work, m->work_floats, ksplit, m->stream));
+        h = next;
+        stride = next_stride;
+    }
+    return POE2D_OK;
+}
+
+// Whether p is memory of the network's device (results then go there directly).
+bool on_this_device(const poe2d_mlp *m, const void *p)
+{
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();  // (ordinary host memory)
+        return false;
+    }
+    return at.type == hipMemoryTypeDevice && at.device == m->device;
+}
 
 // Gradients of the mean squared error for member e on the batch in h16[0] / tgt (n rows, n a
 // multiple of 32); loss (mean) to *loss when non-null.
@@ -543,8 +561,24 @@ static poe2d_status alloc_scratch(poe2d_mlp *m, bool predict)
         return st;
     if (predict &&
         ((st = dmalloc(&m->y, (size_t)B * outp)) || (st = dmalloc(&m->tgt, (size_t)B * outp)) ||
-         (st = dmalloc(&m->acc_mean, (size_t)B * sizes[nlayers])) || (st = dmalloc(&m->acc_m2, (size_t)B * sizes[nlayers]))))
+         (st = dmalloc(&m->acc_mean, (size_t)B * sizes[nlayers])) ||
+         (st = dmalloc(&m->ens_part, ensemble_part_doubles(B, sizes[nlayers])))))
         return st;
+    if (predict) {
+        const size_t E = m->members.size();
+        m->hens.assign(nlayers + 1, nullptr);
+        m->ens_w.assign(nlayers, nullptr);
+        m->ens_b.assign(nlayers, nullptr);
+        for (int li = 0; li < nlayers; ++li) {
+            if (li > 0 && (st = dmalloc(&m->hens[li], E * B * pad128(sizes[li])))) return st;
+            if ((st = dmalloc(&m->ens_w[li], E)) || (st = dmalloc(&m->ens_b[li], E))) return st;
+            std::vector<const uint16_t *> w(E);
+            std::vector<const float *> b(E);
+            for (size_t k = 0; k < E; ++k) w[k] = m->members[k].layers[li].w16, b[k] = m->members[k].layers[li].b;
+            HIP_TRY(hipMemcpy(m->ens_w[li], w.data(), E * sizeof(w[0]), hipMemcpyHostToDevice));
+            HIP_TRY(hipMemcpy(m->ens_b[li], b.data(), E * sizeof(b[0]), hipMemcpyHostToDevice));
+        }
+    }
     return POE2D_OK;
 }
 
@@ -811,33 +845,25 @@ poe2d_status poe2d_mlp_predict(poe2d_mlp *m, int n, const float *x, float *mean,
     poe2d_status st = check_mlp(m);
     if (st) return st;
     if (n < 1 || !x) return fail(POE2D_E_INVALID, "mlp_predict: bad input");
-    const int in = m->sizes[0], out = m->sizes[m->L], outp = pad128(out);
-    const int E = (int)m->members.size();
+    const int in = m->sizes[0], out = m->sizes[m->L];
+    // every input in one copy: a copy per batch from pageable memory would hold the host until the
+    // batch before it is done
+    if ((st = grow(&m->x_all, &m->x_all_cap, (size_t)n * in))) return st;
+    if (spread && (st = grow(&m->spread_all, &m->spread_all_cap, (size_t)n))) return st;
+    HIP_TRY(hipMemcpyAsync(m->x_all, x, (size_t)n * in * sizeof(float), hipMemcpyHostToDevice, m->stream));
+    const bool in_place = mean && on_this_device(m, mean);
     for (int r0 = 0; r0 < n; r0 += m->max_batch) {
         const int nb = std::min(m->max_batch, n - r0);
-        if ((st = load_input(m, x + (size_t)r0 * in, nb))) return st;
-        for (int k = 0; k < E; ++k) {
-            if ((st = forward(m, m->members[k], nb))) return st;
-            welford<<<blocks((size_t)nb * out), 256, 0, m->stream>>>(m->y, outp, nb, out, k, m->acc_mean, m->acc_m2);
-            HIP_TRY(hipGetLastError());
-        }
-        if (spread) {
-            row_spread<<<nb, 256, 0, m->stream>>>(m->acc_mean, m->acc_m2, out, E, m->partial);
-            HIP_TRY(hipGetLastError());
-            HIP_TRY(hipMemcpyAsync(spread + r0, m->partial, nb * sizeof(float), hipMemcpyDefault, m->stream));
-        }
-        if (mean) {
-            // (the spread above is of the unscaled outputs)
-            if (m->oscale) {
-                scale_cols<<<blocks((size_t)nb * out), 256, 0, m->stream>>>(m->acc_mean, nb, out, m->oscale);
-                HIP_TRY(hipGetLastError());
-            }
-            // (host or device memory: the direction comes from the pointers)
-            HIP_TRY(hipMemcpyAsync(mean + (size_t)r0 * out, m->acc_mean, (size_t)nb * out * sizeof(float),
-                                   hipMemcpyDefault, m->stream));
-        }
-        HIP_TRY(hipStreamSynchronize(m->stream));
+        pack_input<<<blocks((size_t)nb * in), 256, 0, m->stream>>>(m->x_all + (size_t)r0 * in, nb, in, m->h16[0], pad128(in));
+        HIP_TRY(hipGetLastError());
+        float *const dst = !mean ? nullptr : in_place ? mean + (size_t)r0 * out : m->acc_mean;
+        if ((st = ensemble_batch(m, nb, dst, spread ? m->spread_all + r0 : nullptr))) return st;
+        if (dst && !in_place)
+            HIP_TRY(hipMemcpyAsync(mean + (size_t)r0 * out, dst, (size_t)nb * out * sizeof(float), hipMemcpyDefault,
+                                   m->stream));
     }
+    if (spread) HIP_TRY(hipMemcpyAsync(spread, m->spread_all, (size_t)n * sizeof(float), hipMemcpyDefault, m->stream));
+    HIP_TRY(hipStreamSynchronize(m->stream));
     return POE2D_OK;
 }
 

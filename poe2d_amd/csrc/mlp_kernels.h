@@ -74,6 +74,21 @@ struct GemmOut {
 hipError_t gemm_bf16(const uint16_t *A, int lda, const uint16_t *B, int ldb, int M, int N, int K, int epi,
                      const GemmOut &out, float *work, size_t work_floats, int ksplit, hipStream_t stream);
 
+// The same hidden-layer product of several members at once: member z's A + z stride_a (0: shared),
+// weights bs[z] and bias biases[z] into b16 + z stride_b16 with GELU; work holds members * ksplit * M * N
+// floats.  Values equal gemm_bf16's with EPI_GELU and the same ksplit > 1.
+hipError_t gemm_bf16_members(const uint16_t *A, int lda, size_t stride_a, const uint16_t *const *bs, int ldb,
+                             const float *const *biases, int members, int M, int N, int K, uint16_t *b16, int ldb16,
+                             size_t stride_b16, float *work, size_t work_floats, int ksplit, hipStream_t stream);
+
+// The members' output layer (A + z stride_a times bs[z]^T + biases[z]) and its statistics: mean over
+// members times scale (either may be null) into mean [M][ldm], and spread[m] = ||standard deviation over
+// members|| / ||unscaled mean|| over the row (null: not formed; part holds ensemble_part_doubles).
+size_t ensemble_part_doubles(int M, int N);
+hipError_t ensemble_output(const uint16_t *A, int lda, size_t stride_a, const uint16_t *const *bs, int ldb,
+                           const float *const *biases, int members, int M, int N, int K, float *mean, size_t ldm,
+                           const float *scale, double *part, float *spread, hipStream_t stream);
+
 // out[c][r] = in[r][c], R x C.
 hipError_t transpose_bf16(const uint16_t *in, int ldi, uint16_t *out, int ldo, int R, int C, hipStream_t stream);
 

@@ -28,6 +28,8 @@ typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int BM = 128, BN = 128, BK = 32;
 constexpr int LDS_ROW = BK + 8;  // bf16 per LDS row (16-byte pad against bank conflicts)
+// products of at least this many 128 x 128 tiles run ensemble_nt on them (two per CU), others on 64 x 64
+constexpr int kEnsembleBigTiles = 512;
 
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
 
@@ -58,11 +60,21 @@ __device__ __forceinline__ float adam_update(float *w, float *mom, float *vel, f
     return x;
 }
 
-// C (+)= A B^T over k in [k0, k1) for the 128 x 128 tile (tm, tn); k0, k1 multiples of BK.
+// C (+)= A B^T over k in [k0, k1) for the 128 x 128 tile (tm, tn); k0, k1 multiples of BK.  Split-K
+// launches may hold several products (blockIdx.z): product z reads A + z stride_a and bs[z], and its
+// partials follow those of product z - 1.
 template <int EPI>
 __global__ void __launch_bounds__(256, 3) gemm_nt(const uint16_t *__restrict__ A, int lda, const uint16_t *__restrict__ B,
-                                               int ldb, int M, int N, int K, int ksplit, GemmOut out)
+                                               int ldb, int M, int N, int K, int ksplit, GemmOut out,
+                                               const uint16_t *const *__restrict__ bs = nullptr, size_t stride_a = 0)
 {
+    if constexpr (EPI == EPI_PARTIAL) {
+        if (bs) {
+            A += blockIdx.z * stride_a;
+            B = bs[blockIdx.z];
+            out.f32 += (size_t)blockIdx.z * ksplit * M * out.ldf;
+        }
+    }
     // operand tiles (la, lb: two k tiles each), reused by the EPI_MSE / EPI_ADAM epilogues for the
     // transposed bf16 tile and the EPI_MSE sums (40 KiB)
     __shared__ uint16_t lds[2 * BM * LDS_ROW + 2 * BN * LDS_ROW];
@@ -354,6 +366,204 @@ __global__ void __launch_bounds__(256, 3) gemm_nt(const uint16_t *__restrict__ A
     }
 }
 
+// The output layer of every ensemble member and their statistics in one pass: tile by tile, member
+// e's product H_e W_e^T + b_e is formed in the accumulators and folded into the running mean and sum
+// of squared deviations (Welford), both in registers.  Stores the mean (times scale[n] when given)
+// and, per row and tile of BN columns, the sums over the tile's columns of the squared deviations and
+// of the squared (unscaled) mean: part[(tn * 2 + 0 / 1) * M + m].
+//
+// What bounds it.  Members one at a time wrote each output array (620 MB of 1024 x 151 500) and read
+// it back with mean and deviations: 0.33 ms of product and 0.51 ms of Welford per member, 0.8 ms of
+// scaling and row sums, 5.3 ms for five members.  Here the mean is the only array that reaches HBM.
+// Waves are 2 x 2 of 32 MI x 32 NJ: MI = NJ = 2 (192 registers of results, two blocks per CU), or 1
+// where that leaves too few blocks.  Tile order as EPI_MSE's: m fastest within an XCD's run, so the
+// m tiles of one n tile share its weights in that L2.
+template <int MI, int NJ>
+__global__ void __launch_bounds__(256, 2)
+    ensemble_nt(const uint16_t *__restrict__ A, int lda, size_t stride_a, const uint16_t *const *__restrict__ bs, int ldb,
+                const float *const *__restrict__ biases, int M, int N, int K, int members, float *__restrict__ mean,
+                size_t ldm, const float *__restrict__ scale, double *__restrict__ part)
+{
+    constexpr int TM = 64 * MI, TN = 64 * NJ;
+    __shared__ uint16_t la[2][TM * LDS_ROW], lb[2][TN * LDS_ROW];
+    __shared__ double red[2][TM][2];
+    const int tiles_m = (M + TM - 1) / TM;
+    const int nb = (int)gridDim.x, q8 = nb >> 3, r8 = nb & 7;
+    const int xcd = (int)blockIdx.x & 7, slot = (int)blockIdx.x >> 3;
+    const int tile = xcd < r8 ? xcd * (q8 + 1) + slot : r8 * (q8 + 1) + (xcd - r8) * q8 + slot;
+    const int tm = tile % tiles_m, tn = tile / tiles_m;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int wm = wave >> 1, wn = wave & 1;
+    const int r0 = t >> 2, kc = t & 3;
+    const int nk = K / BK, steps = nk * members;
+
+    // operand tiles of step g (member g / nk, k tile g % nk), two register sets ahead of the MFMAs
+    u16x8 ra[2][MI], rb[2][NJ];
+    int ge = 0, gk = 0;  // member and k tile of the next load
+    auto load = [&](u16x8 *a, u16x8 *b) {
+        const uint16_t *const pa = A + ge * stride_a + gk * BK + kc * 8;
+        const uint16_t *const pb = bs[ge] + gk * BK + kc * 8;
+#pragma unroll
+        for (int h = 0; h < MI; ++h) a[h] = *(const u16x8 *)(pa + (size_t)min(tm * TM + r0 + h * 64, M - 1) * lda);
+#pragma unroll
+        for (int h = 0; h < NJ; ++h) b[h] = *(const u16x8 *)(pb + (size_t)min(tn * TN + r0 + h * 64, N - 1) * ldb);
+        if (++gk == nk) {
+            gk = 0;
+            if (ge + 1 < members) ++ge;  // (past the last step: re-reads, never used)
+        }
+    };
+    auto store = [&](int buf, const u16x8 *a, const u16x8 *b) {
+#pragma unroll
+        for (int h = 0; h < MI; ++h) *(u16x8 *)(la[buf] + (r0 + h * 64) * LDS_ROW + kc * 8) = a[h];
+#pragma unroll
+        for (int h = 0; h < NJ; ++h) *(u16x8 *)(lb[buf] + (r0 + h * 64) * LDS_ROW + kc * 8) = b[h];
+    };
+    f32x16 acc[MI][NJ], mu[MI][NJ], m2[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = mu[i][j][e] = m2[i][j][e] = 0.f;
+    load(ra[0], rb[0]);
+    load(ra[1], rb[1]);
+    store(0, ra[0], rb[0]);
+    __syncthreads();
+    int kt = 0, e = 0;
+    auto step = [&](int g, int u) {
+        load(ra[u], rb[u]);
+#pragma unroll
+        for (int kk = 0; kk < BK; kk += 16) {
+            bf16x8 fa[MI], fb[NJ];
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+                fa[i] = *(const bf16x8 *)(la[u] + (wm * 32 * MI + i * 32 + (lane & 31)) * LDS_ROW + kk + (lane >> 5) * 8);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+                fb[j] = *(const bf16x8 *)(lb[u] + (wn * 32 * NJ + j * 32 + (lane & 31)) * LDS_ROW + kk + (lane >> 5) * 8);
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+        }
+        if (g + 1 < steps) store(u ^ 1, ra[u ^ 1], rb[u ^ 1]);
+        if (++kt == nk) {
+            // member e's outputs are complete: Welford's update, and the accumulators start over
+            const float count = (float)(e + 1), rcount = 1.0f / count;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int n = tn * TN + wn * 32 * NJ + j * 32 + (lane & 31);
+                const float b = n < N ? biases[e][n] : 0.f;
+#pragma unroll
+                for (int i = 0; i < MI; ++i)
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) {
+                        const float v = acc[i][j][q] + b;
+                        const float d = v - mu[i][j][q];
+                        // d / count, correctly rounded: the quotient by the reciprocal, one step of
+                        // its remainder, and the infinities and NaN
+                        const float q0 = d * rcount;
+                        const float dq = __builtin_amdgcn_div_fixupf(
+                            __builtin_fmaf(__builtin_fmaf(-q0, count, d), rcount, q0), count, d);
+                        const float nm = mu[i][j][q] + dq;
+                        m2[i][j][q] += d * (v - nm);
+                        mu[i][j][q] = nm;
+                        acc[i][j][q] = 0.f;
+                    }
+            }
+            kt = 0;
+            ++e;
+        }
+        __syncthreads();
+    };
+    for (int g = 0; g < steps; g += 2) {
+        step(g, 0);
+        if (g + 1 < steps) step(g + 1, 1);
+    }
+
+    // the mean, and the row sums: lane l's 16 results of a 32 x 32 tile are rows (q / 4) * 8 + (l / 32)
+    // * 4 + q % 4 of column l % 32
+    const bool ok_n[2] = {tn * TN + wn * 32 * NJ + (lane & 31) < N, tn * TN + wn * 32 * NJ + 32 + (lane & 31) < N};
+    float sc[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int n = tn * TN + wn * 32 * NJ + j * 32 + (lane & 31);
+        sc[j] = scale && ok_n[j] ? scale[n] : 1.f;
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        double sv[16], sn[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int m = tm * TM + wm * 32 * MI + i * 32 + (q >> 2) * 8 + (lane >> 5) * 4 + (q & 3);
+            sv[q] = sn[q] = 0.0;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int n = tn * TN + wn * 32 * NJ + j * 32 + (lane & 31);
+                if (ok_n[j]) {
+                    const float v = mu[i][j][q];
+                    sv[q] += m2[i][j][q];
+                    sn[q] += (double)v * v;
+                    if (mean && m < M) mean[(size_t)m * ldm + n] = v * sc[j];
+                }
+            }
+        }
+        if (!part) continue;
+        // sum over the 32 lanes of a half wave: at every step a lane keeps half of its rows, adding
+        // its partner's sums of them; lane l ends with row q = (l % 32) / 2
+        int q0 = 0;
+#pragma unroll
+        for (int h = 16, cnt = 8; cnt >= 1; h >>= 1, cnt >>= 1) {
+            const bool up = lane & h;
+#pragma unroll
+            for (int q = 0; q < cnt; ++q) {
+                const double av = up ? sv[q] : sv[q + cnt], an = up ? sn[q] : sn[q + cnt];
+                sv[q] = (up ? sv[q + cnt] : sv[q]) + __shfl_xor(av, h);
+                sn[q] = (up ? sn[q + cnt] : sn[q]) + __shfl_xor(an, h);
+            }
+            if (up) q0 += cnt;
+        }
+        sv[0] += __shfl_xor(sv[0], 1);
+        sn[0] += __shfl_xor(sn[0], 1);
+        if (!(lane & 1)) {
+            const int row = wm * 32 * MI + i * 32 + (q0 >> 2) * 8 + (lane >> 5) * 4 + (q0 & 3);
+            red[wn][row][0] = sv[0];
+            red[wn][row][1] = sn[0];
+        }
+    }
+    if (!part) return;
+    __syncthreads();
+    for (int r = t; r < 2 * TM; r += 256) {
+        const int row = r % TM, w = r / TM, m = tm * TM + row;
+        if (m < M) part[((size_t)tn * 2 + w) * M + m] = red[0][row][w] + red[1][row][w];
+    }
+}
+
+// spread[m] = ||standard deviation over members|| / ||mean|| from ensemble_nt's sums of `tiles` tiles
+// per row: 64 rows per block, 16 threads a row over the tiles, then over the threads in order.
+__global__ void __launch_bounds__(1024) ensemble_spread(const double *__restrict__ part, int tiles, int M, int members,
+                                                        float *__restrict__ spread)
+{
+    __shared__ double red[2][16][64];
+    const int lane = threadIdx.x & 63, g = threadIdx.x >> 6, m = blockIdx.x * 64 + lane;
+    double var = 0, nrm = 0;
+    if (m < M)
+        for (int t = g; t < tiles; t += 16) {
+            var += part[((size_t)t * 2 + 0) * M + m];
+            nrm += part[((size_t)t * 2 + 1) * M + m];
+        }
+    red[0][g][lane] = var;
+    red[1][g][lane] = nrm;
+    __syncthreads();
+    if (g || m >= M) return;
+    for (int k = 1; k < 16; ++k) {
+        var += red[0][k][lane];
+        nrm += red[1][k][lane];
+    }
+    spread[m] = (float)(sqrt(var / (members > 1 ? members - 1 : 1)) / fmax(sqrt(nrm), 1e-30));
+}
+
 // db[n] = sum over r < rows of part[r][n] (n < N), in order.
 __global__ void column_sums(const float *__restrict__ part, int rows, int ld, int N, float *__restrict__ db)
 {
@@ -364,9 +574,16 @@ __global__ void column_sums(const float *__restrict__ part, int rows, int ld, in
     db[n] = v;
 }
 
-// out[m][n] = sum over splits of part[s][m][n] (+ bias), then as the GEMM epilogue.
-__global__ void reduce_splits(const float *__restrict__ part, int nsplit, int M, int N, int ldf, GemmOut out, int gelu_on)
+// out[m][n] = sum over splits of part[s][m][n] (+ bias), then as the GEMM epilogue; of several
+// products, product blockIdx.y with bias biases[blockIdx.y] into b16 + blockIdx.y stride_b16.
+__global__ void reduce_splits(const float *__restrict__ part, int nsplit, int M, int N, int ldf, GemmOut out, int gelu_on,
+                              const float *const *__restrict__ biases = nullptr, size_t stride_b16 = 0)
 {
+    if (biases) {
+        part += (size_t)blockIdx.y * nsplit * M * ldf;
+        out.bias = biases[blockIdx.y];
+        out.b16 += blockIdx.y * stride_b16;
+    }
     const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
     if (i >= (size_t)M * N) return;
     const int m = (int)(i / N), n = (int)(i % N);
@@ -563,6 +780,52 @@ hipError_t gemm_bf16(const uint16_t *A, int lda, const uint16_t *B, int ldb, int
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     reduce_splits<<<grid_for((size_t)M * N), 256, 0, stream>>>(work, ksplit, M, N, N, out, epi == EPI_GELU);
+    return hipGetLastError();
+}
+
+hipError_t gemm_bf16_members(const uint16_t *A, int lda, size_t stride_a, const uint16_t *const *bs, int ldb,
+                             const float *const *biases, int members, int M, int N, int K, uint16_t *b16, int ldb16,
+                             size_t stride_b16, float *work, size_t work_floats, int ksplit, hipStream_t stream)
+{
+    if (M < 1 || N < 1 || K < BK || K % BK || lda % 8 || ldb % 8 || lda < K || ldb < K || members < 1 || members > 65535 ||
+        ksplit < 1 || ksplit > K / BK || work_floats < (size_t)members * ksplit * M * N)
+        return hipErrorInvalidValue;
+    GemmOut part{}, out{};
+    part.f32 = work;
+    part.ldf = N;
+    out.b16 = b16;
+    out.ldb = ldb16;
+    const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+    gemm_nt<EPI_PARTIAL><<<dim3(tiles, ksplit, members), 256, 0, stream>>>(A, lda, nullptr, ldb, M, N, K, ksplit, part, bs,
+                                                                           stride_a);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    reduce_splits<<<dim3((unsigned)(((size_t)M * N + 255) / 256), members), 256, 0, stream>>>(work, ksplit, M, N, N, out, 1,
+                                                                                            biases, stride_b16);
+    return hipGetLastError();
+}
+
+size_t ensemble_part_doubles(int M, int N) { return (size_t)2 * M * ((N + 63) / 64); }
+
+hipError_t ensemble_output(const uint16_t *A, int lda, size_t stride_a, const uint16_t *const *bs, int ldb,
+                           const float *const *biases, int members, int M, int N, int K, float *mean, size_t ldm,
+                           const float *scale, double *part, float *spread, hipStream_t stream)
+{
+    if (M < 1 || N < 1 || K < BK || K % BK || lda % 8 || ldb % 8 || lda < K || ldb < K || members < 1 || (spread && !part))
+        return hipErrorInvalidValue;
+    if (!spread) part = nullptr;
+    const long long big = (long long)((M + 127) / 128) * ((N + 127) / 128);
+    const int width = big >= kEnsembleBigTiles ? 128 : 64;
+    const int tiles_m = (M + width - 1) / width, tiles_n = (N + width - 1) / width;
+    if (width == 128)
+        ensemble_nt<2, 2><<<tiles_m * tiles_n, 256, 0, stream>>>(A, lda, stride_a, bs, ldb, biases, M, N, K, members, mean,
+                                                                 ldm, scale, part);
+    else
+        ensemble_nt<1, 1><<<tiles_m * tiles_n, 256, 0, stream>>>(A, lda, stride_a, bs, ldb, biases, M, N, K, members, mean,
+                                                                 ldm, scale, part);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || !spread) return e;
+    ensemble_spread<<<(M + 63) / 64, 1024, 0, stream>>>(part, tiles_n, M, members, spread);
     return hipGetLastError();
 }
 

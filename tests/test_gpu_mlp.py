@@ -240,3 +240,22 @@ def test_train_many_equals_training_one_member_at_a_time():
         b.train_many(idx[1][None, :640], 64, 1e-3, members=[1])
         for (wa, ba), (wb, bb) in zip(a.get_params(1), b.get_params(1)):
             assert np.array_equal(wa, wb) and np.array_equal(ba, bb)
+
+
+@pytest.mark.parametrize("sizes,rows,members", [([8, 1], 1, 1), ([8, 63], 65, 2), ([8, 64, 65], 63, 3),
+                                                ([8, 96, 64, 129], 130, 5), ([4, 64, 65600], 130, 2),
+                                                ([4, 160, 70001], 97, 3)])
+def test_predict_statistics_match_the_members_outputs(sizes, rows, members):
+    """The ensemble mean and spread formed with the output layers equal those of the members' own
+    forward passes (sums of up to 512 FP32 products in another order: 1e-5 relative), at the
+    remainders of the 64- and 128-wide tiles, more rows than one batch and one layer alone."""
+    rng = np.random.default_rng(rows)
+    with Network(sizes, members=members, max_batch=96, seed=rows) as net:
+        x = rng.standard_normal((rows, sizes[0])).astype(np.float32)
+        mean, spread = net.predict(x)
+        y = np.stack([np.concatenate([net.forward(x[lo:lo + 96], k) for lo in range(0, rows, 96)])
+                      for k in range(members)]).astype(np.float64)
+    assert rel(mean, y.mean(0)) < 1e-5
+    var = y.var(0, ddof=1) if members > 1 else np.zeros_like(y[0])
+    expect = np.sqrt(var.sum(1)) / np.linalg.norm(y.mean(0), axis=1)
+    assert np.allclose(spread, expect, rtol=1e-4, atol=1e-12)
