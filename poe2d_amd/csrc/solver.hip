@@ -31,6 +31,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "aux_kernels.h"
@@ -44,6 +45,7 @@ namespace {
 const float kRefPiF = 3.1415926535897932f;  // the reference's float PI (seismic_CPML_2d_poroelastic.cpp:9)
 const double kStabilityThreshold = 1.0e25;  // STABILITY_THRESHOLD of the reference (declared, unused there)
 const int kGraphSteps = 32;                 // steps per captured graph
+const int kBandTiles = 8;                   // tile columns to a band of the tile kernel's work order
 const long long kShortTilesMax = 1280;      // launches of up to this many short tiles use them (five per CU)
 
 #define HIP_TRY(expr)                                                                              \
@@ -748,6 +750,12 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
             if (edge.size() + inter.size() > (1u << 28)) return fail(POE2D_E_INVALID, "run: too many tiles in one launch");
         }
     }
+    // Interior tiles run row by row in bands of kBandTiles tile columns, so that the tiles in flight on
+    // an XCD (about 64) make a block of neighbours sharing their halos in its L2.
+    std::stable_sort(inter.begin(), inter.end(), [](const TileItem &a, const TileItem &b) {
+        const int ba = a.x0 / (kBandTiles * kTileCols), bb = b.x0 / (kBandTiles * kTileCols);
+        return std::tie(a.model, ba, a.z0, a.x0) < std::tie(b.model, bb, b.z0, b.x0);
+    });
     // as the two-step kernel's list: every XCD gets an eighth of the edge tiles first, then a run of
     // consecutive interior tiles; shares padded to equal length with empty items
     const int ne = (int)((edge.size() + 7) / 8), ni = (int)((inter.size() + 7) / 8);
