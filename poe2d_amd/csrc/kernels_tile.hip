@@ -1,21 +1,24 @@
 // Two time steps of a tile held on chip.
 //
-// A block of 8 waves loads a region of the state once, advances it two steps in registers and LDS,
-// and stores the points whose halo was complete.  A lane is a column and a thread holds P
-// consecutive rows of it (velocities, strains, C-PML memory variables in registers), so a wave's row
-// of 64 columns needs no other wave for its x neighbours and a thread's inner rows none for their z
-// neighbours: four LDS planes, holding the velocities while stresses are formed and the stresses
-// while velocities are, carry the rest.  A step consumes three rows and columns of the region on
-// each side, so a region of 64 x 8 P points stores 52 x (8 P - 12): 52 x 36 for P = 6 (FP32 tiles
-// away from the border) and 52 x 12 for P = 3 (twice the blocks; and the tiles at C-PML strips and
-// the border, whose twelve memory variables per point stay in registers from load to store).
+// A block of 8 waves loads a region of the state once, advances it two steps, and stores the points
+// whose halo was complete.  A lane is a column and a thread holds P consecutive rows of it
+// (velocities, strains, C-PML memory variables in registers), so x neighbours are the neighbouring
+// lanes' registers (wave shifts, folded into the differences where the instruction allows) and z
+// neighbours the thread's own; only the two or three rows at a wave's ends go through LDS, its
+// velocities before the stresses and its stresses before the velocities, one barrier each.  A step
+// consumes three rows and columns of the region on each side, so a region of 64 x 8 P points stores
+// 52 x (8 P - 12): 52 x 36 for P = 6 (FP32 tiles away from the border) and 52 x 12 for P = 3 (twice
+// the blocks; and the tiles at C-PML strips and the border, whose twelve memory variables per point
+// stay in registers from load to store).
 //
 // What bounds it.  Every load of a tile is issued at the start, so a launch pays one memory latency
 // where a block marching down its rows pays one per row step (about 2 us each, 4 with C-PML records):
-// two steps of a 161^2 grid take 13 us instead of 119, 401^2 14 instead of 122, 701 x 523 FP64 36
-// instead of 127 (two single-step launches).  Large grids are bound by instruction issue: 4001^2
-// takes 274 us per launch at 52 x 36 against 298 for the marching kernel, four waves per SIMD
-// (128 VGPRs, 61 KB of LDS, two blocks per CU).
+// two steps of a 161^2 grid take 12 us instead of 119, 401^2 14 instead of 122, 701 x 523 FP64 33
+// instead of 127 (two single-step launches).  Large grids are bound by HBM: 4001^2 takes 258 us per
+// launch at 52 x 36 against 298 for the marching kernel, 1.17 GB (1.04 compulsory) at 4.5 TB/s, the
+// VALU busy 58 % of the time (128 VGPRs, four waves per SIMD, two blocks per CU).  With every row in
+// LDS planes, x neighbours read from them and four barriers per step it took 262 us, 1201^2 39 us
+// instead of 35.5.
 //
 // The arithmetic is the single-step kernel's expression by expression, so results equal it bit for
 // bit; state buffers alternate as the marching two-step kernel's.
@@ -26,27 +29,59 @@
 
 namespace poe2d {
 
-// LDS planes: the velocities of the region while stresses are formed, the stresses while velocities
-// are.
-enum { PL_VX = 0, PL_VY = 1, PL_WX = 2, PL_WY = 3, PL_SXX = 0, PL_SYY = 1, PL_SXY = 2, PL_P = 3, NPLANES = 4 };
-
 constexpr int kTileThreads = 512, kTileWaves = kTileThreads / 64;
-constexpr int kTilePad = 4;  // plane entries before and after the region, read by the outer lanes only
+
+// Rows a wave publishes to its neighbours, before the stresses (its velocities) and before the
+// velocities (its stresses): of each field the rows a z difference of the wave below or above reads.
+enum { BV_VY_L2, BV_VY_L1, BV_VY_F1, BV_WY_L2, BV_WY_L1, BV_WY_F1, BV_VX_L1, BV_VX_F1, BV_VX_F2, NBOUNDARY };
+enum { BS_SXY_L2, BS_SXY_L1, BS_SXY_F1, BS_SYY_L1, BS_SYY_F1, BS_SYY_F2, BS_P_L1, BS_P_F1, BS_P_F2 };
+
+// The value of the lane one column to the right (zero past the last lane) / to the left.
+__device__ __forceinline__ int dpp_right(int x) { return __builtin_amdgcn_update_dpp(0, x, 0x130, 0xf, 0xf, true); }
+__device__ __forceinline__ int dpp_left(int x) { return __builtin_amdgcn_update_dpp(0, x, 0x138, 0xf, 0xf, true); }
+__device__ __forceinline__ float right(float x) { return __builtin_bit_cast(float, dpp_right(__builtin_bit_cast(int, x))); }
+__device__ __forceinline__ float left(float x) { return __builtin_bit_cast(float, dpp_left(__builtin_bit_cast(int, x))); }
+__device__ __forceinline__ double right(double x)
+{
+    const int2 v = __builtin_bit_cast(int2, x);
+    return __builtin_bit_cast(double, int2{dpp_right(v.x), dpp_right(v.y)});
+}
+__device__ __forceinline__ double left(double x)
+{
+    const int2 v = __builtin_bit_cast(int2, x);
+    return __builtin_bit_cast(double, int2{dpp_left(v.x), dpp_left(v.y)});
+}
+// Staggered x difference between a column and the one to its right / left.
+template <class T>
+__device__ __forceinline__ T ddx_fwd(T f, T rh)
+{
+    const T f1 = right(f);
+    return d4(f1, f, right(f1), left(f), rh);
+}
+template <class T>
+__device__ __forceinline__ T ddx_bwd(T f, T rh)
+{
+    const T f0 = left(f);
+    return d4(f, f0, right(f), left(f0), rh);
+}
 
 // One region: 64 columns (one per lane) x kTileWaves * P rows (P consecutive rows per thread, in
 // registers).  nst steps from step n.
 template <class T, int P, bool AVG, bool PAL, bool EDGE>
 __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem it, const long long n, const int nst,
-                                            T *const pl, const int plane, const Vec4<T> *lpal)
+                                            T (*const bv)[kTileWaves][64], T (*const bs)[kTileWaves][64],
+                                            const Vec4<T> *lpal)
 {
     constexpr uint32_t VB = sizeof(Vec4<T>);
-    constexpr int RH = kTileWaves * P;
+    constexpr int RH = kTileWaves * P;  // the region's rows
     typedef __attribute__((address_space(1))) nvec4<T> GN;
     typedef __attribute__((address_space(1))) T GT;
     typedef __attribute__((address_space(1))) const T GCT;
     typedef __attribute__((address_space(4))) const T KT;
     const int lane = threadIdx.x & 63;
-    const int r0 = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) * P;  // first region row of this wave
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int wb = max(w - 1, 0), wa = min(w + 1, kTileWaves - 1);  // (the region's outer waves read values nothing stored depends on)
+    const int r0 = w * P;  // first region row of this wave
     const int nx = A.nx, nz = A.nz, pitch = A.pitch;
     const int c = it.x0 - kTileHalo + lane;
     const int z0 = it.z0 - kTileHalo + r0;  // grid row of this thread's row 0
@@ -134,20 +169,24 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
     const bool src_p = A.src_kind == POE2D_SRC_PRESSURE_DGAUSS && c == A.src_x;
     const bool src_f = A.src_kind == POE2D_SRC_FORCE_Y_RICKER && c == A.src_x;
 
-    T *const own = pl + kTilePad + r0 * 64 + lane;  // this thread's row 0 of plane 0
-    // row i (which may be another wave's) of plane k; rows off the region read its nearest row,
-    // into values no stored point depends on
-    auto at = [&](int k, int i) -> T { return own[k * plane + (min(max(r0 + i, 0), RH - 1) - r0) * 64]; };
-    typedef int nint4 __attribute__((ext_vector_type(4)));
-    const __attribute__((address_space(1))) nint4 *const rec = (const __attribute__((address_space(1))) nint4 *)A.rec_points;
+    typedef int nint2 __attribute__((ext_vector_type(2)));
+    const __attribute__((address_space(1))) nint2 *const rec = (const __attribute__((address_space(1))) nint2 *)A.rec_entries;
+    kcint *const rec_ptr = (kcint *)A.rec_tile_ptr + it.rec;
 
+    // coefficients of this thread's rows and the one below, from the groups: requested a barrier ahead
+    Vec4<T> mg[PAL ? 1 : P + 1];
+    auto groups = [&](const gchar *g) {
+        if constexpr (!PAL)
 #pragma unroll
-    for (int i = 0; i < P; ++i) {
-        own[PL_VX * plane + i * 64] = V[i].x;
-        own[PL_VY * plane + i * 64] = V[i].y;
-        own[PL_WX * plane + i * 64] = V[i].z;
-        own[PL_WY * plane + i * 64] = V[i].w;
-    }
+            for (int i = 0; i <= P; ++i) mg[i] = ld(g, z0 + i);
+    };
+    auto publish = [&]() {
+        bv[BV_VY_L2][w][lane] = V[P - 2].y, bv[BV_VY_L1][w][lane] = V[P - 1].y, bv[BV_VY_F1][w][lane] = V[0].y;
+        bv[BV_WY_L2][w][lane] = V[P - 2].w, bv[BV_WY_L1][w][lane] = V[P - 1].w, bv[BV_WY_F1][w][lane] = V[0].w;
+        bv[BV_VX_L1][w][lane] = V[P - 1].x, bv[BV_VX_F1][w][lane] = V[0].x, bv[BV_VX_F2][w][lane] = V[1].x;
+    };
+    groups(MSg);
+    publish();
     __syncthreads();
 
     for (int k = 0; k < nst; ++k) {
@@ -157,24 +196,37 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
             const long long q = nk - A.src_n0;
             if (A.src_series && q >= 0 && q < A.src_len) srcv = ((const KT *)A.src_series)[q];
         }
-        const bool rec_on = it.rec_hi > it.rec_lo && nk % A.rec_dec == 0 && nk / A.rec_dec < A.rec_nsamp;
+        const bool rec_on = it.rec >= 0 && nk % A.rec_dec == 0 && nk / A.rec_dec < A.rec_nsamp;
         GT *const trace = (GT *)A.traces + (rec_on ? (long long)(nk / A.rec_dec) * A.rec_ncomp * A.rec_n : 0);
-        auto entry = [&](const nint4 e) -> int { return kTilePad + (e.y - it.z0 + kTileHalo) * 64 + e.x - it.x0 + kTileHalo; };
-        if (rec_on)
-            for (int e = it.rec_lo + (int)threadIdx.x; e < it.rec_hi; e += kTileThreads) {
-                const nint4 en = rec[e];
-                int q = 0;
-                if (A.rec_mask & POE2D_VX) trace[(long long)(q++) * A.rec_n + en.z] = pl[PL_VX * plane + entry(en)];
-                if (A.rec_mask & POE2D_VY) trace[(long long)q * A.rec_n + en.z] = pl[PL_VY * plane + entry(en)];
+        // component q of row i's receivers, one per lane, from the lane that holds their column
+        auto record = [&](int i, int q, T value) {
+            if (r0 + i < kTileHalo || z0 + i >= it.z1) return;
+            const int lo = rec_ptr[z0 + i - it.z0], hi = rec_ptr[z0 + i - it.z0 + 1];
+            for (int e = lo; e < hi; e += 64) {
+                const nint2 en = rec[min(e + lane, hi - 1)];
+                const T v = __shfl(value, en.x - it.x0 + kTileHalo);
+                if (e + lane < hi) trace[(long long)q * A.rec_n + en.y] = v;
             }
+        };
+        if (rec_on) {
+            int q = 0;
+            if (A.rec_mask & POE2D_VX) {
+#pragma unroll
+                for (int i = 0; i < P; ++i) record(i, q, V[i].x);
+                ++q;
+            }
+            if (A.rec_mask & POE2D_VY)
+#pragma unroll
+                for (int i = 0; i < P; ++i) record(i, q, V[i].y);
+        }
 
         // ---- stresses
         T sxx[P], syy[P], p[P];
         {
             T vy[P + 3], wy[P + 3], vx[P + 3];  // rows -2 .. P (vy, wy), -1 .. P + 1 (vx)
-            vy[0] = at(PL_VY, -2), vy[1] = at(PL_VY, -1), vy[P + 2] = at(PL_VY, P);
-            wy[0] = at(PL_WY, -2), wy[1] = at(PL_WY, -1), wy[P + 2] = at(PL_WY, P);
-            vx[0] = at(PL_VX, -1), vx[P + 1] = at(PL_VX, P), vx[P + 2] = at(PL_VX, P + 1);
+            vy[0] = bv[BV_VY_L2][wb][lane], vy[1] = bv[BV_VY_L1][wb][lane], vy[P + 2] = bv[BV_VY_F1][wa][lane];
+            wy[0] = bv[BV_WY_L2][wb][lane], wy[1] = bv[BV_WY_L1][wb][lane], wy[P + 2] = bv[BV_WY_F1][wa][lane];
+            vx[0] = bv[BV_VX_L1][wb][lane], vx[P + 1] = bv[BV_VX_F1][wa][lane], vx[P + 2] = bv[BV_VX_F2][wa][lane];
 #pragma unroll
             for (int i = 0; i < P; ++i) vy[i + 2] = V[i].y, wy[i + 2] = V[i].w, vx[i + 1] = V[i].x;
 #pragma unroll
@@ -182,8 +234,6 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
                 sxx[i] = syy[i] = p[i] = T(0);
                 const int z = z0 + i;
                 if (r0 + i < 3 * k + 1 || r0 + i > RH - 2 - 3 * k) continue;
-                const T *const x0 = own + PL_VX * plane + i * 64, *const x1 = own + PL_WX * plane + i * 64;
-                const T *const x2 = own + PL_VY * plane + i * 64;
                 const int szs = EDGE ? zstrip(A, z) : -1;
                 const bool u1 = xr1 && (!EDGE || (z >= 2 && z < nz - 1)), u2 = xr2 && (!EDGE || (z >= 1 && z < nz - 1));
                 Vec4<T> ms;
@@ -192,17 +242,17 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
                     ms = lpal[PAL_MS * kMaxPalette + id[i]];
                     mu_nxt = lpal[PAL_MS * kMaxPalette + id[i + 1]].w;
                 } else {
-                    ms = ld(MSg, z);
-                    mu_nxt = ld(MSg, z + 1).w;
+                    ms = mg[i];
+                    mu_nxt = mg[i + 1].w;
                 }
                 T az = 0, bz = 1, rkz = 1, azh = 0, bzh = 1;
                 if (szs >= 0) {
                     az = ktab[TB_AZ * A.tn + z], bz = ktab[TB_BZ * A.tn + z], rkz = ktab[TB_RKZ * A.tn + z];
                     azh = ktab[TB_AZH * A.tn + z], bzh = ktab[TB_BZH * A.tn + z];
                 }
+                // (x differences read other lanes' registers: every lane takes part, updated or not)
+                T dvx = ddx_fwd(V[i].x, rdx), dwx = ddx_fwd(V[i].z, rdx), ddx = ddx_bwd(V[i].y, rdx);
                 if (u1) {
-                    T dvx = d4(x0[1], vx[i + 1], x0[2], x0[-1], rdx);
-                    T dwx = d4(x1[1], V[i].z, x1[2], x1[-1], rdx);
                     T dvz = d4(vy[i + 2], vy[i + 1], vy[i + 3], vy[i], rdz);
                     T dwz = d4(wy[i + 2], wy[i + 1], wy[i + 3], wy[i], rdz);
                     if constexpr (EDGE) {
@@ -228,7 +278,6 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
                     }
                 }
                 if (u2) {
-                    T ddx = d4(V[i].y, x2[-1], x2[1], x2[-2], rdx);
                     T ddz = d4(vx[i + 2], vx[i + 1], vx[i + 3], vx[i], rdz);
                     if constexpr (EDGE) {
                         if (sx >= 0) ddx = cpml_held(ddx, qx[i][PX_DVY], ax, bx, rkx);
@@ -240,35 +289,27 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
                 }
             }
         }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < P; ++i) {
-            own[PL_SXX * plane + i * 64] = sxx[i];
-            own[PL_SYY * plane + i * 64] = syy[i];
-            own[PL_SXY * plane + i * 64] = S[i].w;
-            own[PL_P * plane + i * 64] = p[i];
-        }
+        groups(MVg);
+        bs[BS_SXY_L2][w][lane] = S[P - 2].w, bs[BS_SXY_L1][w][lane] = S[P - 1].w, bs[BS_SXY_F1][w][lane] = S[0].w;
+        bs[BS_SYY_L1][w][lane] = syy[P - 1], bs[BS_SYY_F1][w][lane] = syy[0], bs[BS_SYY_F2][w][lane] = syy[1];
+        bs[BS_P_L1][w][lane] = p[P - 1], bs[BS_P_F1][w][lane] = p[0], bs[BS_P_F2][w][lane] = p[1];
         __syncthreads();
         if (rec_on && (A.rec_mask & POE2D_P))
-            for (int e = it.rec_lo + (int)threadIdx.x; e < it.rec_hi; e += kTileThreads) {
-                const nint4 en = rec[e];
-                trace[(long long)(A.rec_ncomp - 1) * A.rec_n + en.z] = pl[PL_P * plane + entry(en)];
-            }
+#pragma unroll
+            for (int i = 0; i < P; ++i) record(i, A.rec_ncomp - 1, p[i]);
 
         // ---- velocities
         {
             T sy[P + 3], pp[P + 3], sh[P + 3];  // rows -1 .. P + 1 (syy, p), -2 .. P (sxy)
-            sy[0] = at(PL_SYY, -1), sy[P + 1] = at(PL_SYY, P), sy[P + 2] = at(PL_SYY, P + 1);
-            pp[0] = at(PL_P, -1), pp[P + 1] = at(PL_P, P), pp[P + 2] = at(PL_P, P + 1);
-            sh[0] = at(PL_SXY, -2), sh[1] = at(PL_SXY, -1), sh[P + 2] = at(PL_SXY, P);
+            sy[0] = bs[BS_SYY_L1][wb][lane], sy[P + 1] = bs[BS_SYY_F1][wa][lane], sy[P + 2] = bs[BS_SYY_F2][wa][lane];
+            pp[0] = bs[BS_P_L1][wb][lane], pp[P + 1] = bs[BS_P_F1][wa][lane], pp[P + 2] = bs[BS_P_F2][wa][lane];
+            sh[0] = bs[BS_SXY_L2][wb][lane], sh[1] = bs[BS_SXY_L1][wb][lane], sh[P + 2] = bs[BS_SXY_F1][wa][lane];
 #pragma unroll
             for (int i = 0; i < P; ++i) sy[i + 1] = syy[i], pp[i + 1] = p[i], sh[i + 2] = S[i].w;
 #pragma unroll
             for (int i = 0; i < P; ++i) {
                 const int z = z0 + i;
                 if (r0 + i < 3 * k + 3 || r0 + i > RH - 4 - 3 * k) continue;
-                const T *const x0 = own + PL_SXX * plane + i * 64, *const x1 = own + PL_P * plane + i * 64;
-                const T *const x2 = own + PL_SXY * plane + i * 64;
                 const int szj = EDGE ? zstrip(A, z) : -1;
                 const bool u4 = xr4 && (!EDGE || (z >= 2 && z < nz)), u5 = xr5 && (!EDGE || (z >= 1 && z < nz - 1));
                 Vec4<T> mv, mv1, cn, cn1;
@@ -280,17 +321,18 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
                         cn1 = lpal[PAL_CN * kMaxPalette + id[i + 1]];
                     }
                 } else {
-                    mv = ld(MVg, z);
-                    mv1 = ld(MVg, z + 1);
+                    mv = mg[i];
+                    mv1 = mg[i + 1];
                 }
                 T az = 0, bz = 1, rkz = 1, azh = 0, bzh = 1, rkzh = 1;
                 if (szj >= 0) {
                     az = ktab[TB_AZ * A.tn + z], bz = ktab[TB_BZ * A.tn + z], rkz = ktab[TB_RKZ * A.tn + z];
                     azh = ktab[TB_AZH * A.tn + z], bzh = ktab[TB_BZH * A.tn + z], rkzh = ktab[TB_RKZH * A.tn + z];
                 }
+                T dsx = ddx_bwd(sxx[i], rdx), dpx = ddx_bwd(p[i], rdx), dhx = ddx_fwd(S[i].w, rdx);
                 if (u4) {
-                    T e1 = d4(sxx[i], x0[-1], x0[1], x0[-2], rdx);
-                    T e2 = d4(p[i], x1[-1], x1[1], x1[-2], rdx);
+                    T e1 = dsx;
+                    T e2 = dpx;
                     T e3 = d4(sh[i + 2], sh[i + 1], sh[i + 3], sh[i], rdz);
                     if constexpr (EDGE) {
                         if (sx >= 0) {
@@ -305,7 +347,7 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
                         biot_velocity(V[i].x, V[i].z, e1 + e3, e2, mv.x, mv.y, mv.z, mv.w, A.inv_dt);
                 }
                 if (u5) {
-                    T e1 = d4(x2[1], S[i].w, x2[2], x2[-1], rdx);
+                    T e1 = dhx;
                     T e2 = d4(sy[i + 2], sy[i + 1], sy[i + 3], sy[i], rdz);
                     T e3 = d4(pp[i + 2], pp[i + 1], pp[i + 3], pp[i], rdz);
                     if constexpr (EDGE) {
@@ -329,14 +371,8 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
             }
         }
         if (k + 1 < nst) {
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < P; ++i) {
-                own[PL_VX * plane + i * 64] = V[i].x;
-                own[PL_VY * plane + i * 64] = V[i].y;
-                own[PL_WX * plane + i * 64] = V[i].z;
-                own[PL_WY * plane + i * 64] = V[i].w;
-            }
+            groups(MSg);
+            publish();  // (every wave has read the velocities before: the stresses' barrier is past)
             __syncthreads();
         }
     }
@@ -374,9 +410,7 @@ __global__ void __launch_bounds__(kTileThreads, sizeof(T) == 4 ? 4 : 2)
     tile_steps(const StepArgs<T> *__restrict__ models, const TileItem *__restrict__ work, int nwork, int per_xcd,
                const long long *__restrict__ base, int k, int nst)
 {
-    constexpr int PMAX = sizeof(T) == 4 ? 6 : 3;
-    constexpr int plane = kTileWaves * PMAX * 64 + 2 * kTilePad;
-    __shared__ T pl[NPLANES * plane];
+    __shared__ T bv[NBOUNDARY][kTileWaves][64], bs[NBOUNDARY][kTileWaves][64];
     __shared__ Vec4<T> lpal[PAL ? PAL_SECTIONS * kMaxPalette : 1];
     const int wi = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
     if (wi >= nwork) return;
@@ -394,9 +428,9 @@ __global__ void __launch_bounds__(kTileThreads, sizeof(T) == 4 ? 4 : 2)
             lpal[e] = Vec4<T>{v.x, v.y, v.z, v.w};
         }
     }
-    if (it.kind == TILE_EDGE) tile_region<T, 3, AVG, PAL, true>(A, it, n, nst, pl, plane, lpal);
-    else if (it.kind == TILE_SHORT) tile_region<T, 3, AVG, PAL, false>(A, it, n, nst, pl, plane, lpal);
-    else if constexpr (sizeof(T) == 4) tile_region<T, 6, AVG, PAL, false>(A, it, n, nst, pl, plane, lpal);
+    if (it.kind == TILE_EDGE) tile_region<T, 3, AVG, PAL, true>(A, it, n, nst, bv, bs, lpal);
+    else if (it.kind == TILE_SHORT) tile_region<T, 3, AVG, PAL, false>(A, it, n, nst, bv, bs, lpal);
+    else if constexpr (sizeof(T) == 4) tile_region<T, 6, AVG, PAL, false>(A, it, n, nst, bv, bs, lpal);
 }
 
 template <class T>

@@ -133,7 +133,7 @@ struct StepList {
     void *models = nullptr;      // StepArgs<T>[nmodels]
     void *work = nullptr;        // WorkItem[nwork], or TileItem[nwork] (tile kernel)
     int *rec_ptr = nullptr;      // receiver offsets per (row, tile column), all models
-    void *rec_ent = nullptr;     // receiver entries, all models: int2, or int4 (tile kernel)
+    int2 *rec_ent = nullptr;     // receiver entries, all models
     long long *base = nullptr;   // step of launch 0 of the current chunk
     long long *h_base = nullptr; // pinned host staging of base
     size_t cap_models = 0, cap_work = 0, cap_ptr = 0, cap_ent = 0;
@@ -174,7 +174,7 @@ struct StepList {
         dev_free(models);
         dev_free(work);
         void *q = rec_ptr; dev_free(q); rec_ptr = nullptr;
-        dev_free(rec_ent);
+        q = rec_ent; dev_free(q); rec_ent = nullptr;
         q = base; dev_free(q); base = nullptr;
         if (h_base) (void)hipHostFree(h_base);
         h_base = nullptr;
@@ -550,8 +550,7 @@ poe2d_status upload_source(poe2d_solver *s, long long n0, int k)
 // arguments once `fix` has pointed each at its receivers.  Waits for `stream` first.
 template <class T, class F>
 poe2d_status upload_list(StepList &L, std::vector<StepArgs<T>> &args, const void *work, size_t work_bytes,
-                         const std::vector<int> &ptr, const void *ent, size_t nent, size_t ent_size, hipStream_t stream,
-                         F fix)
+                         const std::vector<int> &ptr, const int2 *ent, size_t nent, hipStream_t stream, F fix)
 {
     poe2d_status st;
     HIP_TRY(hipStreamSynchronize(stream));
@@ -561,7 +560,10 @@ poe2d_status upload_list(StepList &L, std::vector<StepArgs<T>> &args, const void
     st = grow(&pp, &L.cap_ptr, std::max<size_t>(ptr.size(), 1) * sizeof(int));
     L.rec_ptr = (int *)pp;
     if (st) return st;
-    if ((st = grow(&L.rec_ent, &L.cap_ent, std::max<size_t>(nent, 1) * ent_size))) return st;
+    void *pe = L.rec_ent;
+    st = grow(&pe, &L.cap_ent, std::max<size_t>(nent, 1) * sizeof(int2));
+    L.rec_ent = (int2 *)pe;
+    if (st) return st;
     for (size_t i = 0; i < args.size(); ++i) fix(args[i], (int)i);
     if (!L.base) {
         void *q = nullptr;
@@ -572,7 +574,7 @@ poe2d_status upload_list(StepList &L, std::vector<StepArgs<T>> &args, const void
     HIP_TRY(hipMemcpy(L.models, args.data(), args.size() * sizeof(StepArgs<T>), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(L.work, work, work_bytes, hipMemcpyHostToDevice));
     if (!ptr.empty()) HIP_TRY(hipMemcpy(L.rec_ptr, ptr.data(), ptr.size() * sizeof(int), hipMemcpyHostToDevice));
-    if (nent) HIP_TRY(hipMemcpy(L.rec_ent, ent, nent * ent_size, hipMemcpyHostToDevice));
+    if (nent) HIP_TRY(hipMemcpy(L.rec_ent, ent, nent * sizeof(int2), hipMemcpyHostToDevice));
     return POE2D_OK;
 }
 
@@ -671,9 +673,9 @@ poe2d_status build_list(StepList &L, const std::vector<poe2d_solver *> &members,
         }
     }
     const poe2d_status st = upload_list<T>(L, args, work.data(), work.size() * sizeof(WorkItem), ptr, ent.data(),
-                                           ent.size(), sizeof(int2), stream, [&](StepArgs<T> &A, int i) {
+                                           ent.size(), stream, [&](StepArgs<T> &A, int i) {
                                                A.rec_tile_ptr = L.rec_ptr + ptr_off[i];
-                                               A.rec_entries = (const int2 *)L.rec_ent + ent_off[i];
+                                               A.rec_entries = L.rec_ent + ent_off[i];
                                            });
     if (st) return st;
     L.nmodels = nm;
@@ -701,7 +703,8 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
     tall = tall && sizeof(T) == 4;
     std::vector<StepArgs<T>> args(nm);
     std::vector<TileItem> edge, inter;
-    std::vector<int4> ent;
+    std::vector<int> ptr;
+    std::vector<int2> ent;
     for (int i = 0; i < nm; ++i) {
         const poe2d_solver *s = members[i];
         const Model *md = s->m;
@@ -738,12 +741,18 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
                 it.z0 = z0;
                 it.kind = tall && inside(kTileTall) ? TILE_TALL : inside(kTileShort) ? TILE_SHORT : TILE_EDGE;
                 it.z1 = std::min(z0 + (it.kind == TILE_TALL ? kTileTall : kTileShort), nz + 1);
-                it.rec_lo = (int)ent.size();
-                while (next < order.size() && s->hrx[order[next]] < x0 + kTileCols && s->hrz[order[next]] < it.z1) {
-                    const int r = order[next++];
-                    ent.push_back(int4{s->hrx[r], s->hrz[r], r, 0});
+                it.rec = -1;
+                auto pending = [&](int z) {
+                    return next < order.size() && s->hrx[order[next]] < x0 + kTileCols && s->hrz[order[next]] < z;
+                };
+                if (pending(it.z1)) {
+                    it.rec = (int)ptr.size();
+                    for (int z = z0; z < it.z1; ++z) {
+                        ptr.push_back((int)ent.size());
+                        for (; pending(z + 1); ++next) ent.push_back(int2{s->hrx[order[next]], order[next]});
+                    }
+                    ptr.push_back((int)ent.size());
                 }
-                it.rec_hi = (int)ent.size();
                 (it.kind == TILE_EDGE ? edge : inter).push_back(it);
                 z0 = it.z1;
             }
@@ -767,9 +776,11 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
         for (size_t e = x; e < edge.size(); e += 8) work[o++] = edge[e];
         for (size_t q = (size_t)x * ni; q < std::min(inter.size(), (size_t)(x + 1) * ni); ++q) work[o++] = inter[q];
     }
-    const poe2d_status st = upload_list<T>(L, args, work.data(), work.size() * sizeof(TileItem), {}, ent.data(), ent.size(),
-                                           sizeof(int4), stream,
-                                           [&](StepArgs<T> &A, int) { A.rec_points = (const int4 *)L.rec_ent; });
+    const poe2d_status st = upload_list<T>(L, args, work.data(), work.size() * sizeof(TileItem), ptr, ent.data(),
+                                           ent.size(), stream, [&](StepArgs<T> &A, int) {
+                                               A.rec_tile_ptr = L.rec_ptr;
+                                               A.rec_entries = L.rec_ent;
+                                           });
     if (st) return st;
     L.nmodels = nm;
     L.nint = (int)inter.size();

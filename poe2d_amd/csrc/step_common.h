@@ -122,7 +122,6 @@ struct StepArgs {
     // n / rec_dec of traces ([slot][comp][receiver], components of rec_mask).
     const int *rec_tile_ptr;
     const int2 *rec_entries;
-    const int4 *rec_points;  // the tile kernel's: (x, z, receiver index, -), the tiles' runs one after the other
     T *traces;
     int rec_n, rec_ncomp, rec_dec, rec_nsamp;
     unsigned rec_mask;
@@ -344,11 +343,12 @@ constexpr int kFused2RowsBefore = 10, kFused2RowsAfter = 12, kFused2ColsBefore =
 // work item owns columns [x0, x0 + kTileCols) and rows [z0, z1), at most kTileShort rows (TILE_EDGE,
 // TILE_SHORT) or kTileTall (TILE_TALL).  TILE_EDGE items are those whose region (the owned points and
 // kTileHalo on every side) reaches a C-PML strip or the grid's two outer rows or columns; the others
-// run without that code.  Receivers rec_points[rec_lo .. rec_hi) are the item's.
+// run without that code.  Items with receivers have rec >= 0: rec_tile_ptr[rec + k] .. [rec + k + 1]
+// are the rec_entries of row z0 + k.
 enum { TILE_EDGE = 0, TILE_SHORT = 1, TILE_TALL = 2 };
 constexpr int kTileHalo = 6, kTileCols = 64 - 2 * kTileHalo, kTileShort = 24 - 2 * kTileHalo, kTileTall = 48 - 2 * kTileHalo;
 struct TileItem {
-    int model, x0, z0, z1, kind, rec_lo, rec_hi, unused;
+    int model, x0, z0, z1, kind, rec;
 };
 // nst (1 or 2) steps from step n = *base + k; buffers as the two-step kernel's launches use them.
 template <class T>
