@@ -168,15 +168,17 @@ poe2d_status poe2d_set_receivers(poe2d_solver *s, const poe2d_receivers *rec);
  *     point.
  *   schedule 1: a stress launch and a velocity launch per step, intermediates through memory.
  *   schedule 2: as schedule 0, always reading the per-point coefficient arrays.
- *   schedule 3 (the default): two time steps per launch.  block_w 64 runs the tile kernel: regions
- *     of 64 columns held on chip for both steps, owning 52 columns by 12 rows or, with tile_rows of
- *     36 or more on FP32 handles, by 36 rows away from the border; coefficients as schedule 0.
+ *   schedule 3 (the default): several time steps per launch.  block_w 64 runs the tile kernel:
+ *     regions of 64 columns held on chip, tile_rows 36 or more for two steps per launch on tall
+ *     regions (owning 52 columns by 36 rows, or 20 in FP64 or without a palette; 12 rows at the
+ *     border), 12 for two steps on short ones (12 rows), 13 to 35 and 4 to 11 for three steps on
+ *     tall and on short regions; coefficients as schedule 0.
  *     block_w 128 or 256 runs, on FP32 handles, blocks that march down tiles of block_w - 12 columns
  *     by tile_rows rows (multiples of 6 best), the coefficients through a palette of at most 28
  *     entries, or from the per-point coefficient groups on grids without one; an odd last step of
  *     a run takes one schedule-0 launch.  On FP64 handles those widths run schedule 0.
- * Until this call (or poe2d_autotune) a handle runs schedule 3 on the tile kernel, its tile height
- * by the size of the grid, or of the whole batch.
+ * Until this call (or poe2d_autotune) a handle runs schedule 3 on the tile kernel's tall regions,
+ * two or three steps per launch by the size of the grid, or of the whole batch.
  * Tile heights do not change a bit; schedules and block widths agree to rounding.  The choice
  * only changes speed. */
 poe2d_status poe2d_set_schedule(poe2d_solver *s, int schedule, int block_w, int tile_rows);
@@ -227,7 +229,7 @@ poe2d_status poe2d_reset(poe2d_solver *s);
 
 /* Pick the fastest tile shape of the handle's schedule for its grid: times nsteps steps (after
  * one warm-up step) for each block width in {128, 256, 512} and tile height in {8, 14, 20, 26,
- * 32, 44, 62, 98} (two-step schedule: 64 by 12 or 36, widths {128, 256}, heights {6, 12, ..., 60}), times the
+ * 32, 44, 62, 98} (schedule 3: 64 by 6, 12, 30 or 36, widths {128, 256}, heights {6, 12, ..., 60}), times the
  * three fastest again, twice each over 3 nsteps steps, keeps the best and resets the handle.  The result is cached for the process per grid class (device,
  * precision, schedule, grid size, palette): a later call for the same class applies the cached
  * shape without timing.  nsteps = 0 means 10; nsteps < 0 times -nsteps steps and ignores the

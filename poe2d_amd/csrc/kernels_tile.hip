@@ -68,7 +68,7 @@ __device__ __forceinline__ T ddx_bwd(T f, T rh)
 // One region: 64 columns (one per lane) x kTileWaves * P rows (P consecutive rows per thread, in
 // registers).  nst steps from step n.
 template <class T, int P, bool AVG, bool PAL, bool EDGE>
-__device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem it, const long long n, const int nst,
+__device__ __forceinline__ void tile_region(const __attribute__((address_space(4))) StepArgs<T> &A, const TileItem it, const long long n, const int in, const int halo, const int nst,
                                             T (*const bv)[kTileWaves][64], T (*const bs)[kTileWaves][64],
                                             const Vec4<T> *lpal)
 {
@@ -83,10 +83,11 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
     const int wb = max(w - 1, 0), wa = min(w + 1, kTileWaves - 1);  // (the region's outer waves read values nothing stored depends on)
     const int r0 = w * P;  // first region row of this wave
     const int nx = A.nx, nz = A.nz, pitch = A.pitch;
-    const int c = it.x0 - kTileHalo + lane;
-    const int z0 = it.z0 - kTileHalo + r0;  // grid row of this thread's row 0
-    const int in = (int)((((n - A.pair0) >> 1) + A.pcur) & 1);
+    const int c = it.x0 - halo + lane;
+    const int z0 = it.z0 - halo + r0;  // grid row of this thread's row 0
     const T rdx = A.rdx, rdz = A.rdz, dt = A.dt;
+    const int ztop = A.ztop, zbot = A.zbot;
+    auto strip = [&](int z) -> int { return z < 0 ? -1 : z < ztop ? z : z < zbot ? -1 : z <= nz ? ztop + (z - zbot) : -1; };
 
     gchar *const gb = (gchar *)A.grp;
     const long long gsb = A.group_stride * (long long)VB;
@@ -148,7 +149,7 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
                     qx[i][2 * q] = v.x, qx[i][2 * q + 1] = v.y;
                 }
             }
-            const int s = zstrip(A, z);
+            const int s = strip(z);
             if (s >= 0 && inx) {
                 const GP *const r = (const GP *)pz(in, s);
 #pragma unroll
@@ -173,19 +174,22 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
     const __attribute__((address_space(1))) nint2 *const rec = (const __attribute__((address_space(1))) nint2 *)A.rec_entries;
     kcint *const rec_ptr = (kcint *)A.rec_tile_ptr + it.rec;
 
-    // coefficients of this thread's rows and the one below, from the groups: requested a barrier ahead
-    Vec4<T> mg[PAL ? 1 : P + 1];
-    auto groups = [&](const gchar *g) {
-        if constexpr (!PAL)
+    // without a palette: coefficients of this thread's rows and the one below, from the groups, read
+    // once and held for every step where the registers allow (no memory variables, FP32, no means of
+    // rows), else requested a barrier ahead of each use
+    constexpr bool HOLD = !PAL && !EDGE && !AVG && sizeof(T) == 4;
+    Vec4<T> mg[PAL ? 1 : P + 1], mh[HOLD ? P + 1 : 1];
+    auto groups = [&](const gchar *g, Vec4<T> *m) {
 #pragma unroll
-            for (int i = 0; i <= P; ++i) mg[i] = ld(g, z0 + i);
+        for (int i = 0; i <= P; ++i) m[i] = ld(g, z0 + i);
     };
+    if constexpr (HOLD) groups(MSg, mg), groups(MVg, mh);
     auto publish = [&]() {
         bv[BV_VY_L2][w][lane] = V[P - 2].y, bv[BV_VY_L1][w][lane] = V[P - 1].y, bv[BV_VY_F1][w][lane] = V[0].y;
         bv[BV_WY_L2][w][lane] = V[P - 2].w, bv[BV_WY_L1][w][lane] = V[P - 1].w, bv[BV_WY_F1][w][lane] = V[0].w;
         bv[BV_VX_L1][w][lane] = V[P - 1].x, bv[BV_VX_F1][w][lane] = V[0].x, bv[BV_VX_F2][w][lane] = V[1].x;
     };
-    groups(MSg);
+    if constexpr (!PAL && !HOLD) groups(MSg, mg);
     publish();
     __syncthreads();
 
@@ -200,11 +204,11 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
         GT *const trace = (GT *)A.traces + (rec_on ? (long long)(nk / A.rec_dec) * A.rec_ncomp * A.rec_n : 0);
         // component q of row i's receivers, one per lane, from the lane that holds their column
         auto record = [&](int i, int q, T value) {
-            if (r0 + i < kTileHalo || z0 + i >= it.z1) return;
+            if (r0 + i < halo || z0 + i >= it.z1) return;
             const int lo = rec_ptr[z0 + i - it.z0], hi = rec_ptr[z0 + i - it.z0 + 1];
             for (int e = lo; e < hi; e += 64) {
                 const nint2 en = rec[min(e + lane, hi - 1)];
-                const T v = __shfl(value, en.x - it.x0 + kTileHalo);
+                const T v = __shfl(value, en.x - it.x0 + halo);
                 if (e + lane < hi) trace[(long long)q * A.rec_n + en.y] = v;
             }
         };
@@ -234,7 +238,7 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
                 sxx[i] = syy[i] = p[i] = T(0);
                 const int z = z0 + i;
                 if (r0 + i < 3 * k + 1 || r0 + i > RH - 2 - 3 * k) continue;
-                const int szs = EDGE ? zstrip(A, z) : -1;
+                const int szs = EDGE ? strip(z) : -1;
                 const bool u1 = xr1 && (!EDGE || (z >= 2 && z < nz - 1)), u2 = xr2 && (!EDGE || (z >= 1 && z < nz - 1));
                 Vec4<T> ms;
                 T mu_nxt;
@@ -289,7 +293,7 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
                 }
             }
         }
-        groups(MVg);
+        if constexpr (!PAL && !HOLD) groups(MVg, mg);
         bs[BS_SXY_L2][w][lane] = S[P - 2].w, bs[BS_SXY_L1][w][lane] = S[P - 1].w, bs[BS_SXY_F1][w][lane] = S[0].w;
         bs[BS_SYY_L1][w][lane] = syy[P - 1], bs[BS_SYY_F1][w][lane] = syy[0], bs[BS_SYY_F2][w][lane] = syy[1];
         bs[BS_P_L1][w][lane] = p[P - 1], bs[BS_P_F1][w][lane] = p[0], bs[BS_P_F2][w][lane] = p[1];
@@ -310,7 +314,7 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
             for (int i = 0; i < P; ++i) {
                 const int z = z0 + i;
                 if (r0 + i < 3 * k + 3 || r0 + i > RH - 4 - 3 * k) continue;
-                const int szj = EDGE ? zstrip(A, z) : -1;
+                const int szj = EDGE ? strip(z) : -1;
                 const bool u4 = xr4 && (!EDGE || (z >= 2 && z < nz)), u5 = xr5 && (!EDGE || (z >= 1 && z < nz - 1));
                 Vec4<T> mv, mv1, cn, cn1;
                 if constexpr (PAL) {
@@ -321,8 +325,8 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
                         cn1 = lpal[PAL_CN * kMaxPalette + id[i + 1]];
                     }
                 } else {
-                    mv = mg[i];
-                    mv1 = mg[i + 1];
+                    mv = HOLD ? mh[i] : mg[i];
+                    mv1 = HOLD ? mh[i + 1] : mg[i + 1];
                 }
                 T az = 0, bz = 1, rkz = 1, azh = 0, bzh = 1, rkzh = 1;
                 if (szj >= 0) {
@@ -371,20 +375,20 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
             }
         }
         if (k + 1 < nst) {
-            groups(MSg);
+            if constexpr (!PAL && !HOLD) groups(MSg, mg);
             publish();  // (every wave has read the velocities before: the stresses' barrier is past)
             __syncthreads();
         }
     }
 
     // ---- the owned points
-    if (lane < kTileHalo || lane >= 64 - kTileHalo || c > nx) return;
+    if (lane < halo || lane >= 64 - halo || c > nx) return;
     gchar *const Vn = gb + group_v(in ^ 1) * gsb;
     gchar *const Sn = gb + group_s(in ^ 1) * gsb;
 #pragma unroll
     for (int i = 0; i < P; ++i) {
         const int z = z0 + i;
-        if (r0 + i < kTileHalo || z >= it.z1) continue;
+        if (r0 + i < halo || z >= it.z1) continue;
         *(GN *)(Vn + off(z)) = nvec4<T>{V[i].x, V[i].y, V[i].z, V[i].w};
         *(GN *)(Sn + off(z)) = nvec4<T>{S[i].x, S[i].y, S[i].z, S[i].w};
         if constexpr (EDGE) {
@@ -395,7 +399,7 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
 #pragma unroll
                 for (int q = 0; q < NPSI_X / 2; ++q) r[q] = pair{qx[i][2 * q], qx[i][2 * q + 1]};
             }
-            const int s = zstrip(A, z);
+            const int s = strip(z);
             if (s >= 0) {
                 GP *const r = (GP *)pz(in ^ 1, s);
 #pragma unroll
@@ -408,7 +412,7 @@ __device__ __forceinline__ void tile_region(const StepArgs<T> &A, const TileItem
 template <class T, bool AVG, bool PAL>
 __global__ void __launch_bounds__(kTileThreads, sizeof(T) == 4 ? 4 : 2)
     tile_steps(const StepArgs<T> *__restrict__ models, const TileItem *__restrict__ work, int nwork, int per_xcd,
-               const long long *__restrict__ base, int k, int nst)
+               const long long *__restrict__ base, int launch, int steps, int nst)
 {
     __shared__ T bv[NBOUNDARY][kTileWaves][64], bs[NBOUNDARY][kTileWaves][64];
     __shared__ Vec4<T> lpal[PAL ? PAL_SECTIONS * kMaxPalette : 1];
@@ -416,8 +420,11 @@ __global__ void __launch_bounds__(kTileThreads, sizeof(T) == 4 ? 4 : 2)
     if (wi >= nwork) return;
     const TileItem it = work[wi];
     if (it.model < 0) return;
-    const StepArgs<T> A = models[it.model];
-    const long long n = *(const kcll *)base + k;
+    // (fields are read where used: held from the start, a hundred of them would spill)
+    const __attribute__((address_space(4))) StepArgs<T> &A =
+        *((const __attribute__((address_space(4))) StepArgs<T> *)models + it.model);
+    const long long n = *(const kcll *)base + (long long)launch * steps;
+    const int in = (launch + A.pcur) & 1, halo = 3 * steps;
     if constexpr (PAL) {
         typedef __attribute__((address_space(1))) nvec4<T> GN;
         const GN *const pal = (const GN *)A.pal;
@@ -428,30 +435,31 @@ __global__ void __launch_bounds__(kTileThreads, sizeof(T) == 4 ? 4 : 2)
             lpal[e] = Vec4<T>{v.x, v.y, v.z, v.w};
         }
     }
-    if (it.kind == TILE_EDGE) tile_region<T, 3, AVG, PAL, true>(A, it, n, nst, bv, bs, lpal);
-    else if (it.kind == TILE_SHORT) tile_region<T, 3, AVG, PAL, false>(A, it, n, nst, bv, bs, lpal);
-    else if constexpr (sizeof(T) == 4) tile_region<T, 6, AVG, PAL, false>(A, it, n, nst, bv, bs, lpal);
+    if (it.kind == TILE_EDGE) tile_region<T, 3, AVG, PAL, true>(A, it, n, in, halo, nst, bv, bs, lpal);
+    else if (it.kind == TILE_SHORT) tile_region<T, 3, AVG, PAL, false>(A, it, n, in, halo, nst, bv, bs, lpal);
+    else tile_region<T, tile_tall_p(sizeof(T) == 4, PAL), AVG, PAL, false>(A, it, n, in, halo, nst, bv, bs, lpal);
 }
 
 template <class T>
 hipError_t launch_tiles(const StepArgs<T> *models, const TileItem *work, int nwork, int per_xcd, bool palette, bool avg,
-                        const long long *base, int k, int nst, hipStream_t stream)
+                        const long long *base, int launch, int steps, int nst, hipStream_t stream)
 {
-    if (nwork < 1 || per_xcd < 1 || 8LL * per_xcd < nwork || nst < 1 || nst > 2) return hipErrorInvalidValue;
+    if (nwork < 1 || per_xcd < 1 || 8LL * per_xcd < nwork || steps < 2 || steps > kTileStepsMax || nst < 1 || nst > steps)
+        return hipErrorInvalidValue;
     const dim3 grid(8 * per_xcd);
     if (palette) {
-        if (avg) tile_steps<T, true, true><<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, k, nst);
-        else tile_steps<T, false, true><<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, k, nst);
+        if (avg) tile_steps<T, true, true><<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, launch, steps, nst);
+        else tile_steps<T, false, true><<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, launch, steps, nst);
     } else {
-        if (avg) tile_steps<T, true, false><<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, k, nst);
-        else tile_steps<T, false, false><<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, k, nst);
+        if (avg) tile_steps<T, true, false><<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, launch, steps, nst);
+        else tile_steps<T, false, false><<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, launch, steps, nst);
     }
     return hipGetLastError();
 }
 
 template hipError_t launch_tiles<float>(const StepArgs<float> *, const TileItem *, int, int, bool, bool, const long long *, int,
-                                        int, hipStream_t);
+                                        int, int, hipStream_t);
 template hipError_t launch_tiles<double>(const StepArgs<double> *, const TileItem *, int, int, bool, bool, const long long *,
-                                         int, int, hipStream_t);
+                                         int, int, int, hipStream_t);
 
 }  // namespace poe2d

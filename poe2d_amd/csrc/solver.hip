@@ -45,8 +45,9 @@ namespace {
 const float kRefPiF = 3.1415926535897932f;  // the reference's float PI (seismic_CPML_2d_poroelastic.cpp:9)
 const double kStabilityThreshold = 1.0e25;  // STABILITY_THRESHOLD of the reference (declared, unused there)
 const int kGraphSteps = 32;                 // steps per captured graph
+const int kTileSlots = 512;                 // tiles of the FP32 tile kernel the chip holds at once (half as many FP64)
 const int kBandTiles = 8;                   // tile columns to a band of the tile kernel's work order
-const long long kShortTilesMax = 1280;      // launches of up to this many short tiles use them (five per CU)
+const int kGraphTileLaunches = 32;          // launches of the tile kernel per captured graph
 
 #define HIP_TRY(expr)                                                                              \
     do {                                                                                           \
@@ -142,18 +143,19 @@ struct StepList {
     bool avg = false;  // POE2D_MATERIAL_AVERAGED (all members alike)
     bool two = false;  // two-step or tile kernel: each launch advances two steps
     bool tiles = false;  // tile kernel
+    int steps = 2;       // its steps per launch
     int nint = 0;      // two-step kernel: interior tiles in the list
     int precision = POE2D_F32;
     // graph of kGraphSteps launches plus the base advance, and the launch it was captured for
     hipGraphExec_t exec = nullptr;
     struct Sig {
         void *models, *work, *base;
-        int nwork, nint, per_xcd, bw, palette, avg, two, tiles, precision;
+        int nwork, nint, per_xcd, bw, palette, avg, two, tiles, steps, precision;
         bool operator==(const Sig &o) const
         {
             return models == o.models && work == o.work && base == o.base && nwork == o.nwork && nint == o.nint &&
                    per_xcd == o.per_xcd && bw == o.bw && palette == o.palette && avg == o.avg && two == o.two &&
-                   tiles == o.tiles && precision == o.precision;
+                   tiles == o.tiles && steps == o.steps && precision == o.precision;
         }
     } sig{};
 
@@ -162,7 +164,7 @@ struct StepList {
         Sig g{};
         g.models = models; g.work = work; g.base = base;
         g.nwork = nwork; g.nint = nint; g.per_xcd = per_xcd; g.bw = bw; g.palette = palette; g.avg = avg; g.two = two;
-        g.tiles = tiles;
+        g.tiles = tiles; g.steps = steps;
         g.precision = precision;
         return g;
     }
@@ -691,78 +693,100 @@ poe2d_status build_list(StepList &L, const std::vector<poe2d_solver *> &members,
     return POE2D_OK;
 }
 
-// As build_list, for the tile kernel: each member's grid cut into tiles of kTileCols columns, their
-// rows in tiles of kTileShort rows where the region reaches a C-PML strip or the border (edge tiles)
-// and of kTileTall rows elsewhere (`tall`; else kTileShort), each with its receivers.
+// The tiles of member i's grid for `steps` steps per launch, with their receivers: short rows where
+// the region reaches a C-PML strip or the border (edge tiles), tall_rows (if more) elsewhere.
+void cut_tiles(const poe2d_solver *s, int i, int steps, int tall_rows, std::vector<TileItem> &edge,
+               std::vector<TileItem> &inter, std::vector<int> &ptr, std::vector<int2> &ent)
+{
+    const Model *md = s->m;
+    const int halo = tile_halo(steps), cols = tile_cols(steps), short_rows = tile_rows(3, steps);
+    const int nx = s->grid.nx, nz = s->grid.nz;
+    // receivers by tile column and row
+    std::vector<int> order(s->nrec);
+    for (int r = 0; r < s->nrec; ++r) order[r] = r;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+        const int ta = s->hrx[a] / cols, tb = s->hrx[b] / cols;
+        return ta != tb ? ta < tb : s->hrz[a] < s->hrz[b];
+    });
+    size_t next = 0;
+    const int zlo = std::max(md->ztop, 2), zhi = std::min(md->zbot, nz - 1);
+    for (int x0 = 0; x0 <= nx; x0 += cols) {
+        const int c0 = x0 - halo, c1 = c0 + 63;  // the region's columns
+        const bool xs = c0 < std::max(md->xlo, 2) || c1 >= std::min(md->xhi, nx - 1);
+        for (int z0 = 0; z0 <= nz;) {
+            // rows [z0 - halo, z0 + rows + halo) of the region within [zlo, zhi)
+            auto inside = [&](int rows) { return !xs && z0 - halo >= zlo && z0 + rows + halo <= zhi; };
+            TileItem it{};
+            it.model = i;
+            it.x0 = x0;
+            it.z0 = z0;
+            it.kind = tall_rows > short_rows && inside(tall_rows) ? TILE_TALL : inside(short_rows) ? TILE_SHORT : TILE_EDGE;
+            it.z1 = std::min(z0 + (it.kind == TILE_TALL ? tall_rows : short_rows), nz + 1);
+            it.rec = -1;
+            auto pending = [&](int z) {
+                return next < order.size() && s->hrx[order[next]] < x0 + cols && s->hrz[order[next]] < z;
+            };
+            if (pending(it.z1)) {
+                it.rec = (int)ptr.size();
+                for (int z = z0; z < it.z1; ++z) {
+                    ptr.push_back((int)ent.size());
+                    for (; pending(z + 1); ++next) ent.push_back(int2{s->hrx[order[next]], order[next]});
+                }
+                ptr.push_back((int)ent.size());
+            }
+            (it.kind == TILE_EDGE ? edge : inter).push_back(it);
+            z0 = it.z1;
+        }
+    }
+}
+
+// As build_list, for the tile kernel, `steps` steps per launch.  steps = 0: three where the chip holds
+// every tile of the launch at once, else two: such launches are bound by latency and the cost of a
+// launch, which three steps share (us per step, three / two: 161^2 4.9 / 5.9, 401^2 6.4 / 6.5, 401^2
+// continuous 7.3 / 7.8), others by HBM or instruction issue, where the wider halo costs more (1201^2
+// 20.0 / 16.9, 2001^2 40.4 / 36.1, FP64 401^2 10.5 / 8.8).
 template <class T>
-poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members, bool tall, bool palette,
+poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members, int steps, bool tall, bool palette,
                          hipStream_t stream)
 {
     const int nm = (int)members.size();
     const int material = members[0]->grid.staggered_material;
-    tall = tall && sizeof(T) == 4;
-    std::vector<StepArgs<T>> args(nm);
-    std::vector<TileItem> edge, inter;
-    std::vector<int> ptr;
-    std::vector<int2> ent;
-    for (int i = 0; i < nm; ++i) {
-        const poe2d_solver *s = members[i];
-        const Model *md = s->m;
-        if (palette && (md->npal < 1 || !md->mid || !md->pal))
+    for (const poe2d_solver *s : members) {
+        if (palette && (s->m->npal < 1 || !s->m->mid || !s->m->pal))
             return fail(POE2D_E_INVALID, "run: a palette launch over a grid without a palette");
         if (s->grid.staggered_material != material)
             return fail(POE2D_E_INVALID, "run: batch members differ in staggered material");
-        args[i] = step_args<T>(s, 0, 1, 64, kTileShort, true);
+    }
+    std::vector<TileItem> edge, inter;
+    std::vector<int> ptr;
+    std::vector<int2> ent;
+    const bool choose = steps == 0;
+    if (choose) steps = 3;
+    for (int i = 0; i < nm; ++i) {
+        cut_tiles(members[i], i, steps, tall ? tile_rows(tile_tall_p(sizeof(T) == 4, palette), steps) : 0, edge, inter, ptr, ent);
+        if (edge.size() + inter.size() > (1u << 28)) return fail(POE2D_E_INVALID, "run: too many tiles in one launch");
+        if (choose && steps == 3 && edge.size() + inter.size() > (size_t)kTileSlots * 4 / sizeof(T)) {
+            edge.clear(), inter.clear(), ptr.clear(), ent.clear();
+            steps = 2;
+            i = -1;  // again, for two steps
+        }
+    }
+    const int cols = tile_cols(steps);
+    std::vector<StepArgs<T>> args(nm);
+    for (int i = 0; i < nm; ++i) {
+        const poe2d_solver *s = members[i];
+        args[i] = step_args<T>(s, 0, 1, 64, 12, true);
         args[i].rec_n = s->nrec;
         args[i].rec_ncomp = s->ncomp;
         args[i].rec_dec = s->dec;
         args[i].rec_nsamp = s->nsamp;
         args[i].rec_mask = s->mask;
         args[i].traces = (T *)s->traces;
-        const int nx = s->grid.nx, nz = s->grid.nz;
-        // receivers by tile column and row
-        std::vector<int> order(s->nrec);
-        for (int r = 0; r < s->nrec; ++r) order[r] = r;
-        std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-            const int ta = s->hrx[a] / kTileCols, tb = s->hrx[b] / kTileCols;
-            return ta != tb ? ta < tb : s->hrz[a] < s->hrz[b];
-        });
-        size_t next = 0;
-        for (int x0 = 0; x0 <= nx; x0 += kTileCols) {
-            const int c0 = x0 - kTileHalo, c1 = c0 + 63;  // the region's columns
-            const bool xs = c0 < std::max(md->xlo, 2) || c1 >= std::min(md->xhi, nx - 1);
-            const int zlo = std::max(md->ztop, 2), zhi = std::min(md->zbot, nz - 1);
-            for (int z0 = 0; z0 <= nz;) {
-                // rows [z0 - halo, z0 + rows + halo) of the region within [zlo, zhi)
-                auto inside = [&](int rows) { return !xs && z0 - kTileHalo >= zlo && z0 + rows + kTileHalo <= zhi; };
-                TileItem it{};
-                it.model = i;
-                it.x0 = x0;
-                it.z0 = z0;
-                it.kind = tall && inside(kTileTall) ? TILE_TALL : inside(kTileShort) ? TILE_SHORT : TILE_EDGE;
-                it.z1 = std::min(z0 + (it.kind == TILE_TALL ? kTileTall : kTileShort), nz + 1);
-                it.rec = -1;
-                auto pending = [&](int z) {
-                    return next < order.size() && s->hrx[order[next]] < x0 + kTileCols && s->hrz[order[next]] < z;
-                };
-                if (pending(it.z1)) {
-                    it.rec = (int)ptr.size();
-                    for (int z = z0; z < it.z1; ++z) {
-                        ptr.push_back((int)ent.size());
-                        for (; pending(z + 1); ++next) ent.push_back(int2{s->hrx[order[next]], order[next]});
-                    }
-                    ptr.push_back((int)ent.size());
-                }
-                (it.kind == TILE_EDGE ? edge : inter).push_back(it);
-                z0 = it.z1;
-            }
-            if (edge.size() + inter.size() > (1u << 28)) return fail(POE2D_E_INVALID, "run: too many tiles in one launch");
-        }
     }
     // Interior tiles run row by row in bands of kBandTiles tile columns, so that the tiles in flight on
     // an XCD (about 64) make a block of neighbours sharing their halos in its L2.
-    std::stable_sort(inter.begin(), inter.end(), [](const TileItem &a, const TileItem &b) {
-        const int ba = a.x0 / (kBandTiles * kTileCols), bb = b.x0 / (kBandTiles * kTileCols);
+    std::stable_sort(inter.begin(), inter.end(), [&](const TileItem &a, const TileItem &b) {
+        const int ba = a.x0 / (kBandTiles * cols), bb = b.x0 / (kBandTiles * cols);
         return std::tie(a.model, ba, a.z0, a.x0) < std::tie(b.model, bb, b.z0, b.x0);
     });
     // as the two-step kernel's list: every XCD gets an eighth of the edge tiles first, then a run of
@@ -791,6 +815,7 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
     L.avg = material == POE2D_MATERIAL_AVERAGED;
     L.two = true;
     L.tiles = true;
+    L.steps = steps;
     L.precision = sizeof(T) == 4 ? POE2D_F32 : POE2D_F64;
     return POE2D_OK;
 }
@@ -803,10 +828,10 @@ hipError_t launch_list_chunk(const StepList &L, int count, hipStream_t stream)
     if (L.tiles) {
         for (int k = 0; k < count; ++k) {
             const hipError_t e = launch_tiles<T>((const StepArgs<T> *)L.models, (const TileItem *)L.work, L.nwork, L.per_xcd,
-                                                 L.palette, L.avg, L.base, 2 * k, 2, stream);
+                                                 L.palette, L.avg, L.base, k, L.steps, L.steps, stream);
             if (e != hipSuccess) return e;
         }
-        return launch_base_advance(L.base, 2 * count, stream);
+        return launch_base_advance(L.base, L.steps * count, stream);
     }
     if (L.two) {
         if constexpr (sizeof(T) == 4) {
@@ -835,7 +860,8 @@ poe2d_status run_list(StepList &L, long long n0, int k, bool graphs, hipStream_t
     *L.h_base = n0;
     HIP_TRY(hipMemcpyAsync(L.base, L.h_base, sizeof(long long), hipMemcpyHostToDevice, stream));
     int done = 0;
-    const int chunk = L.two ? kGraphSteps / 2 : kGraphSteps;
+    // (the tile kernel's state buffers alternate by launch within a chunk: an even number of launches)
+    const int chunk = L.tiles ? kGraphTileLaunches : L.two ? kGraphSteps / 2 : kGraphSteps;
     if (graphs && k >= chunk) {
         const StepList::Sig sig = L.signature();
         if (!L.exec || !(L.sig == sig)) {
@@ -864,16 +890,21 @@ poe2d_status run_list(StepList &L, long long n0, int k, bool graphs, hipStream_t
     return POE2D_OK;
 }
 
-// nsteps steps of the members (all at step n0) on the tile kernel: step pairs, and a launch of one
-// step for an odd last one.
+// nsteps steps of the members (all at step n0) on the tile kernel: launches of L.steps steps, and one
+// of the remainder.  *flips = launches, the times the state changed buffers.
 template <class T>
-poe2d_status run_tiles(StepList &L, long long n0, int nsteps, bool graphs, hipStream_t stream)
+poe2d_status run_tiles(StepList &L, long long n0, int nsteps, bool graphs, hipStream_t stream, int *flips)
 {
     poe2d_status st;
-    if ((st = run_list<T>(L, n0, nsteps / 2, graphs, stream))) return st;
-    if (nsteps & 1)
+    const int full = nsteps / L.steps, rest = nsteps % L.steps;
+    if ((st = run_list<T>(L, n0, full, graphs, stream))) return st;
+    if (rest) {
+        // (the counter is past the full launches; an odd number of them leaves the state in the other buffer)
+        HIP_TRY(launch_base_advance(L.base, -(full & 1) * L.steps, stream));
         HIP_TRY(launch_tiles<T>((const StepArgs<T> *)L.models, (const TileItem *)L.work, L.nwork, L.per_xcd, L.palette, L.avg,
-                                L.base, 0, 1, stream));
+                                L.base, full & 1, L.steps, rest, stream));
+    }
+    *flips = full + (rest > 0);
     return POE2D_OK;
 }
 
@@ -902,23 +933,21 @@ bool two_step_kernel(const poe2d_solver *s)
 // Whether the two-step kernel reads handle s through its palette.
 bool two_step_palette(const poe2d_solver *s) { return s->m->npal > 0 && s->m->npal <= kMaxPalette2; }
 struct TileShape {
-    bool tiles;  // the tile kernel
+    bool tiles;  // the tile kernel, its steps per launch (0: by size) and tile kind
+    int steps;
+    bool tall;
     int bw, th;
 };
 
-// The tile shape the members advance with: the chosen one, or (auto_shape) the tile kernel, whose
-// short tiles (twice the blocks, half the rows per thread) serve launches that tall ones would not
-// spread over the chip: us per step, short / tall, 401^2 continuous 7.4 / 9.3, 1001 x 777 14.9 /
-// 15.1 (1300 short tiles), 1201^2 22.3 / 20.1 (2400), 4001^2 190.6 / 137.1.  FP64 has short tiles only.
+// The tile shape the members advance with: the chosen one (block width 64: the tile kernel, the
+// height selecting steps per launch and tile kind), or by default the tile kernel on tall tiles
+// (never slower than short ones: 161^2 5.9 / 5.9, 401^2 6.5 / 6.6 us per step, 4001^2 127 / 172).
 TileShape tile_shape(const std::vector<poe2d_solver *> &members, bool auto_shape, int bw, int th)
 {
     for (const poe2d_solver *s : members)
-        if (s->schedule != SCHED_FUSED2) return {false, bw, th};
-    if (!auto_shape) return {bw == 64, bw, th};
-    long long tiles = 0;
-    for (const poe2d_solver *s : members)
-        tiles += (long long)(s->grid.nx / kTileCols + 1) * (s->grid.nz / kTileShort + 1);
-    return {true, 64, tiles > kShortTilesMax ? kTileTall : kTileShort};
+        if (s->schedule != SCHED_FUSED2) return {false, 2, false, bw, th};
+    if (auto_shape) return {true, 0, true, 64, 36};
+    return {bw == 64, th < 12 || (th > 12 && th < 36) ? 3 : 2, th > 12, bw, th};
 }
 
 // Shapes an autotuner times: of the two-step schedule (the tile kernel's two and the marching
@@ -933,8 +962,8 @@ std::vector<std::pair<int, int>> tune_shapes(const std::vector<poe2d_solver *> &
         nz = std::max(nz, s->grid.nz);
     }
     std::vector<std::pair<int, int>> out;
-    if (tiles) out.push_back({64, kTileShort});
-    if (two) out.push_back({64, kTileTall});
+    if (tiles)
+        for (int h : {6, 12, 30, 36}) out.push_back({64, h});
     // Tile heights of 6k + 2 rows (6k for the two-step kernel) make whole groups of the kernels'
     // 6-step row loops.
     const std::vector<int> widths = two ? std::vector<int>{128, 256} : std::vector<int>{128, 256, 512};
@@ -968,11 +997,12 @@ poe2d_status run_steps(poe2d_solver *s, int nsteps)
         HIP_TRY(hipEventRecord(s->ev1, s->stream));
     } else if (const TileShape shape = tile_shape({s}, s->auto_shape, s->block_w, s->tile_rows); shape.tiles) {
         if ((st = upload_source<T>(s, s->step, nsteps))) return st;
-        if ((st = build_tiles<T>(s->list2, {s}, shape.th >= kTileTall, s->m->npal > 0, s->stream))) return st;
+        if ((st = build_tiles<T>(s->list2, {s}, shape.steps, shape.tall, s->m->npal > 0, s->stream))) return st;
+        int flips = 0;
         HIP_TRY(hipEventRecord(s->ev0, s->stream));
-        if ((st = run_tiles<T>(s->list2, s->step, nsteps, s->graphs, s->stream))) return st;
+        if ((st = run_tiles<T>(s->list2, s->step, nsteps, s->graphs, s->stream, &flips))) return st;
         HIP_TRY(hipEventRecord(s->ev1, s->stream));
-        s->cur = (s->cur + nsteps / 2 + (nsteps & 1)) & 1;
+        s->cur = (s->cur + flips) & 1;
     } else if (sizeof(T) == 4 && two_step_kernel(s)) {
         // step pairs on the two-step kernel, an odd last step on the single-step kernel
         const int pairs = nsteps / 2, rem = nsteps & 1;
@@ -1116,9 +1146,10 @@ poe2d_status batch_run_steps(poe2d_batch *b, int nsteps)
         return fail(POE2D_E_INVALID, "batch_run: the two-step kernel takes block widths 64, 128 or 256");
     two = two || shape.tiles;
     const int pairs = two ? nsteps / 2 : 0, rem = two ? nsteps & 1 : nsteps;
+    int flips = pairs + rem;
     poe2d_status st;
     if (shape.tiles) {
-        if ((st = build_tiles<T>(b->list2, b->members, shape.th >= kTileTall, tile_palette, b->stream))) return st;
+        if ((st = build_tiles<T>(b->list2, b->members, shape.steps, shape.tall, tile_palette, b->stream))) return st;
     } else if (pairs) {
         for (poe2d_solver *s : b->members)
             if (!s->psi_mid && (st = dev_alloc(&s->psi_mid, std::max<size_t>(s->m->psi_half_elems(), 1) * s->rs)))
@@ -1130,7 +1161,7 @@ poe2d_status batch_run_steps(poe2d_batch *b, int nsteps)
         return st;
     HIP_TRY(hipEventRecord(b->ev0, b->stream));
     if (shape.tiles) {
-        if ((st = run_tiles<T>(b->list2, n0, nsteps, b->graphs, b->stream))) return st;
+        if ((st = run_tiles<T>(b->list2, n0, nsteps, b->graphs, b->stream, &flips))) return st;
     } else {
         if (pairs && (st = run_list<T>(b->list2, n0, pairs, b->graphs, b->stream))) return st;
         if (rem && (st = run_list<T>(b->list, n0 + 2LL * pairs, rem, b->graphs, b->stream))) return st;
@@ -1143,7 +1174,7 @@ poe2d_status batch_run_steps(poe2d_batch *b, int nsteps)
     b->last_steps = nsteps;
     poe2d_status first = POE2D_OK;
     for (poe2d_solver *s : b->members) {
-        s->cur = (s->cur + pairs + rem) & 1;
+        s->cur = (s->cur + flips) & 1;
         s->step += nsteps;
         s->last_ms = ms;
         s->last_steps = nsteps;

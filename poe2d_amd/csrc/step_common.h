@@ -339,20 +339,27 @@ hipError_t launch_fused2(const StepArgs<T> *models, const WorkItem *work, int nw
 // outer rows or columns on either side, in this range is an edge tile.
 constexpr int kFused2RowsBefore = 10, kFused2RowsAfter = 12, kFused2ColsBefore = 6;
 
-// The tile kernel (kernels_tile.hip): one or two steps of a region of 64 columns held on chip.  A
-// work item owns columns [x0, x0 + kTileCols) and rows [z0, z1), at most kTileShort rows (TILE_EDGE,
-// TILE_SHORT) or kTileTall (TILE_TALL).  TILE_EDGE items are those whose region (the owned points and
-// kTileHalo on every side) reaches a C-PML strip or the grid's two outer rows or columns; the others
-// run without that code.  Items with receivers have rec >= 0: rec_tile_ptr[rec + k] .. [rec + k + 1]
-// are the rec_entries of row z0 + k.
+// The tile kernel (kernels_tile.hip): `steps` (two or three) steps of a region of 64 columns held on
+// chip.  A step consumes three rows and columns of the region on every side, so a work item owns
+// columns [x0, x0 + tile_cols) and rows [z0, z1), at most 24 - 6 steps rows (TILE_EDGE, TILE_SHORT) or
+// 8 tile_tall_p - 6 steps (TILE_TALL).  TILE_EDGE items are those whose region reaches a C-PML strip or
+// the grid's two outer rows or columns; the others run without that code.  Items with receivers have
+// rec >= 0: rec_tile_ptr[rec + k] .. [rec + k + 1] are the rec_entries of row z0 + k.
 enum { TILE_EDGE = 0, TILE_SHORT = 1, TILE_TALL = 2 };
-constexpr int kTileHalo = 6, kTileCols = 64 - 2 * kTileHalo, kTileShort = 24 - 2 * kTileHalo, kTileTall = 48 - 2 * kTileHalo;
+constexpr int kTileStepsMax = 3;
+// Rows per thread of a tall tile: 6 with an FP32 palette; 4 where the registers also hold FP64 values
+// or the coefficients of every row (at 6 those spill).
+__host__ __device__ constexpr int tile_tall_p(bool f32, bool palette) { return f32 && palette ? 6 : 4; }
+__host__ __device__ constexpr int tile_halo(int steps) { return 3 * steps; }
+__host__ __device__ constexpr int tile_cols(int steps) { return 64 - 2 * tile_halo(steps); }
+__host__ __device__ constexpr int tile_rows(int p, int steps) { return 8 * p - 2 * tile_halo(steps); }
 struct TileItem {
     int model, x0, z0, z1, kind, rec;
 };
-// nst (1 or 2) steps from step n = *base + k; buffers as the two-step kernel's launches use them.
+// nst <= steps steps from step n = *base + launch * steps; reads state buffer (launch + pcur) & 1 and
+// writes the other.
 template <class T>
 hipError_t launch_tiles(const StepArgs<T> *models, const TileItem *work, int nwork, int per_xcd, bool palette, bool avg,
-                        const long long *base, int k, int nst, hipStream_t stream);
+                        const long long *base, int launch, int steps, int nst, hipStream_t stream);
 
 }  // namespace poe2d

@@ -57,7 +57,8 @@ def _same(a, b, label):
 def test_tiles_equal_the_single_step_kernel(nx, nz, npml, entries, precision):
     prob = _problem(nx, nz, npml, entries)
     ref = _run(prob, precision, (0, 256, 14), [9])
-    for shape, steps in (((3, 64, 12), [4, 5]), ((3, 64, 36), [9]), (None, [1, 2, 6])):
+    for shape, steps in (((3, 64, 12), [4, 5]), ((3, 64, 36), [9]), ((3, 64, 6), [8, 1]), ((3, 64, 30), [2, 7]),
+                         (None, [1, 2, 6])):
         _same(_run(prob, precision, shape, steps), ref, f"{nx}x{nz} npml {npml} {entries} entries shape {shape}")
 
 
