@@ -29,12 +29,15 @@
 
 namespace poe2d {
 
+constexpr int kTileCus = 256;  // compute units
 constexpr int kTileThreads = 512, kTileWaves = kTileThreads / 64;
 
 // Rows a wave publishes to its neighbours, before the stresses (its velocities) and before the
 // velocities (its stresses): of each field the rows a z difference of the wave below or above reads.
 enum { BV_VY_L2, BV_VY_L1, BV_VY_F1, BV_WY_L2, BV_WY_L1, BV_WY_F1, BV_VX_L1, BV_VX_F1, BV_VX_F2, NBOUNDARY };
 enum { BS_SXY_L2, BS_SXY_L1, BS_SXY_F1, BS_SYY_L1, BS_SYY_F1, BS_SYY_F2, BS_P_L1, BS_P_F1, BS_P_F2 };
+
+constexpr int NXTAB = TB_RKXH - TB_AX + 1;  // C-PML profiles of a column
 
 // The value of the lane one column to the right (zero past the last lane) / to the left.
 __device__ __forceinline__ int dpp_right(int x) { return __builtin_amdgcn_update_dpp(0, x, 0x130, 0xf, 0xf, true); }
@@ -67,10 +70,10 @@ __device__ __forceinline__ T ddx_bwd(T f, T rh)
 
 // One region: 64 columns (one per lane) x kTileWaves * P rows (P consecutive rows per thread, in
 // registers).  nst steps from step n.
-template <class T, int P, bool AVG, bool PAL, bool EDGE>
-__device__ __forceinline__ void tile_region(const __attribute__((address_space(4))) StepArgs<T> &A, const TileItem it, const long long n, const int in, const int halo, const int nst,
+template <class T, int P, bool AVG, bool PAL, bool EDGE, bool ROOM>
+__device__ __forceinline__ void tile_region(const __attribute__((address_space(4))) StepArgs<T> &A, const TileItem it, const long long n, const int in, const int halo, const int nst, const bool stream,
                                             T (*const bv)[kTileWaves][64], T (*const bs)[kTileWaves][64],
-                                            const Vec4<T> *lpal)
+                                            T (*const xtab)[64], const Vec4<T> *lpal)
 {
     constexpr uint32_t VB = sizeof(Vec4<T>);
     constexpr int RH = kTileWaves * P;  // the region's rows
@@ -109,31 +112,40 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
     for (int i = 0; i < P; ++i) S[i] = ld(So, z0 + i);
 
     // material: palette entries of rows 0 .. P, or the coefficient groups (read where used)
-    int id[P + 1];
+    constexpr bool PACK = EDGE;  // entries of four rows in one register (P = 3)
+    static_assert(!PACK || P == 3, "four bytes");
+    int id[PACK ? 1 : P + 1];
+    auto entry = [&](int i) -> int {
+        if constexpr (PACK) return (id[0] >> (8 * i)) & 255;
+        else return id[i];
+    };
     const gchar *const MSg = (const gchar *)A.mat + G_MS * gsb;
     const gchar *const MVg = (const gchar *)A.mat + G_MV * gsb;
     if constexpr (PAL) {
         gcuchar *const mid = (gcuchar *)A.mid;
+        if constexpr (PACK) id[0] = 0;
 #pragma unroll
-        for (int i = 0; i <= P; ++i) id[i] = mid[(uint32_t)(cc + kPadCols) + prow(z0 + i) * (uint32_t)pitch];
+        for (int i = 0; i <= P; ++i) {
+            const int e = mid[(uint32_t)(cc + kPadCols) + prow(z0 + i) * (uint32_t)pitch];
+            if constexpr (PACK) id[0] |= e << (8 * i);
+            else id[i] = e;
+        }
     }
 
     // C-PML: memory variables of this thread's points and the profiles of its column and rows
+    // (a column's profiles in registers; in LDS, a few per cent slower on launches of one tile per CU,
+    // where FP32 blocks share a CU: there they would spill)
+    constexpr bool XLDS = EDGE && sizeof(T) == 4 && !ROOM;
     const bool inx = c >= 0 && c <= nx;
     const int sx = (EDGE && inx) ? ((gcint *)A.xmap)[c] : -1;
     T qx[EDGE ? P : 1][NPSI_X], qz[EDGE ? P : 1][NPSI_Z];
-    T ax = 0, bx = 1, rkx = 1, axh = 0, bxh = 1, rkxh = 1;
     GT *const psi = (GT *)A.psi;
     auto px = [&](int b, int z) -> GT * { return psi + ((long long)b * A.pxn + (long long)z * A.wxs + sx) * NPSI_X; };
     auto pz = [&](int b, int s) -> GT * {
         return psi + 2LL * NPSI_X * A.pxn + ((long long)b * A.pzn + (long long)s * pitch + c) * NPSI_Z;
     };
     if constexpr (EDGE) {
-        const GCT *const tab = (const GCT *)A.tab;
-        if (sx >= 0) {
-            ax = tab[TB_AX * A.tn + c], bx = tab[TB_BX * A.tn + c], rkx = tab[TB_RKX * A.tn + c];
-            axh = tab[TB_AXH * A.tn + c], bxh = tab[TB_BXH * A.tn + c], rkxh = tab[TB_RKXH * A.tn + c];
-        }
+        if (XLDS && w < NXTAB && inx) xtab[w][lane] = ((const GCT *)A.tab)[(TB_AX + w) * A.tn + c];
         typedef T pair __attribute__((ext_vector_type(2)));
         typedef __attribute__((address_space(1))) const pair GP;
 #pragma unroll
@@ -161,6 +173,11 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
         }
     }
     const KT *const ktab = (const KT *)A.tab;
+    T xr[EDGE && !XLDS ? NXTAB : 1];
+    if constexpr (EDGE && !XLDS)
+#pragma unroll
+        for (int k = 0; k < NXTAB; ++k) xr[k] = inx ? ((const GCT *)A.tab)[(TB_AX + k) * A.tn + c] : T(0);
+    auto xt = [&](int k) -> T { return XLDS ? xtab[k - TB_AX][lane] : xr[EDGE && !XLDS ? k - TB_AX : 0]; };
 
     const bool xr1 = !EDGE || (c >= 1 && c < nx);      // stress1
     const bool xr2 = !EDGE || (c >= 2 && c < nx);      // stress2
@@ -177,7 +194,7 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
     // without a palette: coefficients of this thread's rows and the one below, from the groups, read
     // once and held for every step where the registers allow (no memory variables, FP32, no means of
     // rows), else requested a barrier ahead of each use
-    constexpr bool HOLD = !PAL && !EDGE && !AVG && sizeof(T) == 4;
+    constexpr bool HOLD = !PAL && sizeof(T) == 4 && (ROOM || (!EDGE && !AVG));
     Vec4<T> mg[PAL ? 1 : P + 1], mh[HOLD ? P + 1 : 1];
     auto groups = [&](const gchar *g, Vec4<T> *m) {
 #pragma unroll
@@ -243,8 +260,8 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
                 Vec4<T> ms;
                 T mu_nxt;
                 if constexpr (PAL) {
-                    ms = lpal[PAL_MS * kMaxPalette + id[i]];
-                    mu_nxt = lpal[PAL_MS * kMaxPalette + id[i + 1]].w;
+                    ms = lpal[PAL_MS * kMaxPalette + entry(i)];
+                    mu_nxt = lpal[PAL_MS * kMaxPalette + entry(i + 1)].w;
                 } else {
                     ms = mg[i];
                     mu_nxt = mg[i + 1].w;
@@ -261,8 +278,8 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
                     T dwz = d4(wy[i + 2], wy[i + 1], wy[i + 3], wy[i], rdz);
                     if constexpr (EDGE) {
                         if (sx >= 0) {
-                            dvx = cpml_held(dvx, qx[i][PX_DVX], axh, bxh, rkxh);
-                            dwx = cpml_held(dwx, qx[i][PX_DWX], axh, bxh, rkxh);
+                            dvx = cpml_held(dvx, qx[i][PX_DVX], xt(TB_AXH), xt(TB_BXH), xt(TB_RKXH));
+                            dwx = cpml_held(dwx, qx[i][PX_DWX], xt(TB_AXH), xt(TB_BXH), xt(TB_RKXH));
                         }
                         if (szs >= 0) {
                             dvz = cpml_held(dvz, qz[i][PZ_DVZ], az, bz, rkz);
@@ -284,7 +301,7 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
                 if (u2) {
                     T ddz = d4(vx[i + 2], vx[i + 1], vx[i + 3], vx[i], rdz);
                     if constexpr (EDGE) {
-                        if (sx >= 0) ddx = cpml_held(ddx, qx[i][PX_DVY], ax, bx, rkx);
+                        if (sx >= 0) ddx = cpml_held(ddx, qx[i][PX_DVY], xt(TB_AX), xt(TB_BX), xt(TB_RKX));
                         // half-grid memory coefficients, full-grid K_z divisor (reference :224-226)
                         if (szs >= 0) ddz = cpml_held(ddz, qz[i][PZ_DVX], azh, bzh, rkz);
                     }
@@ -318,11 +335,11 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
                 const bool u4 = xr4 && (!EDGE || (z >= 2 && z < nz)), u5 = xr5 && (!EDGE || (z >= 1 && z < nz - 1));
                 Vec4<T> mv, mv1, cn, cn1;
                 if constexpr (PAL) {
-                    mv = lpal[PAL_MV * kMaxPalette + id[i]];
-                    mv1 = lpal[PAL_MV * kMaxPalette + id[i + 1]];
+                    mv = lpal[PAL_MV * kMaxPalette + entry(i)];
+                    mv1 = lpal[PAL_MV * kMaxPalette + entry(i + 1)];
                     if constexpr (sizeof(T) == 4) {
-                        cn = lpal[PAL_CN * kMaxPalette + id[i]];
-                        cn1 = lpal[PAL_CN * kMaxPalette + id[i + 1]];
+                        cn = lpal[PAL_CN * kMaxPalette + entry(i)];
+                        cn1 = lpal[PAL_CN * kMaxPalette + entry(i + 1)];
                     }
                 } else {
                     mv = HOLD ? mh[i] : mg[i];
@@ -340,8 +357,8 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
                     T e3 = d4(sh[i + 2], sh[i + 1], sh[i + 3], sh[i], rdz);
                     if constexpr (EDGE) {
                         if (sx >= 0) {
-                            e1 = cpml_held(e1, qx[i][PX_DSXX], ax, bx, rkx);
-                            e2 = cpml_held(e2, qx[i][PX_DPX], ax, bx, rkx);
+                            e1 = cpml_held(e1, qx[i][PX_DSXX], xt(TB_AX), xt(TB_BX), xt(TB_RKX));
+                            e2 = cpml_held(e2, qx[i][PX_DPX], xt(TB_AX), xt(TB_BX), xt(TB_RKX));
                         }
                         if (szj >= 0) e3 = cpml_held(e3, qz[i][PZ_DSXY], az, bz, rkz);
                     }
@@ -355,7 +372,7 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
                     T e2 = d4(sy[i + 2], sy[i + 1], sy[i + 3], sy[i], rdz);
                     T e3 = d4(pp[i + 2], pp[i + 1], pp[i + 3], pp[i], rdz);
                     if constexpr (EDGE) {
-                        if (sx >= 0) e1 = cpml_held(e1, qx[i][PX_DSXY], axh, bxh, rkxh);
+                        if (sx >= 0) e1 = cpml_held(e1, qx[i][PX_DSXY], xt(TB_AXH), xt(TB_BXH), xt(TB_RKXH));
                         if (szj >= 0) {
                             e2 = cpml_held(e2, qz[i][PZ_DSYY], azh, bzh, rkzh);
                             e3 = cpml_held(e3, qz[i][PZ_DPZ], azh, bzh, rkzh);
@@ -389,8 +406,16 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
     for (int i = 0; i < P; ++i) {
         const int z = z0 + i;
         if (r0 + i < halo || z >= it.z1) continue;
-        *(GN *)(Vn + off(z)) = nvec4<T>{V[i].x, V[i].y, V[i].z, V[i].w};
-        *(GN *)(Sn + off(z)) = nvec4<T>{S[i].x, S[i].y, S[i].z, S[i].w};
+        const nvec4<T> v = {V[i].x, V[i].y, V[i].z, V[i].w}, t = {S[i].x, S[i].y, S[i].z, S[i].w};
+        if (stream) {
+            asm volatile("" ::: "memory");  // (or the two branches' stores merge into ordinary ones)
+            __builtin_nontemporal_store(v, (GN *)(Vn + off(z)));
+            __builtin_nontemporal_store(t, (GN *)(Sn + off(z)));
+            asm volatile("" ::: "memory");
+        } else {
+            *(GN *)(Vn + off(z)) = v;
+            *(GN *)(Sn + off(z)) = t;
+        }
         if constexpr (EDGE) {
             typedef T pair __attribute__((ext_vector_type(2)));
             typedef __attribute__((address_space(1))) pair GP;
@@ -409,12 +434,15 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
     }
 }
 
-template <class T, bool AVG, bool PAL>
-__global__ void __launch_bounds__(kTileThreads, sizeof(T) == 4 ? 4 : 2)
+// ROOM: launches of at most one block per CU, which may then use twice the registers.  FP64 blocks
+// always do.
+template <class T, bool AVG, bool PAL, bool ROOM>
+__global__ void __launch_bounds__(kTileThreads, sizeof(T) == 4 && !ROOM ? 4 : 2)
     tile_steps(const StepArgs<T> *__restrict__ models, const TileItem *__restrict__ work, int nwork, int per_xcd,
-               const long long *__restrict__ base, int launch, int steps, int nst)
+               const long long *__restrict__ base, int launch, int steps, int nst, int stream)
 {
     __shared__ T bv[NBOUNDARY][kTileWaves][64], bs[NBOUNDARY][kTileWaves][64];
+    __shared__ T xtab[NXTAB][64];
     __shared__ Vec4<T> lpal[PAL ? PAL_SECTIONS * kMaxPalette : 1];
     const int wi = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
     if (wi >= nwork) return;
@@ -435,31 +463,37 @@ __global__ void __launch_bounds__(kTileThreads, sizeof(T) == 4 ? 4 : 2)
             lpal[e] = Vec4<T>{v.x, v.y, v.z, v.w};
         }
     }
-    if (it.kind == TILE_EDGE) tile_region<T, 3, AVG, PAL, true>(A, it, n, in, halo, nst, bv, bs, lpal);
-    else if (it.kind == TILE_SHORT) tile_region<T, 3, AVG, PAL, false>(A, it, n, in, halo, nst, bv, bs, lpal);
-    else tile_region<T, tile_tall_p(sizeof(T) == 4, PAL), AVG, PAL, false>(A, it, n, in, halo, nst, bv, bs, lpal);
+    if (it.kind == TILE_EDGE) tile_region<T, 3, AVG, PAL, true, ROOM>(A, it, n, in, halo, nst, stream, bv, bs, xtab, lpal);
+    else if (it.kind == TILE_SHORT) tile_region<T, 3, AVG, PAL, false, ROOM>(A, it, n, in, halo, nst, stream, bv, bs, xtab, lpal);
+    else tile_region<T, tile_tall_p(sizeof(T) == 4, PAL), AVG, PAL, false, ROOM>(A, it, n, in, halo, nst, stream, bv, bs, xtab, lpal);
 }
 
 template <class T>
 hipError_t launch_tiles(const StepArgs<T> *models, const TileItem *work, int nwork, int per_xcd, bool palette, bool avg,
-                        const long long *base, int launch, int steps, int nst, hipStream_t stream)
+                        const long long *base, int launch, int steps, int nst, bool stream_out, hipStream_t stream)
 {
     if (nwork < 1 || per_xcd < 1 || 8LL * per_xcd < nwork || steps < 2 || steps > kTileStepsMax || nst < 1 || nst > steps)
         return hipErrorInvalidValue;
-    const dim3 grid(8 * per_xcd);
-    if (palette) {
-        if (avg) tile_steps<T, true, true><<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, launch, steps, nst);
-        else tile_steps<T, false, true><<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, launch, steps, nst);
-    } else {
-        if (avg) tile_steps<T, true, false><<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, launch, steps, nst);
-        else tile_steps<T, false, false><<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, launch, steps, nst);
-    }
+    auto launch_as = [&](auto av, auto pal) {
+        constexpr bool AVG = decltype(av)::value, PAL = decltype(pal)::value;
+        const dim3 grid(8 * per_xcd);
+        if (sizeof(T) == 8 || nwork <= kTileCus)
+            tile_steps<T, AVG, PAL, true>
+                <<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, launch, steps, nst, stream_out);
+        else if constexpr (sizeof(T) == 4)
+            tile_steps<T, AVG, PAL, false>
+                <<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, launch, steps, nst, stream_out);
+    };
+    using Yes = std::true_type;
+    using No = std::false_type;
+    if (palette) avg ? launch_as(Yes{}, Yes{}) : launch_as(No{}, Yes{});
+    else avg ? launch_as(Yes{}, No{}) : launch_as(No{}, No{});
     return hipGetLastError();
 }
 
 template hipError_t launch_tiles<float>(const StepArgs<float> *, const TileItem *, int, int, bool, bool, const long long *, int,
-                                        int, int, hipStream_t);
+                                        int, int, bool, hipStream_t);
 template hipError_t launch_tiles<double>(const StepArgs<double> *, const TileItem *, int, int, bool, bool, const long long *,
-                                         int, int, int, hipStream_t);
+                                         int, int, int, bool, hipStream_t);
 
 }  // namespace poe2d

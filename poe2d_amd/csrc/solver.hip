@@ -45,6 +45,8 @@ namespace {
 const float kRefPiF = 3.1415926535897932f;  // the reference's float PI (seismic_CPML_2d_poroelastic.cpp:9)
 const double kStabilityThreshold = 1.0e25;  // STABILITY_THRESHOLD of the reference (declared, unused there)
 const int kGraphSteps = 32;                 // steps per captured graph
+const size_t kL2Bytes = size_t(32) << 20;   // the eight L2s together
+const size_t kMallBytes = size_t(256) << 20;  // the memory-side cache
 const int kTileSlots = 512;                 // tiles of the FP32 tile kernel the chip holds at once (half as many FP64)
 const int kBandTiles = 8;                   // tile columns to a band of the tile kernel's work order
 const int kGraphTileLaunches = 32;          // launches of the tile kernel per captured graph
@@ -144,18 +146,19 @@ struct StepList {
     bool two = false;  // two-step or tile kernel: each launch advances two steps
     bool tiles = false;  // tile kernel
     int steps = 2;       // its steps per launch
+    bool stream_out = false;  // it stores the state past the caches (see build_tiles)
     int nint = 0;      // two-step kernel: interior tiles in the list
     int precision = POE2D_F32;
     // graph of kGraphSteps launches plus the base advance, and the launch it was captured for
     hipGraphExec_t exec = nullptr;
     struct Sig {
         void *models, *work, *base;
-        int nwork, nint, per_xcd, bw, palette, avg, two, tiles, steps, precision;
+        int nwork, nint, per_xcd, bw, palette, avg, two, tiles, steps, stream_out, precision;
         bool operator==(const Sig &o) const
         {
             return models == o.models && work == o.work && base == o.base && nwork == o.nwork && nint == o.nint &&
                    per_xcd == o.per_xcd && bw == o.bw && palette == o.palette && avg == o.avg && two == o.two &&
-                   tiles == o.tiles && steps == o.steps && precision == o.precision;
+                   tiles == o.tiles && steps == o.steps && stream_out == o.stream_out && precision == o.precision;
         }
     } sig{};
 
@@ -164,7 +167,7 @@ struct StepList {
         Sig g{};
         g.models = models; g.work = work; g.base = base;
         g.nwork = nwork; g.nint = nint; g.per_xcd = per_xcd; g.bw = bw; g.palette = palette; g.avg = avg; g.two = two;
-        g.tiles = tiles; g.steps = steps;
+        g.tiles = tiles; g.steps = steps; g.stream_out = stream_out;
         g.precision = precision;
         return g;
     }
@@ -816,6 +819,16 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
     L.two = true;
     L.tiles = true;
     L.steps = steps;
+    // Stores past the caches where a launch's state, both buffers of it, fits neither the L2s nor the
+    // memory-side cache (the halos neighbours read stay in L2 instead), and where it fits the L2s with
+    // room to spare (less to write back at the launch's end); between the two the next launch reads
+    // what this one left there.  us per step, cached / past: 701^2 9.0 / 8.7 (31 MB), 801^2 12.2 / 13.0,
+    // 2001^2 35.6 / 37.4 (256 MB), 2201^2 43.4 / 42.5, 4001^2 126 / 118; FP64, which HBM does not bound,
+    // 401^2 9.05 / 8.6, 1201^2 41.5 / 46.4, 2801^2 200 / 214.
+    size_t state = 0;
+    for (const poe2d_solver *s : members)
+        state += (size_t)(s->grid.nx + 1) * (s->grid.nz + 1) * (palette ? 16 : 24) * sizeof(T);
+    L.stream_out = state < kL2Bytes || (state > kMallBytes && sizeof(T) == 4);
     L.precision = sizeof(T) == 4 ? POE2D_F32 : POE2D_F64;
     return POE2D_OK;
 }
@@ -828,7 +841,7 @@ hipError_t launch_list_chunk(const StepList &L, int count, hipStream_t stream)
     if (L.tiles) {
         for (int k = 0; k < count; ++k) {
             const hipError_t e = launch_tiles<T>((const StepArgs<T> *)L.models, (const TileItem *)L.work, L.nwork, L.per_xcd,
-                                                 L.palette, L.avg, L.base, k, L.steps, L.steps, stream);
+                                                 L.palette, L.avg, L.base, k, L.steps, L.steps, L.stream_out, stream);
             if (e != hipSuccess) return e;
         }
         return launch_base_advance(L.base, L.steps * count, stream);
@@ -902,7 +915,7 @@ poe2d_status run_tiles(StepList &L, long long n0, int nsteps, bool graphs, hipSt
         // (the counter is past the full launches; an odd number of them leaves the state in the other buffer)
         HIP_TRY(launch_base_advance(L.base, -(full & 1) * L.steps, stream));
         HIP_TRY(launch_tiles<T>((const StepArgs<T> *)L.models, (const TileItem *)L.work, L.nwork, L.per_xcd, L.palette, L.avg,
-                                L.base, full & 1, L.steps, rest, stream));
+                                L.base, full & 1, L.steps, rest, L.stream_out, stream));
     }
     *flips = full + (rest > 0);
     return POE2D_OK;
