@@ -238,9 +238,9 @@ poe2d_status poe2d_reset(poe2d_solver *s);
  * (seismic_CPML_2D_poroelastic_withCUDA.cu:1620-1634). */
 poe2d_status poe2d_autotune(poe2d_solver *s, int nsteps, int *block_w, int *tile_rows);
 
-/* Launch mode of the single-pass schedule: with graphs on (the default) a run captures 32 steps
- * (the step kernel and the receiver gather, which also advances the device step counter) in a
- * HIP graph once and replays it; off,
+/* Launch mode of the step kernels other than the tile kernel (which is always launched directly):
+ * with graphs on (the default) a run captures 32 steps (the step kernel, which also gathers the
+ * receivers, and the advance of the device step counter) in a HIP graph once and replays it; off,
  * every step is launched directly.  Results are identical either way.  No counterpart in the
  * reference, which launches six kernels per step (.cu:1628-1634). */
 poe2d_status poe2d_set_graphs(poe2d_solver *s, int enable);

@@ -39,4 +39,26 @@ template <class T>
 void launch_absmax(const StepArgs<T> &A, int buf, float *partials, int nblocks, float *result,
                    hipStream_t stream);
 
+// The same of n members at once: member i's n points of velocity 4-vectors from v on into result[i];
+// partials holds n * nblocks floats.
+struct FieldRange {
+    const void *v;
+    long long n;
+};
+template <class T>
+void launch_absmax_members(const FieldRange *ranges, int n, float *partials, int nblocks, float *result,
+                           hipStream_t stream);
+
+// Zeroes up to kClearRanges ranges of 4-byte words in one launch.
+constexpr int kClearRanges = 5;
+struct ClearRanges {
+    void *p[kClearRanges];
+    size_t words[kClearRanges];
+};
+void launch_clear(const ClearRanges &r, hipStream_t stream);
+
+// out[c][r] = in[r][c], rows x cols.
+template <class T>
+void launch_transpose(const T *in, int rows, int cols, T *out, hipStream_t stream);
+
 }  // namespace poe2d

@@ -2,6 +2,8 @@
 // recompute and component extraction for snapshots, and the stability reduction.
 #include "aux_kernels.h"
 
+#include <algorithm>
+
 namespace poe2d {
 
 namespace {
@@ -76,14 +78,14 @@ __global__ void insert_kernel(StepArgs<T> A, int g, int comp, const T *in)
     else v.w = a;
 }
 
+// Largest |vx|, |vy| of points i = first, first + step, ... < npts (a block's 256 threads), non-finite
+// as +inf.
 template <class T>
-__global__ void __launch_bounds__(256) absmax_blocks(StepArgs<T> A, int buf, float *partial)
+__device__ float block_absmax(const Vec4<T> *V, long long npts, long long first, long long step)
 {
     __shared__ float red[256];
-    const Vec4<T> *V = state_group(A, group_v(buf));
-    const long long npts = (long long)(A.nz + 1) * A.pitch;
     float m = 0.f;
-    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < npts; i += (long long)gridDim.x * blockDim.x) {
+    for (long long i = first; i < npts; i += step) {
         const Vec4<T> v = V[i];  // rows 0..nz, pad columns included (zero)
         float a = fabsf((float)v.x), b = fabsf((float)v.y);
         if (!(a <= 3.0e38f)) a = INFINITY;
@@ -96,13 +98,65 @@ __global__ void __launch_bounds__(256) absmax_blocks(StepArgs<T> A, int buf, flo
         if ((int)threadIdx.x < s) red[threadIdx.x] = fmaxf(red[threadIdx.x], red[threadIdx.x + s]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
+    return red[0];
 }
 
+template <class T>
+__global__ void __launch_bounds__(256) absmax_blocks(StepArgs<T> A, int buf, float *partial)
+{
+    const float m = block_absmax(state_group(A, group_v(buf)), (long long)(A.nz + 1) * A.pitch,
+                                 blockIdx.x * 256LL + threadIdx.x, gridDim.x * 256LL);
+    if (threadIdx.x == 0) partial[blockIdx.x] = m;
+}
+
+// Of several members (blockIdx.y): checked one after the other, 64 members of 1201 x 1201 points cost
+// 128 launches and 64 read-backs after a batch run.
+template <class T>
+__global__ void __launch_bounds__(256) absmax_members(const FieldRange *ranges, float *partial)
+{
+    const FieldRange r = ranges[blockIdx.y];
+    const float m = block_absmax((const Vec4<T> *)r.v, r.n, blockIdx.x * 256LL + threadIdx.x, gridDim.x * 256LL);
+    if (threadIdx.x == 0) partial[blockIdx.y * gridDim.x + blockIdx.x] = m;
+}
+
+// 16-byte stores over the aligned middle of each range, single words at its ends.
+__global__ void __launch_bounds__(256) clear_kernel(ClearRanges r)
+{
+    const size_t first = blockIdx.x * 256ull + threadIdx.x, step = gridDim.x * 256ull;
+    for (int k = 0; k < kClearRanges; ++k) {
+        if (!r.words[k]) continue;
+        unsigned *const p = (unsigned *)r.p[k];
+        const size_t head = min((size_t)(4 - ((size_t)p / 4) % 4) % 4, r.words[k]), mid = (r.words[k] - head) / 4;
+        uint4 *const q = (uint4 *)(p + head);
+        for (size_t i = first; i < mid; i += step) q[i] = make_uint4(0, 0, 0, 0);
+        const size_t tail = head + 4 * mid;
+        if (first < head) p[first] = 0;
+        if (first < r.words[k] - tail) p[tail + first] = 0;
+    }
+}
+
+// 32 x 32 tiles through LDS, a row of 32 values per half wave on either side.
+template <class T>
+__global__ void __launch_bounds__(256) transpose_kernel(const T *in, int rows, int cols, T *out)
+{
+    __shared__ T tile[32][33];
+    const int c0 = blockIdx.x * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    for (int r0 = blockIdx.y * 32; r0 < rows; r0 += gridDim.y * 32) {
+        for (int y = ty; y < 32; y += 8)
+            if (r0 + y < rows && c0 + tx < cols) tile[y][tx] = in[(size_t)(r0 + y) * cols + c0 + tx];
+        __syncthreads();
+        for (int y = ty; y < 32; y += 8)
+            if (c0 + y < cols && r0 + tx < rows) out[(size_t)(c0 + y) * rows + r0 + tx] = tile[tx][y];
+        __syncthreads();
+    }
+}
+
+// out[b] = largest of in[b * n .. b * n + n).
 __global__ void __launch_bounds__(256) absmax_final(const float *in, int n, float *out)
 {
     __shared__ float red[256];
     float m = 0.f;
+    in += (size_t)blockIdx.x * n;
     for (int i = threadIdx.x; i < n; i += blockDim.x) m = fmaxf(m, in[i]);
     red[threadIdx.x] = m;
     __syncthreads();
@@ -110,7 +164,7 @@ __global__ void __launch_bounds__(256) absmax_final(const float *in, int n, floa
         if ((int)threadIdx.x < s) red[threadIdx.x] = fmaxf(red[threadIdx.x], red[threadIdx.x + s]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[0] = red[0];
+    if (threadIdx.x == 0) out[blockIdx.x] = red[0];
 }
 
 }  // namespace
@@ -146,6 +200,28 @@ void launch_absmax(const StepArgs<T> &A, int buf, float *partials, int nblocks, 
     absmax_final<<<1, 256, 0, stream>>>(partials, nblocks, result);
 }
 
+template <class T>
+void launch_absmax_members(const FieldRange *ranges, int n, float *partials, int nblocks, float *result, hipStream_t stream)
+{
+    absmax_members<T><<<dim3(nblocks, n), 256, 0, stream>>>(ranges, partials);
+    absmax_final<<<n, 256, 0, stream>>>(partials, nblocks, result);
+}
+
+void launch_clear(const ClearRanges &r, hipStream_t stream)
+{
+    size_t words = 0;
+    for (size_t w : r.words) words = std::max(words, w);
+    const int blocks = (int)std::min<size_t>(std::max<size_t>((words + 4095) / 4096, 1), 2048);
+    clear_kernel<<<blocks, 256, 0, stream>>>(r);
+}
+
+template <class T>
+void launch_transpose(const T *in, int rows, int cols, T *out, hipStream_t stream)
+{
+    const dim3 grid((cols + 31) / 32, std::min((rows + 31) / 32, 4096));
+    transpose_kernel<T><<<grid, 256, 0, stream>>>(in, rows, cols, out);
+}
+
 __global__ void __launch_bounds__(256) cn_palette_kernel(Vec4<float> *pal, int npal, float inv_dt)
 {
     const int e = (int)threadIdx.x;
@@ -168,7 +244,9 @@ void launch_cn_palette(Vec4<float> *pal, int npal, float inv_dt, hipStream_t str
     template void launch_derived<T>(const StepArgs<T> &, int, int, T *, hipStream_t);                 \
     template void launch_extract<T>(const StepArgs<T> &, int, int, T *, hipStream_t);                 \
     template void launch_insert<T>(const StepArgs<T> &, int, int, const T *, hipStream_t);            \
-    template void launch_absmax<T>(const StepArgs<T> &, int, float *, int, float *, hipStream_t);
+    template void launch_absmax<T>(const StepArgs<T> &, int, float *, int, float *, hipStream_t);         \
+    template void launch_absmax_members<T>(const FieldRange *, int, float *, int, float *, hipStream_t); \
+    template void launch_transpose<T>(const T *, int, int, T *, hipStream_t);
 POE2D_AUX_INSTANTIATE(float)
 POE2D_AUX_INSTANTIATE(double)
 #undef POE2D_AUX_INSTANTIATE

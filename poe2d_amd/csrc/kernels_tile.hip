@@ -439,7 +439,7 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
 template <class T, bool AVG, bool PAL, bool ROOM>
 __global__ void __launch_bounds__(kTileThreads, sizeof(T) == 4 && !ROOM ? 4 : 2)
     tile_steps(const StepArgs<T> *__restrict__ models, const TileItem *__restrict__ work, int nwork, int per_xcd,
-               const long long *__restrict__ base, int launch, int steps, int nst, int stream)
+               long long n, int flip, int steps, int nst, int stream)
 {
     __shared__ T bv[NBOUNDARY][kTileWaves][64], bs[NBOUNDARY][kTileWaves][64];
     __shared__ T xtab[NXTAB][64];
@@ -451,8 +451,7 @@ __global__ void __launch_bounds__(kTileThreads, sizeof(T) == 4 && !ROOM ? 4 : 2)
     // (fields are read where used: held from the start, a hundred of them would spill)
     const __attribute__((address_space(4))) StepArgs<T> &A =
         *((const __attribute__((address_space(4))) StepArgs<T> *)models + it.model);
-    const long long n = *(const kcll *)base + (long long)launch * steps;
-    const int in = (launch + A.pcur) & 1, halo = 3 * steps;
+    const int in = (flip + A.pcur) & 1, halo = 3 * steps;
     if constexpr (PAL) {
         typedef __attribute__((address_space(1))) nvec4<T> GN;
         const GN *const pal = (const GN *)A.pal;
@@ -470,7 +469,7 @@ __global__ void __launch_bounds__(kTileThreads, sizeof(T) == 4 && !ROOM ? 4 : 2)
 
 template <class T>
 hipError_t launch_tiles(const StepArgs<T> *models, const TileItem *work, int nwork, int per_xcd, bool palette, bool avg,
-                        const long long *base, int launch, int steps, int nst, bool stream_out, hipStream_t stream)
+                        long long n, int flip, int steps, int nst, bool stream_out, hipStream_t stream)
 {
     if (nwork < 1 || per_xcd < 1 || 8LL * per_xcd < nwork || steps < 2 || steps > kTileStepsMax || nst < 1 || nst > steps)
         return hipErrorInvalidValue;
@@ -479,10 +478,10 @@ hipError_t launch_tiles(const StepArgs<T> *models, const TileItem *work, int nwo
         const dim3 grid(8 * per_xcd);
         if (sizeof(T) == 8 || nwork <= kTileCus)
             tile_steps<T, AVG, PAL, true>
-                <<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, launch, steps, nst, stream_out);
+                <<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, n, flip, steps, nst, stream_out);
         else if constexpr (sizeof(T) == 4)
             tile_steps<T, AVG, PAL, false>
-                <<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, base, launch, steps, nst, stream_out);
+                <<<grid, kTileThreads, 0, stream>>>(models, work, nwork, per_xcd, n, flip, steps, nst, stream_out);
     };
     using Yes = std::true_type;
     using No = std::false_type;
@@ -491,9 +490,9 @@ hipError_t launch_tiles(const StepArgs<T> *models, const TileItem *work, int nwo
     return hipGetLastError();
 }
 
-template hipError_t launch_tiles<float>(const StepArgs<float> *, const TileItem *, int, int, bool, bool, const long long *, int,
-                                        int, int, bool, hipStream_t);
-template hipError_t launch_tiles<double>(const StepArgs<double> *, const TileItem *, int, int, bool, bool, const long long *,
-                                         int, int, int, bool, hipStream_t);
+template hipError_t launch_tiles<float>(const StepArgs<float> *, const TileItem *, int, int, bool, bool, long long, int, int,
+                                        int, bool, hipStream_t);
+template hipError_t launch_tiles<double>(const StepArgs<double> *, const TileItem *, int, int, bool, bool, long long, int, int,
+                                         int, bool, hipStream_t);
 
 }  // namespace poe2d

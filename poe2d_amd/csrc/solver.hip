@@ -49,7 +49,6 @@ const size_t kL2Bytes = size_t(32) << 20;   // the eight L2s together
 const size_t kMallBytes = size_t(256) << 20;  // the memory-side cache
 const int kTileSlots = 512;                 // tiles of the FP32 tile kernel the chip holds at once (half as many FP64)
 const int kBandTiles = 8;                   // tile columns to a band of the tile kernel's work order
-const int kGraphTileLaunches = 32;          // launches of the tile kernel per captured graph
 
 #define HIP_TRY(expr)                                                                              \
     do {                                                                                           \
@@ -133,13 +132,18 @@ struct Model {
 // graph (which holds those addresses, the item count and the kernel choice) is reused across runs;
 // the per-model arguments it points to are rewritten before every run.
 struct StepList {
+    // device arrays with their page-locked image on the host, filled and copied before every run: the
+    // step of launch 0 of the current chunk, the members' arguments, the work items, the receiver
+    // offsets and entries; and apart from them (a captured graph holds their addresses, and only the
+    // source samples grow with the steps of a run) the members' source samples
+    struct Staged {
+        void *dev = nullptr;
+        char *image = nullptr;
+        size_t cap = 0;
+    } arena, source;
     void *models = nullptr;      // StepArgs<T>[nmodels]
     void *work = nullptr;        // WorkItem[nwork], or TileItem[nwork] (tile kernel)
-    int *rec_ptr = nullptr;      // receiver offsets per (row, tile column), all models
-    int2 *rec_ent = nullptr;     // receiver entries, all models
-    long long *base = nullptr;   // step of launch 0 of the current chunk
-    long long *h_base = nullptr; // pinned host staging of base
-    size_t cap_models = 0, cap_work = 0, cap_ptr = 0, cap_ent = 0;
+    long long *base = nullptr;
     int nmodels = 0, nwork = 0, per_xcd = 0, bw = 0;
     bool palette = false;
     bool avg = false;  // POE2D_MATERIAL_AVERAGED (all members alike)
@@ -176,27 +180,15 @@ struct StepList {
     {
         if (exec) (void)hipGraphExecDestroy(exec);
         exec = nullptr;
-        dev_free(models);
-        dev_free(work);
-        void *q = rec_ptr; dev_free(q); rec_ptr = nullptr;
-        q = rec_ent; dev_free(q); rec_ent = nullptr;
-        q = base; dev_free(q); base = nullptr;
-        if (h_base) (void)hipHostFree(h_base);
-        h_base = nullptr;
-        cap_models = cap_work = cap_ptr = cap_ent = 0;
+        for (Staged *b : {&arena, &source}) {
+            dev_free(b->dev);
+            if (b->image) (void)hipHostFree(b->image);
+            *b = Staged{};
+        }
+        models = work = nullptr;
+        base = nullptr;
     }
 };
-
-poe2d_status grow(void **p, size_t *cap, size_t bytes)
-{
-    if (bytes <= *cap && *p) return POE2D_OK;
-    dev_free(*p);
-    *cap = 0;
-    poe2d_status st = dev_alloc(p, bytes);
-    if (st) return st;
-    *cap = bytes;
-    return POE2D_OK;
-}
 
 }  // namespace
 
@@ -215,10 +207,6 @@ struct poe2d_solver {
     float *red = nullptr;   // reduction scratch: [0] result, [1..] per-block partials
     int red_blocks = 1024;
     void *dense = nullptr;  // (nz+1) x (nx+1) scratch for snapshots, made on first use
-    void *src_dev = nullptr;  // source series of the current run
-    size_t src_cap = 0;
-    long long src_n0 = 0;
-    int src_len = 0;
     // schedule
     int schedule = SCHED_FUSED2;
     int block_w = 256, tile_rows = 14;
@@ -236,6 +224,7 @@ struct poe2d_solver {
     int *rix = nullptr, *riz = nullptr;
     std::vector<int> hrx, hrz;  // their host copies
     void *traces = nullptr;  // [slot][comp][rec]
+    void *traces_out = nullptr;  // [comp][rec][slot], made when they are first read
     int step = 0;
     double last_ms = 0;
     int last_steps = 0;
@@ -267,6 +256,7 @@ struct poe2d_batch {
     bool graphs = true;
     double last_ms = 0;
     int last_steps = 0;
+    void *check = nullptr;  // the stability checks' arguments, partial and final results
     StepList list;   // single-step launches
     StepList list2;  // two-step launches
 };
@@ -291,8 +281,8 @@ void free_handle(poe2d_solver *s)
     q = s->rix; dev_free(q); s->rix = nullptr;
     q = s->riz; dev_free(q); s->riz = nullptr;
     dev_free(s->traces);
+    dev_free(s->traces_out);
     dev_free(s->dense);
-    dev_free(s->src_dev);
     if (s->ev0) (void)hipEventDestroy(s->ev0);
     if (s->ev1) (void)hipEventDestroy(s->ev1);
     if (s->stream) (void)hipStreamDestroy(s->stream);
@@ -514,9 +504,6 @@ StepArgs<T> step_args(const poe2d_solver *s, int in, int out, int bw, int th, bo
     A.src_x = s->have_src ? s->src.ix : -1;
     A.src_z = s->have_src ? s->src.iz : -1;
     A.src_val = T(0);
-    A.src_series = (const T *)s->src_dev;
-    A.src_n0 = s->src_n0;
-    A.src_len = s->src_len;
     // step n = s->step reads state buffer cur
     A.par = (int)(((long long)s->cur - s->step) & 1);
     A.th = th;
@@ -536,60 +523,74 @@ StepArgs<T> step_args(const poe2d_solver *s, int in, int out)
     return step_args<T>(s, in, out, s->block_w, s->tile_rows);
 }
 
-// Source samples of steps [n0, n0 + k) into the handle's device series.
-template <class T>
-poe2d_status upload_source(poe2d_solver *s, long long n0, int k)
+// Room for `bytes` on both sides of b (contents lost when it grows).
+poe2d_status grow(StepList::Staged &b, size_t bytes)
 {
-    poe2d_status st = grow(&s->src_dev, &s->src_cap, (size_t)std::max(k, 1) * sizeof(T));
+    if (bytes <= b.cap) return POE2D_OK;
+    dev_free(b.dev);
+    if (b.image) (void)hipHostFree(b.image);
+    b = StepList::Staged{};
+    poe2d_status st = dev_alloc(&b.dev, bytes);
     if (st) return st;
-    std::vector<T> h(std::max(k, 1), T(0));
-    for (int i = 0; i < k; ++i) h[i] = (T)s->source_value(n0 + i);
-    HIP_TRY(hipStreamSynchronize(s->stream));
-    HIP_TRY(hipMemcpy(s->src_dev, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
-    s->src_n0 = n0;
-    s->src_len = k;
-    return POE2D_OK;
-}
-
-// Device copies of a list's arrays: work items, receiver offsets and entries, and the members'
-// arguments once `fix` has pointed each at its receivers.  Waits for `stream` first.
-template <class T, class F>
-poe2d_status upload_list(StepList &L, std::vector<StepArgs<T>> &args, const void *work, size_t work_bytes,
-                         const std::vector<int> &ptr, const int2 *ent, size_t nent, hipStream_t stream, F fix)
-{
-    poe2d_status st;
-    HIP_TRY(hipStreamSynchronize(stream));
-    if ((st = grow(&L.models, &L.cap_models, args.size() * sizeof(StepArgs<T>)))) return st;
-    if ((st = grow(&L.work, &L.cap_work, work_bytes))) return st;
-    void *pp = L.rec_ptr;
-    st = grow(&pp, &L.cap_ptr, std::max<size_t>(ptr.size(), 1) * sizeof(int));
-    L.rec_ptr = (int *)pp;
-    if (st) return st;
-    void *pe = L.rec_ent;
-    st = grow(&pe, &L.cap_ent, std::max<size_t>(nent, 1) * sizeof(int2));
-    L.rec_ent = (int2 *)pe;
-    if (st) return st;
-    for (size_t i = 0; i < args.size(); ++i) fix(args[i], (int)i);
-    if (!L.base) {
-        void *q = nullptr;
-        if ((st = dev_alloc(&q, sizeof(long long)))) return st;
-        L.base = (long long *)q;
+    if (hipHostMalloc((void **)&b.image, bytes, hipHostMallocDefault) != hipSuccess) {
+        b.image = nullptr;
+        return fail(POE2D_E_NOMEM, "run: page-locked host memory");
     }
-    if (!L.h_base) HIP_TRY(hipHostMalloc((void **)&L.h_base, sizeof(long long), hipHostMallocDefault));
-    HIP_TRY(hipMemcpy(L.models, args.data(), args.size() * sizeof(StepArgs<T>), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(L.work, work, work_bytes, hipMemcpyHostToDevice));
-    if (!ptr.empty()) HIP_TRY(hipMemcpy(L.rec_ptr, ptr.data(), ptr.size() * sizeof(int), hipMemcpyHostToDevice));
-    if (nent) HIP_TRY(hipMemcpy(L.rec_ent, ent, nent * sizeof(int2), hipMemcpyHostToDevice));
+    b.cap = bytes;
     return POE2D_OK;
 }
 
-// Fill `L` for the members (all at the same step, current source series uploaded): per-member
+// Device copies of a list's arrays: the first step n0, work items, receiver offsets
+// and entries (member i's ptr_off[i] and ent_off[i] on), the members' source samples of steps [n0, n0 +
+// nsteps), and the members' arguments pointing at them.
+template <class T>
+poe2d_status upload_list(StepList &L, const std::vector<poe2d_solver *> &members, std::vector<StepArgs<T>> &args,
+                         const void *work, size_t work_bytes, const std::vector<int> &ptr, const std::vector<int2> &ent,
+                         const size_t *ptr_off, const size_t *ent_off, long long n0, int nsteps, hipStream_t stream)
+{
+    const size_t nm = args.size();
+    size_t at = 0;
+    auto section = [&](size_t bytes) {
+        const size_t o = at;
+        at += (bytes + 255) / 256 * 256;
+        return o;
+    };
+    const size_t o_base = section(sizeof(long long)), o_models = section(nm * sizeof(StepArgs<T>));
+    const size_t o_work = section(work_bytes), o_ptr = section(ptr.size() * sizeof(int));
+    const size_t o_ent = section(ent.size() * sizeof(int2)), src_bytes = std::max<size_t>(nm * nsteps, 1) * sizeof(T);
+    HIP_TRY(hipStreamSynchronize(stream));  // (the images' last copies, and launches on the old arrays)
+    poe2d_status st;
+    if ((st = grow(L.arena, at)) || (st = grow(L.source, src_bytes))) return st;
+    char *const dev = (char *)L.arena.dev, *const image = L.arena.image;
+    *(long long *)(image + o_base) = n0;
+    std::memcpy(image + o_work, work, work_bytes);
+    if (!ptr.empty()) std::memcpy(image + o_ptr, ptr.data(), ptr.size() * sizeof(int));
+    if (!ent.empty()) std::memcpy(image + o_ent, ent.data(), ent.size() * sizeof(int2));
+    T *const src = (T *)L.source.image;
+    for (size_t i = 0; i < nm; ++i) {
+        for (int k = 0; k < nsteps; ++k) src[i * nsteps + k] = (T)members[i]->source_value(n0 + k);
+        args[i].src_series = (const T *)L.source.dev + i * nsteps;
+        args[i].src_n0 = n0;
+        args[i].src_len = nsteps;
+        args[i].rec_tile_ptr = (const int *)(dev + o_ptr) + (ptr_off ? ptr_off[i] : 0);
+        args[i].rec_entries = (const int2 *)(dev + o_ent) + (ent_off ? ent_off[i] : 0);
+    }
+    std::memcpy(image + o_models, args.data(), nm * sizeof(StepArgs<T>));
+    HIP_TRY(hipMemcpyAsync(L.arena.dev, image, at, hipMemcpyHostToDevice, stream));
+    HIP_TRY(hipMemcpyAsync(L.source.dev, src, src_bytes, hipMemcpyHostToDevice, stream));
+    L.base = (long long *)(dev + o_base);
+    L.models = dev + o_models;
+    L.work = dev + o_work;
+    return POE2D_OK;
+}
+
+// Fill `L` for nsteps steps from step n0 of the members (all at the same step): per-member
 // arguments, the (member, tile) work list with block width bw and tile height th, and each
 // member's receivers sorted by row and column with their offsets per (row, tile column).  The
 // uploads wait for `stream` first.
 template <class T>
 poe2d_status build_list(StepList &L, const std::vector<poe2d_solver *> &members, int bw, int th, bool palette,
-                        hipStream_t stream, bool two = false, int par_shift = 0)
+                        long long n0, int nsteps, hipStream_t stream, bool two = false, int par_shift = 0)
 {
     const int nm = (int)members.size();
     const int material = members[0]->grid.staggered_material;
@@ -677,11 +678,8 @@ poe2d_status build_list(StepList &L, const std::vector<poe2d_solver *> &members,
             for (size_t q = (size_t)x * ni; q < std::min(inter.size(), (size_t)(x + 1) * ni); ++q) work[o++] = inter[q];
         }
     }
-    const poe2d_status st = upload_list<T>(L, args, work.data(), work.size() * sizeof(WorkItem), ptr, ent.data(),
-                                           ent.size(), stream, [&](StepArgs<T> &A, int i) {
-                                               A.rec_tile_ptr = L.rec_ptr + ptr_off[i];
-                                               A.rec_entries = L.rec_ent + ent_off[i];
-                                           });
+    const poe2d_status st = upload_list<T>(L, members, args, work.data(), work.size() * sizeof(WorkItem), ptr, ent,
+                                           ptr_off.data(), ent_off.data(), n0, nsteps, stream);
     if (st) return st;
     L.nmodels = nm;
     L.nint = two ? nint : (int)work.size();
@@ -750,7 +748,7 @@ void cut_tiles(const poe2d_solver *s, int i, int steps, int tall_rows, std::vect
 // 20.0 / 16.9, 2001^2 40.4 / 36.1, FP64 401^2 10.5 / 8.8).
 template <class T>
 poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members, int steps, bool tall, bool palette,
-                         hipStream_t stream)
+                         int nsteps, hipStream_t stream)
 {
     const int nm = (int)members.size();
     const int material = members[0]->grid.staggered_material;
@@ -803,11 +801,8 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
         for (size_t e = x; e < edge.size(); e += 8) work[o++] = edge[e];
         for (size_t q = (size_t)x * ni; q < std::min(inter.size(), (size_t)(x + 1) * ni); ++q) work[o++] = inter[q];
     }
-    const poe2d_status st = upload_list<T>(L, args, work.data(), work.size() * sizeof(TileItem), ptr, ent.data(),
-                                           ent.size(), stream, [&](StepArgs<T> &A, int) {
-                                               A.rec_tile_ptr = L.rec_ptr;
-                                               A.rec_entries = L.rec_ent;
-                                           });
+    const poe2d_status st = upload_list<T>(L, members, args, work.data(), work.size() * sizeof(TileItem), ptr, ent, nullptr,
+                                           nullptr, members[0]->step, nsteps, stream);
     if (st) return st;
     L.nmodels = nm;
     L.nint = (int)inter.size();
@@ -838,14 +833,6 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
 template <class T>
 hipError_t launch_list_chunk(const StepList &L, int count, hipStream_t stream)
 {
-    if (L.tiles) {
-        for (int k = 0; k < count; ++k) {
-            const hipError_t e = launch_tiles<T>((const StepArgs<T> *)L.models, (const TileItem *)L.work, L.nwork, L.per_xcd,
-                                                 L.palette, L.avg, L.base, k, L.steps, L.steps, L.stream_out, stream);
-            if (e != hipSuccess) return e;
-        }
-        return launch_base_advance(L.base, L.steps * count, stream);
-    }
     if (L.two) {
         if constexpr (sizeof(T) == 4) {
             for (int k = 0; k < count; ++k) {
@@ -865,16 +852,13 @@ hipError_t launch_list_chunk(const StepList &L, int count, hipStream_t stream)
     return launch_base_advance(L.base, count, stream);
 }
 
-// k launches of list L from step n0 on `stream` (k steps, or k step pairs): graph replays of
+// k launches of list L, as it was filled, on `stream` (k steps, or k step pairs): graph replays of
 // kGraphSteps steps, the remainder launched directly.
 template <class T>
-poe2d_status run_list(StepList &L, long long n0, int k, bool graphs, hipStream_t stream)
+poe2d_status run_list(StepList &L, int k, bool graphs, hipStream_t stream)
 {
-    *L.h_base = n0;
-    HIP_TRY(hipMemcpyAsync(L.base, L.h_base, sizeof(long long), hipMemcpyHostToDevice, stream));
     int done = 0;
-    // (the tile kernel's state buffers alternate by launch within a chunk: an even number of launches)
-    const int chunk = L.tiles ? kGraphTileLaunches : L.two ? kGraphSteps / 2 : kGraphSteps;
+    const int chunk = L.two ? kGraphSteps / 2 : kGraphSteps;
     if (graphs && k >= chunk) {
         const StepList::Sig sig = L.signature();
         if (!L.exec || !(L.sig == sig)) {
@@ -903,33 +887,24 @@ poe2d_status run_list(StepList &L, long long n0, int k, bool graphs, hipStream_t
     return POE2D_OK;
 }
 
-// nsteps steps of the members (all at step n0) on the tile kernel: launches of L.steps steps, and one
-// of the remainder.  *flips = launches, the times the state changed buffers.
+// nsteps steps of the members L was filled for (from step n0) on the tile kernel: launches of L.steps
+// steps, the last of the remainder.  Launched directly, the step by value: a launch takes the host
+// less time than the GPU even on the smallest grids, and replayed graphs were never faster (161^2 4.84
+// us per step in graphs of 32 launches, 4.82 direct; 2001^2 35.0, 34.9).  *flips = launches, the times
+// the state changed buffers.
 template <class T>
-poe2d_status run_tiles(StepList &L, long long n0, int nsteps, bool graphs, hipStream_t stream, int *flips)
+poe2d_status run_tiles(StepList &L, long long n0, int nsteps, hipStream_t stream, int *flips)
 {
-    poe2d_status st;
-    const int full = nsteps / L.steps, rest = nsteps % L.steps;
-    if ((st = run_list<T>(L, n0, full, graphs, stream))) return st;
-    if (rest) {
-        // (the counter is past the full launches; an odd number of them leaves the state in the other buffer)
-        HIP_TRY(launch_base_advance(L.base, -(full & 1) * L.steps, stream));
+    *flips = 0;
+    for (int done = 0; done < nsteps; done += L.steps, ++*flips)
         HIP_TRY(launch_tiles<T>((const StepArgs<T> *)L.models, (const TileItem *)L.work, L.nwork, L.per_xcd, L.palette, L.avg,
-                                L.base, full & 1, L.steps, rest, L.stream_out, stream));
-    }
-    *flips = full + (rest > 0);
+                                n0 + done, *flips & 1, L.steps, std::min(L.steps, nsteps - done), L.stream_out, stream));
     return POE2D_OK;
 }
 
-// Largest |v| of the handle's current state; POE2D_E_UNSTABLE above the reference's threshold.
-template <class T>
-poe2d_status stability_check(poe2d_solver *s)
+// POE2D_E_UNSTABLE when the largest |v| of handle s's state is above the reference's threshold.
+poe2d_status stability_check(const poe2d_solver *s, float vmax)
 {
-    StepArgs<T> A = step_args<T>(s, s->cur, s->cur);
-    launch_absmax<T>(A, s->cur, s->red + 1, s->red_blocks, s->red, s->stream);
-    float vmax = 0.f;
-    HIP_TRY(hipMemcpyAsync(&vmax, s->red, sizeof(float), hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipStreamSynchronize(s->stream));
     if (!(vmax <= kStabilityThreshold))
         return fail(POE2D_E_UNSTABLE, "run: wavefield became unstable (max |v| = " + std::to_string(vmax) +
                                           ") by step " + std::to_string(s->step));
@@ -1009,11 +984,10 @@ poe2d_status run_steps(poe2d_solver *s, int nsteps)
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipEventRecord(s->ev1, s->stream));
     } else if (const TileShape shape = tile_shape({s}, s->auto_shape, s->block_w, s->tile_rows); shape.tiles) {
-        if ((st = upload_source<T>(s, s->step, nsteps))) return st;
-        if ((st = build_tiles<T>(s->list2, {s}, shape.steps, shape.tall, s->m->npal > 0, s->stream))) return st;
+        if ((st = build_tiles<T>(s->list2, {s}, shape.steps, shape.tall, s->m->npal > 0, nsteps, s->stream))) return st;
         int flips = 0;
         HIP_TRY(hipEventRecord(s->ev0, s->stream));
-        if ((st = run_tiles<T>(s->list2, s->step, nsteps, s->graphs, s->stream, &flips))) return st;
+        if ((st = run_tiles<T>(s->list2, s->step, nsteps, s->stream, &flips))) return st;
         HIP_TRY(hipEventRecord(s->ev1, s->stream));
         s->cur = (s->cur + flips) & 1;
     } else if (sizeof(T) == 4 && two_step_kernel(s)) {
@@ -1021,34 +995,36 @@ poe2d_status run_steps(poe2d_solver *s, int nsteps)
         const int pairs = nsteps / 2, rem = nsteps & 1;
         if (!s->psi_mid && (st = dev_alloc(&s->psi_mid, std::max<size_t>(s->m->psi_half_elems(), 1) * s->rs)))
             return st;
-        if ((st = upload_source<T>(s, s->step, nsteps))) return st;
-        if (pairs && (st = build_list<T>(s->list2, {s}, shape.bw, shape.th, two_step_palette(s), s->stream, true)))
+        if (pairs && (st = build_list<T>(s->list2, {s}, shape.bw, shape.th, two_step_palette(s), s->step, nsteps, s->stream, true)))
             return st;
         // (the single-step kernel reads the palette whenever the grid has one, which may be larger
         // than the two-step kernel's)
-        if (rem && (st = build_list<T>(s->list, {s}, shape.bw, shape.th, s->m->npal > 0, s->stream, false, pairs)))
+        if (rem && (st = build_list<T>(s->list, {s}, shape.bw, shape.th, s->m->npal > 0, s->step + 2LL * pairs, 1,
+                                       s->stream, false, pairs)))
             return st;
         HIP_TRY(hipEventRecord(s->ev0, s->stream));
-        if (pairs && (st = run_list<T>(s->list2, s->step, pairs, s->graphs, s->stream))) return st;
-        if (rem && (st = run_list<T>(s->list, s->step + 2LL * pairs, 1, s->graphs, s->stream))) return st;
+        if (pairs && (st = run_list<T>(s->list2, pairs, s->graphs, s->stream))) return st;
+        if (rem && (st = run_list<T>(s->list, 1, s->graphs, s->stream))) return st;
         HIP_TRY(hipEventRecord(s->ev1, s->stream));
         s->cur = (s->cur + pairs + rem) & 1;
     } else {
-        if ((st = upload_source<T>(s, s->step, nsteps))) return st;
         const bool palette = (s->schedule == SCHED_FUSED || s->schedule == SCHED_FUSED2) && s->m->npal > 0;
-        if ((st = build_list<T>(s->list, {s}, shape.bw, shape.th, palette, s->stream))) return st;
+        if ((st = build_list<T>(s->list, {s}, shape.bw, shape.th, palette, s->step, nsteps, s->stream))) return st;
         HIP_TRY(hipEventRecord(s->ev0, s->stream));
-        if ((st = run_list<T>(s->list, s->step, nsteps, s->graphs, s->stream))) return st;
+        if ((st = run_list<T>(s->list, nsteps, s->graphs, s->stream))) return st;
         HIP_TRY(hipEventRecord(s->ev1, s->stream));
         s->cur = (s->cur + nsteps) & 1;
     }
-    HIP_TRY(hipEventSynchronize(s->ev1));
+    float vmax = 0.f;
+    launch_absmax<T>(step_args<T>(s, s->cur, s->cur), s->cur, s->red + 1, s->red_blocks, s->red, s->stream);
+    HIP_TRY(hipMemcpyAsync(&vmax, s->red, sizeof(float), hipMemcpyDeviceToHost, s->stream));
+    HIP_TRY(hipStreamSynchronize(s->stream));
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, s->ev0, s->ev1));
     s->last_ms = ms;
     s->last_steps = nsteps;
     s->step += nsteps;
-    return stability_check<T>(s);
+    return stability_check(s, vmax);
 }
 
 // One field of the current state (or p / sxx / syy recomputed from it) to the host.
@@ -1146,8 +1122,6 @@ poe2d_status batch_run_steps(poe2d_batch *b, int nsteps)
     const long long n0 = b->members[0]->step;
     bool palette = true, two = sizeof(T) == 4, palette2 = true, tile_palette = true;
     for (poe2d_solver *s : b->members) {
-        poe2d_status st = upload_source<T>(s, n0, nsteps);
-        if (st) return st;
         palette = palette && (s->schedule == SCHED_FUSED || s->schedule == SCHED_FUSED2) && s->m->npal > 0;
         two = two && two_step_kernel(s);
         palette2 = palette2 && two_step_palette(s);
@@ -1162,36 +1136,53 @@ poe2d_status batch_run_steps(poe2d_batch *b, int nsteps)
     int flips = pairs + rem;
     poe2d_status st;
     if (shape.tiles) {
-        if ((st = build_tiles<T>(b->list2, b->members, shape.steps, shape.tall, tile_palette, b->stream))) return st;
+        if ((st = build_tiles<T>(b->list2, b->members, shape.steps, shape.tall, tile_palette, nsteps, b->stream))) return st;
     } else if (pairs) {
         for (poe2d_solver *s : b->members)
             if (!s->psi_mid && (st = dev_alloc(&s->psi_mid, std::max<size_t>(s->m->psi_half_elems(), 1) * s->rs)))
                 return st;
-        if ((st = build_list<T>(b->list2, b->members, shape.bw, shape.th, palette2, b->stream, true))) return st;
+        if ((st = build_list<T>(b->list2, b->members, shape.bw, shape.th, palette2, n0, nsteps, b->stream, true))) return st;
     }
     if (rem && !shape.tiles &&
-        (st = build_list<T>(b->list, b->members, std::max(shape.bw, 128), shape.th, palette, b->stream, false, pairs)))
+        (st = build_list<T>(b->list, b->members, std::max(shape.bw, 128), shape.th, palette, n0 + 2LL * pairs, rem, b->stream,
+                             false, pairs)))
         return st;
     HIP_TRY(hipEventRecord(b->ev0, b->stream));
     if (shape.tiles) {
-        if ((st = run_tiles<T>(b->list2, n0, nsteps, b->graphs, b->stream, &flips))) return st;
+        if ((st = run_tiles<T>(b->list2, n0, nsteps, b->stream, &flips))) return st;
     } else {
-        if (pairs && (st = run_list<T>(b->list2, n0, pairs, b->graphs, b->stream))) return st;
-        if (rem && (st = run_list<T>(b->list, n0 + 2LL * pairs, rem, b->graphs, b->stream))) return st;
+        if (pairs && (st = run_list<T>(b->list2, pairs, b->graphs, b->stream))) return st;
+        if (rem && (st = run_list<T>(b->list, rem, b->graphs, b->stream))) return st;
     }
     HIP_TRY(hipEventRecord(b->ev1, b->stream));
-    HIP_TRY(hipEventSynchronize(b->ev1));
+    // the stability checks of all members, in one launch
+    const int nm = (int)b->members.size(), blocks = std::min(1024, std::max(8, 4096 / nm));
+    std::vector<FieldRange> ranges(nm);
+    std::vector<float> vmax(nm, 0.f);
+    for (int i = 0; i < nm; ++i) {
+        poe2d_solver *s = b->members[i];
+        s->cur = (s->cur + flips) & 1;
+        ranges[i] = {s->group_ptr(group_v(s->cur)) + s->m->origin() * 4 * sizeof(T),
+                     (long long)(s->grid.nz + 1) * (long long)s->m->pitch};
+    }
+    const size_t range_bytes = (nm * sizeof(FieldRange) + 255) / 256 * 256;
+    if (!b->check && (st = dev_alloc(&b->check, range_bytes + (size_t)nm * (blocks + 1) * sizeof(float)))) return st;
+    float *const result = (float *)((char *)b->check + range_bytes);
+    HIP_TRY(hipMemcpyAsync(b->check, ranges.data(), nm * sizeof(FieldRange), hipMemcpyHostToDevice, b->stream));
+    launch_absmax_members<T>((const FieldRange *)b->check, nm, result + nm, blocks, result, b->stream);
+    HIP_TRY(hipMemcpyAsync(vmax.data(), result, nm * sizeof(float), hipMemcpyDeviceToHost, b->stream));
+    HIP_TRY(hipStreamSynchronize(b->stream));
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, b->ev0, b->ev1));
     b->last_ms = ms;
     b->last_steps = nsteps;
     poe2d_status first = POE2D_OK;
-    for (poe2d_solver *s : b->members) {
-        s->cur = (s->cur + flips) & 1;
+    for (int i = 0; i < nm; ++i) {
+        poe2d_solver *s = b->members[i];
         s->step += nsteps;
         s->last_ms = ms;
         s->last_steps = nsteps;
-        const poe2d_status c = stability_check<T>(s);
+        const poe2d_status c = stability_check(s, vmax[i]);
         if (c && !first) first = c;
     }
     return first;
@@ -1426,6 +1417,7 @@ poe2d_status poe2d_set_receivers(poe2d_solver *s, const poe2d_receivers *r)
     void *q = s->rix; dev_free(q); s->rix = nullptr;
     q = s->riz; dev_free(q); s->riz = nullptr;
     dev_free(s->traces);
+    dev_free(s->traces_out);
     s->nrec = r->n;
     s->mask = r->comp_mask;
     s->ncomp = ((r->comp_mask & 1) != 0) + ((r->comp_mask & 2) != 0) + ((r->comp_mask & 4) != 0);
@@ -1477,17 +1469,15 @@ poe2d_status poe2d_seismograms(poe2d_solver *s, void *out, size_t bytes)
     const size_t need = s->trace_bytes();
     if (bytes < need) return fail(POE2D_E_INVALID, "seismograms: output buffer too small");
     if (need == 0) return POE2D_OK;
-    std::vector<unsigned char> tmp(need);
+    // device layout [slot][comp][rec] -> caller layout [comp][rec][slot], transposed on the device
+    if (!s->traces_out && (st = dev_alloc(&s->traces_out, need))) return st;
+    if (s->precision == POE2D_F32)
+        launch_transpose<float>((const float *)s->traces, s->nsamp, s->ncomp * s->nrec, (float *)s->traces_out, s->stream);
+    else
+        launch_transpose<double>((const double *)s->traces, s->nsamp, s->ncomp * s->nrec, (double *)s->traces_out, s->stream);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(out, s->traces_out, need, hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    HIP_TRY(hipMemcpy(tmp.data(), s->traces, need, hipMemcpyDeviceToHost));
-    // device layout [slot][comp][rec] -> caller layout [comp][rec][slot]
-    const size_t rs = s->rs;
-    unsigned char *o = (unsigned char *)out;
-    for (int k = 0; k < s->nsamp; ++k)
-        for (int c = 0; c < s->ncomp; ++c)
-            for (int r = 0; r < s->nrec; ++r)
-                std::memcpy(o + (((size_t)c * s->nrec + r) * s->nsamp + k) * rs,
-                            tmp.data() + (((size_t)k * s->ncomp + c) * s->nrec + r) * rs, rs);
     return POE2D_OK;
 }
 
@@ -1589,9 +1579,15 @@ poe2d_status poe2d_reset(poe2d_solver *s)
 {
     poe2d_status st = check_handle(s);
     if (st) return st;
-    HIP_TRY(hipMemsetAsync(s->arena, 0, NSTATE_GROUPS * s->group_bytes(), s->stream));
-    HIP_TRY(hipMemsetAsync(s->psi, 0, 2 * s->m->psi_half_elems() * s->rs, s->stream));
-    if (s->traces) HIP_TRY(hipMemsetAsync(s->traces, 0, s->trace_bytes(), s->stream));
+    // the buffer the next step reads: a step writes every grid point of the other one, whose pads (and
+    // whose memory variables no update reaches) stay zero from the start
+    const Model *md = s->m;
+    unsigned char *const psi = (unsigned char *)s->psi;
+    launch_clear({{s->group_ptr(group_v(0)), s->group_ptr(group_s(0)), psi, psi + 2 * NPSI_X * md->pxn() * s->rs, s->traces},
+                  {s->group_bytes() / 4, s->group_bytes() / 4, NPSI_X * md->pxn() * s->rs / 4, NPSI_Z * md->pzn() * s->rs / 4,
+                   s->traces ? s->trace_bytes() / 4 : 0}},
+                 s->stream);
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s->stream));
     s->step = 0;
     s->cur = 0;
@@ -1855,6 +1851,7 @@ void poe2d_batch_destroy(poe2d_batch *b)
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     b->list.release();
     b->list2.release();
+    dev_free(b->check);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
     if (b->stream) (void)hipStreamDestroy(b->stream);

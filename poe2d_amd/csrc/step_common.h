@@ -356,11 +356,10 @@ __host__ __device__ constexpr int tile_rows(int p, int steps) { return 8 * p - 2
 struct TileItem {
     int model, x0, z0, z1, kind, rec;
 };
-// nst <= steps steps from step n = *base + launch * steps; reads state buffer (launch + pcur) & 1 and
-// writes the other, past the caches with stream_out.
+// nst <= steps steps from step n; reads state buffer (flip + pcur) & 1 and writes the other, past the
+// caches with stream_out.
 template <class T>
 hipError_t launch_tiles(const StepArgs<T> *models, const TileItem *work, int nwork, int per_xcd, bool palette, bool avg,
-                        const long long *base, int launch, int steps, int nst, bool stream_out,
-                        hipStream_t stream);
+                        long long n, int flip, int steps, int nst, bool stream_out, hipStream_t stream);
 
 }  // namespace poe2d

@@ -218,9 +218,9 @@ class SolverPool:
 
     def batch(self, k):
         """The batch of the first k members.  On first use it is made, its tile shape autotuned and
-        its step graph captured by a warm-up run (the members are reset afterwards): nothing else
-        may use the GPU from another thread meanwhile, as HIP refuses other threads' calls while a
-        stream captures.  Later runs replay the graph."""
+        (where a kernel replayed from a graph is the fastest) its step graph captured by a warm-up run
+        (the members are reset afterwards): nothing else may use the GPU from another thread
+        meanwhile, as HIP refuses other threads' calls while a stream captures."""
         if k not in self.batches:
             b = Batch(self.solvers[:k])
             self.batches[k] = b

@@ -84,3 +84,44 @@ def test_ragged_fp64_batch_on_tiles():
             assert np.array_equal(s.seismograms(), ref)
     for s in solvers:
         s.close()
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+def test_reset_after_a_run_starts_from_zero(precision):
+    # reset clears the buffer the next step reads; a run after it equals a new handle's, whichever
+    # buffer the earlier run ended in and whichever kernel ran before
+    prob = _problem(104, 131, 10, 2)
+    ref = None
+    for before in (None, (3, 64, 36), (0, 256, 14), (1, 256, 14)):
+        with Solver(prob, precision=precision) as s:
+            if before:
+                s.set_schedule(*before)
+                s.set_field("vx", np.ones((prob.nz + 1, prob.nx + 1)) * 1e-6)
+                s.run(5)
+                s.reset()
+                s.set_schedule(3, 64, 36)
+            s.run(9)
+            got = s.seismograms(), {f: s.snapshot(f) for f in STATE}, s.checkpoint()
+        if ref is None:
+            ref = got
+        _same(got, ref, f"after {before}")
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (3, 2), (33, 31), (64, 65), (5, 1000)])
+def test_traces_keep_their_order(shape):
+    # (samples, receivers) around the transposing kernel's 32 x 32 tiles: trace k of receiver r is
+    # what a snapshot holds at its point
+    nt, nrec = shape
+    rng = np.random.default_rng(nt)
+    prob = _problem(104, 131, 10, 2)
+    prob.receivers = ReceiverSpec(ix=rng.integers(0, 105, nrec), iz=rng.integers(0, 132, nrec), comp_mask=_abi.VX | _abi.P)
+    prob.nt = nt
+    with Solver(prob) as s:
+        s.set_field("vx", rng.standard_normal((132, 105)) * 1e-6)
+        snaps = []
+        for _ in range(nt):
+            snaps.append(s.snapshot("vx")[prob.receivers.iz, prob.receivers.ix])
+            s.run(1)
+        g = s.seismograms()
+    assert g.shape == (2, nrec, nt)
+    assert np.array_equal(g[0], np.stack(snaps, axis=1))
