@@ -69,8 +69,11 @@ poe2d_status dmalloc(P **p, size_t count)
     if (e != hipSuccess)
         return fail(e == hipErrorOutOfMemory ? POE2D_E_NOMEM : POE2D_E_HIP,
                     std::string("hipMalloc: ") + hipGetErrorString(e));
-    HIP_TRY(hipMemset(q, 0, std::max<size_t>(count * sizeof(P), 1)));
     *p = (P *)q;
+    // (the fill runs on the null stream, which the networks' own streams do not wait for: what they
+    // write first could otherwise be cleared after it)
+    HIP_TRY(hipMemset(q, 0, std::max<size_t>(count * sizeof(P), 1)));
+    HIP_TRY(hipStreamSynchronize(nullptr));
     return POE2D_OK;
 }
 

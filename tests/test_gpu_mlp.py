@@ -242,6 +242,20 @@ def test_train_many_equals_training_one_member_at_a_time():
             assert np.array_equal(wa, wb) and np.array_equal(ba, bb)
 
 
+def test_settings_made_right_after_creation_hold():
+    """Factors set while a new network's arrays may still be being cleared (512 MB of partials here)
+    are not cleared with them."""
+    rng = np.random.default_rng(4)
+    x = rng.standard_normal((37, 4)).astype(np.float32)
+    for seed in range(3):
+        with Network([4, 1024, 5000], members=2, max_batch=1024, seed=seed) as net:
+            net.set_output_scale(np.full(5000, 2.0))
+            scaled = net.predict(x)[0]
+            net.set_output_scale(None)
+            plain = net.predict(x)[0]
+        assert np.array_equal(scaled, 2.0 * plain) and np.all(plain.any(axis=0))
+
+
 @pytest.mark.parametrize("sizes,rows,members", [([8, 1], 1, 1), ([8, 63], 65, 2), ([8, 64, 65], 63, 3),
                                                 ([8, 96, 64, 129], 130, 5), ([4, 64, 65600], 130, 2),
                                                 ([4, 160, 70001], 97, 3)])
