@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "mlp_kernels.h"
 
@@ -28,8 +29,14 @@ typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int BM = 128, BN = 128, BK = 32;
 constexpr int LDS_ROW = BK + 8;  // bf16 per LDS row (16-byte pad against bank conflicts)
-// products of at least this many 128 x 128 tiles run ensemble_nt on them (two per CU), others on 64 x 64
-constexpr int kEnsembleBigTiles = 512;
+// The shape of ensemble_output's tiles.  Wide tiles are 128 x 128, two blocks per CU; of fewer than
+// kEnsembleWideTiles of them, tiles of 64 x 64 fill the chip better (us per pass, five members of 512
+// hidden: 40 x 6300 in 50 wide tiles 129, in small ones 122; 300 x 6300 in 150: 161 and 163).  256 x 128
+// tiles read a sixth less per product, about kEnsembleTallGain of the time (2048 x 151500: 2618 against
+// 3007 us), so they are taken where the rows that pad them out cost less than that (130 rows in one tile:
+// 276 against 292; 300 rows in two: 715 against 640).
+constexpr int kEnsembleWideTiles = 128;
+constexpr float kEnsembleTallGain = 1.15f;
 
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
 
@@ -366,6 +373,106 @@ __global__ void __launch_bounds__(256, 3) gemm_nt(const uint16_t *__restrict__ A
     }
 }
 
+// Welford's update by member e's outputs.  The accumulators hold the outputs' differences from the
+// running mean: they start at bias - mean (the first at the bias) instead of 0, which saves the sum
+// and the difference, two operations of six; b is the next member's bias (per column).
+template <int MI, int NJ>
+__device__ __forceinline__ void welford_update(f32x16 (&acc)[MI][NJ], f32x16 (&mu)[MI][NJ], f32x16 (&m2)[MI][NJ], int e,
+                                               const float (&b)[NJ])
+{
+    const float rcount = 1.0f / (float)(e + 1), weight = (float)e / (float)(e + 1);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const float d = acc[i][j][q];
+                mu[i][j][q] = __builtin_fmaf(d, rcount, mu[i][j][q]);
+                m2[i][j][q] = __builtin_fmaf(d * weight, d, m2[i][j][q]);
+                acc[i][j][q] = b[j] - mu[i][j][q];
+            }
+}
+
+// Stores a wave's means (scaled) and its row sums of the squared deviations and squared means into
+// red[wn][row][0 / 1].  Lane l's 16 results of a 32 x 32 tile are rows (q / 4) * 8 + (l / 32) * 4 + q % 4
+// of column l % 32.
+template <int MI, int NJ, int ROWS>
+__device__ __forceinline__ void ensemble_store(const f32x16 (&mu)[MI][NJ], const f32x16 (&m2)[MI][NJ], int m0, int n0, int wm,
+                                               int wn, int M, int N, float *__restrict__ mean, size_t ldm,
+                                               const float *__restrict__ scale, bool sums, double (*red)[ROWS][2])
+{
+    const int lane = threadIdx.x & 63;
+    const bool full = m0 + ROWS <= M && n0 + 64 * NJ <= N;  // (the tile's columns: two waves of 32 NJ)
+    bool ok_n[NJ];
+    float sc[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int n = n0 + wn * 32 * NJ + j * 32 + (lane & 31);
+        ok_n[j] = n < N;
+        sc[j] = scale && ok_n[j] ? scale[n] : 1.f;
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        double sv[16], sn[16];
+        if (full) {
+            float *const row = mean + (size_t)(m0 + wm * 32 * MI + i * 32 + (lane >> 5) * 4) * ldm + n0 + wn * 32 * NJ + (lane & 31);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                sv[q] = sn[q] = 0.0;
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    const float v = mu[i][j][q];
+                    sv[q] += m2[i][j][q];
+                    sn[q] += (double)v * v;
+                    if (mean) row[((q >> 2) * 8 + (q & 3)) * ldm + j * 32] = v * sc[j];
+                }
+            }
+        } else
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int m = m0 + wm * 32 * MI + i * 32 + (q >> 2) * 8 + (lane >> 5) * 4 + (q & 3);
+            sv[q] = sn[q] = 0.0;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int n = n0 + wn * 32 * NJ + j * 32 + (lane & 31);
+                if (ok_n[j]) {
+                    const float v = mu[i][j][q];
+                    sv[q] += m2[i][j][q];
+                    sn[q] += (double)v * v;
+                    if (mean && m < M) mean[(size_t)m * ldm + n] = v * sc[j];
+                }
+            }
+        }
+        if (!sums) continue;
+        // sum over the 32 lanes of a half wave: at every step a lane keeps half of its rows, adding
+        // its partner's sums of them; lane l ends with row q0, the bits 16, 8, 4 and 2 of l
+        int q0 = 0;
+        auto halve = [&](auto half) {
+            constexpr int cnt = decltype(half)::value, h = 2 * cnt;
+            const bool up = lane & h;
+#pragma unroll
+            for (int q = 0; q < cnt; ++q) {
+                const double av = up ? sv[q] : sv[q + cnt], an = up ? sn[q] : sn[q + cnt];
+                sv[q] = (up ? sv[q + cnt] : sv[q]) + __shfl_xor(av, h);
+                sn[q] = (up ? sn[q + cnt] : sn[q]) + __shfl_xor(an, h);
+            }
+            if (up) q0 += cnt;
+        };
+        halve(std::integral_constant<int, 8>{});
+        halve(std::integral_constant<int, 4>{});
+        halve(std::integral_constant<int, 2>{});
+        halve(std::integral_constant<int, 1>{});
+        sv[0] += __shfl_xor(sv[0], 1);
+        sn[0] += __shfl_xor(sn[0], 1);
+        if (!(lane & 1)) {
+            const int row = wm * 32 * MI + i * 32 + (q0 >> 2) * 8 + (lane >> 5) * 4 + (q0 & 3);
+            red[wn][row][0] = sv[0];
+            red[wn][row][1] = sn[0];
+        }
+    }
+}
+
 // The output layer of every ensemble member and their statistics in one pass: tile by tile, member
 // e's product H_e W_e^T + b_e is formed in the accumulators and folded into the running mean and sum
 // of squared deviations (Welford), both in registers.  Stores the mean (times scale[n] when given)
@@ -375,9 +482,8 @@ __global__ void __launch_bounds__(256, 3) gemm_nt(const uint16_t *__restrict__ A
 // What bounds it.  Members one at a time wrote each output array (620 MB of 1024 x 151 500) and read
 // it back with mean and deviations: 0.33 ms of product and 0.51 ms of Welford per member, 0.8 ms of
 // scaling and row sums, 5.3 ms for five members.  Here the mean is the only array that reaches HBM.
-// Waves are 2 x 2 of 32 MI x 32 NJ: MI = NJ = 2 (192 registers of results, two blocks per CU), or 1
-// where that leaves too few blocks.  Tile order as EPI_MSE's: m fastest within an XCD's run, so the
-// m tiles of one n tile share its weights in that L2.
+// Waves are 2 x 2 of 32 MI x 32 NJ.  Tile order as EPI_MSE's: m fastest within an XCD's run, so the m
+// tiles of one n tile share its weights in that L2.
 template <int MI, int NJ>
 __global__ void __launch_bounds__(256, 2)
     ensemble_nt(const uint16_t *__restrict__ A, int lda, size_t stride_a, const uint16_t *const *__restrict__ bs, int ldb,
@@ -424,7 +530,19 @@ __global__ void __launch_bounds__(256, 2)
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = mu[i][j][e] = m2[i][j][e] = 0.f;
+            for (int e = 0; e < 16; ++e) mu[i][j][e] = m2[i][j][e] = 0.f;
+    auto bias_of = [&](int e, int j) {
+        const int n = tn * TN + wn * 32 * NJ + j * 32 + (lane & 31);
+        return n < N ? biases[e][n] : 0.f;
+    };
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const float b = bias_of(0, j);
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = b;
+    }
     load(ra[0], rb[0]);
     load(ra[1], rb[1]);
     store(0, ra[0], rb[0]);
@@ -449,29 +567,10 @@ __global__ void __launch_bounds__(256, 2)
         }
         if (g + 1 < steps) store(u ^ 1, ra[u ^ 1], rb[u ^ 1]);
         if (++kt == nk) {
-            // member e's outputs are complete: Welford's update, and the accumulators start over
-            const float count = (float)(e + 1), rcount = 1.0f / count;
+            float b[NJ];
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                const int n = tn * TN + wn * 32 * NJ + j * 32 + (lane & 31);
-                const float b = n < N ? biases[e][n] : 0.f;
-#pragma unroll
-                for (int i = 0; i < MI; ++i)
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) {
-                        const float v = acc[i][j][q] + b;
-                        const float d = v - mu[i][j][q];
-                        // d / count, correctly rounded: the quotient by the reciprocal, one step of
-                        // its remainder, and the infinities and NaN
-                        const float q0 = d * rcount;
-                        const float dq = __builtin_amdgcn_div_fixupf(
-                            __builtin_fmaf(__builtin_fmaf(-q0, count, d), rcount, q0), count, d);
-                        const float nm = mu[i][j][q] + dq;
-                        m2[i][j][q] += d * (v - nm);
-                        mu[i][j][q] = nm;
-                        acc[i][j][q] = 0.f;
-                    }
-            }
+            for (int j = 0; j < NJ; ++j) b[j] = bias_of(min(e + 1, members - 1), j);
+            welford_update<MI, NJ>(acc, mu, m2, e, b);
             kt = 0;
             ++e;
         }
@@ -482,56 +581,7 @@ __global__ void __launch_bounds__(256, 2)
         if (g + 1 < steps) step(g + 1, 1);
     }
 
-    // the mean, and the row sums: lane l's 16 results of a 32 x 32 tile are rows (q / 4) * 8 + (l / 32)
-    // * 4 + q % 4 of column l % 32
-    const bool ok_n[2] = {tn * TN + wn * 32 * NJ + (lane & 31) < N, tn * TN + wn * 32 * NJ + 32 + (lane & 31) < N};
-    float sc[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        const int n = tn * TN + wn * 32 * NJ + j * 32 + (lane & 31);
-        sc[j] = scale && ok_n[j] ? scale[n] : 1.f;
-    }
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-        double sv[16], sn[16];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const int m = tm * TM + wm * 32 * MI + i * 32 + (q >> 2) * 8 + (lane >> 5) * 4 + (q & 3);
-            sv[q] = sn[q] = 0.0;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                const int n = tn * TN + wn * 32 * NJ + j * 32 + (lane & 31);
-                if (ok_n[j]) {
-                    const float v = mu[i][j][q];
-                    sv[q] += m2[i][j][q];
-                    sn[q] += (double)v * v;
-                    if (mean && m < M) mean[(size_t)m * ldm + n] = v * sc[j];
-                }
-            }
-        }
-        if (!part) continue;
-        // sum over the 32 lanes of a half wave: at every step a lane keeps half of its rows, adding
-        // its partner's sums of them; lane l ends with row q = (l % 32) / 2
-        int q0 = 0;
-#pragma unroll
-        for (int h = 16, cnt = 8; cnt >= 1; h >>= 1, cnt >>= 1) {
-            const bool up = lane & h;
-#pragma unroll
-            for (int q = 0; q < cnt; ++q) {
-                const double av = up ? sv[q] : sv[q + cnt], an = up ? sn[q] : sn[q + cnt];
-                sv[q] = (up ? sv[q + cnt] : sv[q]) + __shfl_xor(av, h);
-                sn[q] = (up ? sn[q + cnt] : sn[q]) + __shfl_xor(an, h);
-            }
-            if (up) q0 += cnt;
-        }
-        sv[0] += __shfl_xor(sv[0], 1);
-        sn[0] += __shfl_xor(sn[0], 1);
-        if (!(lane & 1)) {
-            const int row = wm * 32 * MI + i * 32 + (q0 >> 2) * 8 + (lane >> 5) * 4 + (q0 & 3);
-            red[wn][row][0] = sv[0];
-            red[wn][row][1] = sn[0];
-        }
-    }
+    ensemble_store<MI, NJ>(mu, m2, tm * TM, tn * TN, wm, wn, M, N, mean, ldm, scale, part != nullptr, red);
     if (!part) return;
     __syncthreads();
     for (int r = t; r < 2 * TM; r += 256) {
@@ -540,7 +590,202 @@ __global__ void __launch_bounds__(256, 2)
     }
 }
 
-// spread[m] = ||standard deviation over members|| / ||mean|| from ensemble_nt's sums of `tiles` tiles
+// The same for large products: a block of WM x WN waves, each 64 x 64, owns a tile of 64 WM x 64 WN, and
+// its operand tiles of BKL k values reach LDS by direct loads, STAGES of them in a ring, so no register
+// carries them and STAGES - 1 tiles are in flight (the results of 64 x 64 outputs take 192 of the 256
+// registers).  A wave's direct load writes 1 KiB of consecutive LDS, so rows are unpadded; the 16-byte
+// chunks of a row are exchanged by its row bits instead, which spreads the sixteen rows that a phase of
+// a fragment read touches over all 64 banks (by the low row bits alone, two rows met in each: 45 % of
+// the LDS cycles, 3 % of the time).
+//
+// What bounds it: on 1024 x 151500 x 512 and five members 1.17 ms (2.1 of ensemble_nt on 128 x 128 tiles),
+// 680 TFLOP/s; the matrix cores are busy a third of the cycles, the mean's 620 MB take 0.2 ms in which
+// nothing else runs (one block per CU), the statistics 0.07, and each of the 8 k tiles of a member begins
+// with a barrier and a round trip to LDS.
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(1))) void global_void;
+// pointers in memory that no kernel writes: read by scalar loads, which no load in flight delays
+typedef __attribute__((address_space(4))) const uint64_t const_u64;
+
+constexpr int kWideBiases = 16;  // members whose biases are in LDS at a time
+
+template <int WM, int WN, int BKL, int STAGES>
+__global__ void __launch_bounds__(64 * WM * WN, 2)
+    ensemble_wide(const uint16_t *__restrict__ A, int lda, size_t stride_a, const uint16_t *const *__restrict__ bs, int ldb,
+                  const float *const *__restrict__ biases, int M, int N, int K, int members, float *__restrict__ mean,
+                  size_t ldm, const float *__restrict__ scale, double *__restrict__ part)
+{
+    static_assert(STAGES >= 2 && STAGES <= 4, "the loop over the steps");
+    constexpr int TM = 64 * WM, TN = 64 * WN, THREADS = 64 * WM * WN;
+    constexpr int CH = BKL / 8;                         // 16-byte chunks of a row
+    constexpr int RPL = 64 / CH;                        // rows one wave's load covers
+    constexpr int LOADS = (TM + TN) / RPL / (WM * WN);  // loads per wave and tile
+    // One array for the stages and, behind them, the biases (read from memory at a member's end, they
+    // would wait for every load in flight).  Of several arrays, or with its end out of the compiler's
+    // sight, the compiler holds reads until all direct loads in flight have landed; the waits for the
+    // tile that is read are written out below.
+    constexpr int STAGE = (TM + TN) * BKL;  // bf16 per stage
+    __shared__ __align__(1024) uint16_t ring[STAGES * STAGE + 2 * kWideBiases * TN];
+    uint16_t *const s0 = ring, *const s1 = ring + STAGE, *const s2 = ring + (STAGES > 2 ? 2 : 0) * STAGE,
+                   *const s3 = ring + (STAGES - 1) * STAGE;
+    float *const lbias = (float *)(ring + STAGES * STAGE);
+    const int tiles_m = (M + TM - 1) / TM;
+    const int nb = (int)gridDim.x, q8 = nb >> 3, r8 = nb & 7;
+    const int xcd = (int)blockIdx.x & 7, slot = (int)blockIdx.x >> 3;
+    const int tile = xcd < r8 ? xcd * (q8 + 1) + slot : r8 * (q8 + 1) + (xcd - r8) * q8 + slot;
+    const int tm = tile % tiles_m, tn = tile / tiles_m;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = wave / WN, wn = wave % WN;
+    const int nk = K / BKL, steps = nk * members;
+    // swizzle: chunk c of row r sits at chunk c ^ swz(r)
+    auto swz = [](int r) -> int {
+        return CH == 8 ? (r >> 1 & 3) << 1 | (r >> 3 & 1) : (r >> 2 & 1) << 1 | (r >> 3 & 1);
+    };
+    const_u64 *const b_at = (const_u64 *)(uintptr_t)bs, *const bias_at = (const_u64 *)(uintptr_t)biases;
+
+    // the byte this lane loads, from the tile's first row: load l of the wave covers rows (wave * LOADS +
+    // l) * RPL .. of the stage (A's rows, then B's)
+    uint32_t off[LOADS];
+#pragma unroll
+    for (int l = 0; l < LOADS; ++l) {
+        const int r = (wave * LOADS + l) * RPL + lane / CH, c = (lane % CH) ^ swz(r);
+        off[l] = r < TM ? (uint32_t)(min(r, M - 1 - tm * TM) * lda + c * 8) * 2u
+                        : (uint32_t)(min(r - TM, N - 1 - tn * TN) * ldb + c * 8) * 2u;
+    }
+    int ge = 0, gk = 0;  // member and k tile of the next load
+    // the loads first <= l < last of a tile
+    auto load = [&](uint16_t *stage, int first, int last) {
+        const uint64_t pa = (uint64_t)(uintptr_t)(A + ge * stride_a + (size_t)tm * TM * lda + gk * BKL);
+        const uint64_t pb = b_at[ge] + ((size_t)tn * TN * ldb + gk * BKL) * 2;
+#pragma unroll
+        for (int l = 0; l < LOADS; ++l) {
+            if (l < first || l >= last) continue;
+            const int r0 = (wave * LOADS + l) * RPL;  // (a load's rows are all A's or all B's)
+            __builtin_amdgcn_global_load_lds(
+                (global_void *)((__attribute__((address_space(1))) char *)(r0 < TM ? pa : pb) + off[l]),
+                (lds_void *)(stage + r0 * BKL), 16, 0, 0);
+        }
+    };
+    auto next_tile = [&] {
+        if (++gk == nk) {
+            gk = 0;
+            if (ge + 1 < members) ++ge;  // (past the last step: re-reads, never used)
+        }
+    };
+    auto fill_biases = [&](int e0) {
+        for (int i = t; i < min(members - e0, kWideBiases) * TN; i += THREADS) {
+            const int n = tn * TN + i % TN;
+            lbias[i] = n < N ? ((const __attribute__((address_space(1))) float *)bias_at[e0 + i / TN])[n] : 0.f;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    };
+    f32x16 acc[2][2], mu[2][2], m2[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) mu[i][j][e] = m2[i][j][e] = 0.f;
+    fill_biases(0);
+    __syncthreads();
+    float b[2];
+    auto bias_of = [&](int e) {
+        const float *const l = lbias + (e % kWideBiases) * TN + wn * 64 + (lane & 31);
+        b[0] = l[0], b[1] = l[32];
+    };
+    bias_of(0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = b[j];
+    load(s0, 0, LOADS), next_tile();
+    if constexpr (STAGES > 2) load(s1, 0, LOADS), next_tile();
+    if constexpr (STAGES > 3) load(s2, 0, LOADS), next_tile();
+
+    int kt = 0, e = 0;
+    // this lane's fragments: rows ar, ar + 32 of A and br, br + 32 of B, chunk (kk / 8 + lane / 32) ^ swz of
+    // k step kk (32 rows on the swizzle is the same), as offsets into a stage
+    const int ar = wm * 64 + (lane & 31), br = TM + wn * 64 + (lane & 31);
+    int ao[BKL / 16], bo[BKL / 16];
+#pragma unroll
+    for (int q = 0; q < BKL / 16; ++q) {
+        ao[q] = ar * BKL + ((2 * q + (lane >> 5)) ^ swz(ar)) * 8;
+        bo[q] = br * BKL + ((2 * q + (lane >> 5)) ^ swz(br)) * 8;
+    }
+    // one tile, in stage `at`; the next load goes to `to`, the stage of the tile before
+    auto step = [&](const uint16_t *at, uint16_t *to) {
+        // the tile has landed when no more than the STAGES - 2 tiles after it are in flight; past the
+        // barrier that holds for every wave, and every wave is done with the tile before
+        constexpr int PENDING = LOADS * (STAGES - 2);
+        static_assert(PENDING == 0 || PENDING == 6 || PENDING == 8, "a wait for each");
+        if constexpr (PENDING == 6) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+        else if constexpr (PENDING == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        if (kt == nk - 1 && (e + 1) % kWideBiases == 0 && e + 1 < members) {
+            fill_biases(e + 1);  // (every wave is past the member before)
+            __builtin_amdgcn_s_barrier();
+        }
+        asm volatile("" ::: "memory");
+        bf16x8 fa[2][2], fb[2][2];  // the fragments of k step q and the next
+        auto read = [&](int q) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                fa[q & 1][i] = *(const bf16x8 *)(at + ao[q] + i * 32 * BKL);
+                fb[q & 1][i] = *(const bf16x8 *)(at + bo[q] + i * 32 * BKL);
+            }
+        };
+        read(0);
+#pragma unroll
+        for (int q = 0; q < BKL / 16; ++q) {
+            if (q + 1 < BKL / 16) read(q + 1);
+            load(to, q * LOADS / (BKL / 16), (q + 1) * LOADS / (BKL / 16));
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[q & 1][i], fb[q & 1][j], acc[i][j], 0, 0, 0);
+        }
+        next_tile();
+        if (++kt == nk) {
+            bias_of(e + 1);  // (of no use after the last)
+            welford_update<2, 2>(acc, mu, m2, e, b);
+            kt = 0;
+            ++e;
+        }
+        // (this wave's reads of the tile are done before it reaches the next barrier)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    };
+    // (left from the middle: an edge back from there would have the first step wait for all loads)
+    for (int g = 0;;) {
+        step(s0, s3);
+        if (++g == steps) break;
+        step(s1, s0);
+        if (++g == steps) break;
+        if constexpr (STAGES > 2) {
+            step(s2, s1);
+            if (++g == steps) break;
+        }
+        if constexpr (STAGES > 3) {
+            step(s3, s2);
+            if (++g == steps) break;
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the re-reads, before a stage is used again
+    __syncthreads();
+    double(*const red)[TM][2] = (double(*)[TM][2])s0;
+    ensemble_store<2, 2>(mu, m2, tm * TM, tn * TN, wm, wn, M, N, mean, ldm, scale, part != nullptr, red);
+    if (!part) return;
+    __syncthreads();
+    for (int r = t; r < 2 * TM; r += THREADS) {
+        const int row = r % TM, w = r / TM, m = tm * TM + row;
+        if (m < M) part[((size_t)tn * 2 + w) * M + m] = red[0][row][w] + red[1][row][w];
+    }
+}
+
+// spread[m] = ||standard deviation over members|| / ||mean|| from the sums of `tiles` tiles
 // per row: 64 rows per block, 16 threads a row over the tiles, then over the threads in order.
 __global__ void __launch_bounds__(1024) ensemble_spread(const double *__restrict__ part, int tiles, int M, int members,
                                                         float *__restrict__ spread)
@@ -814,15 +1059,18 @@ hipError_t ensemble_output(const uint16_t *A, int lda, size_t stride_a, const ui
     if (M < 1 || N < 1 || K < BK || K % BK || lda % 8 || ldb % 8 || lda < K || ldb < K || members < 1 || (spread && !part))
         return hipErrorInvalidValue;
     if (!spread) part = nullptr;
-    const long long big = (long long)((M + 127) / 128) * ((N + 127) / 128);
-    const int width = big >= kEnsembleBigTiles ? 128 : 64;
-    const int tiles_m = (M + width - 1) / width, tiles_n = (N + width - 1) / width;
-    if (width == 128)
-        ensemble_nt<2, 2><<<tiles_m * tiles_n, 256, 0, stream>>>(A, lda, stride_a, bs, ldb, biases, M, N, K, members, mean,
-                                                                 ldm, scale, part);
-    else
-        ensemble_nt<1, 1><<<tiles_m * tiles_n, 256, 0, stream>>>(A, lda, stride_a, bs, ldb, biases, M, N, K, members, mean,
-                                                                 ldm, scale, part);
+    const auto tiles = [&](int tm, int tn) { return (long long)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
+    const bool wide = tiles(128, 128) >= kEnsembleWideTiles;
+    const bool tall = wide && K % 64 == 0 && tiles(256, 128) * 256 <= tiles(128, 128) * 128 * kEnsembleTallGain;
+    const int rows = tall ? 256 : wide ? 128 : 64, width = wide ? 128 : 64;
+    const int tiles_n = (N + width - 1) / width, blocks = (int)tiles(rows, width);
+    auto launch = [&](auto kernel, int threads) {
+        kernel<<<blocks, threads, 0, stream>>>(A, lda, stride_a, bs, ldb, biases, M, N, K, members, mean, ldm, scale, part);
+    };
+    if (tall) launch(ensemble_wide<4, 2, 64, 3>, 512);
+    else if (wide && K % 64 == 0) launch(ensemble_wide<2, 2, 64, 2>, 256);
+    else if (wide) launch(ensemble_wide<2, 2, 32, 4>, 256);
+    else launch(ensemble_nt<1, 1>, 256);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !spread) return e;
     ensemble_spread<<<(M + 63) / 64, 1024, 0, stream>>>(part, tiles_n, M, members, spread);
