@@ -29,14 +29,20 @@ typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int BM = 128, BN = 128, BK = 32;
 constexpr int LDS_ROW = BK + 8;  // bf16 per LDS row (16-byte pad against bank conflicts)
-// The shape of ensemble_output's tiles.  Wide tiles are 128 x 128, two blocks per CU; of fewer than
-// kEnsembleWideTiles of them, tiles of 64 x 64 fill the chip better (us per pass, five members of 512
-// hidden: 40 x 6300 in 50 wide tiles 129, in small ones 122; 300 x 6300 in 150: 161 and 163).  256 x 128
-// tiles read a sixth less per product, about kEnsembleTallGain of the time (2048 x 151500: 2618 against
-// 3007 us), so they are taken where the rows that pad them out cost less than that (130 rows in one tile:
-// 276 against 292; 300 rows in two: 715 against 640).
-constexpr int kEnsembleWideTiles = 128;
-constexpr float kEnsembleTallGain = 1.15f;
+// The shape of ensemble_output's tiles: the one with the least work per CU, tiles per block slot (two
+// blocks a CU of the 64 x 64 and 128 x 128, one of the 256 x 128; less than one slot each costs a whole
+// tile) times a tile's cost relative to 64 x 64.  Larger tiles read their operands less often, but pad
+// more rows and fill the chip later.  Measured, us per pass, five members of 512 hidden, rows x outputs:
+//                 64 x 64   128 x 128   256 x 128
+//   37 x 6300         100         121
+//   130 x 20000       140         157         153
+//   300 x 20000       193         174         219
+//   130 x 75750       286         292         276
+//   300 x 151500      949 *       636         743
+//   1024 x 6300       267         252         245
+//   2048 x 151500    4960 *      3000        2614      (* operands carried through registers)
+constexpr int kCus = 256;
+constexpr float kCostSquare = 3.0f, kCostTall = 2.7f;
 
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
 
@@ -482,141 +488,33 @@ __device__ __forceinline__ void ensemble_store(const f32x16 (&mu)[MI][NJ], const
 // What bounds it.  Members one at a time wrote each output array (620 MB of 1024 x 151 500) and read
 // it back with mean and deviations: 0.33 ms of product and 0.51 ms of Welford per member, 0.8 ms of
 // scaling and row sums, 5.3 ms for five members.  Here the mean is the only array that reaches HBM.
-// Waves are 2 x 2 of 32 MI x 32 NJ.  Tile order as EPI_MSE's: m fastest within an XCD's run, so the m
-// tiles of one n tile share its weights in that L2.
-template <int MI, int NJ>
-__global__ void __launch_bounds__(256, 2)
-    ensemble_nt(const uint16_t *__restrict__ A, int lda, size_t stride_a, const uint16_t *const *__restrict__ bs, int ldb,
-                const float *const *__restrict__ biases, int M, int N, int K, int members, float *__restrict__ mean,
-                size_t ldm, const float *__restrict__ scale, double *__restrict__ part)
-{
-    constexpr int TM = 64 * MI, TN = 64 * NJ;
-    __shared__ uint16_t la[2][TM * LDS_ROW], lb[2][TN * LDS_ROW];
-    __shared__ double red[2][TM][2];
-    const int tiles_m = (M + TM - 1) / TM;
-    const int nb = (int)gridDim.x, q8 = nb >> 3, r8 = nb & 7;
-    const int xcd = (int)blockIdx.x & 7, slot = (int)blockIdx.x >> 3;
-    const int tile = xcd < r8 ? xcd * (q8 + 1) + slot : r8 * (q8 + 1) + (xcd - r8) * q8 + slot;
-    const int tm = tile % tiles_m, tn = tile / tiles_m;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int r0 = t >> 2, kc = t & 3;
-    const int nk = K / BK, steps = nk * members;
-
-    // operand tiles of step g (member g / nk, k tile g % nk), two register sets ahead of the MFMAs
-    u16x8 ra[2][MI], rb[2][NJ];
-    int ge = 0, gk = 0;  // member and k tile of the next load
-    auto load = [&](u16x8 *a, u16x8 *b) {
-        const uint16_t *const pa = A + ge * stride_a + gk * BK + kc * 8;
-        const uint16_t *const pb = bs[ge] + gk * BK + kc * 8;
-#pragma unroll
-        for (int h = 0; h < MI; ++h) a[h] = *(const u16x8 *)(pa + (size_t)min(tm * TM + r0 + h * 64, M - 1) * lda);
-#pragma unroll
-        for (int h = 0; h < NJ; ++h) b[h] = *(const u16x8 *)(pb + (size_t)min(tn * TN + r0 + h * 64, N - 1) * ldb);
-        if (++gk == nk) {
-            gk = 0;
-            if (ge + 1 < members) ++ge;  // (past the last step: re-reads, never used)
-        }
-    };
-    auto store = [&](int buf, const u16x8 *a, const u16x8 *b) {
-#pragma unroll
-        for (int h = 0; h < MI; ++h) *(u16x8 *)(la[buf] + (r0 + h * 64) * LDS_ROW + kc * 8) = a[h];
-#pragma unroll
-        for (int h = 0; h < NJ; ++h) *(u16x8 *)(lb[buf] + (r0 + h * 64) * LDS_ROW + kc * 8) = b[h];
-    };
-    f32x16 acc[MI][NJ], mu[MI][NJ], m2[MI][NJ];
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) mu[i][j][e] = m2[i][j][e] = 0.f;
-    auto bias_of = [&](int e, int j) {
-        const int n = tn * TN + wn * 32 * NJ + j * 32 + (lane & 31);
-        return n < N ? biases[e][n] : 0.f;
-    };
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        const float b = bias_of(0, j);
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = b;
-    }
-    load(ra[0], rb[0]);
-    load(ra[1], rb[1]);
-    store(0, ra[0], rb[0]);
-    __syncthreads();
-    int kt = 0, e = 0;
-    auto step = [&](int g, int u) {
-        load(ra[u], rb[u]);
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 16) {
-            bf16x8 fa[MI], fb[NJ];
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-                fa[i] = *(const bf16x8 *)(la[u] + (wm * 32 * MI + i * 32 + (lane & 31)) * LDS_ROW + kk + (lane >> 5) * 8);
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-                fb[j] = *(const bf16x8 *)(lb[u] + (wn * 32 * NJ + j * 32 + (lane & 31)) * LDS_ROW + kk + (lane >> 5) * 8);
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                for (int j = 0; j < NJ; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-        }
-        if (g + 1 < steps) store(u ^ 1, ra[u ^ 1], rb[u ^ 1]);
-        if (++kt == nk) {
-            float b[NJ];
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) b[j] = bias_of(min(e + 1, members - 1), j);
-            welford_update<MI, NJ>(acc, mu, m2, e, b);
-            kt = 0;
-            ++e;
-        }
-        __syncthreads();
-    };
-    for (int g = 0; g < steps; g += 2) {
-        step(g, 0);
-        if (g + 1 < steps) step(g + 1, 1);
-    }
-
-    ensemble_store<MI, NJ>(mu, m2, tm * TM, tn * TN, wm, wn, M, N, mean, ldm, scale, part != nullptr, red);
-    if (!part) return;
-    __syncthreads();
-    for (int r = t; r < 2 * TM; r += 256) {
-        const int row = r % TM, w = r / TM, m = tm * TM + row;
-        if (m < M) part[((size_t)tn * 2 + w) * M + m] = red[0][row][w] + red[1][row][w];
-    }
-}
-
-// The same for large products: a block of WM x WN waves, each 64 x 64, owns a tile of 64 WM x 64 WN, and
-// its operand tiles of BKL k values reach LDS by direct loads, STAGES of them in a ring, so no register
-// carries them and STAGES - 1 tiles are in flight (the results of 64 x 64 outputs take 192 of the 256
-// registers).  A wave's direct load writes 1 KiB of consecutive LDS, so rows are unpadded; the 16-byte
-// chunks of a row are exchanged by its row bits instead, which spreads the sixteen rows that a phase of
-// a fragment read touches over all 64 banks (by the low row bits alone, two rows met in each: 45 % of
-// the LDS cycles, 3 % of the time).
+// A block of WM x WN waves, each with MI x NJ results of 32 x 32, owns a tile; the operand tiles of 64 k
+// values reach LDS by direct loads, STAGES of them in a ring, so no register carries them and STAGES - 1
+// are in flight (results of 64 x 64 a wave take 192 of its 256 registers).  A wave's direct load writes
+// 1 KiB of consecutive LDS, so rows are unpadded; the 16-byte chunks of a row are exchanged by its row
+// bits instead, which spreads the sixteen rows that a phase of a fragment read touches over all 64 banks
+// (by the low row bits alone, two rows met in each: 45 % of the LDS cycles, 3 % of the time).  Tile order
+// as EPI_MSE's: m fastest within an XCD's run, so the m tiles of one n tile share its weights in that L2.
 //
-// What bounds it: on 1024 x 151500 x 512 and five members 1.17 ms (2.1 of ensemble_nt on 128 x 128 tiles),
-// 680 TFLOP/s; the matrix cores are busy a third of the cycles, the mean's 620 MB take 0.2 ms in which
-// nothing else runs (one block per CU), the statistics 0.07, and each of the 8 k tiles of a member begins
-// with a barrier and a round trip to LDS.
+// On 1024 x 151500 x 512 and five members in 256 x 128 tiles 1.19 ms, 670 TFLOP/s (operands through
+// registers, 128 x 128 tiles: 2.13): the matrix cores are busy a third of the cycles, the mean's 620 MB
+// take 0.2 ms in which nothing else runs (one block per CU), the statistics 0.07, and each of the 8 k
+// tiles of a member begins with a barrier and a round trip to LDS.
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) void global_void;
 // pointers in memory that no kernel writes: read by scalar loads, which no load in flight delays
 typedef __attribute__((address_space(4))) const uint64_t const_u64;
 
-constexpr int kWideBiases = 16;  // members whose biases are in LDS at a time
+constexpr int kBiasMembers = 16;  // members whose biases are in LDS at a time
 
-template <int WM, int WN, int BKL, int STAGES>
+template <int WM, int WN, int MI, int NJ, int STAGES>
 __global__ void __launch_bounds__(64 * WM * WN, 2)
-    ensemble_wide(const uint16_t *__restrict__ A, int lda, size_t stride_a, const uint16_t *const *__restrict__ bs, int ldb,
+    ensemble_tiles(const uint16_t *__restrict__ A, int lda, size_t stride_a, const uint16_t *const *__restrict__ bs, int ldb,
                   const float *const *__restrict__ biases, int M, int N, int K, int members, float *__restrict__ mean,
                   size_t ldm, const float *__restrict__ scale, double *__restrict__ part)
 {
     static_assert(STAGES >= 2 && STAGES <= 4, "the loop over the steps");
-    constexpr int TM = 64 * WM, TN = 64 * WN, THREADS = 64 * WM * WN;
+    constexpr int TM = 32 * MI * WM, TN = 32 * NJ * WN, THREADS = 64 * WM * WN, BKL = 64;
     constexpr int CH = BKL / 8;                         // 16-byte chunks of a row
     constexpr int RPL = 64 / CH;                        // rows one wave's load covers
     constexpr int LOADS = (TM + TN) / RPL / (WM * WN);  // loads per wave and tile
@@ -625,7 +523,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2)
     // sight, the compiler holds reads until all direct loads in flight have landed; the waits for the
     // tile that is read are written out below.
     constexpr int STAGE = (TM + TN) * BKL;  // bf16 per stage
-    __shared__ __align__(1024) uint16_t ring[STAGES * STAGE + 2 * kWideBiases * TN];
+    __shared__ __align__(1024) uint16_t ring[STAGES * STAGE + 2 * kBiasMembers * TN];
     uint16_t *const s0 = ring, *const s1 = ring + STAGE, *const s2 = ring + (STAGES > 2 ? 2 : 0) * STAGE,
                    *const s3 = ring + (STAGES - 1) * STAGE;
     float *const lbias = (float *)(ring + STAGES * STAGE);
@@ -638,9 +536,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2)
     const int wm = wave / WN, wn = wave % WN;
     const int nk = K / BKL, steps = nk * members;
     // swizzle: chunk c of row r sits at chunk c ^ swz(r)
-    auto swz = [](int r) -> int {
-        return CH == 8 ? (r >> 1 & 3) << 1 | (r >> 3 & 1) : (r >> 2 & 1) << 1 | (r >> 3 & 1);
-    };
+    auto swz = [](int r) -> int { return (r >> 1 & 3) << 1 | (r >> 3 & 1); };
     const_u64 *const b_at = (const_u64 *)(uintptr_t)bs, *const bias_at = (const_u64 *)(uintptr_t)biases;
 
     // the byte this lane loads, from the tile's first row: load l of the wave covers rows (wave * LOADS +
@@ -673,31 +569,31 @@ __global__ void __launch_bounds__(64 * WM * WN, 2)
         }
     };
     auto fill_biases = [&](int e0) {
-        for (int i = t; i < min(members - e0, kWideBiases) * TN; i += THREADS) {
+        for (int i = t; i < min(members - e0, kBiasMembers) * TN; i += THREADS) {
             const int n = tn * TN + i % TN;
             lbias[i] = n < N ? ((const __attribute__((address_space(1))) float *)bias_at[e0 + i / TN])[n] : 0.f;
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
-    f32x16 acc[2][2], mu[2][2], m2[2][2];
+    f32x16 acc[MI][NJ], mu[MI][NJ], m2[MI][NJ];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) mu[i][j][e] = m2[i][j][e] = 0.f;
     fill_biases(0);
     __syncthreads();
-    float b[2];
+    float b[NJ];
     auto bias_of = [&](int e) {
-        const float *const l = lbias + (e % kWideBiases) * TN + wn * 64 + (lane & 31);
-        b[0] = l[0], b[1] = l[32];
+        #pragma unroll
+        for (int j = 0; j < NJ; ++j) b[j] = lbias[(e % kBiasMembers) * TN + wn * 32 * NJ + j * 32 + (lane & 31)];
     };
     bias_of(0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = b[j];
     load(s0, 0, LOADS), next_tile();
@@ -707,7 +603,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2)
     int kt = 0, e = 0;
     // this lane's fragments: rows ar, ar + 32 of A and br, br + 32 of B, chunk (kk / 8 + lane / 32) ^ swz of
     // k step kk (32 rows on the swizzle is the same), as offsets into a stage
-    const int ar = wm * 64 + (lane & 31), br = TM + wn * 64 + (lane & 31);
+    const int ar = wm * 32 * MI + (lane & 31), br = TM + wn * 32 * NJ + (lane & 31);
     int ao[BKL / 16], bo[BKL / 16];
 #pragma unroll
     for (int q = 0; q < BKL / 16; ++q) {
@@ -719,23 +615,19 @@ __global__ void __launch_bounds__(64 * WM * WN, 2)
         // the tile has landed when no more than the STAGES - 2 tiles after it are in flight; past the
         // barrier that holds for every wave, and every wave is done with the tile before
         constexpr int PENDING = LOADS * (STAGES - 2);
-        static_assert(PENDING == 0 || PENDING == 6 || PENDING == 8, "a wait for each");
-        if constexpr (PENDING == 6) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-        else if constexpr (PENDING == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(PENDING) : "memory");
         __builtin_amdgcn_s_barrier();
-        if (kt == nk - 1 && (e + 1) % kWideBiases == 0 && e + 1 < members) {
+        if (kt == nk - 1 && (e + 1) % kBiasMembers == 0 && e + 1 < members) {
             fill_biases(e + 1);  // (every wave is past the member before)
             __builtin_amdgcn_s_barrier();
         }
         asm volatile("" ::: "memory");
-        bf16x8 fa[2][2], fb[2][2];  // the fragments of k step q and the next
+        bf16x8 fa[2][MI], fb[2][NJ];  // the fragments of k step q and the next
         auto read = [&](int q) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                fa[q & 1][i] = *(const bf16x8 *)(at + ao[q] + i * 32 * BKL);
-                fb[q & 1][i] = *(const bf16x8 *)(at + bo[q] + i * 32 * BKL);
-            }
+            for (int i = 0; i < MI; ++i) fa[q & 1][i] = *(const bf16x8 *)(at + ao[q] + i * 32 * BKL);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) fb[q & 1][j] = *(const bf16x8 *)(at + bo[q] + j * 32 * BKL);
         };
         read(0);
 #pragma unroll
@@ -743,15 +635,15 @@ __global__ void __launch_bounds__(64 * WM * WN, 2)
             if (q + 1 < BKL / 16) read(q + 1);
             load(to, q * LOADS / (BKL / 16), (q + 1) * LOADS / (BKL / 16));
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < MI; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+                for (int j = 0; j < NJ; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[q & 1][i], fb[q & 1][j], acc[i][j], 0, 0, 0);
         }
         next_tile();
         if (++kt == nk) {
             bias_of(e + 1);  // (of no use after the last)
-            welford_update<2, 2>(acc, mu, m2, e, b);
+            welford_update<MI, NJ>(acc, mu, m2, e, b);
             kt = 0;
             ++e;
         }
@@ -776,7 +668,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the re-reads, before a stage is used again
     __syncthreads();
     double(*const red)[TM][2] = (double(*)[TM][2])s0;
-    ensemble_store<2, 2>(mu, m2, tm * TM, tn * TN, wm, wn, M, N, mean, ldm, scale, part != nullptr, red);
+    ensemble_store<MI, NJ>(mu, m2, tm * TM, tn * TN, wm, wn, M, N, mean, ldm, scale, part != nullptr, red);
     if (!part) return;
     __syncthreads();
     for (int r = t; r < 2 * TM; r += THREADS) {
@@ -785,26 +677,31 @@ __global__ void __launch_bounds__(64 * WM * WN, 2)
     }
 }
 
-// spread[m] = ||standard deviation over members|| / ||mean|| from the sums of `tiles` tiles
-// per row: 64 rows per block, 16 threads a row over the tiles, then over the threads in order.
+// spread[m] = ||standard deviation over members|| / ||mean|| from the sums of `tiles` tiles per row:
+// kSpreadRows rows per block, 64 threads a row over the tiles, then over the threads in order.  Latency
+// bounds it: 64 rows and 16 threads a row took 40 us on 1024 rows of 1184 tiles (16 blocks on 256 CUs),
+// this 14 us.
+constexpr int kSpreadRows = 16;
+
 __global__ void __launch_bounds__(1024) ensemble_spread(const double *__restrict__ part, int tiles, int M, int members,
                                                         float *__restrict__ spread)
 {
-    __shared__ double red[2][16][64];
-    const int lane = threadIdx.x & 63, g = threadIdx.x >> 6, m = blockIdx.x * 64 + lane;
+    __shared__ double red[2][64][kSpreadRows];
+    const int r = threadIdx.x % kSpreadRows, g = threadIdx.x / kSpreadRows, m = blockIdx.x * kSpreadRows + r;
     double var = 0, nrm = 0;
     if (m < M)
-        for (int t = g; t < tiles; t += 16) {
+#pragma unroll 4
+        for (int t = g; t < tiles; t += 64) {
             var += part[((size_t)t * 2 + 0) * M + m];
             nrm += part[((size_t)t * 2 + 1) * M + m];
         }
-    red[0][g][lane] = var;
-    red[1][g][lane] = nrm;
+    red[0][g][r] = var;
+    red[1][g][r] = nrm;
     __syncthreads();
     if (g || m >= M) return;
-    for (int k = 1; k < 16; ++k) {
-        var += red[0][k][lane];
-        nrm += red[1][k][lane];
+    for (int k = 1; k < 64; ++k) {
+        var += red[0][k][r];
+        nrm += red[1][k][r];
     }
     spread[m] = (float)(sqrt(var / (members > 1 ? members - 1 : 1)) / fmax(sqrt(nrm), 1e-30));
 }
@@ -1056,24 +953,24 @@ hipError_t ensemble_output(const uint16_t *A, int lda, size_t stride_a, const ui
                            const float *const *biases, int members, int M, int N, int K, float *mean, size_t ldm,
                            const float *scale, double *part, float *spread, hipStream_t stream)
 {
-    if (M < 1 || N < 1 || K < BK || K % BK || lda % 8 || ldb % 8 || lda < K || ldb < K || members < 1 || (spread && !part))
+    if (M < 1 || N < 1 || K < 64 || K % 64 || lda % 8 || ldb % 8 || lda < K || ldb < K || members < 1 || (spread && !part))
         return hipErrorInvalidValue;
     if (!spread) part = nullptr;
     const auto tiles = [&](int tm, int tn) { return (long long)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
-    const bool wide = tiles(128, 128) >= kEnsembleWideTiles;
-    const bool tall = wide && K % 64 == 0 && tiles(256, 128) * 256 <= tiles(128, 128) * 128 * kEnsembleTallGain;
-    const int rows = tall ? 256 : wide ? 128 : 64, width = wide ? 128 : 64;
-    const int tiles_n = (N + width - 1) / width, blocks = (int)tiles(rows, width);
+    const auto cost = [&](int tm, int tn, int slots, float tile) { return std::max(1.f, tiles(tm, tn) / (float)slots) * tile; };
+    const float c64 = cost(64, 64, 2 * kCus, 1.f), c128 = cost(128, 128, 2 * kCus, kCostSquare);
+    const bool tall = cost(256, 128, kCus, kCostTall) < std::min(c64, c128), square = !tall && c128 < c64;
+    const int tiles_n = (N + (tall || square ? 127 : 63)) / (tall || square ? 128 : 64);
+    const int blocks = (int)(tall ? tiles(256, 128) : square ? tiles(128, 128) : tiles(64, 64));
     auto launch = [&](auto kernel, int threads) {
         kernel<<<blocks, threads, 0, stream>>>(A, lda, stride_a, bs, ldb, biases, M, N, K, members, mean, ldm, scale, part);
     };
-    if (tall) launch(ensemble_wide<4, 2, 64, 3>, 512);
-    else if (wide && K % 64 == 0) launch(ensemble_wide<2, 2, 64, 2>, 256);
-    else if (wide) launch(ensemble_wide<2, 2, 32, 4>, 256);
-    else launch(ensemble_nt<1, 1>, 256);
+    if (tall) launch(ensemble_tiles<4, 2, 2, 2, 3>, 512);
+    else if (square) launch(ensemble_tiles<2, 2, 2, 2, 2>, 256);
+    else launch(ensemble_tiles<2, 2, 1, 1, 4>, 256);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !spread) return e;
-    ensemble_spread<<<(M + 63) / 64, 1024, 0, stream>>>(part, tiles_n, M, members, spread);
+    ensemble_spread<<<(M + kSpreadRows - 1) / kSpreadRows, 1024, 0, stream>>>(part, tiles_n, M, members, spread);
     return hipGetLastError();
 }
 

@@ -256,17 +256,17 @@ def test_settings_made_right_after_creation_hold():
         assert np.array_equal(scaled, 2.0 * plain) and np.all(plain.any(axis=0))
 
 
-@pytest.mark.parametrize("sizes,rows,members,batch", [([8, 1], 1, 1, 96), ([8, 63], 65, 2, 96),
+@pytest.mark.parametrize("sizes,rows,members,batch", [([8, 1], 1, 1, 96), ([8, 63], 65, 20, 96),
                                                       ([8, 64, 65], 63, 3, 96), ([8, 96, 64, 129], 130, 5, 96),
                                                       ([4, 64, 65600], 130, 2, 96), ([4, 160, 70001], 97, 3, 96),
                                                       ([8, 200, 16500], 300, 3, 320), ([8, 16513], 257, 18, 288),
-                                                      ([4, 500, 8200], 700, 18, 512),
-                                                      ([4, 500, 8200], 300, 17, 320)])
+                                                      ([4, 500, 17000], 700, 18, 704),
+                                                      ([4, 500, 34000], 257, 17, 288)])
 def test_predict_statistics_match_the_members_outputs(sizes, rows, members, batch):
     """The ensemble mean and spread formed with the output layers equal those of the members' own
     forward passes (sums of up to 512 FP32 products in another order: 1e-5 relative), at the
-    remainders of the 64 x 64, 128 x 128 and 256 x 128 tiles, with k tiles of 32 and 64, more rows than
-    one batch, one layer alone, and more members than the wide kernel holds biases of."""
+    remainders of the 64 x 64, 128 x 128 and 256 x 128 tiles, more rows than one batch, one layer alone,
+    and more members than a block holds biases of."""
     rng = np.random.default_rng(rows)
     with Network(sizes, members=members, max_batch=batch, seed=rows) as net:
         x = rng.standard_normal((rows, sizes[0])).astype(np.float32)
