@@ -7,18 +7,19 @@
 // neighbours the thread's own; only the two or three rows at a wave's ends go through LDS, its
 // velocities before the stresses and its stresses before the velocities, one barrier each.  A step
 // consumes three rows and columns of the region on each side, so a region of 64 x 8 P points stores
-// 52 x (8 P - 12): 52 x 36 for P = 6 (FP32 tiles away from the border) and 52 x 12 for P = 3 (twice
-// the blocks; and the tiles at C-PML strips and the border, whose twelve memory variables per point
-// stay in registers from load to store).
+// 52 x (8 P - 12) of two steps: 52 x 36 for P = 6 (FP32 tiles away from the border), 52 x 20 for P = 4
+// (tiles at the C-PML strips or the border of one axis, whose six memory variables per point stay in
+// registers from load to store) and 52 x 12 for P = 3 (corners, with twelve; or twice the blocks).  Lower
+// tiles load and compute only the rows they need.
 //
 // What bounds it.  Every load of a tile is issued at the start, so a launch pays one memory latency
 // where a block marching down its rows pays one per row step (about 2 us each, 4 with C-PML records):
-// two steps of a 161^2 grid take 12 us instead of 119, 401^2 14 instead of 122, 701 x 523 FP64 33
-// instead of 127 (two single-step launches).  Large grids are bound by HBM: 4001^2 takes 258 us per
-// launch at 52 x 36 against 298 for the marching kernel, 1.17 GB (1.04 compulsory) at 4.5 TB/s, the
-// VALU busy 58 % of the time (128 VGPRs, four waves per SIMD, two blocks per CU).  With every row in
-// LDS planes, x neighbours read from them and four barriers per step it took 262 us, 1201^2 39 us
-// instead of 35.5.
+// two steps of a 161^2 grid take 11 us instead of 119, 401^2 12 instead of 122, 701 x 523 FP64 28
+// instead of 127 (two single-step launches).  Large grids are bound by HBM: 4001^2 takes 231 us per
+// launch against 298 for the marching kernel, 1.17 GB (1.04 compulsory) at 5.0 TB/s (128 VGPRs, four
+// waves per SIMD, two blocks per CU).  Mid-sized ones by their edges' wider halo: with P = 3 and both
+// axes' code along every edge, 401^2 took 6.1 us a step instead of 5.0 (three steps per launch), 801^2
+// 12.0 instead of 8.8, 1201^2 16.7 instead of 15.1, 64 models of 401^2 127 instead of 103.
 //
 // The arithmetic is the single-step kernel's expression by expression, so results equal it bit for
 // bit; state buffers alternate as the marching two-step kernel's.
@@ -29,7 +30,6 @@
 
 namespace poe2d {
 
-constexpr int kTileCus = 256;  // compute units
 constexpr int kTileThreads = 512, kTileWaves = kTileThreads / 64;
 
 // Rows a wave publishes to its neighbours, before the stresses (its velocities) and before the
@@ -69,14 +69,17 @@ __device__ __forceinline__ T ddx_bwd(T f, T rh)
 }
 
 // One region: 64 columns (one per lane) x kTileWaves * P rows (P consecutive rows per thread, in
-// registers).  nst steps from step n.
-template <class T, int P, bool AVG, bool PAL, bool EDGE, bool ROOM>
+// registers).  nst steps from step n.  EDGE: the region reaches x strips or the outer columns (EDGE_X),
+// z strips or the outer rows (EDGE_Z).
+enum { EDGE_X = 1, EDGE_Z = 2 };
+template <class T, int P, bool AVG, bool PAL, int EDGE, bool ROOM>
 __device__ __forceinline__ void tile_region(const __attribute__((address_space(4))) StepArgs<T> &A, const TileItem it, const long long n, const int in, const int halo, const int nst, const bool stream,
                                             T (*const bv)[kTileWaves][64], T (*const bs)[kTileWaves][64],
                                             T (*const xtab)[64], const Vec4<T> *lpal)
 {
     constexpr uint32_t VB = sizeof(Vec4<T>);
-    constexpr int RH = kTileWaves * P;  // the region's rows
+    constexpr bool EX = EDGE & EDGE_X, EZ = EDGE & EDGE_Z;
+    const int rows = min(it.z1 - it.z0 + 2 * halo, kTileWaves * P);  // the region's rows (the last waves' may be past it)
     typedef __attribute__((address_space(1))) nvec4<T> GN;
     typedef __attribute__((address_space(1))) T GT;
     typedef __attribute__((address_space(1))) const T GCT;
@@ -96,7 +99,7 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
     const long long gsb = A.group_stride * (long long)VB;
     const int cc = min(max(c, -kPadCols), nx + 1);
     const uint32_t rowb = (uint32_t)pitch * VB;
-    const int last_row = nz + kPadRows;
+    const int last_row = min(nz + kPadRows, it.z0 - halo + rows - 1);
     auto prow = [&](int z) -> uint32_t { return (uint32_t)(min(z, last_row) + kPadRows); };
     auto off = [&](int z) -> uint32_t { return (uint32_t)(cc + kPadCols) * VB + prow(z) * rowb; };
     auto ld = [&](const gchar *g, int z) -> Vec4<T> {
@@ -112,22 +115,22 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
     for (int i = 0; i < P; ++i) S[i] = ld(So, z0 + i);
 
     // material: palette entries of rows 0 .. P, or the coefficient groups (read where used)
-    constexpr bool PACK = EDGE;  // entries of four rows in one register (P = 3)
-    static_assert(!PACK || P == 3, "four bytes");
-    int id[PACK ? 1 : P + 1];
+    constexpr bool PACK = EDGE;  // entries of four rows in one register
+    int id[PACK ? P / 4 + 1 : P + 1];
     auto entry = [&](int i) -> int {
-        if constexpr (PACK) return (id[0] >> (8 * i)) & 255;
+        if constexpr (PACK) return (id[i / 4] >> (8 * (i % 4))) & 255;
         else return id[i];
     };
     const gchar *const MSg = (const gchar *)A.mat + G_MS * gsb;
     const gchar *const MVg = (const gchar *)A.mat + G_MV * gsb;
     if constexpr (PAL) {
         gcuchar *const mid = (gcuchar *)A.mid;
-        if constexpr (PACK) id[0] = 0;
+        if constexpr (PACK)
+            for (int &q : id) q = 0;
 #pragma unroll
         for (int i = 0; i <= P; ++i) {
             const int e = mid[(uint32_t)(cc + kPadCols) + prow(z0 + i) * (uint32_t)pitch];
-            if constexpr (PACK) id[0] |= e << (8 * i);
+            if constexpr (PACK) id[i / 4] |= e << (8 * (i % 4));
             else id[i] = e;
         }
     }
@@ -135,10 +138,10 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
     // C-PML: memory variables of this thread's points and the profiles of its column and rows
     // (a column's profiles in registers; in LDS, a few per cent slower on launches of one tile per CU,
     // where FP32 blocks share a CU: there they would spill)
-    constexpr bool XLDS = EDGE && sizeof(T) == 4 && !ROOM;
+    constexpr bool XLDS = EX && sizeof(T) == 4 && !ROOM;
     const bool inx = c >= 0 && c <= nx;
-    const int sx = (EDGE && inx) ? ((gcint *)A.xmap)[c] : -1;
-    T qx[EDGE ? P : 1][NPSI_X], qz[EDGE ? P : 1][NPSI_Z];
+    const int sx = (EX && inx) ? ((gcint *)A.xmap)[c] : -1;
+    T qx[EX ? P : 1][NPSI_X], qz[EZ ? P : 1][NPSI_Z];
     GT *const psi = (GT *)A.psi;
     auto px = [&](int b, int z) -> GT * { return psi + ((long long)b * A.pxn + (long long)z * A.wxs + sx) * NPSI_X; };
     auto pz = [&](int b, int s) -> GT * {
@@ -151,39 +154,45 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
 #pragma unroll
         for (int i = 0; i < P; ++i) {
 #pragma unroll
-            for (int q = 0; q < NPSI_X; ++q) qx[i][q] = qz[i][q] = T(0);
-            const int z = z0 + i;
-            if (sx >= 0 && z >= 0 && z <= nz) {
-                const GP *const r = (const GP *)px(in, z);
-#pragma unroll
-                for (int q = 0; q < NPSI_X / 2; ++q) {
-                    const pair v = r[q];
-                    qx[i][2 * q] = v.x, qx[i][2 * q + 1] = v.y;
-                }
+            for (int q = 0; q < NPSI_X; ++q) {
+                if constexpr (EX) qx[i][q] = T(0);
+                if constexpr (EZ) qz[i][q] = T(0);
             }
-            const int s = strip(z);
-            if (s >= 0 && inx) {
-                const GP *const r = (const GP *)pz(in, s);
+            const int z = z0 + i;
+            if constexpr (EX)
+                if (sx >= 0 && z >= 0 && z <= min(nz, last_row)) {
+                    const GP *const r = (const GP *)px(in, z);
 #pragma unroll
-                for (int q = 0; q < NPSI_Z / 2; ++q) {
-                    const pair v = r[q];
-                    qz[i][2 * q] = v.x, qz[i][2 * q + 1] = v.y;
+                    for (int q = 0; q < NPSI_X / 2; ++q) {
+                        const pair v = r[q];
+                        qx[i][2 * q] = v.x, qx[i][2 * q + 1] = v.y;
+                    }
+                }
+            if constexpr (EZ) {
+                const int s = strip(z);
+                if (s >= 0 && inx && z <= last_row) {
+                    const GP *const r = (const GP *)pz(in, s);
+#pragma unroll
+                    for (int q = 0; q < NPSI_Z / 2; ++q) {
+                        const pair v = r[q];
+                        qz[i][2 * q] = v.x, qz[i][2 * q + 1] = v.y;
+                    }
                 }
             }
         }
     }
     const KT *const ktab = (const KT *)A.tab;
-    T xr[EDGE && !XLDS ? NXTAB : 1];
-    if constexpr (EDGE && !XLDS)
+    T xr[EX && !XLDS ? NXTAB : 1];
+    if constexpr (EX && !XLDS)
 #pragma unroll
         for (int k = 0; k < NXTAB; ++k) xr[k] = inx ? ((const GCT *)A.tab)[(TB_AX + k) * A.tn + c] : T(0);
-    auto xt = [&](int k) -> T { return XLDS ? xtab[k - TB_AX][lane] : xr[EDGE && !XLDS ? k - TB_AX : 0]; };
+    auto xt = [&](int k) -> T { return XLDS ? xtab[k - TB_AX][lane] : xr[EX && !XLDS ? k - TB_AX : 0]; };
 
-    const bool xr1 = !EDGE || (c >= 1 && c < nx);      // stress1
-    const bool xr2 = !EDGE || (c >= 2 && c < nx);      // stress2
-    const bool xr3 = !EDGE || (c >= 1 && c < nx - 1);  // stress3
-    const bool xr4 = !EDGE || (c >= 2 && c < nx);      // vx
-    const bool xr5 = !EDGE || (c >= 1 && c < nx - 1);  // vz
+    const bool xr1 = !EX || (c >= 1 && c < nx);      // stress1
+    const bool xr2 = !EX || (c >= 2 && c < nx);      // stress2
+    const bool xr3 = !EX || (c >= 1 && c < nx - 1);  // stress3
+    const bool xr4 = !EX || (c >= 2 && c < nx);      // vx
+    const bool xr5 = !EX || (c >= 1 && c < nx - 1);  // vz
     const bool src_p = A.src_kind == POE2D_SRC_PRESSURE_DGAUSS && c == A.src_x;
     const bool src_f = A.src_kind == POE2D_SRC_FORCE_Y_RICKER && c == A.src_x;
 
@@ -254,9 +263,9 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
             for (int i = 0; i < P; ++i) {
                 sxx[i] = syy[i] = p[i] = T(0);
                 const int z = z0 + i;
-                if (r0 + i < 3 * k + 1 || r0 + i > RH - 2 - 3 * k) continue;
-                const int szs = EDGE ? strip(z) : -1;
-                const bool u1 = xr1 && (!EDGE || (z >= 2 && z < nz - 1)), u2 = xr2 && (!EDGE || (z >= 1 && z < nz - 1));
+                if (r0 + i < 3 * k + 1 || r0 + i > rows - 2 - 3 * k) continue;
+                const int szs = EZ ? strip(z) : -1;
+                const bool u1 = xr1 && (!EZ || (z >= 2 && z < nz - 1)), u2 = xr2 && (!EZ || (z >= 1 && z < nz - 1));
                 Vec4<T> ms;
                 T mu_nxt;
                 if constexpr (PAL) {
@@ -276,16 +285,16 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
                 if (u1) {
                     T dvz = d4(vy[i + 2], vy[i + 1], vy[i + 3], vy[i], rdz);
                     T dwz = d4(wy[i + 2], wy[i + 1], wy[i + 3], wy[i], rdz);
-                    if constexpr (EDGE) {
+                    if constexpr (EX)
                         if (sx >= 0) {
                             dvx = cpml_held(dvx, qx[i][PX_DVX], xt(TB_AXH), xt(TB_BXH), xt(TB_RKXH));
                             dwx = cpml_held(dwx, qx[i][PX_DWX], xt(TB_AXH), xt(TB_BXH), xt(TB_RKXH));
                         }
+                    if constexpr (EZ)
                         if (szs >= 0) {
                             dvz = cpml_held(dvz, qz[i][PZ_DVZ], az, bz, rkz);
                             dwz = cpml_held(dwz, qz[i][PZ_DWZ], az, bz, rkz);
                         }
-                    }
                     S[i].x = S[i].x + dt * dvx;
                     S[i].y = S[i].y + dt * dvz;
                     S[i].z = (S[i].z - dwx * dt) - dwz * dt;
@@ -300,11 +309,11 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
                 }
                 if (u2) {
                     T ddz = d4(vx[i + 2], vx[i + 1], vx[i + 3], vx[i], rdz);
-                    if constexpr (EDGE) {
+                    if constexpr (EX)
                         if (sx >= 0) ddx = cpml_held(ddx, qx[i][PX_DVY], xt(TB_AX), xt(TB_BX), xt(TB_RKX));
-                        // half-grid memory coefficients, full-grid K_z divisor (reference :224-226)
+                    // half-grid memory coefficients, full-grid K_z divisor (reference :224-226)
+                    if constexpr (EZ)
                         if (szs >= 0) ddz = cpml_held(ddz, qz[i][PZ_DVX], azh, bzh, rkz);
-                    }
                     const T mu_xy = AVG ? harmonic_mu(ms.w, mu_nxt) : mu_nxt;
                     S[i].w = S[i].w + mu_xy * (ddx + ddz) * dt;
                 }
@@ -330,9 +339,9 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
 #pragma unroll
             for (int i = 0; i < P; ++i) {
                 const int z = z0 + i;
-                if (r0 + i < 3 * k + 3 || r0 + i > RH - 4 - 3 * k) continue;
-                const int szj = EDGE ? strip(z) : -1;
-                const bool u4 = xr4 && (!EDGE || (z >= 2 && z < nz)), u5 = xr5 && (!EDGE || (z >= 1 && z < nz - 1));
+                if (r0 + i < 3 * k + 3 || r0 + i > rows - 4 - 3 * k) continue;
+                const int szj = EZ ? strip(z) : -1;
+                const bool u4 = xr4 && (!EZ || (z >= 2 && z < nz)), u5 = xr5 && (!EZ || (z >= 1 && z < nz - 1));
                 Vec4<T> mv, mv1, cn, cn1;
                 if constexpr (PAL) {
                     mv = lpal[PAL_MV * kMaxPalette + entry(i)];
@@ -355,13 +364,13 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
                     T e1 = dsx;
                     T e2 = dpx;
                     T e3 = d4(sh[i + 2], sh[i + 1], sh[i + 3], sh[i], rdz);
-                    if constexpr (EDGE) {
+                    if constexpr (EX)
                         if (sx >= 0) {
                             e1 = cpml_held(e1, qx[i][PX_DSXX], xt(TB_AX), xt(TB_BX), xt(TB_RKX));
                             e2 = cpml_held(e2, qx[i][PX_DPX], xt(TB_AX), xt(TB_BX), xt(TB_RKX));
                         }
+                    if constexpr (EZ)
                         if (szj >= 0) e3 = cpml_held(e3, qz[i][PZ_DSXY], az, bz, rkz);
-                    }
                     if constexpr (PAL && sizeof(T) == 4)
                         biot_velocity_cn(V[i].x, V[i].z, e1 + e3, e2, mv.x, mv.y, mv.z, cn);
                     else
@@ -371,13 +380,13 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
                     T e1 = dhx;
                     T e2 = d4(sy[i + 2], sy[i + 1], sy[i + 3], sy[i], rdz);
                     T e3 = d4(pp[i + 2], pp[i + 1], pp[i + 3], pp[i], rdz);
-                    if constexpr (EDGE) {
+                    if constexpr (EX)
                         if (sx >= 0) e1 = cpml_held(e1, qx[i][PX_DSXY], xt(TB_AXH), xt(TB_BXH), xt(TB_RKXH));
+                    if constexpr (EZ)
                         if (szj >= 0) {
                             e2 = cpml_held(e2, qz[i][PZ_DSYY], azh, bzh, rkzh);
                             e3 = cpml_held(e3, qz[i][PZ_DPZ], azh, bzh, rkzh);
                         }
-                    }
                     T div = e1 + e2;
                     if (src_f && z == A.src_z) div += srcv;
                     if constexpr (AVG) {
@@ -419,16 +428,19 @@ __device__ __forceinline__ void tile_region(const __attribute__((address_space(4
         if constexpr (EDGE) {
             typedef T pair __attribute__((ext_vector_type(2)));
             typedef __attribute__((address_space(1))) pair GP;
-            if (sx >= 0) {
-                GP *const r = (GP *)px(in ^ 1, z);
+            if constexpr (EX)
+                if (sx >= 0) {
+                    GP *const r = (GP *)px(in ^ 1, z);
 #pragma unroll
-                for (int q = 0; q < NPSI_X / 2; ++q) r[q] = pair{qx[i][2 * q], qx[i][2 * q + 1]};
-            }
-            const int s = strip(z);
-            if (s >= 0) {
-                GP *const r = (GP *)pz(in ^ 1, s);
+                    for (int q = 0; q < NPSI_X / 2; ++q) r[q] = pair{qx[i][2 * q], qx[i][2 * q + 1]};
+                }
+            if constexpr (EZ) {
+                const int s = strip(z);
+                if (s >= 0) {
+                    GP *const r = (GP *)pz(in ^ 1, s);
 #pragma unroll
-                for (int q = 0; q < NPSI_Z / 2; ++q) r[q] = pair{qz[i][2 * q], qz[i][2 * q + 1]};
+                    for (int q = 0; q < NPSI_Z / 2; ++q) r[q] = pair{qz[i][2 * q], qz[i][2 * q + 1]};
+                }
             }
         }
     }
@@ -462,9 +474,16 @@ __global__ void __launch_bounds__(kTileThreads, sizeof(T) == 4 && !ROOM ? 4 : 2)
             lpal[e] = Vec4<T>{v.x, v.y, v.z, v.w};
         }
     }
-    if (it.kind == TILE_EDGE) tile_region<T, 3, AVG, PAL, true, ROOM>(A, it, n, in, halo, nst, stream, bv, bs, xtab, lpal);
-    else if (it.kind == TILE_SHORT) tile_region<T, 3, AVG, PAL, false, ROOM>(A, it, n, in, halo, nst, stream, bv, bs, xtab, lpal);
-    else tile_region<T, tile_tall_p(sizeof(T) == 4, PAL), AVG, PAL, false, ROOM>(A, it, n, in, halo, nst, stream, bv, bs, xtab, lpal);
+    auto region = [&](auto p, auto edge) {
+        tile_region<T, decltype(p)::value, AVG, PAL, decltype(edge)::value, ROOM>(A, it, n, in, halo, nst, stream, bv, bs, xtab, lpal);
+    };
+    using std::integral_constant;
+    constexpr integral_constant<int, tile_edge_p(PAL)> edge_p{};
+    if (it.kind == TILE_EDGE) region(integral_constant<int, 3>{}, integral_constant<int, EDGE_X | EDGE_Z>{});
+    else if (it.kind == TILE_EDGE_X) region(edge_p, integral_constant<int, EDGE_X>{});
+    else if (it.kind == TILE_EDGE_Z) region(edge_p, integral_constant<int, EDGE_Z>{});
+    else if (it.kind == TILE_SHORT) region(integral_constant<int, 3>{}, integral_constant<int, 0>{});
+    else region(integral_constant<int, tile_tall_p(sizeof(T) == 4, PAL)>{}, integral_constant<int, 0>{});
 }
 
 template <class T>

@@ -47,7 +47,6 @@ const double kStabilityThreshold = 1.0e25;  // STABILITY_THRESHOLD of the refere
 const int kGraphSteps = 32;                 // steps per captured graph
 const size_t kL2Bytes = size_t(32) << 20;   // the eight L2s together
 const size_t kMallBytes = size_t(256) << 20;  // the memory-side cache
-const int kTileSlots = 512;                 // tiles of the FP32 tile kernel the chip holds at once (half as many FP64)
 const int kBandTiles = 8;                   // tile columns to a band of the tile kernel's work order
 
 #define HIP_TRY(expr)                                                                              \
@@ -694,14 +693,25 @@ poe2d_status build_list(StepList &L, const std::vector<poe2d_solver *> &members,
     return POE2D_OK;
 }
 
-// The tiles of member i's grid for `steps` steps per launch, with their receivers: short rows where
-// the region reaches a C-PML strip or the border (edge tiles), tall_rows (if more) elsewhere.
-void cut_tiles(const poe2d_solver *s, int i, int steps, int tall_rows, std::vector<TileItem> &edge,
-               std::vector<TileItem> &inter, std::vector<int> &ptr, std::vector<int2> &ent)
+// The tiles of a launch and their receivers.
+struct TileCut {
+    std::vector<TileItem> edge, inter;
+    std::vector<int> ptr;
+    std::vector<int2> ent;
+
+    size_t tiles() const { return edge.size() + inter.size(); }
+};
+
+// Member i's part of it, `steps` steps per launch.  A column of tiles is three bands: the rows whose region
+// reaches the upper z strip or border, those away from both, and the lower ones; the tiles of a band are
+// of equal height (+- 1), at most short_rows at a corner, edge_rows along an edge and tall_rows elsewhere.
+void cut_tiles(const poe2d_solver *s, int i, int steps, int short_rows, int edge_rows, int tall_rows, TileCut &out)
 {
     const Model *md = s->m;
-    const int halo = tile_halo(steps), cols = tile_cols(steps), short_rows = tile_rows(3, steps);
+    const int halo = tile_halo(steps), cols = tile_cols(steps);
     const int nx = s->grid.nx, nz = s->grid.nz;
+    const int xlo = std::max(md->xlo, 2), xhi = std::min(md->xhi, nx - 1);
+    const int zlo = std::max(md->ztop, 2), zhi = std::min(md->zbot, nz - 1);
     // receivers by tile column and row
     std::vector<int> order(s->nrec);
     for (int r = 0; r < s->nrec; ++r) order[r] = r;
@@ -710,42 +720,46 @@ void cut_tiles(const poe2d_solver *s, int i, int steps, int tall_rows, std::vect
         return ta != tb ? ta < tb : s->hrz[a] < s->hrz[b];
     });
     size_t next = 0;
-    const int zlo = std::max(md->ztop, 2), zhi = std::min(md->zbot, nz - 1);
     for (int x0 = 0; x0 <= nx; x0 += cols) {
         const int c0 = x0 - halo, c1 = c0 + 63;  // the region's columns
-        const bool xs = c0 < std::max(md->xlo, 2) || c1 >= std::min(md->xhi, nx - 1);
+        const bool xs = c0 < xlo || c1 >= xhi;
+        const int upper = std::min(zlo + halo, nz + 1), lower = std::max(zhi - halo, upper);
         for (int z0 = 0; z0 <= nz;) {
-            // rows [z0 - halo, z0 + rows + halo) of the region within [zlo, zhi)
-            auto inside = [&](int rows) { return !xs && z0 - halo >= zlo && z0 + rows + halo <= zhi; };
+            const bool zs = z0 < upper || z0 >= lower;
+            const int end = z0 < upper ? upper : z0 < lower ? std::min(lower, nz + 1) : nz + 1;
+            const int most = xs && zs ? short_rows : xs || zs ? edge_rows : tall_rows;
+            const int count = (end - z0 + most - 1) / most;
             TileItem it{};
             it.model = i;
             it.x0 = x0;
             it.z0 = z0;
-            it.kind = tall_rows > short_rows && inside(tall_rows) ? TILE_TALL : inside(short_rows) ? TILE_SHORT : TILE_EDGE;
-            it.z1 = std::min(z0 + (it.kind == TILE_TALL ? tall_rows : short_rows), nz + 1);
+            it.z1 = z0 + (end - z0 + count - 1) / count;
+            it.kind = !xs && !zs ? (tall_rows > short_rows ? TILE_TALL : TILE_SHORT)
+                      : tall_rows == short_rows || (xs && zs) ? TILE_EDGE : xs ? TILE_EDGE_X : TILE_EDGE_Z;
             it.rec = -1;
             auto pending = [&](int z) {
                 return next < order.size() && s->hrx[order[next]] < x0 + cols && s->hrz[order[next]] < z;
             };
             if (pending(it.z1)) {
-                it.rec = (int)ptr.size();
+                it.rec = (int)out.ptr.size();
                 for (int z = z0; z < it.z1; ++z) {
-                    ptr.push_back((int)ent.size());
-                    for (; pending(z + 1); ++next) ent.push_back(int2{s->hrx[order[next]], order[next]});
+                    out.ptr.push_back((int)out.ent.size());
+                    for (; pending(z + 1); ++next) out.ent.push_back(int2{s->hrx[order[next]], order[next]});
                 }
-                ptr.push_back((int)ent.size());
+                out.ptr.push_back((int)out.ent.size());
             }
-            (it.kind == TILE_EDGE ? edge : inter).push_back(it);
+            (xs || zs ? out.edge : out.inter).push_back(it);
             z0 = it.z1;
         }
     }
 }
 
-// As build_list, for the tile kernel, `steps` steps per launch.  steps = 0: three where the chip holds
-// every tile of the launch at once, else two: such launches are bound by latency and the cost of a
-// launch, which three steps share (us per step, three / two: 161^2 4.9 / 5.9, 401^2 6.4 / 6.5, 401^2
-// continuous 7.3 / 7.8), others by HBM or instruction issue, where the wider halo costs more (1201^2
-// 20.0 / 16.9, 2001^2 40.4 / 36.1, FP64 401^2 10.5 / 8.8).
+// As build_list, for the tile kernel, `steps` steps per launch.  steps = 0: three or two, by the rounds in
+// which the chip takes the tiles (two blocks per CU, one of FP64; up to one block per CU a round is a
+// fifth shorter), since three steps take a block 1.28 times as long as two, 0.85 of it per step.  us per
+// step, three / two (tiles): 401^2 4.97 / 5.79 (196 / 132), 601^2 6.4 / 7.5 (422 / 268), 701^2 9.2 / 7.9
+// (532 / 359), 1201^2 15.5 / 15.0 (1356 / 948); averaged material, 1001 x 777 12.3 / 14.1 (724 / 554); no
+// palette, 401^2 6.6 / 6.0 (379 / 214); FP64, 241^2 6.4 / 7.6 (126 / 74), 401^2 9.2 / 8.0 (287 / 180).
 template <class T>
 poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members, int steps, bool tall, bool palette,
                          int nsteps, hipStream_t stream)
@@ -758,20 +772,28 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
         if (s->grid.staggered_material != material)
             return fail(POE2D_E_INVALID, "run: batch members differ in staggered material");
     }
-    std::vector<TileItem> edge, inter;
-    std::vector<int> ptr;
-    std::vector<int2> ent;
-    const bool choose = steps == 0;
-    if (choose) steps = 3;
-    for (int i = 0; i < nm; ++i) {
-        cut_tiles(members[i], i, steps, tall ? tile_rows(tile_tall_p(sizeof(T) == 4, palette), steps) : 0, edge, inter, ptr, ent);
-        if (edge.size() + inter.size() > (1u << 28)) return fail(POE2D_E_INVALID, "run: too many tiles in one launch");
-        if (choose && steps == 3 && edge.size() + inter.size() > (size_t)kTileSlots * 4 / sizeof(T)) {
-            edge.clear(), inter.clear(), ptr.clear(), ent.clear();
-            steps = 2;
-            i = -1;  // again, for two steps
-        }
+    const auto cut = [&](int k) {
+        const int rows = tile_rows(3, k);
+        TileCut c;
+        for (int i = 0; i < nm; ++i)
+            cut_tiles(members[i], i, k, rows, tall ? tile_rows(tile_edge_p(palette), k) : rows,
+                      tall ? tile_rows(tile_tall_p(sizeof(T) == 4, palette), k) : rows, c);
+        return c;
+    };
+    const auto rounds = [](size_t tiles) {
+        const size_t slots = kTileCus * (sizeof(T) == 4 ? 2 : 1);
+        return tiles <= (size_t)kTileCus ? 1.0 : (sizeof(T) == 4 ? 1.25 : 1.0) * (double)((tiles + slots - 1) / slots);
+    };
+    TileCut tiles = cut(steps ? steps : 2);
+    if (!steps) {
+        TileCut three = cut(3);
+        steps = 0.85 * rounds(three.tiles()) < rounds(tiles.tiles()) ? 3 : 2;
+        if (steps == 3) std::swap(tiles, three);
     }
+    if (tiles.tiles() > (1u << 28)) return fail(POE2D_E_INVALID, "run: too many tiles in one launch");
+    std::vector<TileItem> &edge = tiles.edge, &inter = tiles.inter;
+    const std::vector<int> &ptr = tiles.ptr;
+    const std::vector<int2> &ent = tiles.ent;
     const int cols = tile_cols(steps);
     std::vector<StepArgs<T>> args(nm);
     for (int i = 0; i < nm; ++i) {

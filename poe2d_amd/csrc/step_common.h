@@ -341,15 +341,22 @@ constexpr int kFused2RowsBefore = 10, kFused2RowsAfter = 12, kFused2ColsBefore =
 
 // The tile kernel (kernels_tile.hip): `steps` (two or three) steps of a region of 64 columns held on
 // chip.  A step consumes three rows and columns of the region on every side, so a work item owns
-// columns [x0, x0 + tile_cols) and rows [z0, z1), at most 24 - 6 steps rows (TILE_EDGE, TILE_SHORT) or
-// 8 tile_tall_p - 6 steps (TILE_TALL).  TILE_EDGE items are those whose region reaches a C-PML strip or
-// the grid's two outer rows or columns; the others run without that code.  Items with receivers have
+// columns [x0, x0 + tile_cols) and rows [z0, z1), at most tile_rows(P, steps) for the P rows a thread of
+// its kind holds: 3 of TILE_SHORT and TILE_EDGE, tile_tall_p of TILE_TALL, tile_edge_p of the others.
+// TILE_EDGE items are those whose region reaches a C-PML strip or the grid's two outer rows or columns
+// on both axes (or, among short tiles, on one), TILE_EDGE_X and TILE_EDGE_Z those whose region reaches
+// them along x or along z alone; the others run without that code.  Items with receivers have
 // rec >= 0: rec_tile_ptr[rec + k] .. [rec + k + 1] are the rec_entries of row z0 + k.
-enum { TILE_EDGE = 0, TILE_SHORT = 1, TILE_TALL = 2 };
+enum { TILE_EDGE = 0, TILE_SHORT = 1, TILE_TALL = 2, TILE_EDGE_X = 3, TILE_EDGE_Z = 4 };
 constexpr int kTileStepsMax = 3;
+constexpr int kTileCus = 256;  // compute units; a CU holds two FP32 tiles at a time, one of FP64
 // Rows per thread of a tall tile: 6 with an FP32 palette; 4 where the registers also hold FP64 values
 // or the coefficients of every row (at 6 those spill).
 __host__ __device__ constexpr int tile_tall_p(bool f32, bool palette) { return f32 && palette ? 6 : 4; }
+// Rows per thread of a tile at one edge: 4 (six memory variables a point, as many registers as a corner's
+// twelve at 3); 3 where the registers also hold coefficients (4 spills 67).  5 spills: 1201^2 17.9 us a
+// step instead of 15.1.
+__host__ __device__ constexpr int tile_edge_p(bool palette) { return palette ? 4 : 3; }
 __host__ __device__ constexpr int tile_halo(int steps) { return 3 * steps; }
 __host__ __device__ constexpr int tile_cols(int steps) { return 64 - 2 * tile_halo(steps); }
 __host__ __device__ constexpr int tile_rows(int p, int steps) { return 8 * p - 2 * tile_halo(steps); }

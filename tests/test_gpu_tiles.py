@@ -1,6 +1,6 @@
 """The tile kernel (schedule 3, block width 64, and what a handle runs until a shape is chosen)
 against the single-step kernel it must reproduce bit for bit: from a random state, on grids at the
-remainders of its 52-column tiles and 12- and 36-row tiles, with a material palette, one beyond the
+remainders of its 52-column tiles and 12-, 20- and 36-row tiles, with a material palette, one beyond the
 marching kernel's limit and none, in both precisions, over odd and even step counts."""
 import numpy as np
 import pytest
@@ -60,6 +60,18 @@ def test_tiles_equal_the_single_step_kernel(nx, nz, npml, entries, precision):
     for shape, steps in (((3, 64, 12), [4, 5]), ((3, 64, 36), [9]), ((3, 64, 6), [8, 1]), ((3, 64, 30), [2, 7]),
                          (None, [1, 2, 6])):
         _same(_run(prob, precision, shape, steps), ref, f"{nx}x{nz} npml {npml} {entries} entries shape {shape}")
+
+
+@pytest.mark.parametrize("nz", [40, 41, 42, 57, 58])
+@pytest.mark.parametrize("entries", [2, 0])
+@pytest.mark.parametrize("precision", [32, 64])
+def test_tile_bands_at_the_heights_of_their_tiles(nz, entries, precision):
+    """Edge and tall bands of 19 to 37 rows (13 to 31 with three steps): one row less, as many and one
+    more than a tile of 20 or 36 (14 or 30) takes."""
+    prob = _problem(150, nz, 4, entries)
+    ref = _run(prob, precision, (0, 256, 14), [6])
+    for shape in ((3, 64, 36), (3, 64, 30), (3, 64, 12)):
+        _same(_run(prob, precision, shape, [6]), ref, f"{nz} rows {entries} entries shape {shape}")
 
 
 @pytest.mark.parametrize("opts", [dict(stress_law=1), dict(staggered_material=1)])
