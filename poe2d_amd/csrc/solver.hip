@@ -702,16 +702,47 @@ struct TileCut {
     size_t tiles() const { return edge.size() + inter.size(); }
 };
 
-// Member i's part of it, `steps` steps per launch.  A column of tiles is three bands: the rows whose region
-// reaches the upper z strip or border, those away from both, and the lower ones; the tiles of a band are
-// of equal height (+- 1), at most short_rows at a corner, edge_rows along an edge and tall_rows elsewhere.
-void cut_tiles(const poe2d_solver *s, int i, int steps, int short_rows, int edge_rows, int tall_rows, TileCut &out)
+// Where a grid's tiles lie with `steps` steps per launch.  A column of tiles is three bands: the rows whose
+// region reaches the upper z strip or border, those away from both, and the lower ones; the tiles of a
+// band are of equal height (+- 1), at most short_rows at a corner, edge_rows along an edge and tall_rows
+// elsewhere.
+struct TileGrid {
+    int steps, short_rows, edge_rows, tall_rows;
+
+    bool x_edge(const poe2d_solver *s, int x0) const
+    {
+        const int c0 = x0 - tile_halo(steps), c1 = c0 + 63;  // the region's columns
+        return c0 < std::max(s->m->xlo, 2) || c1 >= std::min(s->m->xhi, s->grid.nx - 1);
+    }
+    // the tile of a column (xs: x_edge) that begins at row z0: its end, and whether it is a z edge's
+    int end(const poe2d_solver *s, bool xs, int z0, bool &zs) const
+    {
+        const int halo = tile_halo(steps), nz = s->grid.nz;
+        const int upper = std::min(std::max(s->m->ztop, 2) + halo, nz + 1);
+        const int lower = std::max(std::min(s->m->zbot, nz - 1) - halo, upper);
+        zs = z0 < upper || z0 >= lower;
+        const int left = (z0 < upper ? upper : z0 < lower ? std::min(lower, nz + 1) : nz + 1) - z0;
+        const int most = xs && zs ? short_rows : xs || zs ? edge_rows : tall_rows, count = (left + most - 1) / most;
+        return z0 + (left + count - 1) / count;
+    }
+    size_t count(const poe2d_solver *s) const
+    {
+        size_t columns[2] = {0, 0}, n = 0;
+        for (int x0 = 0; x0 <= s->grid.nx; x0 += tile_cols(steps)) ++columns[x_edge(s, x0)];
+        for (int xs = 0; xs < 2; ++xs) {
+            bool zs;
+            if (columns[xs])
+                for (int z0 = 0; z0 <= s->grid.nz; z0 = end(s, xs, z0, zs)) n += columns[xs];
+        }
+        return n;
+    }
+};
+
+// Member i's part of the cut, interior tiles row by row in bands of kBandTiles tile columns, so that the
+// tiles in flight on an XCD (about 64) make a block of neighbours sharing their halos in its L2.
+void cut_tiles(const poe2d_solver *s, int i, const TileGrid &grid, TileCut &out)
 {
-    const Model *md = s->m;
-    const int halo = tile_halo(steps), cols = tile_cols(steps);
-    const int nx = s->grid.nx, nz = s->grid.nz;
-    const int xlo = std::max(md->xlo, 2), xhi = std::min(md->xhi, nx - 1);
-    const int zlo = std::max(md->ztop, 2), zhi = std::min(md->zbot, nz - 1);
+    const int cols = tile_cols(grid.steps), nx = s->grid.nx, nz = s->grid.nz;
     // receivers by tile column and row
     std::vector<int> order(s->nrec);
     for (int r = 0; r < s->nrec; ++r) order[r] = r;
@@ -720,22 +751,18 @@ void cut_tiles(const poe2d_solver *s, int i, int steps, int short_rows, int edge
         return ta != tb ? ta < tb : s->hrz[a] < s->hrz[b];
     });
     size_t next = 0;
+    std::vector<TileItem> inter;  // column by column, every column cut alike
     for (int x0 = 0; x0 <= nx; x0 += cols) {
-        const int c0 = x0 - halo, c1 = c0 + 63;  // the region's columns
-        const bool xs = c0 < xlo || c1 >= xhi;
-        const int upper = std::min(zlo + halo, nz + 1), lower = std::max(zhi - halo, upper);
+        const bool xs = grid.x_edge(s, x0);
         for (int z0 = 0; z0 <= nz;) {
-            const bool zs = z0 < upper || z0 >= lower;
-            const int end = z0 < upper ? upper : z0 < lower ? std::min(lower, nz + 1) : nz + 1;
-            const int most = xs && zs ? short_rows : xs || zs ? edge_rows : tall_rows;
-            const int count = (end - z0 + most - 1) / most;
+            bool zs;
             TileItem it{};
             it.model = i;
             it.x0 = x0;
             it.z0 = z0;
-            it.z1 = z0 + (end - z0 + count - 1) / count;
-            it.kind = !xs && !zs ? (tall_rows > short_rows ? TILE_TALL : TILE_SHORT)
-                      : tall_rows == short_rows || (xs && zs) ? TILE_EDGE : xs ? TILE_EDGE_X : TILE_EDGE_Z;
+            it.z1 = grid.end(s, xs, z0, zs);
+            const bool tall = grid.tall_rows > grid.short_rows;
+            it.kind = !xs && !zs ? (tall ? TILE_TALL : TILE_SHORT) : !tall || (xs && zs) ? TILE_EDGE : xs ? TILE_EDGE_X : TILE_EDGE_Z;
             it.rec = -1;
             auto pending = [&](int z) {
                 return next < order.size() && s->hrx[order[next]] < x0 + cols && s->hrz[order[next]] < z;
@@ -748,9 +775,18 @@ void cut_tiles(const poe2d_solver *s, int i, int steps, int short_rows, int edge
                 }
                 out.ptr.push_back((int)out.ent.size());
             }
-            (xs || zs ? out.edge : out.inter).push_back(it);
+            (xs || zs ? out.edge : inter).push_back(it);
             z0 = it.z1;
         }
+    }
+    size_t rows = 0;
+    while (rows < inter.size() && inter[rows].x0 == inter[0].x0) ++rows;
+    for (size_t c0 = 0; c0 < inter.size();) {
+        size_t c1 = c0;
+        while (c1 < inter.size() && inter[c1].x0 / (kBandTiles * cols) == inter[c0].x0 / (kBandTiles * cols)) c1 += rows;
+        for (size_t r = 0; r < rows; ++r)
+            for (size_t c = c0; c < c1; c += rows) out.inter.push_back(inter[c + r]);
+        c0 = c1;
     }
 }
 
@@ -772,29 +808,28 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
         if (s->grid.staggered_material != material)
             return fail(POE2D_E_INVALID, "run: batch members differ in staggered material");
     }
-    const auto cut = [&](int k) {
+    const auto grid = [&](int k) {
         const int rows = tile_rows(3, k);
-        TileCut c;
-        for (int i = 0; i < nm; ++i)
-            cut_tiles(members[i], i, k, rows, tall ? tile_rows(tile_edge_p(palette), k) : rows,
-                      tall ? tile_rows(tile_tall_p(sizeof(T) == 4, palette), k) : rows, c);
-        return c;
+        if (!tall) return TileGrid{k, rows, rows, rows};
+        return TileGrid{k, rows, tile_rows(tile_edge_p(palette), k), tile_rows(tile_tall_p(sizeof(T) == 4, palette), k)};
     };
-    const auto rounds = [](size_t tiles) {
-        const size_t slots = kTileCus * (sizeof(T) == 4 ? 2 : 1);
-        return tiles <= (size_t)kTileCus ? 1.0 : (sizeof(T) == 4 ? 1.25 : 1.0) * (double)((tiles + slots - 1) / slots);
-    };
-    TileCut tiles = cut(steps ? steps : 2);
     if (!steps) {
-        TileCut three = cut(3);
-        steps = 0.85 * rounds(three.tiles()) < rounds(tiles.tiles()) ? 3 : 2;
-        if (steps == 3) std::swap(tiles, three);
+        const auto rounds = [&](int k) {
+            size_t n = 0;
+            for (const poe2d_solver *s : members) n += grid(k).count(s);
+            const size_t slots = kTileCus * (sizeof(T) == 4 ? 2 : 1);
+            return n <= (size_t)kTileCus ? 1.0 : (sizeof(T) == 4 ? 1.25 : 1.0) * (double)((n + slots - 1) / slots);
+        };
+        steps = 0.85 * rounds(3) < rounds(2) ? 3 : 2;
     }
-    if (tiles.tiles() > (1u << 28)) return fail(POE2D_E_INVALID, "run: too many tiles in one launch");
+    TileCut tiles;
+    for (int i = 0; i < nm; ++i) {
+        cut_tiles(members[i], i, grid(steps), tiles);
+        if (tiles.tiles() > (1u << 28)) return fail(POE2D_E_INVALID, "run: too many tiles in one launch");
+    }
     std::vector<TileItem> &edge = tiles.edge, &inter = tiles.inter;
     const std::vector<int> &ptr = tiles.ptr;
     const std::vector<int2> &ent = tiles.ent;
-    const int cols = tile_cols(steps);
     std::vector<StepArgs<T>> args(nm);
     for (int i = 0; i < nm; ++i) {
         const poe2d_solver *s = members[i];
@@ -806,12 +841,6 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
         args[i].rec_mask = s->mask;
         args[i].traces = (T *)s->traces;
     }
-    // Interior tiles run row by row in bands of kBandTiles tile columns, so that the tiles in flight on
-    // an XCD (about 64) make a block of neighbours sharing their halos in its L2.
-    std::stable_sort(inter.begin(), inter.end(), [&](const TileItem &a, const TileItem &b) {
-        const int ba = a.x0 / (kBandTiles * cols), bb = b.x0 / (kBandTiles * cols);
-        return std::tie(a.model, ba, a.z0, a.x0) < std::tie(b.model, bb, b.z0, b.x0);
-    });
     // as the two-step kernel's list: every XCD gets an eighth of the edge tiles first, then a run of
     // consecutive interior tiles; shares padded to equal length with empty items
     const int ne = (int)((edge.size() + 7) / 8), ni = (int)((inter.size() + 7) / 8);
