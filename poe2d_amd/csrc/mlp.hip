@@ -117,7 +117,6 @@ struct poe2d_mlp {
     std::vector<float *> pre;      // pre-activations Z_l, l = 0..L-1
     std::vector<uint16_t *> g16;   // gradients at Z_l (bf16)
     std::vector<uint16_t *> g16t;  // their transposes
-    float *dh = nullptr;           // G_l W_l (FP32), largest hidden width
     float *y = nullptr;            // outputs Z_{L-1} (FP32)
     float *tgt = nullptr;          // targets of the batch
     float *xin = nullptr;          // network input of the batch (FP32)
@@ -179,7 +178,7 @@ void free_mlp(poe2d_mlp *m)
     for (auto &p : m->pre) dfree(p);
     for (auto &p : m->g16) dfree(p);
     for (auto &p : m->g16t) dfree(p);
-    dfree(m->dh); dfree(m->y); dfree(m->tgt); dfree(m->xin); dfree(m->work); dfree(m->partial);
+    dfree(m->y); dfree(m->tgt); dfree(m->xin); dfree(m->work); dfree(m->partial);
     for (auto &p : m->hens) dfree(p);
     for (auto &p : m->ens_w) dfree(p);
     for (auto &p : m->ens_b) dfree(p);
@@ -238,7 +237,8 @@ poe2d_status copy_rows(poe2d_mlp *m, float *host, float *dev, int ld, int rows, 
 poe2d_status sync_copies(poe2d_mlp *m, Layer &l)
 {
     HIP_TRY(convert_bf16(l.w, l.w16, (size_t)l.outp * l.inp, m->stream));
-    HIP_TRY(transpose_bf16(l.w16, l.inp, l.w16t, l.outp, l.outp, l.inp, m->stream));
+    const Transpose w16t{l.w16, l.w16t, l.inp, l.outp, l.outp, l.inp};
+    HIP_TRY(transpose_bf16(&w16t, 1, m->stream));
     return POE2D_OK;
 }
 
@@ -249,13 +249,14 @@ __global__ void pack_input(const float *__restrict__ x, int n, int in, uint16_t 
     h[(size_t)(i / in) * ldh + i % in] = bf16_rne(x[i]);
 }
 
-__global__ void gather_rows(const float *__restrict__ src, int ld_src, const int *__restrict__ idx, int n, int cols,
-                            float *__restrict__ dst, int ld_dst)
+// Rows idx[0 .. n) of src into h as pack_input.
+__global__ void gather_input(const float *__restrict__ src, const int *__restrict__ idx, int n, int in,
+                             uint16_t *__restrict__ h, int ldh)
 {
-    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (i >= (size_t)n * cols) return;
-    const int r = (int)(i / cols), c = (int)(i % cols);
-    dst[(size_t)r * ld_dst + c] = src[(size_t)idx[r] * ld_src + c];
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n * in) return;
+    const int r = i / in, c = i % in;
+    h[(size_t)r * ldh + c] = bf16_rne(src[(size_t)idx[r] * in + c]);
 }
 
 int blocks(size_t n) { return (int)std::min<size_t>((n + 255) / 256, 1u << 20); }
@@ -393,6 +394,26 @@ bool on_this_device(const poe2d_mlp *m, const void *p)
     return at.type == hipMemoryTypeDevice && at.device == m->device;
 }
 
+// The layers' inputs of the batch of n rows, transposed for the weight gradients.
+poe2d_status transpose_activations(poe2d_mlp *m, const Member &e, int n)
+{
+    std::vector<Transpose> list;
+    for (int li = 0; li < m->L; ++li)
+        list.push_back({m->h16[li], m->h16t[li], e.layers[li].inp, m->max_batch, n, e.layers[li].inp});
+    HIP_TRY(transpose_bf16(list.data(), m->L, m->stream));
+    return POE2D_OK;
+}
+
+// G_{li-1} = (G_li W_li) * gelu'(Z_{li-1}) and its transpose: A = G_li [n][outp], B = W_li^T [inp][outp].
+poe2d_status input_gradient(poe2d_mlp *m, const Layer &l, int li, int n)
+{
+    const int ksplit = product_splits(m, n, l.in, l.outp);
+    HIP_TRY(gemm_partials(m->g16[li], l.outp, l.w16t, l.outp, n, l.in, l.outp, m->work, m->work_floats, ksplit, m->stream));
+    HIP_TRY(hidden_gradients(m->work, ksplit, m->pre[li - 1], l.inp, n, l.in, m->g16[li - 1], l.inp, m->g16t[li - 1],
+                             m->max_batch, m->stream));
+    return POE2D_OK;
+}
+
 // Gradients of the mean squared error for member e on the batch in h16[0] / tgt (n rows, n a
 // multiple of 32); loss (mean) to *loss when non-null.
 poe2d_status backward(poe2d_mlp *m, Member &e, int n, float *loss)
@@ -410,27 +431,18 @@ poe2d_status backward(poe2d_mlp *m, Member &e, int n, float *loss)
         for (float v : part) s += v;
         *loss = (float)(s / ((double)n * top.out));
     }
+    poe2d_status st = transpose_activations(m, e, n);
+    if (st) return st;
     for (int li = L - 1; li >= 0; --li) {
         Layer &l = e.layers[li];
         // dW = G^T H: A = G^T [outp][n], B = H^T [inp][n]
-        if (li < L - 1) HIP_TRY(transpose_bf16(m->g16[li], l.outp, m->g16t[li], m->max_batch, n, l.outp, m->stream));
-        HIP_TRY(transpose_bf16(m->h16[li], l.inp, m->h16t[li], m->max_batch, n, l.inp, m->stream));
         GemmOut o;
         o.f32 = l.gw;
         o.ldf = l.inp;
         HIP_TRY(gemm_bf16(m->g16t[li], m->max_batch, m->h16t[li], m->max_batch, l.outp, l.inp, n, EPI_LINEAR, o,
                           m->work, m->work_floats, product_splits(m, l.outp, l.inp, n), m->stream));
         if (li < L - 1) HIP_TRY(bias_gradient(m->g16t[li], m->max_batch, l.outp, n, l.gb, m->stream));
-        if (li == 0) break;
-        // G_{l-1} = (G_l W_l) * gelu'(Z_{l-1}): A = G_l [n][outp], B = W_l^T [inp][outp]
-        const int K = l.outp;
-        const int ksplit = product_splits(m, n, l.in, K);
-        GemmOut od;
-        od.f32 = m->dh;
-        od.ldf = l.inp;
-        HIP_TRY(gemm_bf16(m->g16[li], l.outp, l.w16t, l.outp, n, l.in, K, EPI_LINEAR, od, m->work, m->work_floats,
-                          ksplit, m->stream));
-        HIP_TRY(gelu_bwd(m->dh, m->pre[li - 1], n, l.in, l.inp, m->g16[li - 1], l.inp, m->stream));
+        if (li > 0 && (st = input_gradient(m, l, li, n))) return st;
     }
     return POE2D_OK;
 }
@@ -476,29 +488,21 @@ poe2d_status train_step(poe2d_mlp *m, Member &e, int n, const float *tgt, int ld
         HIP_TRY(gemm_bf16(m->h16[L - 1], top.inp, top.w16, top.inp, n, top.out, top.inp, EPI_MSE, o, m->work,
                           m->work_floats, 1, m->stream));
     }
-    HIP_TRY(sum_rows(m->work, (n + 127) / 128, top.outp, top.out, top.gb, m->stream));
+    e.t += 1;
+    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+    const float c1 = 1.f - powf(b1, (float)e.t), c2 = 1.f - powf(b2, (float)e.t);
+    HIP_TRY(output_bias_step(m->work, (n + 127) / 128, top.outp, top.out, top.b, top.mb, top.vb, lr, b1, b2, eps, e.t,
+                             m->stream));
     if (loss_dev) {
         loss_sum<<<1, 256, 0, m->stream>>>(m->partial, gemm_tiles(n, top.out), 1.0 / ((double)n * top.out), loss_dev);
         HIP_TRY(hipGetLastError());
     }
-    e.t += 1;
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float c1 = 1.f - powf(b1, (float)e.t), c2 = 1.f - powf(b2, (float)e.t);
+    poe2d_status st = transpose_activations(m, e, n);
+    if (st) return st;
     for (int li = L - 1; li >= 0; --li) {
         Layer &l = e.layers[li];
-        if (li < L - 1) HIP_TRY(transpose_bf16(m->g16[li], l.outp, m->g16t[li], m->max_batch, n, l.outp, m->stream));
-        HIP_TRY(transpose_bf16(m->h16[li], l.inp, m->h16t[li], m->max_batch, n, l.inp, m->stream));
-        if (li > 0) {
-            // G_{l-1} = (G_l W_l) * gelu'(Z_{l-1}) with the weights of this step
-            const int K = l.outp;
-            const int ksplit = product_splits(m, n, l.in, K);
-            GemmOut od;
-            od.f32 = m->dh;
-            od.ldf = l.inp;
-            HIP_TRY(gemm_bf16(m->g16[li], l.outp, l.w16t, l.outp, n, l.in, K, EPI_LINEAR, od, m->work, m->work_floats,
-                              ksplit, m->stream));
-            HIP_TRY(gelu_bwd(m->dh, m->pre[li - 1], n, l.in, l.inp, m->g16[li - 1], l.inp, m->stream));
-        }
+        // (with the weights of this step)
+        if (li > 0 && (st = input_gradient(m, l, li, n))) return st;
         if (li == L - 1) {
             // dW = G^T H and the Adam step in one product: A = G^T [outp][n], B = H^T [inp][n]
             GemmOut ow;
@@ -519,17 +523,14 @@ poe2d_status train_step(poe2d_mlp *m, Member &e, int n, const float *tgt, int ld
                               m->work, m->work_floats, 1, m->stream));
         } else {
             // (the hidden layers' 512 x 512 products make 16 tiles: too few blocks to stream the
-            // optimiser state from the product's epilogue; a separate Adam pass over 64 tiles is faster)
-            GemmOut o;
-            o.f32 = l.gw;
-            o.ldf = l.inp;
-            HIP_TRY(gemm_bf16(m->g16t[li], m->max_batch, m->h16t[li], m->max_batch, l.outp, l.inp, n, EPI_LINEAR, o,
-                              m->work, m->work_floats, product_splits(m, l.outp, l.inp, n), m->stream));
-            HIP_TRY(bias_gradient(m->g16t[li], m->max_batch, l.outp, n, l.gb, m->stream));
-            HIP_TRY(adam_matrix_step(l.w, l.mw, l.vw, l.gw, l.outp, l.inp, lr, b1, b2, eps, e.t, l.w16, l.w16t,
-                                     m->stream));
+            // optimiser state from the product's epilogue; a separate Adam pass over 128 tiles is faster)
+            const int ksplit = product_splits(m, l.outp, l.inp, n);
+            float *const part = ksplit > 1 ? m->work : l.gw;  // (one partial may be more than work holds)
+            HIP_TRY(gemm_partials(m->g16t[li], m->max_batch, m->h16t[li], m->max_batch, l.outp, l.inp, n, part,
+                                  ksplit > 1 ? m->work_floats : (size_t)l.outp * l.inp, ksplit, m->stream));
+            HIP_TRY(adam_layer_step(l.w, l.mw, l.vw, part, ksplit, l.outp, l.inp, lr, b1, b2, eps, e.t, l.w16, l.w16t,
+                                    m->g16t[li], m->max_batch, n, l.b, l.mb, l.vb, m->stream));
         }
-        HIP_TRY(adam_step(l.b, l.mb, l.vb, l.gb, (size_t)l.outp, lr, b1, b2, eps, e.t, nullptr, m->stream));
     }
     return POE2D_OK;
 }
@@ -559,8 +560,7 @@ static poe2d_status dataset_step(poe2d_mlp *lane, const poe2d_mlp *data, Member 
                                  float *loss_dev)
 {
     const int in = lane->sizes[0], out = lane->sizes[lane->L];
-    gather_rows<<<blocks((size_t)batch * in), 256, 0, lane->stream>>>(data->data_x, in, idx, batch, in, lane->xin, in);
-    pack_input<<<blocks((size_t)batch * in), 256, 0, lane->stream>>>(lane->xin, batch, in, lane->h16[0], pad128(in));
+    gather_input<<<blocks((size_t)batch * in), 256, 0, lane->stream>>>(data->data_x, idx, batch, in, lane->h16[0], pad128(in));
     HIP_TRY(hipGetLastError());
     return train_step(lane, e, batch, data->data_t, out, idx, lr, loss_dev);
 }
@@ -593,8 +593,7 @@ static poe2d_status alloc_scratch(poe2d_mlp *m, bool predict)
     // split-K partials of the input-gradient products, and the output bias gradient's per-tile sums
     m->work_floats = std::max((size_t)128 * B * hidden_max, (size_t)((B + 127) / 128) * pad128(sizes[nlayers]));
     m->nred = std::max({m->nred, B, mse_blocks(sizes[nlayers]), gemm_tiles(B, sizes[nlayers])});
-    if ((st = dmalloc(&m->dh, (size_t)B * std::max(hidden_max, pad128(sizes[0])))) ||
-        (st = dmalloc(&m->xin, (size_t)B * sizes[0])) || (st = dmalloc(&m->work, m->work_floats)) ||
+    if ((st = dmalloc(&m->xin, (size_t)B * sizes[0])) || (st = dmalloc(&m->work, m->work_floats)) ||
         (st = dmalloc(&m->partial, m->nred)) || (st = dmalloc(&m->idx, (size_t)kIndexSteps * B)) ||
         (st = dmalloc(&m->dloss, kIndexSteps)))
         return st;

@@ -89,11 +89,26 @@ hipError_t ensemble_output(const uint16_t *A, int lda, size_t stride_a, const ui
                            const float *const *biases, int members, int M, int N, int K, float *mean, size_t ldm,
                            const float *scale, double *part, float *spread, hipStream_t stream);
 
-// out[c][r] = in[r][c], R x C.
-hipError_t transpose_bf16(const uint16_t *in, int ldi, uint16_t *out, int ldo, int R, int C, hipStream_t stream);
+// The partial products of a GEMM split over ksplit ranges of K, part [ksplit][M][N] floats, not summed.
+hipError_t gemm_partials(const uint16_t *A, int lda, const uint16_t *B, int ldb, int M, int N, int K, float *part,
+                         size_t part_floats, int ksplit, hipStream_t stream);
 
-// g = dh * gelu'(pre) (bf16), M x N with leading dimension ld (ldg for g).
-hipError_t gelu_bwd(const float *dh, const float *pre, int M, int N, int ld, uint16_t *g, int ldg, hipStream_t stream);
+// out[c][r] = in[r][c], R x C, for n matrices (kTransposes to a launch).
+struct Transpose {
+    const uint16_t *in;
+    uint16_t *out;
+    int ldi, ldo, R, C;
+};
+constexpr int kTransposes = 8;
+struct TransposeList {
+    Transpose m[kTransposes];
+};
+hipError_t transpose_bf16(const Transpose *m, int n, hipStream_t stream);
+
+// An activation's gradient g = dh * gelu'(pre) (bf16, M x N, leading dimension ldg; pre: ld) and its
+// transpose gt [N][ldgt], dh the sum of gemm_partials' nsplit partials.
+hipError_t hidden_gradients(const float *part, int nsplit, const float *pre, int ld, int M, int N, uint16_t *g, int ldg,
+                            uint16_t *gt, int ldgt, hipStream_t stream);
 
 // Mean squared error over M x N: gradient 2 (y - t) / (M N) as bf16 into g and its transpose gt
 // ([N][ldgt]), its column sums (the bias gradient) into db[N], and per-block sums of squares into
@@ -104,20 +119,20 @@ inline int gemm_tiles(int M, int N) { return ((M + 127) / 128) * ((N + 127) / 12
 hipError_t mse(const float *y, int ldy, const float *t, int ldt, int M, int N, uint16_t *g, int ldg, uint16_t *gt,
                int ldgt, float *db, float *partial, hipStream_t stream);
 
-// db[n] = sum over r < rows of part[r * ld + n], n < N (the bias gradient from EPI_MSE's dbp).
-hipError_t sum_rows(const float *part, int rows, int ld, int N, float *db, hipStream_t stream);
+// Adam step t (1-based) of the output bias b[N], its gradient the sum over r < rows of part[r * ld + n]
+// (EPI_MSE's dbp).
+hipError_t output_bias_step(const float *part, int rows, int ld, int N, float *b, float *mom, float *vel, float lr, float b1,
+                            float b2, float eps, long long t, hipStream_t stream);
 
 // db[r] = sum_k gt[r][k] over the K = batch entries of the transposed gradient gt [R][ldgt].
 hipError_t bias_gradient(const uint16_t *gt, int ldgt, int R, int K, float *db, hipStream_t stream);
 
-// Adam step t (1-based) on n FP32 master weights; their bf16 copy w16 (may be null) follows.
-hipError_t adam_step(float *w, float *m, float *v, const float *g, size_t n, float lr, float b1, float b2, float eps,
-                     long long t, uint16_t *w16, hipStream_t stream);
-
-// Adam step t on an R x C weight matrix (R, C multiples of 64) refreshing its bf16 copy w16 and
-// the transposed copy w16t [C][R].
-hipError_t adam_matrix_step(float *w, float *m, float *v, const float *g, int R, int C, float lr, float b1, float b2,
-                            float eps, long long t, uint16_t *w16, uint16_t *w16t, hipStream_t stream);
+// Adam step t of a layer: its R x C weights (R a multiple of 32, C of 64) from the sum of gemm_partials'
+// nsplit partials, refreshing their bf16 copy w16 and the transposed copy w16t [C][R], and its bias from
+// the sums over the K = batch entries of the transposed gradient gt [R][ldgt].
+hipError_t adam_layer_step(float *w, float *m, float *v, const float *part, int nsplit, int R, int C, float lr, float b1,
+                           float b2, float eps, long long t, uint16_t *w16, uint16_t *w16t, const uint16_t *gt, int ldgt, int K,
+                           float *b, float *bm, float *bv, hipStream_t stream);
 
 hipError_t convert_bf16(const float *in, uint16_t *out, size_t n, hipStream_t stream);
 

@@ -706,16 +706,6 @@ __global__ void __launch_bounds__(1024) ensemble_spread(const double *__restrict
     spread[m] = (float)(sqrt(var / (members > 1 ? members - 1 : 1)) / fmax(sqrt(nrm), 1e-30));
 }
 
-// db[n] = sum over r < rows of part[r][n] (n < N), in order.
-__global__ void column_sums(const float *__restrict__ part, int rows, int ld, int N, float *__restrict__ db)
-{
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
-    float v = 0.f;
-    for (int r = 0; r < rows; ++r) v += part[(size_t)r * ld + n];
-    db[n] = v;
-}
-
 // out[m][n] = sum over splits of part[s][m][n] (+ bias), then as the GEMM epilogue; of several
 // products, product blockIdx.y with bias biases[blockIdx.y] into b16 + blockIdx.y stride_b16.
 __global__ void reduce_splits(const float *__restrict__ part, int nsplit, int M, int N, int ldf, GemmOut out, int gelu_on,
@@ -749,31 +739,25 @@ __global__ void reduce_splits(const float *__restrict__ part, int nsplit, int M,
     if (out.b16) out.b16[(size_t)m * out.ldb + n] = bf16_rne(v);
 }
 
-// out[c][r] = in[r][c] for an R x C bf16 matrix (leading dimensions ldi, ldo), 32 x 32 tiles.
-__global__ void transpose16(const uint16_t *__restrict__ in, int ldi, uint16_t *__restrict__ out, int ldo, int R, int C)
+// out[c][r] = in[r][c] for the R x C bf16 matrices of a list (blockIdx.z), 32 x 32 tiles.
+__global__ void transpose16(const TransposeList list)
 {
     __shared__ uint16_t tile[32][33];
+    const Transpose &t = list.m[blockIdx.z];
     const int c0 = blockIdx.x * 32, r0 = blockIdx.y * 32;
+    if (c0 >= t.C || r0 >= t.R) return;
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 256 threads: 8 rows per pass
+#pragma unroll
     for (int y = ty; y < 32; y += 8) {
         const int r = r0 + y, c = c0 + tx;
-        tile[y][tx] = (r < R && c < C) ? in[(size_t)r * ldi + c] : 0;
+        tile[y][tx] = (r < t.R && c < t.C) ? t.in[(size_t)r * t.ldi + c] : 0;
     }
     __syncthreads();
+#pragma unroll
     for (int y = ty; y < 32; y += 8) {
         const int c = c0 + y, r = r0 + tx;
-        if (c < C && r < R) out[(size_t)c * ldo + r] = tile[tx][y];
+        if (c < t.C && r < t.R) t.out[(size_t)c * t.ldo + r] = tile[tx][y];
     }
-}
-
-// g[m][n] = dh[m][n] * gelu'(pre[m][n]) as bf16 (the gradient at the pre-activation).
-__global__ void gelu_backward(const float *__restrict__ dh, const float *__restrict__ pre, int M, int N, int ld,
-                              uint16_t *__restrict__ g, int ldg)
-{
-    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (i >= (size_t)M * N) return;
-    const int m = (int)(i / N), n = (int)(i % N);
-    g[(size_t)m * ldg + n] = bf16_rne(dh[(size_t)m * ld + n] * gelu_grad(pre[(size_t)m * ld + n]));
 }
 
 // The kernels below work on 64-column strips with 256 threads: thread (group q = t / 64, lane)
@@ -839,39 +823,121 @@ __global__ void __launch_bounds__(256) bias_grad(const uint16_t *__restrict__ gt
     if (lane == 0) db[r] = s;
 }
 
-// One Adam step on n master weights (FP32), refreshing their bf16 copy (when given).
-__global__ void adam(float *__restrict__ w, float *__restrict__ mom, float *__restrict__ vel, const float *__restrict__ grad,
-                     size_t n, float lr, float b1, float b2, float eps, float c1, float c2, uint16_t *__restrict__ w16)
+// v[k] = the sum of a split product's partials at offset at(k), in split order as reduce_splits (one
+// partial: itself); the loads of U splits in flight together.
+template <int U, int N, class At>
+__device__ __forceinline__ void split_sums(const float *__restrict__ part, int nsplit, size_t stride, float (&v)[N], const At &at)
 {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const float x = adam_update(w, mom, vel, grad[i], i, lr, b1, b2, eps, c1, c2);
-        if (w16) w16[i] = bf16_rne(x);
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = nsplit > 1 ? 0.f : -0.f;
+    int s = 0;
+    for (; s + U <= nsplit; s += U, part += U * stride) {
+        float q[U][N];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int k = 0; k < N; ++k) q[u][k] = part[u * stride + at(k)];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int k = 0; k < N; ++k) v[k] += q[u][k];
+    }
+    for (; s < nsplit; ++s, part += stride)
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] += part[at(k)];
+}
+
+// The training step's small kernels are bound by launches and latency (3 to 5 us each, 13 of a 512 x 512
+// Adam pass that loaded a row at a time): one per stage of a layer, loads first.
+
+// An activation's gradient g = bf16(dh gelu'(pre)) and its transpose gt, dh from the product's nsplit
+// partials (part [nsplit][M][ldp]); tiles of 32 x 32.
+__global__ void __launch_bounds__(256) hidden_gradient(const float *__restrict__ part, int nsplit, int ldp,
+                                                       const float *__restrict__ pre, int ld, int M, int N,
+                                                       uint16_t *__restrict__ g, int ldg, uint16_t *__restrict__ gt, int ldgt)
+{
+    __shared__ uint16_t tile[32][33];
+    const int c0 = blockIdx.x * 32, r0 = blockIdx.y * 32;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const int c = c0 + tx;
+    float dh[4], z[4];
+    auto row = [&](int k) { return (size_t)min(r0 + ty + 8 * k, M - 1); };
+    const int cc = min(c, N - 1);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) z[k] = pre[row(k) * ld + cc];
+    split_sums<8>(part, nsplit, (size_t)M * ldp, dh, [&](int k) { return row(k) * ldp + cc; });
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int y = ty + 8 * k, r = r0 + y;
+        const uint16_t v = bf16_rne(dh[k] * gelu_grad(z[k]));
+        if (r < M && c < N) g[(size_t)r * ldg + c] = v;
+        tile[y][tx] = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int y = ty + 8 * k;
+        if (c0 + y < N && r0 + tx < M) gt[(size_t)(c0 + y) * ldgt + r0 + tx] = tile[tx][y];
     }
 }
 
-// Adam on an R x C weight matrix (row-major, leading dimension C) refreshing its bf16 copy w16
-// and the transposed copy w16t ([C][R]); one 64 x 64 tile per block (R, C multiples of 64).
-__global__ void __launch_bounds__(256) adam_matrix(float *__restrict__ w, float *__restrict__ mom,
-                                                   float *__restrict__ vel, const float *__restrict__ grad, int R, int C,
-                                                   float lr, float b1, float b2, float eps, float c1, float c2,
-                                                   uint16_t *__restrict__ w16, uint16_t *__restrict__ w16t)
+// A layer's Adam step: the weights [R][C] (gradient: the sum of nsplit partials [R][C]), their bf16 copy
+// w16 and its transpose w16t [C][R], in tiles of 32 x 64; in the blocks after those, a wave per row of the
+// transposed gradient gt [R][ldgt], the bias (gradient: the sum over the batch's K entries).
+__global__ void __launch_bounds__(256) adam_layer(float *__restrict__ w, float *__restrict__ mom, float *__restrict__ vel,
+                                                  const float *__restrict__ part, int nsplit, int R, int C, float lr,
+                                                  float b1, float b2, float eps, float c1, float c2,
+                                                  uint16_t *__restrict__ w16, uint16_t *__restrict__ w16t,
+                                                  const uint16_t *__restrict__ gt, int ldgt, int K, float *__restrict__ b,
+                                                  float *__restrict__ bmom, float *__restrict__ bvel)
 {
-    __shared__ uint16_t tile[64][66];
+    __shared__ uint16_t tile[32][66];
     const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
-    const int tiles_c = C / 64;
-    const int r0 = (blockIdx.x / tiles_c) * 64, c0 = (blockIdx.x % tiles_c) * 64;
-    for (int k = 0; k < 16; ++k) {
+    const int tiles_c = C / 64, tiles = R / 32 * tiles_c;
+    if ((int)blockIdx.x >= tiles) {
+        const int r = ((int)blockIdx.x - tiles) * 4 + q;
+        if (r >= R) return;
+        float s = 0.f;
+        for (int k = lane; k < K; k += 64) s += bf16_to_f32(gt[(size_t)r * ldgt + k]);
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+        if (lane == 0) adam_update(b, bmom, bvel, s, r, lr, b1, b2, eps, c1, c2);
+        return;
+    }
+    const int r0 = (int)blockIdx.x / tiles_c * 32, c0 = (int)blockIdx.x % tiles_c * 64;
+    float x[8], m[8], v[8], g[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const size_t i = (size_t)(r0 + q + 4 * k) * C + c0 + lane;
+        x[k] = w[i], m[k] = mom[i], v[k] = vel[i];
+    }
+    split_sums<4>(part, nsplit, (size_t)R * C, g, [&](int k) { return (size_t)(r0 + q + 4 * k) * C + c0 + lane; });
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
         const int rr = q + 4 * k;
         const size_t i = (size_t)(r0 + rr) * C + c0 + lane;
-        const uint16_t v = bf16_rne(adam_update(w, mom, vel, grad[i], i, lr, b1, b2, eps, c1, c2));
-        w16[i] = v;
-        tile[rr][lane] = v;
+        x[k] = adam_value(x[k], m[k], v[k], g[k], lr, b1, b2, eps, c1, c2);
+        const uint16_t h = bf16_rne(x[k]);
+        w[i] = x[k], mom[i] = m[k], vel[i] = v[k], w16[i] = h;
+        tile[rr][lane] = h;
     }
     __syncthreads();
-    for (int k = 0; k < 16; ++k) {
-        const int cc = q + 4 * k;
-        w16t[(size_t)(c0 + cc) * R + r0 + lane] = tile[lane][cc];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int cc = (threadIdx.x >> 5) + 8 * k, rr = threadIdx.x & 31;
+        w16t[(size_t)(c0 + cc) * R + r0 + rr] = tile[rr][cc];
     }
+}
+
+// The output bias's Adam step from its gradient, the sum over r < rows of part[r][n] in order.
+__global__ void adam_output_bias(const float *__restrict__ part, int rows, int ld, int N,
+                                 float *__restrict__ b, float *__restrict__ mom, float *__restrict__ vel, float lr, float b1,
+                                 float b2, float eps, float c1, float c2)
+{
+    const int n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= N) return;
+    float v = 0.f;
+    for (int r = 0; r < rows; ++r) v += part[(size_t)r * ld + n];
+    adam_update(b, mom, vel, v, n, lr, b1, b2, eps, c1, c2);
 }
 
 __global__ void to_bf16(const float *__restrict__ in, uint16_t *__restrict__ out, size_t n)
@@ -974,16 +1040,22 @@ hipError_t ensemble_output(const uint16_t *A, int lda, size_t stride_a, const ui
     return hipGetLastError();
 }
 
-hipError_t transpose_bf16(const uint16_t *in, int ldi, uint16_t *out, int ldo, int R, int C, hipStream_t stream)
+hipError_t transpose_bf16(const Transpose *m, int n, hipStream_t stream)
 {
-    transpose16<<<dim3((C + 31) / 32, (R + 31) / 32), 256, 0, stream>>>(in, ldi, out, ldo, R, C);
-    return hipGetLastError();
-}
-
-hipError_t gelu_bwd(const float *dh, const float *pre, int M, int N, int ld, uint16_t *g, int ldg, hipStream_t stream)
-{
-    gelu_backward<<<grid_for((size_t)M * N), 256, 0, stream>>>(dh, pre, M, N, ld, g, ldg);
-    return hipGetLastError();
+    for (int i0 = 0; i0 < n; i0 += kTransposes) {
+        TransposeList list{};
+        const int k = std::min(n - i0, kTransposes);
+        int rows = 0, cols = 0;
+        for (int i = 0; i < k; ++i) {
+            list.m[i] = m[i0 + i];
+            rows = std::max(rows, list.m[i].R);
+            cols = std::max(cols, list.m[i].C);
+        }
+        transpose16<<<dim3((cols + 31) / 32, (rows + 31) / 32, k), 256, 0, stream>>>(list);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 int mse_blocks(int N) { return (N + 63) / 64; }
@@ -995,9 +1067,32 @@ hipError_t mse(const float *y, int ldy, const float *t, int ldt, int M, int N, u
     return hipGetLastError();
 }
 
-hipError_t sum_rows(const float *part, int rows, int ld, int N, float *db, hipStream_t stream)
+hipError_t output_bias_step(const float *part, int rows, int ld, int N, float *b, float *mom, float *vel, float lr,
+                            float b1, float b2, float eps, long long t, hipStream_t stream)
 {
-    column_sums<<<(N + 255) / 256, 256, 0, stream>>>(part, rows, ld, N, db);
+    const float c1 = 1.f - powf(b1, (float)t), c2 = 1.f - powf(b2, (float)t);
+    adam_output_bias<<<(N + 255) / 256, 256, 0, stream>>>(part, rows, ld, N, b, mom, vel, lr, b1, b2, eps, c1, c2);
+    return hipGetLastError();
+}
+
+hipError_t gemm_partials(const uint16_t *A, int lda, const uint16_t *B, int ldb, int M, int N, int K, float *work,
+                         size_t work_floats, int ksplit, hipStream_t stream)
+{
+    if (M < 1 || N < 1 || K < BK || K % BK || lda % 8 || ldb % 8 || lda < K || ldb < K || ksplit < 1 || ksplit > K / BK ||
+        work_floats < (size_t)ksplit * M * N)
+        return hipErrorInvalidValue;
+    GemmOut part{};
+    part.f32 = work;
+    part.ldf = N;
+    gemm_nt<EPI_PARTIAL><<<dim3(((M + BM - 1) / BM) * ((N + BN - 1) / BN), ksplit), 256, 0, stream>>>(A, lda, B, ldb, M, N, K,
+                                                                                                     ksplit, part);
+    return hipGetLastError();
+}
+
+hipError_t hidden_gradients(const float *part, int nsplit, const float *pre, int ld, int M, int N, uint16_t *g, int ldg,
+                            uint16_t *gt, int ldgt, hipStream_t stream)
+{
+    hidden_gradient<<<dim3((N + 31) / 32, (M + 31) / 32), 256, 0, stream>>>(part, nsplit, N, pre, ld, M, N, g, ldg, gt, ldgt);
     return hipGetLastError();
 }
 
@@ -1007,20 +1102,14 @@ hipError_t bias_gradient(const uint16_t *gt, int ldgt, int R, int K, float *db, 
     return hipGetLastError();
 }
 
-hipError_t adam_step(float *w, float *m, float *v, const float *g, size_t n, float lr, float b1, float b2, float eps,
-                     long long t, uint16_t *w16, hipStream_t stream)
+hipError_t adam_layer_step(float *w, float *m, float *v, const float *part, int nsplit, int R, int C, float lr, float b1,
+                           float b2, float eps, long long t, uint16_t *w16, uint16_t *w16t, const uint16_t *gt, int ldgt, int K,
+                           float *b, float *bm, float *bv, hipStream_t stream)
 {
+    if (R % 32 || C % 64) return hipErrorInvalidValue;
     const float c1 = 1.f - powf(b1, (float)t), c2 = 1.f - powf(b2, (float)t);
-    adam<<<grid_for(n), 256, 0, stream>>>(w, m, v, g, n, lr, b1, b2, eps, c1, c2, w16);
-    return hipGetLastError();
-}
-
-hipError_t adam_matrix_step(float *w, float *m, float *v, const float *g, int R, int C, float lr, float b1, float b2,
-                            float eps, long long t, uint16_t *w16, uint16_t *w16t, hipStream_t stream)
-{
-    if (R % 64 || C % 64) return hipErrorInvalidValue;
-    const float c1 = 1.f - powf(b1, (float)t), c2 = 1.f - powf(b2, (float)t);
-    adam_matrix<<<(R / 64) * (C / 64), 256, 0, stream>>>(w, m, v, g, R, C, lr, b1, b2, eps, c1, c2, w16, w16t);
+    adam_layer<<<R / 32 * (C / 64) + (R + 3) / 4, 256, 0, stream>>>(w, m, v, part, nsplit, R, C, lr, b1, b2, eps, c1, c2, w16,
+                                                                  w16t, gt, ldgt, K, b, bm, bv);
     return hipGetLastError();
 }
 

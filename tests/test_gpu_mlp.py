@@ -175,6 +175,31 @@ def test_adam_matches_the_bias_corrected_update():
             assert np.array_equal(a, b) and np.array_equal(c, d)
 
 
+@pytest.mark.parametrize("sizes,batch", [([4, 96, 20000], 32), ([40, 130, 70, 3000], 224), ([5000, 64, 40, 300], 32),
+                                         ([3, 7], 64)])
+def test_gradients_and_first_step_over_split_products(sizes, batch):
+    """The layers' gradients against the reference and the first Adam step against the update restated
+    from them (both at the tolerances of the tests above), where the input gradient sums 128 partials,
+    where batch and splits leave remainders, where one partial of a weight gradient exceeds the
+    workspace, and with one layer."""
+    rng = np.random.default_rng(batch + len(sizes))
+    params = random_params(sizes, rng)
+    x = rng.uniform(-1, 1, (batch, sizes[0])).astype(np.float32)
+    t = rng.normal(size=(batch, sizes[-1])).astype(np.float32)
+    with Network(sizes, members=1, max_batch=batch) as net:
+        net.set_params(params)
+        net.set_dataset(x, t)
+        _, grads = net.gradients(x, t)
+        _, ref = loss_and_grads(params, x, t, emulate=True)
+        for (gw, gb), (rw, rb) in zip(grads, ref):
+            assert rel(gw, rw) < 2e-3 and rel(gb, rb) < 2e-3
+        net.train(np.arange(batch, dtype=np.int32), batch, 1e-3)
+        for old, new, grad in zip(params, net.get_params(), grads):
+            for a, b, g in zip(old, new, grad):
+                upd = 1e-3 * g.astype(np.float64) / (np.abs(g.astype(np.float64)) + 1e-8)
+                assert np.abs(b - (a.astype(np.float64) - upd)).max() < 1e-3 * np.abs(upd).max()
+
+
 def test_predict_into_page_locked_memory_with_output_scale():
     """predict writes the ensemble mean into a caller's page-locked array, the same bits as into
     its own; the device-side output scale multiplies the mean as a host FP32 product would and
