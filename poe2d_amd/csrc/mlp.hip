@@ -330,32 +330,51 @@ int product_splits(const poe2d_mlp *m, int M, int N, int K)
     return ksplit;
 }
 
-// Forward pass of member e on the first n rows of m->xin (already packed into h16[0]).
-poe2d_status forward(poe2d_mlp *m, Member &e, int n)
+// Hidden layer l on n rows in h, into out (and before the activation into pre when given).
+poe2d_status hidden(poe2d_mlp *m, const Layer &l, const uint16_t *h, int n, float *pre, uint16_t *out)
 {
-    for (int li = 0; li < m->L; ++li) {
-        Layer &l = e.layers[li];
-        const bool last = li == m->L - 1;
-        GemmOut o;
-        o.bias = l.b;
-        o.pre = last ? nullptr : m->pre[li];
-        o.ldp = l.outp;
-        if (last) {
-            o.f32 = m->y;
-            o.ldf = l.outp;
-        } else {
-            o.b16 = m->h16[li + 1];
-            o.ldb = l.outp;
-        }
-        HIP_TRY(gemm_bf16(m->h16[li], l.inp, l.w16, l.inp, n, l.out, l.inp, last ? EPI_LINEAR : EPI_GELU, o, m->work,
-                          m->work_floats, product_splits(m, n, l.out, l.inp), m->stream));
+    const int ksplit = product_splits(m, n, l.out, l.inp);
+    if (hidden_in_registers(1, n, l.out, l.inp)) {
+        HIP_TRY(hidden_layer(h, l.inp, 0, l.w16, nullptr, l.inp, l.b, nullptr, 1, n, l.out, l.inp, ksplit, pre, l.outp, out, l.outp,
+                             0, m->stream));
+        return POE2D_OK;
+    }
+    GemmOut o;
+    o.bias = l.b;
+    o.pre = pre;
+    o.ldp = l.outp;
+    o.b16 = out;
+    o.ldb = l.outp;
+    HIP_TRY(gemm_bf16(h, l.inp, l.w16, l.inp, n, l.out, l.inp, EPI_GELU, o, m->work, m->work_floats, ksplit, m->stream));
+    return POE2D_OK;
+}
+
+poe2d_status hidden_layers(poe2d_mlp *m, const Member &e, int n)
+{
+    for (int li = 0; li < m->L - 1; ++li) {
+        poe2d_status st = hidden(m, e.layers[li], m->h16[li], n, m->pre[li], m->h16[li + 1]);
+        if (st) return st;
     }
     return POE2D_OK;
 }
 
+// Forward pass of member e on the first n rows of m->xin (already packed into h16[0]).
+poe2d_status forward(poe2d_mlp *m, Member &e, int n)
+{
+    poe2d_status st = hidden_layers(m, e, n);
+    if (st) return st;
+    const Layer &l = e.layers[m->L - 1];
+    GemmOut o;
+    o.bias = l.b;
+    o.f32 = m->y;
+    o.ldf = l.outp;
+    HIP_TRY(gemm_bf16(m->h16[m->L - 1], l.inp, l.w16, l.inp, n, l.out, l.inp, EPI_LINEAR, o, m->work, m->work_floats,
+                      product_splits(m, n, l.out, l.inp), m->stream));
+    return POE2D_OK;
+}
 
-// The ensemble on the nb rows in h16[0]: the hidden layers of every member, layer by layer (as many
-// members to a launch as the partials buffer holds), then their output layers and statistics in one
+
+// The ensemble on the nb rows in h16[0]: the hidden layers of every member, layer by layer, then their output layers and statistics in one
 // pass.  mean [nb][outputs] (scaled) and spread [nb] are device memory; either may be null.
 poe2d_status ensemble_batch(poe2d_mlp *m, int nb, float *mean, float *spread)
 {
@@ -372,11 +391,14 @@ poe2d_status ensemble_batch(poe2d_mlp *m, int nb, float *mean, float *spread)
         uint16_t *const next = m->hens[li + 1];
         const size_t next_stride = (size_t)B * l.outp;
         const int ksplit = product_splits(m, nb, l.out, l.inp);
-        const int group = std::max<int>(1, (int)std::min<size_t>(E, m->work_floats / ((size_t)ksplit * nb * l.out)));
-        for (int k = 0; k < E; k += group)
-            HIP_TRY(gemm_bf16_members(h + k * stride, l.inp, stride, m->ens_w[li] + k, l.inp, m->ens_b[li] + k,
-                                      std::min(group, E - k), nb, l.out, l.inp, next + k * next_stride, l.outp, next_stride,
-                                      m->work, m->work_floats, ksplit, m->stream));
+        if (hidden_in_registers(E, nb, l.out, l.inp))
+            HIP_TRY(hidden_layer(h, l.inp, stride, nullptr, m->ens_w[li], l.inp, nullptr, m->ens_b[li], E, nb, l.out, l.inp, ksplit,
+                                 nullptr, 0, next, l.outp, next_stride, m->stream));
+        else
+            for (int k = 0; k < E; ++k) {
+                poe2d_status st = hidden(m, m->members[k].layers[li], h + k * stride, nb, nullptr, next + k * next_stride);
+                if (st) return st;
+            }
         h = next;
         stride = next_stride;
     }
@@ -459,17 +481,8 @@ poe2d_status train_step(poe2d_mlp *m, Member &e, int n, const float *tgt, int ld
                         float *loss_dev)
 {
     const int L = m->L;
-    for (int li = 0; li < L - 1; ++li) {
-        Layer &l = e.layers[li];
-        GemmOut o;
-        o.bias = l.b;
-        o.pre = m->pre[li];
-        o.ldp = l.outp;
-        o.b16 = m->h16[li + 1];
-        o.ldb = l.outp;
-        HIP_TRY(gemm_bf16(m->h16[li], l.inp, l.w16, l.inp, n, l.out, l.inp, EPI_GELU, o, m->work, m->work_floats,
-                          product_splits(m, n, l.out, l.inp), m->stream));
-    }
+    poe2d_status st = hidden_layers(m, e, n);
+    if (st) return st;
     Layer &top = e.layers[L - 1];
     {
         GemmOut o;
@@ -497,8 +510,7 @@ poe2d_status train_step(poe2d_mlp *m, Member &e, int n, const float *tgt, int ld
         loss_sum<<<1, 256, 0, m->stream>>>(m->partial, gemm_tiles(n, top.out), 1.0 / ((double)n * top.out), loss_dev);
         HIP_TRY(hipGetLastError());
     }
-    poe2d_status st = transpose_activations(m, e, n);
-    if (st) return st;
+    if ((st = transpose_activations(m, e, n))) return st;
     for (int li = L - 1; li >= 0; --li) {
         Layer &l = e.layers[li];
         // (with the weights of this step)

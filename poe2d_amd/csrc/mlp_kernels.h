@@ -74,12 +74,14 @@ struct GemmOut {
 hipError_t gemm_bf16(const uint16_t *A, int lda, const uint16_t *B, int ldb, int M, int N, int K, int epi,
                      const GemmOut &out, float *work, size_t work_floats, int ksplit, hipStream_t stream);
 
-// The same hidden-layer product of several members at once: member z's A + z stride_a (0: shared),
-// weights bs[z] and bias biases[z] into b16 + z stride_b16 with GELU; work holds members * ksplit * M * N
-// floats.  Values equal gemm_bf16's with EPI_GELU and the same ksplit > 1.
-hipError_t gemm_bf16_members(const uint16_t *A, int lda, size_t stride_a, const uint16_t *const *bs, int ldb,
-                             const float *const *biases, int members, int M, int N, int K, uint16_t *b16, int ldb16,
-                             size_t stride_b16, float *work, size_t work_floats, int ksplit, hipStream_t stream);
+// A hidden layer gelu(A B^T + bias) into b16 (and before the activation into pre when given): of one
+// member (B, bias), or of several at once, member z's A + z stride_a (0: shared), bs[z] and biases[z] into
+// b16 + z stride_b16.  Values equal gemm_bf16's with EPI_GELU and the same ksplit > 1.  K a multiple of 64.
+hipError_t hidden_layer(const uint16_t *A, int lda, size_t stride_a, const uint16_t *B, const uint16_t *const *bs, int ldb,
+                        const float *bias, const float *const *biases, int members, int M, int N, int K, int ksplit, float *pre,
+                        int ldp, uint16_t *b16, int ldb16, size_t stride_b16, hipStream_t stream);
+// Whether that is the faster way (gemm_bf16 the other).
+bool hidden_in_registers(int members, int M, int N, int K);
 
 // The members' output layer (A + z stride_a times bs[z]^T + biases[z]) and its statistics: mean over
 // members times scale (either may be null) into mean [M][ldm], and spread[m] = ||standard deviation over

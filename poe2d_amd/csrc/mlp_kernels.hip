@@ -44,6 +44,10 @@ constexpr int LDS_ROW = BK + 8;  // bf16 per LDS row (16-byte pad against bank c
 constexpr int kCus = 256;
 constexpr float kCostSquare = 3.0f, kCostTall = 2.7f;
 
+// hidden layers with at most this many inputs form their sums one after the other in a block; with more,
+// the chain costs more than partials in memory unless the tiles fill the chip
+constexpr int kHiddenChain = 2048;
+
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
 
 __device__ __forceinline__ float gelu_grad(float x)
@@ -73,21 +77,11 @@ __device__ __forceinline__ float adam_update(float *w, float *mom, float *vel, f
     return x;
 }
 
-// C (+)= A B^T over k in [k0, k1) for the 128 x 128 tile (tm, tn); k0, k1 multiples of BK.  Split-K
-// launches may hold several products (blockIdx.z): product z reads A + z stride_a and bs[z], and its
-// partials follow those of product z - 1.
+// C (+)= A B^T over k in [k0, k1) for the 128 x 128 tile (tm, tn); k0, k1 multiples of BK.
 template <int EPI>
 __global__ void __launch_bounds__(256, 3) gemm_nt(const uint16_t *__restrict__ A, int lda, const uint16_t *__restrict__ B,
-                                               int ldb, int M, int N, int K, int ksplit, GemmOut out,
-                                               const uint16_t *const *__restrict__ bs = nullptr, size_t stride_a = 0)
+                                               int ldb, int M, int N, int K, int ksplit, GemmOut out)
 {
-    if constexpr (EPI == EPI_PARTIAL) {
-        if (bs) {
-            A += blockIdx.z * stride_a;
-            B = bs[blockIdx.z];
-            out.f32 += (size_t)blockIdx.z * ksplit * M * out.ldf;
-        }
-    }
     // operand tiles (la, lb: two k tiles each), reused by the EPI_MSE / EPI_ADAM epilogues for the
     // transposed bf16 tile and the EPI_MSE sums (40 KiB)
     __shared__ uint16_t lds[2 * BM * LDS_ROW + 2 * BN * LDS_ROW];
@@ -379,6 +373,130 @@ __global__ void __launch_bounds__(256, 3) gemm_nt(const uint16_t *__restrict__ A
     }
 }
 
+// Products over tiles of 64 k values.  A block of WM x WN waves, each with MI x NJ results of 32 x 32, owns
+// the tile (tm, tn) of C = A B^T (M x N); its operand tiles reach LDS by direct loads, STAGES of them in
+// the ring, so no register carries them and STAGES - 1 are in flight.  A wave's direct load writes 1 KiB
+// of consecutive LDS, so rows are unpadded; the 16-byte chunks of a row are exchanged by its row bits
+// instead, which spreads the sixteen rows that a phase of a fragment read touches over all 64 banks (by
+// the low row bits alone, two rows met in each: 45 % of the LDS cycles, 3 % of the time of a large product).
+//
+// The ring (ring_elems long) is the kernel's only LDS array, what else the kernel keeps there behind it: of
+// several arrays, or with its end out of the compiler's sight, the compiler holds every read until all
+// direct loads in flight have landed.  The waits for the tile that is read are written out here.
+//
+// at(pa, pb) gives the addresses of A's and B's next k tile (the first 64 values of the block's first
+// rows), next() moves on to the one after; they run STAGES - 1 tiles ahead, past the last step too (any
+// readable tile does).  after(q) follows the matrix instructions of k values 16 q .. of a tile.
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(1))) void global_void;
+// pointers in memory that no kernel writes: read by scalar loads, which no load in flight delays
+typedef __attribute__((address_space(4))) const uint64_t const_u64;
+
+constexpr int RING_K = 64;
+constexpr int ring_elems(int tm, int tn, int stages) { return stages * (tm + tn) * RING_K; }
+
+template <int WM, int WN, int MI, int NJ, int STAGES, class At, class Next, class After>
+__device__ __forceinline__ void ring_product(uint16_t *ring, int M, int N, int lda, int ldb, int tm, int tn, int steps,
+                                             f32x16 (&acc)[MI][NJ], const At &at, const Next &next, const After &after)
+{
+    static_assert(STAGES >= 2 && STAGES <= 4, "the loop over the steps");
+    constexpr int TM = 32 * MI * WM, TN = 32 * NJ * WN, BKL = RING_K;
+    constexpr int CH = BKL / 8;                         // 16-byte chunks of a row
+    constexpr int RPL = 64 / CH;                        // rows one wave's load covers
+    constexpr int LOADS = (TM + TN) / RPL / (WM * WN);  // loads per wave and tile
+    constexpr int STAGE = (TM + TN) * BKL;              // bf16 per stage
+    uint16_t *const s0 = ring, *const s1 = ring + STAGE, *const s2 = ring + (STAGES > 2 ? 2 : 0) * STAGE,
+                   *const s3 = ring + (STAGES - 1) * STAGE;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = wave / WN, wn = wave % WN;
+    // swizzle: chunk c of row r sits at chunk c ^ swz(r)
+    auto swz = [](int r) -> int { return (r >> 1 & 3) << 1 | (r >> 3 & 1); };
+
+    // the byte this lane loads, from the tile's first row: load l of the wave covers rows (wave * LOADS +
+    // l) * RPL .. of the stage (A's rows, then B's)
+    uint32_t off[LOADS];
+#pragma unroll
+    for (int l = 0; l < LOADS; ++l) {
+        const int r = (wave * LOADS + l) * RPL + lane / CH, c = (lane % CH) ^ swz(r);
+        off[l] = r < TM ? (uint32_t)(min(r, M - 1 - tm * TM) * lda + c * 8) * 2u
+                        : (uint32_t)(min(r - TM, N - 1 - tn * TN) * ldb + c * 8) * 2u;
+    }
+    // the loads first <= l < last of a tile
+    auto load = [&](uint16_t *stage, int first, int last) {
+        uint64_t pa, pb;
+        at(pa, pb);
+#pragma unroll
+        for (int l = 0; l < LOADS; ++l) {
+            if (l < first || l >= last) continue;
+            const int r0 = (wave * LOADS + l) * RPL;  // (a load's rows are all A's or all B's)
+            __builtin_amdgcn_global_load_lds(
+                (global_void *)((__attribute__((address_space(1))) char *)(r0 < TM ? pa : pb) + off[l]),
+                (lds_void *)(stage + r0 * BKL), 16, 0, 0);
+        }
+    };
+    load(s0, 0, LOADS), next();
+    if constexpr (STAGES > 2) load(s1, 0, LOADS), next();
+    if constexpr (STAGES > 3) load(s2, 0, LOADS), next();
+
+    // this lane's fragments: rows ar, ar + 32 of A and br, br + 32 of B, chunk (kk / 8 + lane / 32) ^ swz of
+    // k step kk (32 rows on the swizzle is the same), as offsets into a stage
+    const int ar = wm * 32 * MI + (lane & 31), br = TM + wn * 32 * NJ + (lane & 31);
+    int ao[BKL / 16], bo[BKL / 16];
+#pragma unroll
+    for (int q = 0; q < BKL / 16; ++q) {
+        ao[q] = ar * BKL + ((2 * q + (lane >> 5)) ^ swz(ar)) * 8;
+        bo[q] = br * BKL + ((2 * q + (lane >> 5)) ^ swz(br)) * 8;
+    }
+    // one tile, in stage `from`; the next load goes to `to`, the stage of the tile before
+    auto step = [&](const uint16_t *from, uint16_t *to) {
+        // the tile has landed when no more than the STAGES - 2 tiles after it are in flight; past the
+        // barrier that holds for every wave, and every wave is done with the tile before
+        constexpr int PENDING = LOADS * (STAGES - 2);
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(PENDING) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        bf16x8 fa[2][MI], fb[2][NJ];  // the fragments of k step q and the next
+        auto read = [&](int q) {
+#pragma unroll
+            for (int i = 0; i < MI; ++i) fa[q & 1][i] = *(const bf16x8 *)(from + ao[q] + i * 32 * BKL);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) fb[q & 1][j] = *(const bf16x8 *)(from + bo[q] + j * 32 * BKL);
+        };
+        read(0);
+#pragma unroll
+        for (int q = 0; q < BKL / 16; ++q) {
+            if (q + 1 < BKL / 16) read(q + 1);
+            load(to, q * LOADS / (BKL / 16), (q + 1) * LOADS / (BKL / 16));
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[q & 1][i], fb[q & 1][j], acc[i][j], 0, 0, 0);
+            if (q + 1 == BKL / 16) next();
+            after(q);
+        }
+        // (this wave's reads of the tile are done before it reaches the next barrier)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    };
+    // (left from the middle: an edge back from there would have the first step wait for all loads)
+    for (int g = 0;;) {
+        step(s0, s3);
+        if (++g == steps) break;
+        step(s1, s0);
+        if (++g == steps) break;
+        if constexpr (STAGES > 2) {
+            step(s2, s1);
+            if (++g == steps) break;
+        }
+        if constexpr (STAGES > 3) {
+            step(s3, s2);
+            if (++g == steps) break;
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the re-reads, before a stage is used again
+    __syncthreads();
+}
+
 // Welford's update by member e's outputs.  The accumulators hold the outputs' differences from the
 // running mean: they start at bias - mean (the first at the bias) instead of 0, which saves the sum
 // and the difference, two operations of six; b is the next member's bias (per column).
@@ -488,23 +606,13 @@ __device__ __forceinline__ void ensemble_store(const f32x16 (&mu)[MI][NJ], const
 // What bounds it.  Members one at a time wrote each output array (620 MB of 1024 x 151 500) and read
 // it back with mean and deviations: 0.33 ms of product and 0.51 ms of Welford per member, 0.8 ms of
 // scaling and row sums, 5.3 ms for five members.  Here the mean is the only array that reaches HBM.
-// A block of WM x WN waves, each with MI x NJ results of 32 x 32, owns a tile; the operand tiles of 64 k
-// values reach LDS by direct loads, STAGES of them in a ring, so no register carries them and STAGES - 1
-// are in flight (results of 64 x 64 a wave take 192 of its 256 registers).  A wave's direct load writes
-// 1 KiB of consecutive LDS, so rows are unpadded; the 16-byte chunks of a row are exchanged by its row
-// bits instead, which spreads the sixteen rows that a phase of a fragment read touches over all 64 banks
-// (by the low row bits alone, two rows met in each: 45 % of the LDS cycles, 3 % of the time).  Tile order
-// as EPI_MSE's: m fastest within an XCD's run, so the m tiles of one n tile share its weights in that L2.
+// Results of 64 x 64 a wave take 192 of its 256 registers.  Tile order as EPI_MSE's: m fastest within an
+// XCD's run, so the m tiles of one n tile share its weights in that L2.
 //
 // On 1024 x 151500 x 512 and five members in 256 x 128 tiles 1.19 ms, 670 TFLOP/s (operands through
 // registers, 128 x 128 tiles: 2.13): the matrix cores are busy a third of the cycles, the mean's 620 MB
 // take 0.2 ms in which nothing else runs (one block per CU), the statistics 0.07, and each of the 8 k
 // tiles of a member begins with a barrier and a round trip to LDS.
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) void global_void;
-// pointers in memory that no kernel writes: read by scalar loads, which no load in flight delays
-typedef __attribute__((address_space(4))) const uint64_t const_u64;
-
 constexpr int kBiasMembers = 16;  // members whose biases are in LDS at a time
 
 template <int WM, int WN, int MI, int NJ, int STAGES>
@@ -513,20 +621,11 @@ __global__ void __launch_bounds__(64 * WM * WN, 2)
                   const float *const *__restrict__ biases, int M, int N, int K, int members, float *__restrict__ mean,
                   size_t ldm, const float *__restrict__ scale, double *__restrict__ part)
 {
-    static_assert(STAGES >= 2 && STAGES <= 4, "the loop over the steps");
-    constexpr int TM = 32 * MI * WM, TN = 32 * NJ * WN, THREADS = 64 * WM * WN, BKL = 64;
-    constexpr int CH = BKL / 8;                         // 16-byte chunks of a row
-    constexpr int RPL = 64 / CH;                        // rows one wave's load covers
-    constexpr int LOADS = (TM + TN) / RPL / (WM * WN);  // loads per wave and tile
-    // One array for the stages and, behind them, the biases (read from memory at a member's end, they
-    // would wait for every load in flight).  Of several arrays, or with its end out of the compiler's
-    // sight, the compiler holds reads until all direct loads in flight have landed; the waits for the
-    // tile that is read are written out below.
-    constexpr int STAGE = (TM + TN) * BKL;  // bf16 per stage
-    __shared__ __align__(1024) uint16_t ring[STAGES * STAGE + 2 * kBiasMembers * TN];
-    uint16_t *const s0 = ring, *const s1 = ring + STAGE, *const s2 = ring + (STAGES > 2 ? 2 : 0) * STAGE,
-                   *const s3 = ring + (STAGES - 1) * STAGE;
-    float *const lbias = (float *)(ring + STAGES * STAGE);
+    constexpr int TM = 32 * MI * WM, TN = 32 * NJ * WN, THREADS = 64 * WM * WN;
+    // behind the ring the biases (read from memory at a member's end, they would wait for every load in
+    // flight)
+    __shared__ __align__(1024) uint16_t ring[ring_elems(TM, TN, STAGES) + 2 * kBiasMembers * TN];
+    float *const lbias = (float *)(ring + ring_elems(TM, TN, STAGES));
     const int tiles_m = (M + TM - 1) / TM;
     const int nb = (int)gridDim.x, q8 = nb >> 3, r8 = nb & 7;
     const int xcd = (int)blockIdx.x & 7, slot = (int)blockIdx.x >> 3;
@@ -534,40 +633,8 @@ __global__ void __launch_bounds__(64 * WM * WN, 2)
     const int tm = tile % tiles_m, tn = tile / tiles_m;
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave / WN, wn = wave % WN;
-    const int nk = K / BKL, steps = nk * members;
-    // swizzle: chunk c of row r sits at chunk c ^ swz(r)
-    auto swz = [](int r) -> int { return (r >> 1 & 3) << 1 | (r >> 3 & 1); };
+    const int nk = K / RING_K;
     const_u64 *const b_at = (const_u64 *)(uintptr_t)bs, *const bias_at = (const_u64 *)(uintptr_t)biases;
-
-    // the byte this lane loads, from the tile's first row: load l of the wave covers rows (wave * LOADS +
-    // l) * RPL .. of the stage (A's rows, then B's)
-    uint32_t off[LOADS];
-#pragma unroll
-    for (int l = 0; l < LOADS; ++l) {
-        const int r = (wave * LOADS + l) * RPL + lane / CH, c = (lane % CH) ^ swz(r);
-        off[l] = r < TM ? (uint32_t)(min(r, M - 1 - tm * TM) * lda + c * 8) * 2u
-                        : (uint32_t)(min(r - TM, N - 1 - tn * TN) * ldb + c * 8) * 2u;
-    }
-    int ge = 0, gk = 0;  // member and k tile of the next load
-    // the loads first <= l < last of a tile
-    auto load = [&](uint16_t *stage, int first, int last) {
-        const uint64_t pa = (uint64_t)(uintptr_t)(A + ge * stride_a + (size_t)tm * TM * lda + gk * BKL);
-        const uint64_t pb = b_at[ge] + ((size_t)tn * TN * ldb + gk * BKL) * 2;
-#pragma unroll
-        for (int l = 0; l < LOADS; ++l) {
-            if (l < first || l >= last) continue;
-            const int r0 = (wave * LOADS + l) * RPL;  // (a load's rows are all A's or all B's)
-            __builtin_amdgcn_global_load_lds(
-                (global_void *)((__attribute__((address_space(1))) char *)(r0 < TM ? pa : pb) + off[l]),
-                (lds_void *)(stage + r0 * BKL), 16, 0, 0);
-        }
-    };
-    auto next_tile = [&] {
-        if (++gk == nk) {
-            gk = 0;
-            if (ge + 1 < members) ++ge;  // (past the last step: re-reads, never used)
-        }
-    };
     auto fill_biases = [&](int e0) {
         for (int i = t; i < min(members - e0, kBiasMembers) * TN; i += THREADS) {
             const int n = tn * TN + i % TN;
@@ -586,7 +653,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2)
     __syncthreads();
     float b[NJ];
     auto bias_of = [&](int e) {
-        #pragma unroll
+#pragma unroll
         for (int j = 0; j < NJ; ++j) b[j] = lbias[(e % kBiasMembers) * TN + wn * 32 * NJ + j * 32 + (lane & 31)];
     };
     bias_of(0);
@@ -596,84 +663,94 @@ __global__ void __launch_bounds__(64 * WM * WN, 2)
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = b[j];
-    load(s0, 0, LOADS), next_tile();
-    if constexpr (STAGES > 2) load(s1, 0, LOADS), next_tile();
-    if constexpr (STAGES > 3) load(s2, 0, LOADS), next_tile();
 
-    int kt = 0, e = 0;
-    // this lane's fragments: rows ar, ar + 32 of A and br, br + 32 of B, chunk (kk / 8 + lane / 32) ^ swz of
-    // k step kk (32 rows on the swizzle is the same), as offsets into a stage
-    const int ar = wm * 32 * MI + (lane & 31), br = TM + wn * 32 * NJ + (lane & 31);
-    int ao[BKL / 16], bo[BKL / 16];
-#pragma unroll
-    for (int q = 0; q < BKL / 16; ++q) {
-        ao[q] = ar * BKL + ((2 * q + (lane >> 5)) ^ swz(ar)) * 8;
-        bo[q] = br * BKL + ((2 * q + (lane >> 5)) ^ swz(br)) * 8;
-    }
-    // one tile, in stage `at`; the next load goes to `to`, the stage of the tile before
-    auto step = [&](const uint16_t *at, uint16_t *to) {
-        // the tile has landed when no more than the STAGES - 2 tiles after it are in flight; past the
-        // barrier that holds for every wave, and every wave is done with the tile before
-        constexpr int PENDING = LOADS * (STAGES - 2);
-        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(PENDING) : "memory");
-        __builtin_amdgcn_s_barrier();
-        if (kt == nk - 1 && (e + 1) % kBiasMembers == 0 && e + 1 < members) {
-            fill_biases(e + 1);  // (every wave is past the member before)
-            __builtin_amdgcn_s_barrier();
-        }
-        asm volatile("" ::: "memory");
-        bf16x8 fa[2][MI], fb[2][NJ];  // the fragments of k step q and the next
-        auto read = [&](int q) {
-#pragma unroll
-            for (int i = 0; i < MI; ++i) fa[q & 1][i] = *(const bf16x8 *)(at + ao[q] + i * 32 * BKL);
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) fb[q & 1][j] = *(const bf16x8 *)(at + bo[q] + j * 32 * BKL);
-        };
-        read(0);
-#pragma unroll
-        for (int q = 0; q < BKL / 16; ++q) {
-            if (q + 1 < BKL / 16) read(q + 1);
-            load(to, q * LOADS / (BKL / 16), (q + 1) * LOADS / (BKL / 16));
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                for (int j = 0; j < NJ; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[q & 1][i], fb[q & 1][j], acc[i][j], 0, 0, 0);
-        }
-        next_tile();
-        if (++kt == nk) {
+    int ge = 0, gk = 0;  // member and k tile of the next load
+    int kt = 0, e = 0;   // k tiles done of member e
+    ring_product<WM, WN, MI, NJ, STAGES>(
+        ring, M, N, lda, ldb, tm, tn, nk * members, acc,
+        [&](uint64_t &pa, uint64_t &pb) {
+            pa = (uint64_t)(uintptr_t)(A + ge * stride_a + (size_t)tm * TM * lda + gk * RING_K);
+            pb = b_at[ge] + ((size_t)tn * TN * ldb + gk * RING_K) * 2;
+        },
+        [&] {
+            if (++gk == nk) {
+                gk = 0;
+                if (ge + 1 < members) ++ge;
+            }
+        },
+        [&](int q) {
+            if (q + 1 < RING_K / 16 || ++kt < nk) return;
+            if ((e + 1) % kBiasMembers == 0 && e + 1 < members) {
+                __builtin_amdgcn_s_barrier();  // every wave has read the biases it needs of these
+                fill_biases(e + 1);
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+            }
             bias_of(e + 1);  // (of no use after the last)
             welford_update<MI, NJ>(acc, mu, m2, e, b);
             kt = 0;
             ++e;
-        }
-        // (this wave's reads of the tile are done before it reaches the next barrier)
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    };
-    // (left from the middle: an edge back from there would have the first step wait for all loads)
-    for (int g = 0;;) {
-        step(s0, s3);
-        if (++g == steps) break;
-        step(s1, s0);
-        if (++g == steps) break;
-        if constexpr (STAGES > 2) {
-            step(s2, s1);
-            if (++g == steps) break;
-        }
-        if constexpr (STAGES > 3) {
-            step(s3, s2);
-            if (++g == steps) break;
-        }
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the re-reads, before a stage is used again
-    __syncthreads();
-    double(*const red)[TM][2] = (double(*)[TM][2])s0;
+        });
+    double(*const red)[TM][2] = (double(*)[TM][2])ring;
     ensemble_store<MI, NJ>(mu, m2, tm * TM, tn * TN, wm, wn, M, N, mean, ldm, scale, part != nullptr, red);
     if (!part) return;
     __syncthreads();
     for (int r = t; r < 2 * TM; r += THREADS) {
         const int row = r % TM, w = r / TM, m = tm * TM + row;
         if (m < M) part[((size_t)tn * 2 + w) * M + m] = red[0][row][w] + red[1][row][w];
+    }
+}
+
+// A hidden layer of one or several members (blockIdx.y): gelu(A B^T + bias) as bf16 (b16), before the
+// activation as FP32 (pre) when given.  The sums over ranges of kper k values are formed one after the
+// other and added up in range order, so the values are those of the product split over K (EPI_PARTIAL and
+// reduce_splits) without the partials' way through memory and the second launch.  Latency bounds it, the k
+// tiles one after the other: five members of 512 x 512 take 8.1 us on 37 rows (10.4 split) and 19.1 us on
+// 1024 (40), one member on 256 rows of a training step 3 us less.
+__global__ void __launch_bounds__(256, 2)
+    hidden_product(const uint16_t *__restrict__ A, int lda, size_t stride_a, const uint16_t *B,
+                   const uint16_t *const *__restrict__ bs, int ldb, const float *bias, const float *const *__restrict__ biases,
+                   int M, int N, int K, int kper, float *__restrict__ pre, int ldp, uint16_t *__restrict__ b16, int ldb16,
+                   size_t stride_b16)
+{
+    constexpr int T = 64;  // 2 x 2 waves of 32 x 32
+    __shared__ __align__(1024) uint16_t ring[ring_elems(T, T, 4)];
+    const int tiles_n = (N + T - 1) / T, tm = (int)blockIdx.x / tiles_n, tn = (int)blockIdx.x % tiles_n;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (bs) B = bs[blockIdx.y], bias = biases[blockIdx.y];
+    const int n = tn * T + (wave & 1) * 32 + (lane & 31);
+    const float b = n < N ? bias[n] : 0.f;
+    const uint64_t a0 = (uint64_t)(uintptr_t)(A + blockIdx.y * stride_a + (size_t)tm * T * lda);
+    const uint64_t b0 = (uint64_t)(uintptr_t)(B + (size_t)tn * T * ldb);
+    f32x16 acc[1][1], sums;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[0][0][e] = sums[e] = 0.f;
+    auto flush = [&] {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            sums[e] += acc[0][0][e];
+            acc[0][0][e] = 0.f;
+        }
+    };
+    int gk = 0, k = 0, end = kper;
+    ring_product<2, 2, 1, 1, 4>(
+        ring, M, N, lda, ldb, tm, tn, K / RING_K, acc,
+        [&](uint64_t &pa, uint64_t &pb) { pa = a0 + gk * 2, pb = b0 + gk * 2; },
+        [&] { gk = min(gk + RING_K, K - RING_K); },
+        [&](int) {
+            if ((k += 16) < end) return;
+            flush();
+            end += kper;
+        });
+    if (k > end - kper) flush();
+    const int m0 = tm * T + (wave >> 1) * 32 + (lane >> 5) * 4;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const int m = m0 + (e >> 2) * 8 + (e & 3);
+        if (m >= M || n >= N) continue;
+        const float v = sums[e] + b;
+        if (pre) pre[(size_t)m * ldp + n] = v;
+        b16[blockIdx.y * stride_b16 + (size_t)m * ldb16 + n] = bf16_rne(gelu(v));
     }
 }
 
@@ -706,16 +783,9 @@ __global__ void __launch_bounds__(1024) ensemble_spread(const double *__restrict
     spread[m] = (float)(sqrt(var / (members > 1 ? members - 1 : 1)) / fmax(sqrt(nrm), 1e-30));
 }
 
-// out[m][n] = sum over splits of part[s][m][n] (+ bias), then as the GEMM epilogue; of several
-// products, product blockIdx.y with bias biases[blockIdx.y] into b16 + blockIdx.y stride_b16.
-__global__ void reduce_splits(const float *__restrict__ part, int nsplit, int M, int N, int ldf, GemmOut out, int gelu_on,
-                              const float *const *__restrict__ biases = nullptr, size_t stride_b16 = 0)
+// out[m][n] = sum over splits of part[s][m][n] (+ bias), then as the GEMM epilogue.
+__global__ void reduce_splits(const float *__restrict__ part, int nsplit, int M, int N, int ldf, GemmOut out, int gelu_on)
 {
-    if (biases) {
-        part += (size_t)blockIdx.y * nsplit * M * ldf;
-        out.bias = biases[blockIdx.y];
-        out.b16 += blockIdx.y * stride_b16;
-    }
     const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
     if (i >= (size_t)M * N) return;
     const int m = (int)(i / N), n = (int)(i % N);
@@ -991,25 +1061,22 @@ hipError_t gemm_bf16(const uint16_t *A, int lda, const uint16_t *B, int ldb, int
     return hipGetLastError();
 }
 
-hipError_t gemm_bf16_members(const uint16_t *A, int lda, size_t stride_a, const uint16_t *const *bs, int ldb,
-                             const float *const *biases, int members, int M, int N, int K, uint16_t *b16, int ldb16,
-                             size_t stride_b16, float *work, size_t work_floats, int ksplit, hipStream_t stream)
+bool hidden_in_registers(int members, int M, int N, int K)
 {
-    if (M < 1 || N < 1 || K < BK || K % BK || lda % 8 || ldb % 8 || lda < K || ldb < K || members < 1 || members > 65535 ||
-        ksplit < 1 || ksplit > K / BK || work_floats < (size_t)members * ksplit * M * N)
+    return K % RING_K == 0 && members <= 65535 &&
+           (K <= kHiddenChain || (long long)members * ((M + 63) / 64) * ((N + 63) / 64) >= 2 * kCus);
+}
+
+hipError_t hidden_layer(const uint16_t *A, int lda, size_t stride_a, const uint16_t *B, const uint16_t *const *bs, int ldb,
+                        const float *bias, const float *const *biases, int members, int M, int N, int K, int ksplit, float *pre,
+                        int ldp, uint16_t *b16, int ldb16, size_t stride_b16, hipStream_t stream)
+{
+    if (M < 1 || N < 1 || K < RING_K || K % RING_K || lda % 8 || ldb % 8 || lda < K || ldb < K || members < 1 ||
+        members > 65535 || ksplit < 1 || ksplit > K / BK || (bs ? !biases : !B || !bias || members > 1))
         return hipErrorInvalidValue;
-    GemmOut part{}, out{};
-    part.f32 = work;
-    part.ldf = N;
-    out.b16 = b16;
-    out.ldb = ldb16;
-    const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    gemm_nt<EPI_PARTIAL><<<dim3(tiles, ksplit, members), 256, 0, stream>>>(A, lda, nullptr, ldb, M, N, K, ksplit, part, bs,
-                                                                           stride_a);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    reduce_splits<<<dim3((unsigned)(((size_t)M * N + 255) / 256), members), 256, 0, stream>>>(work, ksplit, M, N, N, out, 1,
-                                                                                            biases, stride_b16);
+    const int kper = ((K / BK + ksplit - 1) / ksplit) * BK;
+    hidden_product<<<dim3(((M + 63) / 64) * ((N + 63) / 64), members), 256, 0, stream>>>(
+        A, lda, stride_a, B, bs, ldb, bias, biases, M, N, K, kper, pre, ldp, b16, ldb16, stride_b16);
     return hipGetLastError();
 }
 

@@ -176,11 +176,11 @@ def test_adam_matches_the_bias_corrected_update():
 
 
 @pytest.mark.parametrize("sizes,batch", [([4, 96, 20000], 32), ([40, 130, 70, 3000], 224), ([5000, 64, 40, 300], 32),
-                                         ([3, 7], 64)])
+                                         ([4, 300, 90, 40], 64), ([3, 7], 64)])
 def test_gradients_and_first_step_over_split_products(sizes, batch):
     """The layers' gradients against the reference and the first Adam step against the update restated
     from them (both at the tolerances of the tests above), where the input gradient sums 128 partials,
-    where batch and splits leave remainders, where one partial of a weight gradient exceeds the
+    where batch and splits leave remainders, where ranges of k end within a tile's 64, where one partial of a weight gradient exceeds the
     workspace, and with one layer."""
     rng = np.random.default_rng(batch + len(sizes))
     params = random_params(sizes, rng)
