@@ -1,6 +1,6 @@
-// Two time steps of a tile held on chip.
+// Two or three time steps of a tile held on chip.
 //
-// A block of 8 waves loads a region of the state once, advances it two steps, and stores the points
+// A block of 8 waves loads a region of the state once, advances it two or three steps, and stores the points
 // whose halo was complete.  A lane is a column and a thread holds P consecutive rows of it
 // (velocities, strains, C-PML memory variables in registers), so x neighbours are the neighbouring
 // lanes' registers (wave shifts, folded into the differences where the instruction allows) and z

@@ -328,7 +328,7 @@ inline int fused_tile_width(int bw) { return bw - 8; }
 // its one-byte material index and a palette of at most kMaxPalette2 entries, else through the
 // coefficient groups.
 __host__ __device__ constexpr int fused2_tile_width(int bw) { return bw - 12; }
-constexpr int kMaxPalette2 = 28;  // palette entries the two-step kernel keeps in LDS (blocks of 64 threads: 12 per CU)
+constexpr int kMaxPalette2 = 28;  // palette entries the two-step kernel keeps in LDS
 // Items whose tile field is negative (~tile) are edge tiles: tiles touching a C-PML strip or
 // holding receivers (the others run a variant without that code).
 template <class T>

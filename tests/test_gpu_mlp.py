@@ -180,8 +180,8 @@ def test_adam_matches_the_bias_corrected_update():
 def test_gradients_and_first_step_over_split_products(sizes, batch):
     """The layers' gradients against the reference and the first Adam step against the update restated
     from them (both at the tolerances of the tests above), where the input gradient sums 128 partials,
-    where batch and splits leave remainders, where ranges of k end within a tile's 64, where one partial of a weight gradient exceeds the
-    workspace, and with one layer."""
+    where batch and splits leave remainders, where ranges of k end within a tile's 64, where one partial
+    of a weight gradient exceeds the workspace, and with one layer."""
     rng = np.random.default_rng(batch + len(sizes))
     params = random_params(sizes, rng)
     x = rng.uniform(-1, 1, (batch, sizes[0])).astype(np.float32)
