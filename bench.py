@@ -7,19 +7,18 @@ outside the timed region.  value = Gcell-updates/s = 4001^2 * 6000 * K / (device
 hipEvents on the solver's stream).
 
 Roofline: the dominant kernel is the step kernel: the single-pass kernel (one launch per time
-step) or the two-step kernel (one launch per two steps, the intermediate state on chip), whichever
-autotunes faster on the grid; either records the receivers, and the device step counter advances
-once per 32 steps.  The algorithmic traffic of a time step is 104 B per point-update (9 state
-fields read + written, 8 coefficients read, FP32) plus 48 B per C-PML strip point and 96 B per
-corner point; `achieved` divides that by the time per step of the timed solves (hipEvents on the
-solver's stream around the whole run, so launch gaps count against the kernel).  The figure is
-fixed by the algorithm, not by the schedule: the two-step kernel performs two cell-updates per
-point per launch while reading and writing the state once, so its `achieved` (and `frac`) can pass
-the HBM peak; `hbm_gbs` beside it is the measured traffic over the same time.  `traffic` is the
-measured HBM bytes per time step (rocprofv3 FETCH_SIZE and WRITE_SIZE per launch, each scaled by
-what the same counter reads for a plain copy of known size, halved for the two-step kernel), read
-from the committed profile summary when it was taken with the same kernel and tile shape, else
-null.
+step), the tile kernel (one launch per two or three steps of a region held on chip) or the marching
+two-step kernel, whichever autotunes fastest on the grid; all record the receivers.  The algorithmic
+traffic of a time step is 104 B per point-update (9 state fields read + written, 8 coefficients
+read, FP32) plus 48 B per C-PML strip point and 96 B per corner point; `achieved` divides that by
+the time per step of the timed solves (hipEvents on the solver's stream around the whole run, so
+launch gaps count against the kernel).  The figure is fixed by the algorithm, not by the schedule: a
+launch of several steps performs as many cell-updates per point while reading and writing the state
+once, so its `achieved` (and `frac`) can pass the HBM peak; `hbm_gbs` beside it is the measured
+traffic over the same time.  `traffic` is the measured HBM bytes per time step (rocprofv3 FETCH_SIZE
+and WRITE_SIZE per launch, each scaled by what the same counter reads for a plain copy of known
+size, divided by the launch's steps), read from the committed profile summary when it was taken with
+the same kernel and tile shape, else null.
 
 The CPU baseline is the oracle in its reference-structured form (five sweeps plus three full-grid
 receiver scans per step, one thread) timed on a bounded sample of the same model.
@@ -67,9 +66,15 @@ def strip_counts(prob):
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "fused_step_4001x4001_traffic.txt")
 
 
+def steps_per_launch(tile, schedule):
+    """Time steps of one launch: one (schedule 0); two, or on the tile kernel (block width 64) three
+    for tile heights 30 and 6."""
+    return 1 if schedule != 3 else 3 if tile[0] == 64 and tile[1] in (6, 30) else 2
+
+
 def recorded_traffic(tile, n, schedule=0):
     """HBM bytes per time step from the committed PMC summary ("grid_n: N", "tile BWxTH: bytes"
-    for the one-step kernel and "two-step BWxTH: bytes" for the two-step kernel, bytes per
+    for the one-step kernel and "two-step BWxTH: bytes" for schedule 3's kernels, bytes per
     launch), if it was measured on this grid with this kernel and tile shape."""
     try:
         lines = [ln.strip() for ln in open(TRAFFIC_FILE) if ln.strip() and not ln.startswith("#")]
@@ -77,7 +82,7 @@ def recorded_traffic(tile, n, schedule=0):
         return None, None
     kv = dict(ln.split(":", 1) for ln in lines if ":" in ln)
     kv = {k.strip(): v.strip() for k, v in kv.items()}
-    key, per = (f"tile {tile[0]}x{tile[1]}", 1) if schedule == 0 else (f"two-step {tile[0]}x{tile[1]}", 2)
+    key, per = f"{'tile' if schedule == 0 else 'two-step'} {tile[0]}x{tile[1]}", steps_per_launch(tile, schedule)
     try:
         if int(kv.get("grid_n", -1)) != n + 1:
             return None, None
@@ -101,14 +106,15 @@ def trace_rel_l2(g, o, floor=1e-3):
     return num / np.maximum(np.maximum(den, floor * den.max(axis=-1, keepdims=True)), 1e-300)
 
 
-def compulsory_bytes_per_step(npts, strip_points, schedule, palette):
+def compulsory_bytes_per_step(npts, strip_points, schedule, palette, tile):
     """Bytes per time step that the schedule cannot avoid: each launch reads and writes the V and S
     groups (64 B per point, FP32) and reads the one-byte material index (palette) or both coefficient
-    groups (32 B); the two-step kernel does this once per two steps.  Every step reads and writes the
-    six memory variables of each strip record (48 B per strip point and strip)."""
+    groups (32 B), once per steps_per_launch steps.  The six memory variables of each strip record
+    (48 B per strip point and strip) are read and written every step, by the tile kernel every
+    launch."""
     per_point = 64.0 + (1.0 if palette else 32.0)
-    per_launch_steps = 2 if schedule == 3 else 1
-    return per_point * npts / per_launch_steps + 48.0 * strip_points
+    steps = steps_per_launch(tile, schedule)
+    return per_point * npts / steps + 48.0 * strip_points / (steps if schedule == 3 and tile[0] == 64 else 1)
 
 
 def cpu_leg(prob, make, steps, gpu_traces):
@@ -244,7 +250,7 @@ def time_batch(members, nt, warmup, reps, schedules=(0, 3), label="batch", fixed
     return statistics.median(dev_ms), schedule, tile, finite
 
 
-SCHEDULE_NAMES = {0: "one step per launch", 3: "two steps per launch"}
+SCHEDULE_NAMES = {0: "one step per launch", 3: "several steps per launch"}
 
 
 def secondary_continuous(n, nt):
@@ -284,7 +290,7 @@ def secondary_no_palette(prob, nt, label):
             out[f"schedule_{sched}"] = {"kernel": SCHEDULE_NAMES[sched], "tile": f"{t[0]}x{t[1]} (autotuned)",
                                         "us_per_step": round(step_s * 1e6, 1),
                                         "gcell_updates_per_s": round(npts / step_s / 1e9, 2),
-                                        "compulsory_frac": round(compulsory_bytes_per_step(npts, strips, sched, False)
+                                        "compulsory_frac": round(compulsory_bytes_per_step(npts, strips, sched, False, t)
                                                                  / step_s / 1e9 / HBM_PEAK_GBS, 4)}
             print(f"[bench] {label} schedule {sched}: {t[0]}x{t[1]}, {step_s * 1e6:.1f} us per step",
                   file=sys.stderr, flush=True)
@@ -562,7 +568,7 @@ def main():
                     help="tile shape of the step kernel (block width x tile rows); 'auto' runs the "
                          "library's autotuner first")
     ap.add_argument("--schedule", default="auto", choices=("auto", "0", "3"),
-                    help="step kernel: 0 = one step per launch, 3 = two steps per launch, auto = the "
+                    help="step kernel: 0 = one step per launch, 3 = several steps per launch, auto = the "
                          "faster after autotuning both")
     ap.add_argument("--copy-probe", type=int, default=0, metavar="MIB",
                     help="instead of the benchmark: time a plain device copy of MIB MiB (torch; the copy "
@@ -669,7 +675,9 @@ def main():
     achieved = bytes_step / (step_ms / 1e3) / 1e9
     # the committed counter readings are of configuration 1's patchy model
     traffic, traffic_src = recorded_traffic(tile, args.n, schedule) if args.workload == "config1" else (None, None)
-    compulsory = compulsory_bytes_per_step(npts, cols * (prob.nz + 1) + rows * (prob.nx + 1), schedule, palette > 0)
+    compulsory = compulsory_bytes_per_step(npts, cols * (prob.nz + 1) + rows * (prob.nx + 1), schedule, palette > 0,
+                                           tile)
+    launch_steps = steps_per_launch(tile, schedule)
     out = {
         "metric": ("Gcell-updates/s (FP32 Biot C-PML time loop, 4001x4001, 6000 steps)" if args.workload == "config1"
                    else f"Gcell-updates/s (FP32 Biot C-PML time loop, {prob.meta['workload']}, {args.nt} steps)"),
@@ -703,18 +711,18 @@ def main():
                      "frac_compulsory": round(compulsory / (step_ms / 1e3) / 1e9 / HBM_PEAK_GBS, 4),
                      "compulsory_bytes_per_step": round(compulsory),
                      "kernel": ("fused_step (one launch per time step, 32-step HIP graphs)" if schedule == 0 else
-                                "fused_step2 (one launch per two time steps, 32-step HIP graphs); per step: "
-                                "half a launch"),
+                                f"tile_steps (one launch per {launch_steps} time steps)" if tile[0] == 64 else
+                                "fused_step2 (one launch per two time steps, 32-step HIP graphs)"),
                      "step_us": round(step_ms * 1e3, 2),
-                     "per_launch": (("one time step" if schedule == 0 else "two time steps, 2 x") +
+                     "per_launch": (("one time step," if launch_steps == 1 else f"{launch_steps} time steps, {launch_steps} x") +
                                     f" {bytes_step / 1e9:.4f} GB algorithmic per step "
                                     f"(104 B x {npts} points + 48 B x strip points, {cols} strip columns, "
                                     f"{rows} strip rows)"),
                      "hbm_gbs": None if traffic is None else round(traffic / (step_ms / 1e3) / 1e9, 1),
                      "traffic_source": traffic_src,
                      "note": ("frac: algorithmic bytes, 104 B per cell-update (+ C-PML strips) whatever the "
-                              "schedule (the two-step kernel performs two cell-updates per point for each pass "
-                              "over HBM, so it can pass 1); frac_measured: the HBM traffic the counters read per "
+                              "schedule (a launch of several steps performs as many cell-updates per point for "
+                              "each pass over HBM, so it can pass 1); frac_measured: the HBM traffic the counters read per "
                               "step (traffic) over the same time; frac_compulsory: the bytes this schedule cannot "
                               "avoid per step (state read and written once per launch, the one-byte material "
                               "index or the coefficients, C-PML records) over the same time")},
