@@ -29,8 +29,8 @@ typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int BM = 128, BN = 128, BK = 32;
 constexpr int LDS_ROW = BK + 8;  // bf16 per LDS row (16-byte pad against bank conflicts)
-// The shape of ensemble_output's tiles: the one with the least work per CU, tiles per block slot (two
-// blocks a CU of the 64 x 64 and 128 x 128, one of the 256 x 128; less than one slot each costs a whole
+// The shape of ensemble_output's tiles: the one with the least work per CU, tiles per block slot (counted
+// two a CU of the 64 x 64 and 128 x 128, one of the 256 x 128; less than one slot each costs a whole
 // tile) times a tile's cost relative to 64 x 64.  Larger tiles read their operands less often, but pad
 // more rows and fill the chip later.  Measured, us per pass, five members of 512 hidden, rows x outputs:
 //                 64 x 64   128 x 128   256 x 128
@@ -705,8 +705,9 @@ __global__ void __launch_bounds__(64 * WM * WN, 2)
 // activation as FP32 (pre) when given.  The sums over ranges of kper k values are formed one after the
 // other and added up in range order, so the values are those of the product split over K (EPI_PARTIAL and
 // reduce_splits) without the partials' way through memory and the second launch.  Latency bounds it, the k
-// tiles one after the other: five members of 512 x 512 take 8.1 us on 37 rows (10.4 split) and 19.1 us on
-// 1024 (40), one member on 256 rows of a training step 3 us less.
+// tiles one after the other: five members of 512 x 512 take 8.1 us on 37 rows (10.4 split) and 15.0 us on
+// 1024 (40; 19.1 with four stages and two blocks to a CU), one member on 256 rows of a training step 3 us
+// less.
 __global__ void __launch_bounds__(256, 2)
     hidden_product(const uint16_t *__restrict__ A, int lda, size_t stride_a, const uint16_t *B,
                    const uint16_t *const *__restrict__ bs, int ldb, const float *bias, const float *const *__restrict__ biases,
@@ -714,7 +715,7 @@ __global__ void __launch_bounds__(256, 2)
                    size_t stride_b16)
 {
     constexpr int T = 64;  // 2 x 2 waves of 32 x 32
-    __shared__ __align__(1024) uint16_t ring[ring_elems(T, T, 4)];
+    __shared__ __align__(1024) uint16_t ring[ring_elems(T, T, 3)];
     const int tiles_n = (N + T - 1) / T, tm = (int)blockIdx.x / tiles_n, tn = (int)blockIdx.x % tiles_n;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     if (bs) B = bs[blockIdx.y], bias = biases[blockIdx.y];
@@ -733,7 +734,7 @@ __global__ void __launch_bounds__(256, 2)
         }
     };
     int gk = 0, k = 0, end = kper;
-    ring_product<2, 2, 1, 1, 4>(
+    ring_product<2, 2, 1, 1, 3>(
         ring, M, N, lda, ldb, tm, tn, K / RING_K, acc,
         [&](uint64_t &pa, uint64_t &pb) { pa = a0 + gk * 2, pb = b0 + gk * 2; },
         [&] { gk = min(gk + RING_K, K - RING_K); },
@@ -1100,7 +1101,9 @@ hipError_t ensemble_output(const uint16_t *A, int lda, size_t stride_a, const ui
     };
     if (tall) launch(ensemble_tiles<4, 2, 2, 2, 3>, 512);
     else if (square) launch(ensemble_tiles<2, 2, 2, 2, 2>, 256);
-    else launch(ensemble_tiles<2, 2, 1, 1, 4>, 256);
+    // (three stages, three blocks to a CU: four stages leave room for two, 100 x 20000 116 us instead of 109,
+    // 700 x 6300 158 instead of 150, 40 x 151500 261 instead of 254)
+    else launch(ensemble_tiles<2, 2, 1, 1, 3>, 256);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !spread) return e;
     ensemble_spread<<<(M + kSpreadRows - 1) / kSpreadRows, 1024, 0, stream>>>(part, tiles_n, M, members, spread);
