@@ -44,9 +44,12 @@ constexpr int LDS_ROW = BK + 8;  // bf16 per LDS row (16-byte pad against bank c
 constexpr int kCus = 256;
 constexpr float kCostSquare = 3.0f, kCostTall = 2.7f;
 
-// hidden layers with at most this many inputs form their sums one after the other in a block; with more,
-// the chain costs more than partials in memory unless the tiles fill the chip
-constexpr int kHiddenChain = 2048;
+// Hidden layers with at most this many inputs per member form their sums one after the other in a block;
+// with more, the chain costs more than partials in memory unless the tiles fill the chip.  us per
+// prediction, in registers / split (member by member): one member, 37 rows of 2000 inputs 92 / 103, 4000
+// 110 / 112, 16000 214 / 193, 256 rows of 4000 245 / 258, 16000 619 / 600; five members, 37 rows of 4000
+// 121 / 181, 16000 224 / 283.
+constexpr int kHiddenChain = 4096;
 
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
 
@@ -1065,7 +1068,7 @@ hipError_t gemm_bf16(const uint16_t *A, int lda, const uint16_t *B, int ldb, int
 bool hidden_in_registers(int members, int M, int N, int K)
 {
     return K % RING_K == 0 && members <= 65535 &&
-           (K <= kHiddenChain || (long long)members * ((M + 63) / 64) * ((N + 63) / 64) >= 2 * kCus);
+           (K <= (long long)kHiddenChain * members || (long long)members * ((M + 63) / 64) * ((N + 63) / 64) >= 2 * kCus);
 }
 
 hipError_t hidden_layer(const uint16_t *A, int lda, size_t stride_a, const uint16_t *B, const uint16_t *const *bs, int ldb,
