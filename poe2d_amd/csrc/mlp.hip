@@ -23,6 +23,7 @@
 #include "../../include/poe2d.h"
 #include "common.h"
 #include "mlp_kernels.h"
+#include "mlp_plan.h"
 
 using namespace poe2d;
 using namespace poe2d::mlp;
@@ -207,7 +208,7 @@ __global__ void repitch(const float *__restrict__ src, size_t lds, float *__rest
 // rows x cols values of a device array (ld apart) to contiguous host memory or, from_host, back.  A
 // strided copy to or from pageable memory moves a row at a time (75 750 rows of 2 KB: 538 ms, one
 // contiguous copy 9 to 17 ms), so padded rows are packed on the device first, through the partials
-// buffer, as many rows at a time as it holds.
+// buffer, as many rows (or as much of a row) at a time as it holds.
 poe2d_status copy_rows(poe2d_mlp *m, float *host, float *dev, int ld, int rows, int cols, bool from_host)
 {
     if (ld == cols) {
@@ -215,21 +216,22 @@ poe2d_status copy_rows(poe2d_mlp *m, float *host, float *dev, int ld, int rows, 
                                from_host ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, m->stream));
         return POE2D_OK;
     }
-    const int piece = (int)std::min<size_t>(rows, std::max<size_t>(m->work_floats / cols, 1));
-    for (int r = 0; r < rows; r += piece) {
-        const int n = std::min(piece, rows - r);
-        const size_t count = (size_t)n * cols;
-        const int grid = (int)std::min<size_t>((count + 255) / 256, 65536);
-        float *const h = host + (size_t)r * cols, *const d = dev + (size_t)r * ld;
-        if (from_host) {
-            HIP_TRY(hipMemcpyAsync(m->work, h, count * sizeof(float), hipMemcpyHostToDevice, m->stream));
-            repitch<<<grid, 256, 0, m->stream>>>(m->work, cols, d, ld, n, cols);
-        } else {
-            repitch<<<grid, 256, 0, m->stream>>>(d, ld, m->work, cols, n, cols);
-            HIP_TRY(hipMemcpyAsync(h, m->work, count * sizeof(float), hipMemcpyDeviceToHost, m->stream));
+    const Piece piece = staging_piece(m->work_floats, rows, cols);
+    for (int r = 0; r < rows; r += piece.rows)
+        for (int c = 0; c < cols; c += piece.cols) {
+            const int nr = std::min(piece.rows, rows - r), nc = std::min(piece.cols, cols - c);
+            const size_t count = (size_t)nr * nc;
+            const int grid = (int)std::min<size_t>((count + 255) / 256, 65536);
+            float *const h = host + (size_t)r * cols + c, *const d = dev + (size_t)r * ld + c;
+            if (from_host) {
+                HIP_TRY(hipMemcpyAsync(m->work, h, count * sizeof(float), hipMemcpyHostToDevice, m->stream));
+                repitch<<<grid, 256, 0, m->stream>>>(m->work, nc, d, ld, nr, nc);
+            } else {
+                repitch<<<grid, 256, 0, m->stream>>>(d, ld, m->work, nc, nr, nc);
+                HIP_TRY(hipMemcpyAsync(h, m->work, count * sizeof(float), hipMemcpyDeviceToHost, m->stream));
+            }
+            HIP_TRY(hipGetLastError());
         }
-        HIP_TRY(hipGetLastError());
-    }
     return POE2D_OK;
 }
 

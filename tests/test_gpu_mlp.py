@@ -302,3 +302,20 @@ def test_predict_statistics_match_the_members_outputs(sizes, rows, members, batc
     var = y.var(0, ddof=1) if members > 1 else np.zeros_like(y[0])
     expect = np.sqrt(var.sum(1)) / np.linalg.norm(y.mean(0), axis=1)
     assert np.allclose(spread, expect, rtol=1e-4, atol=1e-12)
+
+
+@pytest.mark.parametrize("sizes", [[5000, 8], [9001, 130]])
+def test_rows_longer_than_the_workspace(sizes):
+    """A network without hidden layers has less workspace (4096 floats with batches of 32) than one of its
+    padded rows: weights come back as they were set, gradients are the reference's (tolerance as above)."""
+    rng = np.random.default_rng(sizes[0])
+    params = random_params(sizes, rng)
+    x = rng.uniform(-1, 1, (32, sizes[0])).astype(np.float32)
+    t = rng.normal(size=(32, sizes[-1])).astype(np.float32)
+    with Network(sizes, members=2, max_batch=32) as net:
+        net.set_params(params, member=1)
+        (w, b), = net.get_params(1)
+        assert np.array_equal(w, params[0][0]) and np.array_equal(b, params[0][1])
+        _, ((gw, gb),) = net.gradients(x, t, member=1)
+        _, ((rw, rb),) = loss_and_grads(params, x, t, emulate=True)
+        assert rel(gw, rw) < 2e-3 and rel(gb, rb) < 2e-3

@@ -1,0 +1,27 @@
+"""The host arithmetic of the network's transfers and launches (csrc/mlp_plan.h), in a program of its own
+on the CPU."""
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "poe2d_amd", "csrc")
+
+
+def run(tmp_path, body):
+    src, exe = str(tmp_path / "t.cpp"), str(tmp_path / "t")
+    with open(src, "w") as f:
+        f.write('#include <cstdio>\n#include "mlp_plan.h"\nusing namespace poe2d::mlp;\nint main() {%s}\n' % body)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, src, "-o", exe], check=True)
+    return [[int(v) for v in line.split()] for line in subprocess.run([exe], check=True, capture_output=True,
+                                                                      text=True).stdout.splitlines()]
+
+
+@pytest.mark.parametrize("floats,rows,cols", [(4096, 8, 5000), (4096, 8, 4096), (4096, 8, 4097), (4096, 5, 1000),
+                                              (1, 3, 7), (524288, 64, 524289), (1 << 33, 200000, 20000)])
+def test_a_staged_piece_fits_its_buffer_and_makes_progress(tmp_path, floats, rows, cols):
+    # (a 5000 -> 8 network with batches of 32 has 4096 floats of workspace, less than one of its rows)
+    (r, c), = run(tmp_path, f'auto p = staging_piece({floats}ull, {rows}, {cols}); printf("%d %d\\n", p.rows, p.cols);')
+    assert 1 <= r <= rows and 1 <= c <= cols and r * c <= floats
+    assert r == 1 or c == cols  # several rows only when whole: they are contiguous on the host
+    assert c == cols or c == floats
