@@ -67,9 +67,11 @@ poe2d_status dmalloc(P **p, size_t count)
 {
     void *q = nullptr;
     hipError_t e = hipMalloc(&q, std::max<size_t>(count * sizeof(P), 1));
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // (reported here, not by the check of the next launch)
         return fail(e == hipErrorOutOfMemory ? POE2D_E_NOMEM : POE2D_E_HIP,
                     std::string("hipMalloc: ") + hipGetErrorString(e));
+    }
     *p = (P *)q;
     // (the fill runs on the null stream, which the networks' own streams do not wait for: what they
     // write first could otherwise be cleared after it)
@@ -88,9 +90,11 @@ poe2d_status grow(P **p, size_t *cap, size_t count)
     *cap = 0;
     void *q = nullptr;
     const hipError_t e = hipMalloc(&q, count * sizeof(P));
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // (reported here, not by the check of the next launch)
         return fail(e == hipErrorOutOfMemory ? POE2D_E_NOMEM : POE2D_E_HIP,
                     std::string("hipMalloc: ") + hipGetErrorString(e));
+    }
     *p = (P *)q;
     *cap = count;
     return POE2D_OK;
@@ -1046,6 +1050,7 @@ poe2d_status poe2d_host_alloc(size_t bytes, void **out)
     if (!out || bytes == 0) return fail(POE2D_E_INVALID, "host_alloc: bad arguments");
     *out = nullptr;
     if (hipHostMalloc(out, bytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
         *out = nullptr;
         return fail(POE2D_E_NOMEM, "host_alloc: hipHostMalloc failed");
     }
@@ -1062,6 +1067,7 @@ poe2d_status poe2d_device_alloc(size_t bytes, void **out)
     if (!out || bytes == 0) return fail(POE2D_E_INVALID, "device_alloc: bad arguments");
     *out = nullptr;
     if (hipMalloc(out, bytes) != hipSuccess) {
+        (void)hipGetLastError();
         *out = nullptr;
         return fail(POE2D_E_NOMEM, "device_alloc: hipMalloc failed");
     }

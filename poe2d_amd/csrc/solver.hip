@@ -63,6 +63,7 @@ poe2d_status dev_alloc(void **p, size_t bytes)
 {
     hipError_t e = hipMalloc(p, std::max<size_t>(bytes, 1));
     if (e != hipSuccess) {
+        (void)hipGetLastError();  // (reported here, not by the check of the next launch)
         *p = nullptr;
         return fail(e == hipErrorOutOfMemory ? POE2D_E_NOMEM : POE2D_E_HIP,
                     std::string("hipMalloc(") + std::to_string(bytes) + "): " + hipGetErrorString(e));
@@ -532,6 +533,7 @@ poe2d_status grow(StepList::Staged &b, size_t bytes)
     poe2d_status st = dev_alloc(&b.dev, bytes);
     if (st) return st;
     if (hipHostMalloc((void **)&b.image, bytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
         b.image = nullptr;
         return fail(POE2D_E_NOMEM, "run: page-locked host memory");
     }

@@ -1,0 +1,38 @@
+"""Calls that fail leave the handle, and the thread, as their callers may rely on: later calls work."""
+import numpy as np
+import pytest
+
+from poe2d_amd import _abi
+from poe2d_amd.mlp import DeviceArray, Network
+from poe2d_amd.solver import ReceiverSpec, Solver, SourceSpec
+
+from .helpers import small_problem
+
+pytestmark = pytest.mark.gpu
+
+TOO_LARGE = (1 << 33, 1 << 10)  # 32 TB of floats
+
+
+def shot(nt=9):
+    rec = ReceiverSpec(ix=np.arange(20, 100, 7), iz=np.full(12, 50))
+    src = SourceSpec(kind=_abi.SRC_PRESSURE_DGAUSS, ix=60, iz=60, amp=1e6)
+    return small_problem(src=src, rec=rec, nt=nt)
+
+
+def refused(f):
+    with pytest.raises(_abi.Poe2dError) as e:
+        f()
+    assert e.value.status == _abi.POE2D_E_NOMEM
+
+
+def test_a_refused_allocation_is_not_reported_by_the_next_call():
+    with Solver(shot()) as s, Network([4, 64, 64], max_batch=32) as net:
+        x = np.ones((3, 4), np.float32)
+        y = net.predict(x)[0]
+        for call in (s.reset, lambda: s.run(3), lambda: net.predict(x), lambda: Network([4, 8], max_batch=32).close()):
+            refused(lambda: DeviceArray(TOO_LARGE))
+            call()
+        refused(lambda: Network([1 << 20, 1 << 26], max_batch=32))
+        assert np.array_equal(net.predict(x)[0], y)
+        s.run(1)
+        assert s.step_count() == 4
