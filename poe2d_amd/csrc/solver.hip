@@ -1162,6 +1162,34 @@ poe2d_solver *new_handle(Model *md, poe2d_status *st)
     return s;
 }
 
+void drop_receivers(poe2d_solver *s)
+{
+    void *q = s->rix; dev_free(q); s->rix = nullptr;
+    q = s->riz; dev_free(q); s->riz = nullptr;
+    dev_free(s->traces);
+    dev_free(s->traces_out);
+    s->nrec = 0;
+}
+
+// Positions and traces of r's receivers (at least one) for a handle that has none.
+poe2d_status place_receivers(poe2d_solver *s, const poe2d_receivers *r)
+{
+    s->hrx.assign(r->ix, r->ix + r->n);
+    s->hrz.assign(r->iz, r->iz + r->n);
+    s->nrec = r->n;
+    poe2d_status st;
+    void *q = nullptr;
+    if ((st = dev_alloc(&q, (size_t)r->n * sizeof(int)))) return st;
+    s->rix = (int *)q;
+    if ((st = dev_alloc(&q, (size_t)r->n * sizeof(int)))) return st;
+    s->riz = (int *)q;
+    if ((st = dev_alloc_zero(&s->traces, s->trace_bytes(), s->stream))) return st;
+    HIP_TRY(hipStreamSynchronize(s->stream));
+    HIP_TRY(hipMemcpy(s->rix, r->ix, (size_t)r->n * sizeof(int), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(s->riz, r->iz, (size_t)r->n * sizeof(int), hipMemcpyHostToDevice));
+    return POE2D_OK;
+}
+
 poe2d_status check_batch(poe2d_batch *b)
 {
     if (!b) return fail(POE2D_E_INVALID, "null batch handle");
@@ -1467,27 +1495,16 @@ poe2d_status poe2d_set_receivers(poe2d_solver *s, const poe2d_receivers *r)
         if (r->ix[k] < 0 || r->ix[k] > s->grid.nx || r->iz[k] < 0 || r->iz[k] > s->grid.nz)
             return fail(POE2D_E_INVALID, "set_receivers: receiver " + std::to_string(k) + " outside the grid");
     HIP_TRY(hipStreamSynchronize(s->stream));
-    void *q = s->rix; dev_free(q); s->rix = nullptr;
-    q = s->riz; dev_free(q); s->riz = nullptr;
-    dev_free(s->traces);
-    dev_free(s->traces_out);
-    s->nrec = r->n;
+    drop_receivers(s);
     s->mask = r->comp_mask;
     s->ncomp = ((r->comp_mask & 1) != 0) + ((r->comp_mask & 2) != 0) + ((r->comp_mask & 4) != 0);
     s->dec = r->decimate;
     s->nsamp = r->nsamp;
-    if (s->nrec == 0) return POE2D_OK;
-    if ((st = dev_alloc(&q, (size_t)r->n * sizeof(int)))) return st;
-    s->rix = (int *)q;
-    if ((st = dev_alloc(&q, (size_t)r->n * sizeof(int)))) return st;
-    s->riz = (int *)q;
-    if ((st = dev_alloc_zero(&s->traces, s->trace_bytes(), s->stream))) return st;
-    HIP_TRY(hipStreamSynchronize(s->stream));
-    s->hrx.assign(r->ix, r->ix + r->n);
-    s->hrz.assign(r->iz, r->iz + r->n);
-    HIP_TRY(hipMemcpy(s->rix, r->ix, (size_t)r->n * sizeof(int), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(s->riz, r->iz, (size_t)r->n * sizeof(int), hipMemcpyHostToDevice));
-    return POE2D_OK;
+    if (r->n == 0) return POE2D_OK;
+    // (where the memory is not there the handle has no receivers: a run would read positions and write
+    // traces that do not exist)
+    if ((st = place_receivers(s, r))) drop_receivers(s);
+    return st;
 }
 
 poe2d_status poe2d_run(poe2d_solver *s, int nsteps)

@@ -36,3 +36,20 @@ def test_a_refused_allocation_is_not_reported_by_the_next_call():
         assert np.array_equal(net.predict(x)[0], y)
         s.run(1)
         assert s.step_count() == 4
+
+
+def test_receivers_whose_traces_do_not_fit_leave_the_handle_without_receivers():
+    prob = shot()
+    with Solver(prob) as s:
+        s.run()
+        ref = s.seismograms()
+        # 25 TB of traces, at more positions than the handle had
+        far = ReceiverSpec(ix=np.tile(np.arange(100), 10), iz=np.repeat(np.arange(10), 100), nsamp=2 ** 31 - 1)
+        refused(lambda: s.set_receivers(far))
+        s.reset()
+        s.run(5)
+        assert s.step_count() == 5 and np.isfinite(s.snapshot("vx")).all()
+        s.reset()
+        s.set_receivers(prob.receivers)
+        s.run()
+        assert np.array_equal(s.seismograms(), ref)
