@@ -132,7 +132,7 @@ struct poe2d_mlp {
     // prediction: hidden activations of every member (per layer boundary l = 1..L-1, [members]
     // [max_batch][pad(sizes[l])]), the members' weight and bias pointers (per layer, [members]), the
     // row sums behind the spread, a batch's mean on its way to host memory, and the inputs and spreads
-    // of a whole call (grown to the largest call)
+    // of a call, or of a stretch of a long one (grown to the longest)
     std::vector<uint16_t *> hens;
     std::vector<const uint16_t **> ens_w;
     std::vector<const float **> ens_b;
@@ -899,23 +899,28 @@ poe2d_status poe2d_mlp_predict(poe2d_mlp *m, int n, const float *x, float *mean,
     if (st) return st;
     if (n < 1 || !x) return fail(POE2D_E_INVALID, "mlp_predict: bad input");
     const int in = m->sizes[0], out = m->sizes[m->L];
-    // every input in one copy: a copy per batch from pageable memory would hold the host until the
-    // batch before it is done
-    if ((st = grow(&m->x_all, &m->x_all_cap, (size_t)n * in))) return st;
-    if (spread && (st = grow(&m->spread_all, &m->spread_all_cap, (size_t)n))) return st;
-    HIP_TRY(hipMemcpyAsync(m->x_all, x, (size_t)n * in * sizeof(float), hipMemcpyHostToDevice, m->stream));
+    // Inputs in one copy for many batches: a copy per batch from pageable memory would hold the host until
+    // the batch before it is done.  As many batches as kInputFloats hold, so that a call's device memory
+    // does not grow with its rows.
+    const int stretch = predict_stretch(n, in, m->max_batch);
+    if ((st = grow(&m->x_all, &m->x_all_cap, (size_t)stretch * in))) return st;
+    if (spread && (st = grow(&m->spread_all, &m->spread_all_cap, (size_t)stretch))) return st;
     const bool in_place = mean && on_this_device(m, mean);
-    for (int r0 = 0; r0 < n; r0 += m->max_batch) {
-        const int nb = std::min(m->max_batch, n - r0);
-        pack_input<<<blocks((size_t)nb * in), 256, 0, m->stream>>>(m->x_all + (size_t)r0 * in, nb, in, m->h16[0], pad128(in));
-        HIP_TRY(hipGetLastError());
-        float *const dst = !mean ? nullptr : in_place ? mean + (size_t)r0 * out : m->acc_mean;
-        if ((st = ensemble_batch(m, nb, dst, spread ? m->spread_all + r0 : nullptr))) return st;
-        if (dst && !in_place)
-            HIP_TRY(hipMemcpyAsync(mean + (size_t)r0 * out, dst, (size_t)nb * out * sizeof(float), hipMemcpyDefault,
-                                   m->stream));
+    for (int s0 = 0; s0 < n; s0 += stretch) {
+        const int ns = std::min(stretch, n - s0);
+        HIP_TRY(hipMemcpyAsync(m->x_all, x + (size_t)s0 * in, (size_t)ns * in * sizeof(float), hipMemcpyHostToDevice, m->stream));
+        for (int r0 = 0; r0 < ns; r0 += m->max_batch) {
+            const int nb = std::min(m->max_batch, ns - r0);
+            pack_input<<<blocks((size_t)nb * in), 256, 0, m->stream>>>(m->x_all + (size_t)r0 * in, nb, in, m->h16[0], pad128(in));
+            HIP_TRY(hipGetLastError());
+            float *const rows = mean ? mean + (size_t)(s0 + r0) * out : nullptr, *const dst = !rows || in_place ? rows : m->acc_mean;
+            if ((st = ensemble_batch(m, nb, dst, spread ? m->spread_all + r0 : nullptr))) return st;
+            if (dst && !in_place)
+                HIP_TRY(hipMemcpyAsync(rows, dst, (size_t)nb * out * sizeof(float), hipMemcpyDefault, m->stream));
+        }
+        if (spread)
+            HIP_TRY(hipMemcpyAsync(spread + s0, m->spread_all, (size_t)ns * sizeof(float), hipMemcpyDefault, m->stream));
     }
-    if (spread) HIP_TRY(hipMemcpyAsync(spread, m->spread_all, (size_t)n * sizeof(float), hipMemcpyDefault, m->stream));
     HIP_TRY(hipStreamSynchronize(m->stream));
     return POE2D_OK;
 }

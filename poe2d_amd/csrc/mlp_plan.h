@@ -19,5 +19,14 @@ inline Piece staging_piece(size_t floats, int rows, int cols)
     return {1, (int)floats};
 }
 
+// Rows of a prediction whose inputs (`in` values each) are on the device at a time: all n, or as many
+// batches as kInputFloats hold, at least one.
+constexpr size_t kInputFloats = size_t(16) << 20;
+inline int predict_stretch(int n, int in, int batch)
+{
+    const size_t batches = std::max<size_t>(kInputFloats / in / batch, 1);
+    return (int)std::min<size_t>(n, batches * batch);
+}
+
 }  // namespace mlp
 }  // namespace poe2d

@@ -73,3 +73,13 @@ def trace_rel_l2(g, o, floor=1e-3):
     fl = floor * den.max(axis=-1, keepdims=True)
     return num / np.maximum(np.maximum(den, fl), 1e-300)
 
+
+
+def device_memory_free():
+    """Free device memory in bytes, from the HIP runtime that the library uses."""
+    import ctypes
+
+    from poe2d_amd import _abi
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert _abi.load_library().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value

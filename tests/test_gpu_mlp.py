@@ -6,6 +6,7 @@ import pytest
 
 from poe2d_amd.mlp import DeviceArray, Network, gemm_bf16, pinned_empty
 
+from .helpers import device_memory_free
 from .mlp_reference import bf16, forward, loss_and_grads
 
 pytestmark = pytest.mark.gpu
@@ -319,3 +320,19 @@ def test_rows_longer_than_the_workspace(sizes):
         _, ((gw, gb),) = net.gradients(x, t, member=1)
         _, ((rw, rb),) = loss_and_grads(params, x, t, emulate=True)
         assert rel(gw, rw) < 2e-3 and rel(gb, rb) < 2e-3
+
+
+def test_a_long_prediction_holds_a_bounded_part_of_its_inputs():
+    """1 GB of inputs take at most 256 MB of device memory beside the network, and rows on either side of
+    the parts' seams come out as in a call of their own."""
+    rng = np.random.default_rng(8)
+    with Network([256, 64, 3], members=2, max_batch=8192, seed=4) as net:
+        x = np.empty((1 << 20, 256), np.float32)
+        x[:] = rng.standard_normal((1 << 12, 256)).astype(np.float32).repeat(256, axis=0)
+        x[::7, 0] += 1.0
+        before = device_memory_free()
+        mean, spread = net.predict(x)
+        assert before - device_memory_free() < 256 << 20
+        for lo in (0, 65536 - 50, 15 * 65536 - 50, len(x) - 100):
+            m, s = net.predict(x[lo:lo + 100])
+            assert np.array_equal(m, mean[lo:lo + 100]) and np.array_equal(s, spread[lo:lo + 100])

@@ -25,3 +25,12 @@ def test_a_staged_piece_fits_its_buffer_and_makes_progress(tmp_path, floats, row
     assert 1 <= r <= rows and 1 <= c <= cols and r * c <= floats
     assert r == 1 or c == cols  # several rows only when whole: they are contiguous on the host
     assert c == cols or c == floats
+
+
+@pytest.mark.parametrize("n,inputs,batch", [(37, 207, 1024), (2048, 207, 1024), (1 << 20, 256, 8192), (100000000, 207, 1024),
+                                            (1000, 50000000, 32), (2147483647, 1, 32), (65536, 256, 8192), (65537, 256, 8192)])
+def test_a_prediction_holds_bounded_inputs(tmp_path, n, inputs, batch):
+    (rows,), = run(tmp_path, f'printf("%d\\n", predict_stretch({n}, {inputs}, {batch}));')
+    assert 1 <= rows <= n
+    assert rows * inputs <= max(1 << 24, batch * inputs)
+    assert rows == n or (rows % batch == 0 and (rows + batch) * inputs > 1 << 24)
