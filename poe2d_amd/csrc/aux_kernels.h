@@ -57,8 +57,8 @@ struct ClearRanges {
 };
 void launch_clear(const ClearRanges &r, hipStream_t stream);
 
-// out[c][r] = in[r][c], rows x cols.
+// out[c][r] = in[r][c], rows x cols; rows of `in` ld apart.
 template <class T>
-void launch_transpose(const T *in, int rows, int cols, T *out, hipStream_t stream);
+void launch_transpose(const T *in, size_t ld, int rows, int cols, T *out, hipStream_t stream);
 
 }  // namespace poe2d

@@ -137,13 +137,13 @@ __global__ void __launch_bounds__(256) clear_kernel(ClearRanges r)
 
 // 32 x 32 tiles through LDS, a row of 32 values per half wave on either side.
 template <class T>
-__global__ void __launch_bounds__(256) transpose_kernel(const T *in, int rows, int cols, T *out)
+__global__ void __launch_bounds__(256) transpose_kernel(const T *in, size_t ld, int rows, int cols, T *out)
 {
     __shared__ T tile[32][33];
     const int c0 = blockIdx.x * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     for (int r0 = blockIdx.y * 32; r0 < rows; r0 += gridDim.y * 32) {
         for (int y = ty; y < 32; y += 8)
-            if (r0 + y < rows && c0 + tx < cols) tile[y][tx] = in[(size_t)(r0 + y) * cols + c0 + tx];
+            if (r0 + y < rows && c0 + tx < cols) tile[y][tx] = in[(size_t)(r0 + y) * ld + c0 + tx];
         __syncthreads();
         for (int y = ty; y < 32; y += 8)
             if (c0 + y < cols && r0 + tx < rows) out[(size_t)(c0 + y) * rows + r0 + tx] = tile[tx][y];
@@ -216,10 +216,10 @@ void launch_clear(const ClearRanges &r, hipStream_t stream)
 }
 
 template <class T>
-void launch_transpose(const T *in, int rows, int cols, T *out, hipStream_t stream)
+void launch_transpose(const T *in, size_t ld, int rows, int cols, T *out, hipStream_t stream)
 {
     const dim3 grid((cols + 31) / 32, std::min((rows + 31) / 32, 4096));
-    transpose_kernel<T><<<grid, 256, 0, stream>>>(in, rows, cols, out);
+    transpose_kernel<T><<<grid, 256, 0, stream>>>(in, ld, rows, cols, out);
 }
 
 __global__ void __launch_bounds__(256) cn_palette_kernel(Vec4<float> *pal, int npal, float inv_dt)
@@ -246,7 +246,7 @@ void launch_cn_palette(Vec4<float> *pal, int npal, float inv_dt, hipStream_t str
     template void launch_insert<T>(const StepArgs<T> &, int, int, const T *, hipStream_t);            \
     template void launch_absmax<T>(const StepArgs<T> &, int, float *, int, float *, hipStream_t);         \
     template void launch_absmax_members<T>(const FieldRange *, int, float *, int, float *, hipStream_t); \
-    template void launch_transpose<T>(const T *, int, int, T *, hipStream_t);
+    template void launch_transpose<T>(const T *, size_t, int, int, T *, hipStream_t);
 POE2D_AUX_INSTANTIATE(float)
 POE2D_AUX_INSTANTIATE(double)
 #undef POE2D_AUX_INSTANTIATE

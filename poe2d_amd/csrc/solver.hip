@@ -47,6 +47,7 @@ const double kStabilityThreshold = 1.0e25;  // STABILITY_THRESHOLD of the refere
 const int kGraphSteps = 32;                 // steps per captured graph
 const size_t kL2Bytes = size_t(32) << 20;   // the eight L2s together
 const size_t kMallBytes = size_t(256) << 20;  // the memory-side cache
+const size_t kTraceBytes = size_t(64) << 20;  // traces on their way to the host
 const int kBandTiles = 8;                   // tile columns to a band of the tile kernel's work order
 
 #define HIP_TRY(expr)                                                                              \
@@ -224,7 +225,7 @@ struct poe2d_solver {
     int *rix = nullptr, *riz = nullptr;
     std::vector<int> hrx, hrz;  // their host copies
     void *traces = nullptr;  // [slot][comp][rec]
-    void *traces_out = nullptr;  // [comp][rec][slot], made when they are first read
+    void *traces_out = nullptr;  // some of them as [comp][rec][slot], made when they are first read
     int step = 0;
     double last_ms = 0;
     int last_steps = 0;
@@ -1539,14 +1540,20 @@ poe2d_status poe2d_seismograms(poe2d_solver *s, void *out, size_t bytes)
     const size_t need = s->trace_bytes();
     if (bytes < need) return fail(POE2D_E_INVALID, "seismograms: output buffer too small");
     if (need == 0) return POE2D_OK;
-    // device layout [slot][comp][rec] -> caller layout [comp][rec][slot], transposed on the device
-    if (!s->traces_out && (st = dev_alloc(&s->traces_out, need))) return st;
-    if (s->precision == POE2D_F32)
-        launch_transpose<float>((const float *)s->traces, s->nsamp, s->ncomp * s->nrec, (float *)s->traces_out, s->stream);
-    else
-        launch_transpose<double>((const double *)s->traces, s->nsamp, s->ncomp * s->nrec, (double *)s->traces_out, s->stream);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(out, s->traces_out, need, hipMemcpyDeviceToHost, s->stream));
+    // device layout [slot][comp][rec] -> caller layout [comp][rec][slot], transposed on the device, as many
+    // traces at a time as kTraceBytes hold, so that long records need no second copy of all of them
+    const size_t ncol = (size_t)s->ncomp * s->nrec, col = s->nsamp * s->rs;
+    const size_t piece = std::min(ncol, std::max<size_t>(kTraceBytes / col, 1));
+    if (!s->traces_out && (st = dev_alloc(&s->traces_out, piece * col))) return st;
+    for (size_t c = 0; c < ncol; c += piece) {
+        const size_t nc = std::min(piece, ncol - c);
+        if (s->precision == POE2D_F32)
+            launch_transpose<float>((const float *)s->traces + c, ncol, s->nsamp, (int)nc, (float *)s->traces_out, s->stream);
+        else
+            launch_transpose<double>((const double *)s->traces + c, ncol, s->nsamp, (int)nc, (double *)s->traces_out, s->stream);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipMemcpyAsync((unsigned char *)out + c * col, s->traces_out, nc * col, hipMemcpyDeviceToHost, s->stream));
+    }
     HIP_TRY(hipStreamSynchronize(s->stream));
     return POE2D_OK;
 }
