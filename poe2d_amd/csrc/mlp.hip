@@ -33,8 +33,10 @@ namespace {
 #define HIP_TRY(expr)                                                                              \
     do {                                                                                           \
         hipError_t e_ = (expr);                                                                    \
-        if (e_ != hipSuccess)                                                                      \
+        if (e_ != hipSuccess) {                                                                    \
+            (void)hipGetLastError(); /* (reported here, not by the check of the next launch) */    \
             return fail(POE2D_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_));           \
+        }                                                                                          \
     } while (0)
 
 int pad128(int n) { return (n + 127) / 128 * 128; }

@@ -53,8 +53,10 @@ const int kBandTiles = 8;                   // tile columns to a band of the til
 #define HIP_TRY(expr)                                                                              \
     do {                                                                                           \
         hipError_t e_ = (expr);                                                                    \
-        if (e_ != hipSuccess)                                                                      \
+        if (e_ != hipSuccess) {                                                                    \
+            (void)hipGetLastError(); /* (reported here, not by the check of the next launch) */    \
             return fail(POE2D_E_HIP, std::string(#expr) + ": " + hipGetErrorString(e_));           \
+        }                                                                                          \
     } while (0)
 
 // single-pass (palette when the grid has one), two-pass, single-pass always on the MS/MV groups

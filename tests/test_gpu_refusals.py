@@ -1,4 +1,6 @@
 """Calls that fail leave the handle, and the thread, as their callers may rely on: later calls work."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -53,3 +55,16 @@ def test_receivers_whose_traces_do_not_fit_leave_the_handle_without_receivers():
         s.set_receivers(prob.receivers)
         s.run()
         assert np.array_equal(s.seismograms(), ref)
+
+
+def test_a_copy_that_the_runtime_refuses_is_not_reported_by_the_next_call():
+    with Solver(shot()) as s, Network([4, 64, 64], max_batch=32) as net:
+        x = np.ones((3, 4), np.float32)
+        y = net.predict(x)[0]
+        short = DeviceArray((10, 4096))
+        host = np.zeros((100, 4096), np.float32)
+        for call in (s.reset, lambda: s.run(3), lambda: net.predict(x)):
+            assert s._lib.poe2d_copy(ctypes.c_void_p(short.ptr), ctypes.c_void_p(host.ctypes.data),
+                                     ctypes.c_size_t(host.nbytes)) == _abi.POE2D_E_HIP
+            call()
+        assert np.array_equal(net.predict(x)[0], y)
