@@ -413,15 +413,23 @@ poe2d_status ensemble_batch(poe2d_mlp *m, int nb, float *mean, float *spread)
     return POE2D_OK;
 }
 
-// Whether p is memory of the network's device (results then go there directly).
-bool on_this_device(const poe2d_mlp *m, const void *p)
+// Whether `bytes` bytes from p on lie in one allocation of the network's device (results then go there
+// directly; a shorter one is left to a copy, which the runtime refuses).
+bool on_this_device(const poe2d_mlp *m, const void *p, size_t bytes)
 {
     hipPointerAttribute_t at{};
     if (hipPointerGetAttributes(&at, p) != hipSuccess) {
         (void)hipGetLastError();  // (ordinary host memory)
         return false;
     }
-    return at.type == hipMemoryTypeDevice && at.device == m->device;
+    if (at.type != hipMemoryTypeDevice || at.device != m->device) return false;
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return bytes <= size - ((const char *)p - (const char *)base);
 }
 
 // The layers' inputs of the batch of n rows, transposed for the weight gradients.
@@ -907,7 +915,7 @@ poe2d_status poe2d_mlp_predict(poe2d_mlp *m, int n, const float *x, float *mean,
     const int stretch = predict_stretch(n, in, m->max_batch);
     if ((st = grow(&m->x_all, &m->x_all_cap, (size_t)stretch * in))) return st;
     if (spread && (st = grow(&m->spread_all, &m->spread_all_cap, (size_t)stretch))) return st;
-    const bool in_place = mean && on_this_device(m, mean);
+    const bool in_place = mean && on_this_device(m, mean, (size_t)n * out * sizeof(float));
     for (int s0 = 0; s0 < n; s0 += stretch) {
         const int ns = std::min(stretch, n - s0);
         HIP_TRY(hipMemcpyAsync(m->x_all, x + (size_t)s0 * in, (size_t)ns * in * sizeof(float), hipMemcpyHostToDevice, m->stream));

@@ -68,3 +68,19 @@ def test_a_copy_that_the_runtime_refuses_is_not_reported_by_the_next_call():
                                      ctypes.c_size_t(host.nbytes)) == _abi.POE2D_E_HIP
             call()
         assert np.array_equal(net.predict(x)[0], y)
+
+
+@pytest.mark.parametrize("held", [10, 70])
+def test_a_prediction_into_device_memory_that_is_too_short_is_refused(held):
+    """Batches of 64 rows: the first, or the second, does not fit."""
+    rows = 100
+    rng = np.random.default_rng(5)
+    with Network([8, 64, 4096], members=2, max_batch=64) as net:
+        x = rng.standard_normal((rows, 8)).astype(np.float32)
+        ref, spread = net.predict(x)
+        short, whole = DeviceArray((held, 4096)), DeviceArray((rows, 4096))
+        fp = _abi.c_float_p
+        args = net._h, rows, x.ctypes.data_as(fp)
+        assert net._lib.poe2d_mlp_predict(*args, ctypes.cast(ctypes.c_void_p(short.ptr), fp), None) == _abi.POE2D_E_HIP
+        got, s = net.predict(x, out=whole)
+        assert np.array_equal(got.to_host(), ref) and np.array_equal(s, spread)
