@@ -140,6 +140,7 @@ struct poe2d_mlp {
     std::vector<const float **> ens_b;
     double *ens_part = nullptr;
     float *acc_mean = nullptr;
+    float *acc_m2 = nullptr;  // sums of squared deviations, where output layers may run member by member
     float *x_all = nullptr, *spread_all = nullptr;
     size_t x_all_cap = 0, spread_all_cap = 0;
     float *oscale = nullptr;  // per-output factor of the predicted mean (null: none)
@@ -190,7 +191,7 @@ void free_mlp(poe2d_mlp *m)
     for (auto &p : m->ens_w) dfree(p);
     for (auto &p : m->ens_b) dfree(p);
     dfree(m->ens_part); dfree(m->x_all); dfree(m->spread_all);
-    dfree(m->acc_mean); dfree(m->oscale); dfree(m->data_x); dfree(m->data_t); dfree(m->idx); dfree(m->dloss);
+    dfree(m->acc_mean); dfree(m->acc_m2); dfree(m->oscale); dfree(m->data_x); dfree(m->data_t); dfree(m->idx); dfree(m->dloss);
     dfree(m->idx_all); dfree(m->loss_all);
     for (hipEvent_t ev : m->step_done) (void)hipEventDestroy(ev);
     m->step_done.clear();
@@ -265,6 +266,58 @@ __global__ void gather_input(const float *__restrict__ src, const int *__restric
     if (i >= n * in) return;
     const int r = i / in, c = i % in;
     h[(size_t)r * ldh + c] = bf16_rne(src[(size_t)idx[r] * in + c]);
+}
+
+// The statistics of an output layer formed member by member.  Running mean / sum of squared deviations over
+// members (Welford), k = member index.
+__global__ void welford(const float *__restrict__ y, int ldy, int n, int cols, int k, float *__restrict__ mean,
+                        float *__restrict__ m2)
+{
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < (size_t)n * cols; i += (size_t)gridDim.x * blockDim.x) {
+        const float v = y[i / cols * ldy + i % cols];
+        if (k == 0) {
+            mean[i] = v;
+            m2[i] = 0.f;
+            continue;
+        }
+        const float d = v - mean[i];
+        const float mu = mean[i] + d / (float)(k + 1);
+        m2[i] += d * (v - mu);
+        mean[i] = mu;
+    }
+}
+
+// spread[r] = ||std over members|| / ||mean|| over the outputs of row r (one block per row).
+__global__ void __launch_bounds__(256) row_spread(const float *__restrict__ mean, const float *__restrict__ m2, int cols,
+                                                  int members, float *__restrict__ spread)
+{
+    __shared__ double sv[256], sn[256];
+    const int r = blockIdx.x;
+    double var = 0, nrm = 0;
+    for (int c = threadIdx.x; c < cols; c += blockDim.x) {
+        const float mu = mean[(size_t)r * cols + c];
+        var += m2[(size_t)r * cols + c];
+        nrm += (double)mu * mu;
+    }
+    sv[threadIdx.x] = var;
+    sn[threadIdx.x] = nrm;
+    __syncthreads();
+    for (int s = 128; s > 0; s >>= 1) {
+        if ((int)threadIdx.x < s) {
+            sv[threadIdx.x] += sv[threadIdx.x + s];
+            sn[threadIdx.x] += sn[threadIdx.x + s];
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) spread[r] = (float)(sqrt(sv[0] / (members > 1 ? members - 1 : 1)) / fmax(sqrt(sn[0]), 1e-30));
+}
+
+// mean[r][c] *= scale[c] for n rows of `cols` values.
+__global__ void scale_cols(float *__restrict__ mean, int n, int cols, const float *__restrict__ scale)
+{
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < (size_t)n * cols;
+         i += (size_t)gridDim.x * blockDim.x)
+        mean[i] *= scale[i % cols];
 }
 
 int blocks(size_t n) { return (int)std::min<size_t>((n + 255) / 256, 1u << 20); }
@@ -366,21 +419,44 @@ poe2d_status hidden_layers(poe2d_mlp *m, const Member &e, int n)
     return POE2D_OK;
 }
 
-// Forward pass of member e on the first n rows of m->xin (already packed into h16[0]).
-poe2d_status forward(poe2d_mlp *m, Member &e, int n)
+// Output layer l on n rows in h, into y.
+poe2d_status output(poe2d_mlp *m, const Layer &l, const uint16_t *h, int n)
 {
-    poe2d_status st = hidden_layers(m, e, n);
-    if (st) return st;
-    const Layer &l = e.layers[m->L - 1];
     GemmOut o;
     o.bias = l.b;
     o.f32 = m->y;
     o.ldf = l.outp;
-    HIP_TRY(gemm_bf16(m->h16[m->L - 1], l.inp, l.w16, l.inp, n, l.out, l.inp, EPI_LINEAR, o, m->work, m->work_floats,
+    HIP_TRY(gemm_bf16(h, l.inp, l.w16, l.inp, n, l.out, l.inp, EPI_LINEAR, o, m->work, m->work_floats,
                       product_splits(m, n, l.out, l.inp), m->stream));
     return POE2D_OK;
 }
 
+// Forward pass of member e on the first n rows of m->xin (already packed into h16[0]).
+poe2d_status forward(poe2d_mlp *m, Member &e, int n)
+{
+    const poe2d_status st = hidden_layers(m, e, n);
+    return st ? st : output(m, e.layers[m->L - 1], m->h16[m->L - 1], n);
+}
+
+// The members' output layers on the nb rows in h (member k's k stride on) and their statistics, member by
+// member.
+poe2d_status output_by_member(poe2d_mlp *m, const uint16_t *h, size_t stride, int nb, float *mean, float *spread)
+{
+    const int E = (int)m->members.size(), out = m->sizes[m->L], grid = blocks((size_t)nb * out);
+    float *const mu = mean ? mean : m->acc_mean;
+    for (int k = 0; k < E; ++k) {
+        const Layer &l = m->members[k].layers[m->L - 1];
+        const poe2d_status st = output(m, l, h + k * stride, nb);
+        if (st) return st;
+        welford<<<grid, 256, 0, m->stream>>>(m->y, l.outp, nb, out, k, mu, m->acc_m2);
+        HIP_TRY(hipGetLastError());
+    }
+    if (spread) row_spread<<<nb, 256, 0, m->stream>>>(mu, m->acc_m2, out, E, spread);
+    // (the spread is of the unscaled outputs)
+    if (mean && m->oscale) scale_cols<<<grid, 256, 0, m->stream>>>(mean, nb, out, m->oscale);
+    HIP_TRY(hipGetLastError());
+    return POE2D_OK;
+}
 
 // The ensemble on the nb rows in h16[0]: the hidden layers of every member, layer by layer, then their output layers and statistics in one
 // pass.  mean [nb][outputs] (scaled) and spread [nb] are device memory; either may be null.
@@ -392,6 +468,7 @@ poe2d_status ensemble_batch(poe2d_mlp *m, int nb, float *mean, float *spread)
     for (int li = 0; li < m->L; ++li) {
         const Layer &l = m->members[0].layers[li];
         if (li == m->L - 1) {
+            if (!ensemble_in_registers(nb, l.out, l.inp)) return output_by_member(m, h, stride, nb, mean, spread);
             HIP_TRY(ensemble_output(h, l.inp, stride, m->ens_w[li], l.inp, m->ens_b[li], E, nb, l.out, l.inp, mean, l.out,
                                     m->oscale, m->ens_part, spread, m->stream));
             break;
@@ -629,6 +706,9 @@ static poe2d_status alloc_scratch(poe2d_mlp *m, bool predict)
         ((st = dmalloc(&m->y, (size_t)B * outp)) || (st = dmalloc(&m->tgt, (size_t)B * outp)) ||
          (st = dmalloc(&m->acc_mean, (size_t)B * sizes[nlayers])) ||
          (st = dmalloc(&m->ens_part, ensemble_part_doubles(B, sizes[nlayers])))))
+        return st;
+    if (predict && !ensemble_in_registers(1, sizes[nlayers], pad128(sizes[nlayers - 1])) &&
+        (st = dmalloc(&m->acc_m2, (size_t)B * sizes[nlayers])))
         return st;
     if (predict) {
         const size_t E = m->members.size();

@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "mlp_kernels.h"
+#include "mlp_plan.h"
 
 namespace poe2d {
 namespace mlp {
@@ -1067,7 +1068,7 @@ hipError_t gemm_bf16(const uint16_t *A, int lda, const uint16_t *B, int ldb, int
 
 bool hidden_in_registers(int members, int M, int N, int K)
 {
-    return K % RING_K == 0 && members <= 65535 &&
+    return K % RING_K == 0 && K <= kRingRow && members <= 65535 &&
            (K <= (long long)kHiddenChain * members || (long long)members * ((M + 63) / 64) * ((N + 63) / 64) >= 2 * kCus);
 }
 
@@ -1075,8 +1076,8 @@ hipError_t hidden_layer(const uint16_t *A, int lda, size_t stride_a, const uint1
                         const float *bias, const float *const *biases, int members, int M, int N, int K, int ksplit, float *pre,
                         int ldp, uint16_t *b16, int ldb16, size_t stride_b16, hipStream_t stream)
 {
-    if (M < 1 || N < 1 || K < RING_K || K % RING_K || lda % 8 || ldb % 8 || lda < K || ldb < K || members < 1 ||
-        members > 65535 || ksplit < 1 || ksplit > K / BK || (bs ? !biases : !B || !bias || members > 1))
+    if (M < 1 || N < 1 || K < RING_K || K % RING_K || lda % 8 || ldb % 8 || lda < K || ldb < K || lda > kRingRow ||
+        ldb > kRingRow || members < 1 || members > 65535 || ksplit < 1 || ksplit > K / BK || (bs ? !biases : !B || !bias || members > 1))
         return hipErrorInvalidValue;
     const int kper = ((K / BK + ksplit - 1) / ksplit) * BK;
     hidden_product<<<dim3(((M + 63) / 64) * ((N + 63) / 64), members), 256, 0, stream>>>(
@@ -1090,7 +1091,8 @@ hipError_t ensemble_output(const uint16_t *A, int lda, size_t stride_a, const ui
                            const float *const *biases, int members, int M, int N, int K, float *mean, size_t ldm,
                            const float *scale, double *part, float *spread, hipStream_t stream)
 {
-    if (M < 1 || N < 1 || K < 64 || K % 64 || lda % 8 || ldb % 8 || lda < K || ldb < K || members < 1 || (spread && !part))
+    if (M < 1 || N < 1 || K < 64 || K % 64 || lda % 8 || ldb % 8 || lda < K || ldb < K || lda > kRingRow || ldb > kRingRow ||
+        members < 1 || (spread && !part))
         return hipErrorInvalidValue;
     if (!spread) part = nullptr;
     const auto tiles = [&](int tm, int tn) { return (long long)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };

@@ -336,3 +336,26 @@ def test_a_long_prediction_holds_a_bounded_part_of_its_inputs():
         for lo in (0, 65536 - 50, 15 * 65536 - 50, len(x) - 100):
             m, s = net.predict(x[lo:lo + 100])
             assert np.array_equal(m, mean[lo:lo + 100]) and np.array_equal(s, spread[lo:lo + 100])
+
+
+@pytest.mark.parametrize("sizes,rows,members", [([9000, 40], 37, 3), ([9000, 1], 1, 1), ([4, 8200, 4032], 64, 2),
+                                                ([4, 8200, 4032], 65, 2), ([4, 70, 20000, 300], 150, 5)])
+def test_predict_statistics_of_long_output_layers(sizes, rows, members):
+    """As above where an output layer of many inputs and few tiles runs member by member (and one row more
+    than that takes): mean and spread into host memory and device memory, scaled, and without the mean."""
+    rng = np.random.default_rng(rows)
+    with Network(sizes, members=members, max_batch=96, seed=rows) as net:
+        x = rng.standard_normal((rows, sizes[0])).astype(np.float32)
+        mean, spread = net.predict(x)
+        y = np.stack([np.concatenate([net.forward(x[lo:lo + 96], k) for lo in range(0, rows, 96)])
+                      for k in range(members)]).astype(np.float64)
+        assert rel(mean, y.mean(0)) < 1e-5
+        var = y.var(0, ddof=1) if members > 1 else np.zeros_like(y[0])
+        expect = np.sqrt(var.sum(1)) / np.linalg.norm(y.mean(0), axis=1)
+        assert np.allclose(spread, expect, rtol=1e-4, atol=1e-12)
+        assert np.array_equal(net.predict(x, want_mean=False)[1], spread)
+        dev = DeviceArray((rows, sizes[-1]))
+        assert np.array_equal(net.predict(x, out=dev)[1], spread) and np.array_equal(dev.to_host(), mean)
+        scale = rng.uniform(0.5, 2.0, sizes[-1]).astype(np.float32)
+        net.set_output_scale(scale)
+        assert np.array_equal(net.predict(x, out=dev)[1], spread) and np.array_equal(dev.to_host(), mean * scale[None, :])

@@ -34,3 +34,10 @@ def test_a_prediction_holds_bounded_inputs(tmp_path, n, inputs, batch):
     assert 1 <= rows <= n
     assert rows * inputs <= max(1 << 24, batch * inputs)
     assert rows == n or (rows % batch == 0 and (rows + batch) * inputs > 1 << 24)
+
+
+def test_output_layers_of_many_inputs_and_few_tiles_run_member_by_member(tmp_path):
+    shapes = {(1024, 151500, 512): 1, (37, 6300, 512): 1, (1, 8, 4096): 1, (1, 8, 8192): 0, (64, 4032, 8192): 0,
+              (65, 4032, 8192): 1, (64, 4096, 8192): 1, (256, 300, 65536): 0, (2147483647, 64, 1 << 24): 0}
+    body = "".join(f'printf("%d\\n", ensemble_in_registers({m}, {n}, {k}));' for m, n, k in shapes)
+    assert [v for v, in run(tmp_path, body)] == list(shapes.values())
