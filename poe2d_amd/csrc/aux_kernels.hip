@@ -109,14 +109,14 @@ __global__ void __launch_bounds__(256) absmax_blocks(StepArgs<T> A, int buf, flo
     if (threadIdx.x == 0) partial[blockIdx.x] = m;
 }
 
-// Of several members (blockIdx.y): checked one after the other, 64 members of 1201 x 1201 points cost
-// 128 launches and 64 read-backs after a batch run.
+// Of several members (blockIdx.x, the grid's axis without a limit of 65 535): checked one after the other,
+// 64 members of 1201 x 1201 points cost 128 launches and 64 read-backs after a batch run.
 template <class T>
 __global__ void __launch_bounds__(256) absmax_members(const FieldRange *ranges, float *partial)
 {
-    const FieldRange r = ranges[blockIdx.y];
-    const float m = block_absmax((const Vec4<T> *)r.v, r.n, blockIdx.x * 256LL + threadIdx.x, gridDim.x * 256LL);
-    if (threadIdx.x == 0) partial[blockIdx.y * gridDim.x + blockIdx.x] = m;
+    const FieldRange r = ranges[blockIdx.x];
+    const float m = block_absmax((const Vec4<T> *)r.v, r.n, blockIdx.y * 256LL + threadIdx.x, gridDim.y * 256LL);
+    if (threadIdx.x == 0) partial[(size_t)blockIdx.x * gridDim.y + blockIdx.y] = m;
 }
 
 // 16-byte stores over the aligned middle of each range, single words at its ends.
@@ -203,7 +203,7 @@ void launch_absmax(const StepArgs<T> &A, int buf, float *partials, int nblocks, 
 template <class T>
 void launch_absmax_members(const FieldRange *ranges, int n, float *partials, int nblocks, float *result, hipStream_t stream)
 {
-    absmax_members<T><<<dim3(nblocks, n), 256, 0, stream>>>(ranges, partials);
+    absmax_members<T><<<dim3(n, nblocks), 256, 0, stream>>>(ranges, partials);
     absmax_final<<<n, 256, 0, stream>>>(partials, nblocks, result);
 }
 

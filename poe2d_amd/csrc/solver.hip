@@ -1023,6 +1023,7 @@ template <class T>
 poe2d_status run_steps(poe2d_solver *s, int nsteps)
 {
     poe2d_status st;
+    int flips = 0;  // times the state changes buffers
     if (s->schedule == SCHED_TWOPASS) {
         Receivers R{s->nrec, s->mask, s->rix, s->riz};
         StepArgs<T> A = step_args<T>(s, s->cur, s->cur);
@@ -1041,11 +1042,9 @@ poe2d_status run_steps(poe2d_solver *s, int nsteps)
         HIP_TRY(hipEventRecord(s->ev1, s->stream));
     } else if (const TileShape shape = tile_shape({s}, s->auto_shape, s->block_w, s->tile_rows); shape.tiles) {
         if ((st = build_tiles<T>(s->list2, {s}, shape.steps, shape.tall, s->m->npal > 0, nsteps, s->stream))) return st;
-        int flips = 0;
         HIP_TRY(hipEventRecord(s->ev0, s->stream));
         if ((st = run_tiles<T>(s->list2, s->step, nsteps, s->stream, &flips))) return st;
         HIP_TRY(hipEventRecord(s->ev1, s->stream));
-        s->cur = (s->cur + flips) & 1;
     } else if (sizeof(T) == 4 && two_step_kernel(s)) {
         // step pairs on the two-step kernel, an odd last step on the single-step kernel
         const int pairs = nsteps / 2, rem = nsteps & 1;
@@ -1062,24 +1061,27 @@ poe2d_status run_steps(poe2d_solver *s, int nsteps)
         if (pairs && (st = run_list<T>(s->list2, pairs, s->graphs, s->stream))) return st;
         if (rem && (st = run_list<T>(s->list, 1, s->graphs, s->stream))) return st;
         HIP_TRY(hipEventRecord(s->ev1, s->stream));
-        s->cur = (s->cur + pairs + rem) & 1;
+        flips = pairs + rem;
     } else {
         const bool palette = (s->schedule == SCHED_FUSED || s->schedule == SCHED_FUSED2) && s->m->npal > 0;
         if ((st = build_list<T>(s->list, {s}, shape.bw, shape.th, palette, s->step, nsteps, s->stream))) return st;
         HIP_TRY(hipEventRecord(s->ev0, s->stream));
         if ((st = run_list<T>(s->list, nsteps, s->graphs, s->stream))) return st;
         HIP_TRY(hipEventRecord(s->ev1, s->stream));
-        s->cur = (s->cur + nsteps) & 1;
+        flips = nsteps;
     }
+    // (together, before anything else can fail: the buffer and the step it holds)
+    s->cur = (s->cur + flips) & 1;
+    s->step += nsteps;
     float vmax = 0.f;
     launch_absmax<T>(step_args<T>(s, s->cur, s->cur), s->cur, s->red + 1, s->red_blocks, s->red, s->stream);
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpyAsync(&vmax, s->red, sizeof(float), hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, s->ev0, s->ev1));
     s->last_ms = ms;
     s->last_steps = nsteps;
-    s->step += nsteps;
     return stability_check(s, vmax);
 }
 
@@ -1231,6 +1233,9 @@ poe2d_status batch_run_steps(poe2d_batch *b, int nsteps)
         (st = build_list<T>(b->list, b->members, std::max(shape.bw, 128), shape.th, palette, n0 + 2LL * pairs, rem, b->stream,
                              false, pairs)))
         return st;
+    const int nm = (int)b->members.size(), blocks = std::min(1024, std::max(8, 4096 / nm));
+    const size_t range_bytes = (nm * sizeof(FieldRange) + 255) / 256 * 256;
+    if (!b->check && (st = dev_alloc(&b->check, range_bytes + (size_t)nm * (blocks + 1) * sizeof(float)))) return st;
     HIP_TRY(hipEventRecord(b->ev0, b->stream));
     if (shape.tiles) {
         if ((st = run_tiles<T>(b->list2, n0, nsteps, b->stream, &flips))) return st;
@@ -1239,21 +1244,21 @@ poe2d_status batch_run_steps(poe2d_batch *b, int nsteps)
         if (rem && (st = run_list<T>(b->list, rem, b->graphs, b->stream))) return st;
     }
     HIP_TRY(hipEventRecord(b->ev1, b->stream));
-    // the stability checks of all members, in one launch
-    const int nm = (int)b->members.size(), blocks = std::min(1024, std::max(8, 4096 / nm));
+    // (together, before anything else can fail: the buffers and the step they hold)
     std::vector<FieldRange> ranges(nm);
-    std::vector<float> vmax(nm, 0.f);
     for (int i = 0; i < nm; ++i) {
         poe2d_solver *s = b->members[i];
         s->cur = (s->cur + flips) & 1;
+        s->step += nsteps;
         ranges[i] = {s->group_ptr(group_v(s->cur)) + s->m->origin() * 4 * sizeof(T),
                      (long long)(s->grid.nz + 1) * (long long)s->m->pitch};
     }
-    const size_t range_bytes = (nm * sizeof(FieldRange) + 255) / 256 * 256;
-    if (!b->check && (st = dev_alloc(&b->check, range_bytes + (size_t)nm * (blocks + 1) * sizeof(float)))) return st;
+    // the stability checks of all members, in one launch
+    std::vector<float> vmax(nm, 0.f);
     float *const result = (float *)((char *)b->check + range_bytes);
     HIP_TRY(hipMemcpyAsync(b->check, ranges.data(), nm * sizeof(FieldRange), hipMemcpyHostToDevice, b->stream));
     launch_absmax_members<T>((const FieldRange *)b->check, nm, result + nm, blocks, result, b->stream);
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpyAsync(vmax.data(), result, nm * sizeof(float), hipMemcpyDeviceToHost, b->stream));
     HIP_TRY(hipStreamSynchronize(b->stream));
     float ms = 0.f;
@@ -1263,7 +1268,6 @@ poe2d_status batch_run_steps(poe2d_batch *b, int nsteps)
     poe2d_status first = POE2D_OK;
     for (int i = 0; i < nm; ++i) {
         poe2d_solver *s = b->members[i];
-        s->step += nsteps;
         s->last_ms = ms;
         s->last_steps = nsteps;
         const poe2d_status c = stability_check(s, vmax[i]);
