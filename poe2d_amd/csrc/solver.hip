@@ -544,12 +544,12 @@ poe2d_status grow(StepList::Staged &b, size_t bytes)
     return POE2D_OK;
 }
 
-// Device copies of a list's arrays: the first step n0, work items, receiver offsets
-// and entries (member i's ptr_off[i] and ent_off[i] on), the members' source samples of steps [n0, n0 +
-// nsteps), and the members' arguments pointing at them.
-template <class T>
+// Device copies of a list's arrays: the first step n0, work items (work_bytes of them, by fill_work),
+// receiver offsets and entries (member i's ptr_off[i] and ent_off[i] on), the members' source samples of
+// steps [n0, n0 + nsteps), and the members' arguments pointing at them.
+template <class T, class Fill>
 poe2d_status upload_list(StepList &L, const std::vector<poe2d_solver *> &members, std::vector<StepArgs<T>> &args,
-                         const void *work, size_t work_bytes, const std::vector<int> &ptr, const std::vector<int2> &ent,
+                         const Fill &fill_work, size_t work_bytes, const std::vector<int> &ptr, const std::vector<int2> &ent,
                          const size_t *ptr_off, const size_t *ent_off, long long n0, int nsteps, hipStream_t stream)
 {
     const size_t nm = args.size();
@@ -567,7 +567,7 @@ poe2d_status upload_list(StepList &L, const std::vector<poe2d_solver *> &members
     if ((st = grow(L.arena, at)) || (st = grow(L.source, src_bytes))) return st;
     char *const dev = (char *)L.arena.dev, *const image = L.arena.image;
     *(long long *)(image + o_base) = n0;
-    std::memcpy(image + o_work, work, work_bytes);
+    fill_work(image + o_work);
     if (!ptr.empty()) std::memcpy(image + o_ptr, ptr.data(), ptr.size() * sizeof(int));
     if (!ent.empty()) std::memcpy(image + o_ent, ent.data(), ent.size() * sizeof(int2));
     T *const src = (T *)L.source.image;
@@ -682,8 +682,10 @@ poe2d_status build_list(StepList &L, const std::vector<poe2d_solver *> &members,
             for (size_t q = (size_t)x * ni; q < std::min(inter.size(), (size_t)(x + 1) * ni); ++q) work[o++] = inter[q];
         }
     }
-    const poe2d_status st = upload_list<T>(L, members, args, work.data(), work.size() * sizeof(WorkItem), ptr, ent,
-                                           ptr_off.data(), ent_off.data(), n0, nsteps, stream);
+    const size_t work_bytes = work.size() * sizeof(WorkItem);
+    const auto fill = [&](void *image) { std::memcpy(image, work.data(), work_bytes); };
+    const poe2d_status st = upload_list<T>(L, members, args, fill, work_bytes, ptr, ent, ptr_off.data(), ent_off.data(), n0,
+                                           nsteps, stream);
     if (st) return st;
     L.nmodels = nm;
     L.nint = two ? nint : (int)work.size();
@@ -697,15 +699,6 @@ poe2d_status build_list(StepList &L, const std::vector<poe2d_solver *> &members,
     L.precision = sizeof(T) == 4 ? POE2D_F32 : POE2D_F64;
     return POE2D_OK;
 }
-
-// The tiles of a launch and their receivers.
-struct TileCut {
-    std::vector<TileItem> edge, inter;
-    std::vector<int> ptr;
-    std::vector<int2> ent;
-
-    size_t tiles() const { return edge.size() + inter.size(); }
-};
 
 // Where a grid's tiles lie with `steps` steps per launch.  A column of tiles is three bands: the rows whose
 // region reaches the upper z strip or border, those away from both, and the lower ones; the tiles of a
@@ -730,70 +723,108 @@ struct TileGrid {
         const int most = xs && zs ? short_rows : xs || zs ? edge_rows : tall_rows, count = (left + most - 1) / most;
         return z0 + (left + count - 1) / count;
     }
-    size_t count(const poe2d_solver *s) const
-    {
-        size_t columns[2] = {0, 0}, n = 0;
-        for (int x0 = 0; x0 <= s->grid.nx; x0 += tile_cols(steps)) ++columns[x_edge(s, x0)];
-        for (int xs = 0; xs < 2; ++xs) {
-            bool zs;
-            if (columns[xs])
-                for (int z0 = 0; z0 <= s->grid.nz; z0 = end(s, xs, z0, zs)) n += columns[xs];
-        }
-        return n;
-    }
 };
 
-// Member i's part of the cut, interior tiles row by row in bands of kBandTiles tile columns, so that the
-// tiles in flight on an XCD (about 64) make a block of neighbours sharing their halos in its L2.
-void cut_tiles(const poe2d_solver *s, int i, const TileGrid &grid, TileCut &out)
-{
-    const int cols = tile_cols(grid.steps), nx = s->grid.nx, nz = s->grid.nz;
-    // receivers by tile column and row
-    std::vector<int> order(s->nrec);
-    for (int r = 0; r < s->nrec; ++r) order[r] = r;
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-        const int ta = s->hrx[a] / cols, tb = s->hrx[b] / cols;
-        return ta != tb ? ta < tb : s->hrz[a] < s->hrz[b];
-    });
-    size_t next = 0;
-    std::vector<TileItem> inter;  // column by column, every column cut alike
-    for (int x0 = 0; x0 <= nx; x0 += cols) {
-        const bool xs = grid.x_edge(s, x0);
-        for (int z0 = 0; z0 <= nz;) {
-            bool zs;
-            TileItem it{};
-            it.model = i;
-            it.x0 = x0;
-            it.z0 = z0;
-            it.z1 = grid.end(s, xs, z0, zs);
-            const bool tall = grid.tall_rows > grid.short_rows;
-            it.kind = !xs && !zs ? (tall ? TILE_TALL : TILE_SHORT) : !tall || (xs && zs) ? TILE_EDGE : xs ? TILE_EDGE_X : TILE_EDGE_Z;
-            it.rec = -1;
-            auto pending = [&](int z) {
-                return next < order.size() && s->hrx[order[next]] < x0 + cols && s->hrz[order[next]] < z;
-            };
-            if (pending(it.z1)) {
-                it.rec = (int)out.ptr.size();
-                for (int z = z0; z < it.z1; ++z) {
-                    out.ptr.push_back((int)out.ent.size());
-                    for (; pending(z + 1); ++next) out.ent.push_back(int2{s->hrx[order[next]], order[next]});
-                }
-                out.ptr.push_back((int)out.ent.size());
+// The tiles of member s (number `model` of a launch) and its receivers in them.  Every column away from
+// the x edges is cut alike, and so is every column at them, so a tile is a column and a row of that cut.
+class TileCut {
+public:
+    struct Row {
+        int z0, z1;
+        bool edge;
+    };
+
+    TileCut(const poe2d_solver *s, int model, const TileGrid &grid) : s_(s), model_(model), grid_(grid), cols_(tile_cols(grid.steps))
+    {
+        for (int x0 = 0; x0 <= s->grid.nx; x0 += cols_) x_edge_.push_back(grid.x_edge(s, x0));
+        for (int xs = 0; xs < 2; ++xs)
+            for (int z0 = 0; z0 <= s->grid.nz; z0 = rows_[xs].back().z1) {
+                Row r{z0, 0, false};
+                r.z1 = grid.end(s, xs, z0, r.edge);
+                rows_[xs].push_back(r);
             }
-            (xs || zs ? out.edge : inter).push_back(it);
-            z0 = it.z1;
+        const size_t at_edge = std::count(x_edge_.begin(), x_edge_.end(), true), away = x_edge_.size() - at_edge;
+        const size_t low = std::count_if(rows_[0].begin(), rows_[0].end(), [](const Row &r) { return r.edge; });
+        edge = at_edge * rows_[1].size() + away * low;
+        inter = away * (rows_[0].size() - low);
+    }
+
+    size_t edge, inter;  // tiles at an edge, and away from every edge
+
+    // Adds the receivers to a launch's: of each tile that has some, the offsets of its rows and the entries.
+    void receivers(std::vector<int> &ptr, std::vector<int2> &ent)
+    {
+        if (s_->nrec == 0) return;
+        std::vector<int> order(s_->nrec);
+        for (int r = 0; r < s_->nrec; ++r) order[r] = r;
+        std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+            const int ta = s_->hrx[a] / cols_, tb = s_->hrx[b] / cols_;
+            return ta != tb ? ta < tb : s_->hrz[a] < s_->hrz[b];
+        });
+        first_.assign(x_edge_.size() + 1, 0);
+        size_t next = 0;
+        for (size_t c = 0; c < x_edge_.size(); first_[++c] = (int)recs_.size()) {
+            const auto pending = [&](int z) {
+                return next < order.size() && s_->hrx[order[next]] / cols_ == (int)c && s_->hrz[order[next]] < z;
+            };
+            if (!pending(s_->grid.nz + 1)) continue;
+            for (const Row &row : rows_[x_edge_[c]]) {
+                if (!pending(row.z1)) continue;
+                recs_.push_back({row.z0, (int)ptr.size()});
+                for (int z = row.z0; z < row.z1; ++z) {
+                    ptr.push_back((int)ent.size());
+                    for (; pending(z + 1); ++next) ent.push_back(int2{s_->hrx[order[next]], order[next]});
+                }
+                ptr.push_back((int)ent.size());
+            }
         }
     }
-    size_t rows = 0;
-    while (rows < inter.size() && inter[rows].x0 == inter[0].x0) ++rows;
-    for (size_t c0 = 0; c0 < inter.size();) {
-        size_t c1 = c0;
-        while (c1 < inter.size() && inter[c1].x0 / (kBandTiles * cols) == inter[c0].x0 / (kBandTiles * cols)) c1 += rows;
-        for (size_t r = 0; r < rows; ++r)
-            for (size_t c = c0; c < c1; c += rows) out.inter.push_back(inter[c + r]);
-        c0 = c1;
+
+    // Edge tiles column by column; the others row by row in bands of kBandTiles columns, so that the tiles
+    // in flight on an XCD (about 64) make a block of neighbours sharing their halos in its L2.
+    template <class Put>
+    void put_edges(const Put &put) const
+    {
+        for (size_t c = 0; c < x_edge_.size(); ++c)
+            for (const Row &row : rows_[x_edge_[c]])
+                if (x_edge_[c] || row.edge) put(item(c, row));
     }
-}
+    template <class Put>
+    void put_interior(const Put &put) const
+    {
+        for (size_t c0 = 0; c0 < x_edge_.size(); c0 += kBandTiles)
+            for (const Row &row : rows_[0])
+                if (!row.edge)
+                    for (size_t c = c0; c < std::min(c0 + kBandTiles, x_edge_.size()); ++c)
+                        if (!x_edge_[c]) put(item(c, row));
+    }
+
+private:
+    TileItem item(size_t c, const Row &row) const
+    {
+        const bool xs = x_edge_[c], zs = row.edge, tall = grid_.tall_rows > grid_.short_rows;
+        const int kind = !xs && !zs ? (tall ? TILE_TALL : TILE_SHORT) : !tall || (xs && zs) ? TILE_EDGE : xs ? TILE_EDGE_X : TILE_EDGE_Z;
+        int rec = -1;
+        if (!recs_.empty()) {
+            const auto end = recs_.begin() + first_[c + 1];
+            const auto at = std::lower_bound(recs_.begin() + first_[c], end, row.z0, [](const Rec &r, int z0) { return r.z0 < z0; });
+            if (at != end && at->z0 == row.z0) rec = at->rec;
+        }
+        return {model_, (int)c * cols_, row.z0, row.z1, kind, rec};
+    }
+
+    struct Rec {
+        int z0, rec;
+    };
+    const poe2d_solver *s_;
+    int model_;
+    TileGrid grid_;
+    int cols_;
+    std::vector<unsigned char> x_edge_;  // of every column
+    std::vector<Row> rows_[2];  // of a column away from the x edges, and at one
+    std::vector<Rec> recs_;  // tiles with receivers, column by column
+    std::vector<int> first_;  // recs_ of column c: first_[c] .. first_[c + 1]
+};
 
 // As build_list, for the tile kernel, `steps` steps per launch.  steps = 0: three or two, by the rounds in
 // which the chip takes the tiles (two blocks per CU, one of FP64; up to one block per CU a round is a
@@ -818,23 +849,35 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
         if (!tall) return TileGrid{k, rows, rows, rows};
         return TileGrid{k, rows, tile_rows(tile_edge_p(palette), k), tile_rows(tile_tall_p(sizeof(T) == 4, palette), k)};
     };
+    const auto cut = [&](int k, std::vector<TileCut> &cuts) {
+        size_t n = 0;
+        for (int i = 0; i < nm; ++i) {
+            cuts.emplace_back(members[i], i, grid(k));
+            n += cuts.back().edge + cuts.back().inter;
+        }
+        return n;
+    };
+    std::vector<TileCut> cuts;
     if (!steps) {
-        const auto rounds = [&](int k) {
-            size_t n = 0;
-            for (const poe2d_solver *s : members) n += grid(k).count(s);
+        const auto rounds = [&](size_t n) {
             const size_t slots = kTileCus * (sizeof(T) == 4 ? 2 : 1);
             return n <= (size_t)kTileCus ? 1.0 : (sizeof(T) == 4 ? 1.25 : 1.0) * (double)((n + slots - 1) / slots);
         };
-        steps = 0.85 * rounds(3) < rounds(2) ? 3 : 2;
+        std::vector<TileCut> three;
+        steps = 0.85 * rounds(cut(3, three)) < rounds(cut(2, cuts)) ? 3 : 2;
+        if (steps == 3) cuts.swap(three);
+    } else {
+        cut(steps, cuts);
     }
-    TileCut tiles;
-    for (int i = 0; i < nm; ++i) {
-        cut_tiles(members[i], i, grid(steps), tiles);
-        if (tiles.tiles() > (1u << 28)) return fail(POE2D_E_INVALID, "run: too many tiles in one launch");
+    size_t edge = 0, inter = 0;
+    std::vector<int> ptr;
+    std::vector<int2> ent;
+    for (TileCut &c : cuts) {
+        edge += c.edge;
+        inter += c.inter;
+        if (edge + inter > (1u << 28)) return fail(POE2D_E_INVALID, "run: too many tiles in one launch");
+        c.receivers(ptr, ent);
     }
-    std::vector<TileItem> &edge = tiles.edge, &inter = tiles.inter;
-    const std::vector<int> &ptr = tiles.ptr;
-    const std::vector<int2> &ent = tiles.ent;
     std::vector<StepArgs<T>> args(nm);
     for (int i = 0; i < nm; ++i) {
         const poe2d_solver *s = members[i];
@@ -847,23 +890,38 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
         args[i].traces = (T *)s->traces;
     }
     // as the two-step kernel's list: every XCD gets an eighth of the edge tiles first, then a run of
-    // consecutive interior tiles; shares padded to equal length with empty items
-    const int ne = (int)((edge.size() + 7) / 8), ni = (int)((inter.size() + 7) / 8);
-    TileItem none{};
-    none.model = -1;
-    std::vector<TileItem> work((size_t)8 * (ne + ni), none);
-    for (int x = 0; x < 8; ++x) {
-        size_t o = (size_t)x * (ne + ni);
-        for (size_t e = x; e < edge.size(); e += 8) work[o++] = edge[e];
-        for (size_t q = (size_t)x * ni; q < std::min(inter.size(), (size_t)(x + 1) * ni); ++q) work[o++] = inter[q];
-    }
-    const poe2d_status st = upload_list<T>(L, members, args, work.data(), work.size() * sizeof(TileItem), ptr, ent, nullptr,
-                                           nullptr, members[0]->step, nsteps, stream);
+    // consecutive interior tiles; shares padded to equal length with empty items.  Written where it is
+    // copied from: large grids have 50 000 and more tiles, and through vectors of their own these took
+    // longer than a step (16000 x 16000, a run of two steps: 5.9 ms).
+    const size_t ne = (edge + 7) / 8, ni = (inter + 7) / 8, nwork = 8 * (ne + ni);
+    const auto fill = [&](void *image) {
+        TileItem *const work = (TileItem *)image;
+        size_t e = 0, q = 0;
+        for (const TileCut &c : cuts) {
+            c.put_edges([&](const TileItem &it) {
+                work[e % 8 * (ne + ni) + e / 8] = it;
+                ++e;
+            });
+        }
+        TileItem *at = work + ne, *share = work + ne + ni;  // the next interior tile and the end of its share
+        for (const TileCut &c : cuts)
+            c.put_interior([&](const TileItem &it) {
+                if (at == share) at += ne, share += ne + ni;
+                *at++ = it;
+                ++q;
+            });
+        TileItem none{};
+        none.model = -1;
+        for (; e < 8 * ne; ++e) work[e % 8 * (ne + ni) + e / 8] = none;
+        for (; q < 8 * ni; ++q) work[q / ni * (ne + ni) + ne + q % ni] = none;
+    };
+    const poe2d_status st = upload_list<T>(L, members, args, fill, nwork * sizeof(TileItem), ptr, ent, nullptr, nullptr,
+                                           members[0]->step, nsteps, stream);
     if (st) return st;
     L.nmodels = nm;
-    L.nint = (int)inter.size();
-    L.nwork = (int)work.size();
-    L.per_xcd = ne + ni;
+    L.nint = (int)inter;
+    L.nwork = (int)nwork;
+    L.per_xcd = (int)(ne + ni);
     L.bw = 64;
     L.palette = palette;
     L.avg = material == POE2D_MATERIAL_AVERAGED;
