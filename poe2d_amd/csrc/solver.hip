@@ -47,6 +47,7 @@ const double kStabilityThreshold = 1.0e25;  // STABILITY_THRESHOLD of the refere
 const int kGraphSteps = 32;                 // steps per captured graph
 const size_t kL2Bytes = size_t(32) << 20;   // the eight L2s together
 const size_t kMallBytes = size_t(256) << 20;  // the memory-side cache
+const int kTailWidth = 256, kTailRows = 14;  // tiles of the single-step kernel after launches of the tile kernel
 const size_t kTraceBytes = size_t(64) << 20;  // traces on their way to the host
 const int kBandTiles = 8;                   // tile columns to a band of the tile kernel's work order
 
@@ -1039,7 +1040,22 @@ struct TileShape {
     int steps;
     bool tall;
     int bw, th;
+    bool single_tail;  // an odd last step on the single-step kernel (two steps per launch)
 };
+
+long long grid_points(const poe2d_solver *s) { return (long long)(s->grid.nx + 1) * (s->grid.nz + 1); }
+
+// Whether one step by itself is faster on the single-step kernel, which computes no halo: where the step is
+// bound by arithmetic on grids that fill the chip many times.  us per run of a step, single / tiles: FP64
+// 6 M points 332 / 369, 16 M 694 / 863, 33 M 1302 / 1652 (1000 wide 1662 / 1798); FP32 without a palette 24 M
+// 709 / 772, 128 M 3314 / 3625; with one 128 M 2476 / 2466.
+bool single_step_faster(const std::vector<poe2d_solver *> &members)
+{
+    long long points = 0;
+    bool palette = true;
+    for (const poe2d_solver *s : members) points += grid_points(s), palette = palette && s->m->npal > 0;
+    return members[0]->precision == POE2D_F64 ? points >= 6000000 : !palette && points >= 20000000;
+}
 
 // The tile shape the members advance with: the chosen one (block width 64: the tile kernel, the
 // height selecting steps per launch and tile kind), or by default the tile kernel on tall tiles
@@ -1047,9 +1063,11 @@ struct TileShape {
 TileShape tile_shape(const std::vector<poe2d_solver *> &members, bool auto_shape, int bw, int th)
 {
     for (const poe2d_solver *s : members)
-        if (s->schedule != SCHED_FUSED2) return {false, 2, false, bw, th};
-    if (auto_shape) return {true, 0, true, 64, 36};
-    return {bw == 64, th < 12 || (th > 12 && th < 36) ? 3 : 2, th > 12, bw, th};
+        if (s->schedule != SCHED_FUSED2) return {false, 2, false, bw, th, false};
+    // (the grids of a single tail take two steps per launch by size, too)
+    if (auto_shape && single_step_faster(members)) return {true, 2, true, 64, 36, true};
+    if (auto_shape) return {true, 0, true, 64, 36, false};
+    return {bw == 64, th < 12 || (th > 12 && th < 36) ? 3 : 2, th > 12, bw, th, false};
 }
 
 // Shapes an autotuner times: of the two-step schedule (the tile kernel's two and the marching
@@ -1099,10 +1117,16 @@ poe2d_status run_steps(poe2d_solver *s, int nsteps)
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipEventRecord(s->ev1, s->stream));
     } else if (const TileShape shape = tile_shape({s}, s->auto_shape, s->block_w, s->tile_rows); shape.tiles) {
-        if ((st = build_tiles<T>(s->list2, {s}, shape.steps, shape.tall, s->m->npal > 0, nsteps, s->stream))) return st;
+        const int tail = shape.single_tail ? nsteps & 1 : 0, body = nsteps - tail;
+        if (body && (st = build_tiles<T>(s->list2, {s}, shape.steps, shape.tall, s->m->npal > 0, body, s->stream))) return st;
+        if (tail && (st = build_list<T>(s->list, {s}, kTailWidth, kTailRows, s->m->npal > 0, (long long)s->step + body, 1,
+                                        s->stream, false, body / 2)))
+            return st;
         HIP_TRY(hipEventRecord(s->ev0, s->stream));
-        if ((st = run_tiles<T>(s->list2, s->step, nsteps, s->stream, &flips))) return st;
+        if (body && (st = run_tiles<T>(s->list2, s->step, body, s->stream, &flips))) return st;
+        if (tail && (st = run_list<T>(s->list, 1, s->graphs, s->stream))) return st;
         HIP_TRY(hipEventRecord(s->ev1, s->stream));
+        flips += tail;
     } else if (sizeof(T) == 4 && two_step_kernel(s)) {
         // step pairs on the two-step kernel, an odd last step on the single-step kernel
         const int pairs = nsteps / 2, rem = nsteps & 1;
@@ -1276,31 +1300,33 @@ poe2d_status batch_run_steps(poe2d_batch *b, int nsteps)
     if ((two || shape.tiles) && shape.bw == 512)
         return fail(POE2D_E_INVALID, "batch_run: the two-step kernel takes block widths 64, 128 or 256");
     two = two || shape.tiles;
-    const int pairs = two ? nsteps / 2 : 0, rem = two ? nsteps & 1 : nsteps;
+    const int tail = shape.single_tail ? nsteps & 1 : 0, body = nsteps - tail;  // (tile kernel)
+    const int pairs = two ? nsteps / 2 : 0, rem = shape.tiles ? tail : two ? nsteps & 1 : nsteps;
     int flips = pairs + rem;
     poe2d_status st;
     if (shape.tiles) {
-        if ((st = build_tiles<T>(b->list2, b->members, shape.steps, shape.tall, tile_palette, nsteps, b->stream))) return st;
+        if (body && (st = build_tiles<T>(b->list2, b->members, shape.steps, shape.tall, tile_palette, body, b->stream))) return st;
     } else if (pairs) {
         for (poe2d_solver *s : b->members)
             if (!s->psi_mid && (st = dev_alloc(&s->psi_mid, std::max<size_t>(s->m->psi_half_elems(), 1) * s->rs)))
                 return st;
         if ((st = build_list<T>(b->list2, b->members, shape.bw, shape.th, palette2, n0, nsteps, b->stream, true))) return st;
     }
-    if (rem && !shape.tiles &&
-        (st = build_list<T>(b->list, b->members, std::max(shape.bw, 128), shape.th, palette, n0 + 2LL * pairs, rem, b->stream,
-                             false, pairs)))
+    if (rem && (st = build_list<T>(b->list, b->members, shape.tiles ? kTailWidth : std::max(shape.bw, 128),
+                                   shape.tiles ? kTailRows : shape.th, palette, n0 + 2LL * pairs, rem, b->stream, false, pairs)))
         return st;
     const int nm = (int)b->members.size(), blocks = std::min(1024, std::max(8, 4096 / nm));
     const size_t range_bytes = (nm * sizeof(FieldRange) + 255) / 256 * 256;
     if (!b->check && (st = dev_alloc(&b->check, range_bytes + (size_t)nm * (blocks + 1) * sizeof(float)))) return st;
     HIP_TRY(hipEventRecord(b->ev0, b->stream));
     if (shape.tiles) {
-        if ((st = run_tiles<T>(b->list2, n0, nsteps, b->stream, &flips))) return st;
-    } else {
-        if (pairs && (st = run_list<T>(b->list2, pairs, b->graphs, b->stream))) return st;
-        if (rem && (st = run_list<T>(b->list, rem, b->graphs, b->stream))) return st;
+        flips = 0;
+        if (body && (st = run_tiles<T>(b->list2, n0, body, b->stream, &flips))) return st;
+        flips += tail;
+    } else if (pairs && (st = run_list<T>(b->list2, pairs, b->graphs, b->stream))) {
+        return st;
     }
+    if (rem && (st = run_list<T>(b->list, rem, b->graphs, b->stream))) return st;
     HIP_TRY(hipEventRecord(b->ev1, b->stream));
     // (together, before anything else can fail: the buffers and the step they hold)
     std::vector<FieldRange> ranges(nm);
