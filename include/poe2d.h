@@ -179,7 +179,9 @@ poe2d_status poe2d_set_receivers(poe2d_solver *s, const poe2d_receivers *rec);
  *     a run takes one schedule-0 launch.  On FP64 handles those widths run schedule 0.
  * Until this call (or poe2d_autotune) a handle runs schedule 3 on the tile kernel's tall regions,
  * two or three steps per launch by the size of the grid, or of the whole batch; an odd last step on
- * large grids (6 M points in FP64, 20 M in FP32 without a palette) as schedule 0.
+ * large grids (6 M points in FP64, 20 M in FP32 without a palette) as schedule 0.  FP32 grids of
+ * averaged material 5000 to 18 000 columns wide (20 M points without a palette, 64 M with one) run
+ * block_w 256, tile_rows 24.
  * Tile heights do not change a bit; schedules and block widths agree to rounding.  The choice
  * only changes speed. */
 poe2d_status poe2d_set_schedule(poe2d_solver *s, int schedule, int block_w, int tile_rows);

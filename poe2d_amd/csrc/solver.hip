@@ -1045,6 +1045,19 @@ struct TileShape {
 
 long long grid_points(const poe2d_solver *s) { return (long long)(s->grid.nx + 1) * (s->grid.nz + 1); }
 
+// Whether the marching kernel is the faster default: averaged material on large FP32 grids of rows that
+// are neither short (a tenth of its tile columns and more then hold an edge) nor longer than the tiles an
+// XCD has in flight (tiles of consecutive rows then share no halo in its L2).  us per step, marching /
+// tiles, averaged, no palette: 20 M points 8000 wide 250 / 263, 24 M 4000 wide 326 / 307, 5000 312 / 313,
+// 8000 294 / 312, 18 000 313 / 320, 20 000 332 / 321, 64 M 8000 730 / 813; with a palette 33 M 269 / 269, 64 M
+// 13 600 wide 487 / 506.  Material as written: tiles 0.98 to 2 times as fast up to 16 000 x 16 000.
+bool marching_faster(const poe2d_solver *s)
+{
+    if (!two_step_kernel(s) || s->grid.staggered_material != POE2D_MATERIAL_AVERAGED) return false;
+    if (s->m->npal > 0 && !two_step_palette(s)) return false;  // (it would read the groups instead)
+    return s->grid.nx >= 5000 && s->grid.nx < 18000 && grid_points(s) >= (s->m->npal > 0 ? 64000000 : 20000000);
+}
+
 // Whether one step by itself is faster on the single-step kernel, which computes no halo: where the step is
 // bound by arithmetic on grids that fill the chip many times.  us per run of a step, single / tiles: FP64
 // 6 M points 332 / 369, 16 M 694 / 863, 33 M 1302 / 1652 (1000 wide 1662 / 1798); FP32 without a palette 24 M
@@ -1064,6 +1077,7 @@ TileShape tile_shape(const std::vector<poe2d_solver *> &members, bool auto_shape
 {
     for (const poe2d_solver *s : members)
         if (s->schedule != SCHED_FUSED2) return {false, 2, false, bw, th, false};
+    if (auto_shape && std::all_of(members.begin(), members.end(), marching_faster)) return {false, 2, false, 256, 24, false};
     // (the grids of a single tail take two steps per launch by size, too)
     if (auto_shape && single_step_faster(members)) return {true, 2, true, 64, 36, true};
     if (auto_shape) return {true, 0, true, 64, 36, false};

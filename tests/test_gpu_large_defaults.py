@@ -54,3 +54,9 @@ def test_single_last_steps_of_a_large_batch():
             _same((s.seismograms(), {f: s.snapshot(f) for f in STATE + ("p",)}, s.checkpoint()), ref, "batch")
     for s in solvers:
         s.close()
+
+
+@pytest.mark.parametrize("steps", [(1, 2, 1), (4,)])
+def test_averaged_material_on_a_large_grid(steps):
+    prob = problem(5200, 3900, 0, staggered_material=_abi.MATERIAL_AVERAGED)
+    _same(_run(prob, 32, None, steps), _run(prob, 32, (0, 256, 14), [4]), f"averaged {steps}")
