@@ -151,8 +151,8 @@ struct StepList {
     int nmodels = 0, nwork = 0, per_xcd = 0, bw = 0;
     bool palette = false;
     bool avg = false;  // POE2D_MATERIAL_AVERAGED (all members alike)
-    bool two = false;  // two-step or tile kernel: each launch advances two steps
-    bool tiles = false;  // tile kernel
+    bool two = false;  // marching two-step kernel
+    bool tiles = false;  // tile kernel (never in a graph)
     int steps = 2;       // its steps per launch
     bool stream_out = false;  // it stores the state past the caches (see build_tiles)
     int nint = 0;      // two-step kernel: interior tiles in the list
@@ -161,12 +161,12 @@ struct StepList {
     hipGraphExec_t exec = nullptr;
     struct Sig {
         void *models, *work, *base;
-        int nwork, nint, per_xcd, bw, palette, avg, two, tiles, steps, stream_out, precision;
+        int nwork, nint, per_xcd, bw, palette, avg, two, precision;
         bool operator==(const Sig &o) const
         {
             return models == o.models && work == o.work && base == o.base && nwork == o.nwork && nint == o.nint &&
                    per_xcd == o.per_xcd && bw == o.bw && palette == o.palette && avg == o.avg && two == o.two &&
-                   tiles == o.tiles && steps == o.steps && stream_out == o.stream_out && precision == o.precision;
+                   precision == o.precision;
         }
     } sig{};
 
@@ -175,7 +175,6 @@ struct StepList {
         Sig g{};
         g.models = models; g.work = work; g.base = base;
         g.nwork = nwork; g.nint = nint; g.per_xcd = per_xcd; g.bw = bw; g.palette = palette; g.avg = avg; g.two = two;
-        g.tiles = tiles; g.steps = steps; g.stream_out = stream_out;
         g.precision = precision;
         return g;
     }
@@ -926,7 +925,7 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
     L.bw = 64;
     L.palette = palette;
     L.avg = material == POE2D_MATERIAL_AVERAGED;
-    L.two = true;
+    L.two = false;
     L.tiles = true;
     L.steps = steps;
     // Stores past the caches where a launch's state, both buffers of it, fits neither the L2s nor the
@@ -948,6 +947,7 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
 template <class T>
 hipError_t launch_list_chunk(const StepList &L, int count, hipStream_t stream)
 {
+    if (L.tiles) return hipErrorInvalidValue;  // (its items are the tile kernel's: run_tiles)
     if (L.two) {
         if constexpr (sizeof(T) == 4) {
             for (int k = 0; k < count; ++k) {
