@@ -68,8 +68,8 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "fused_step_4001x4001_traffic.txt"
 
 def steps_per_launch(tile, schedule):
     """Time steps of one launch: one (schedule 0); two, or on the tile kernel (block width 64) three
-    for tile heights 30 and 6."""
-    return 1 if schedule != 3 else 3 if tile[0] == 64 and tile[1] in (6, 30) else 2
+    for the tile heights poe2d_set_schedule gives three steps."""
+    return 1 if schedule != 3 else 3 if tile[0] == 64 and (tile[1] < 12 or 12 < tile[1] < 36) else 2
 
 
 def recorded_traffic(tile, n, schedule=0):

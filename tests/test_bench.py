@@ -44,3 +44,14 @@ def test_recorded_traffic_is_per_time_step():
     # another grid, or a shape that was not profiled: no figure
     assert bench.recorded_traffic((256, 8), 1200, 0) == (None, None)
     assert bench.recorded_traffic((128, 30), 4000, 3) == (None, None)
+
+
+def test_steps_of_a_launch_follow_the_library():
+    # poe2d_set_schedule: width 64 takes three steps for heights 4 to 11 and 13 to 35, two for 12 and from 36 on
+    three = [h for h in range(4, 80) if bench.steps_per_launch((64, h), 3) == 3]
+    assert three == list(range(4, 12)) + list(range(13, 36))
+    assert all(bench.steps_per_launch((w, h), 3) == 2 for w in (128, 256) for h in (6, 24, 30))
+    assert all(bench.steps_per_launch((w, h), 0) == 1 for w in (128, 256, 512) for h in (8, 30))
+    prob_points, strips = 4001 * 4001, 44 * 4001 * 2
+    assert bench.compulsory_bytes_per_step(prob_points, strips, 3, True, (64, 24)) == pytest.approx(
+        (65.0 * prob_points + 48.0 * strips) / 3)
