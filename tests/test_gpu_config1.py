@@ -163,3 +163,31 @@ def test_continuous_model_whole_grid_two_step_vs_single_step():
         assert np.abs(two[1][f]).max() > 0, f
         assert np.array_equal(two[1][f], one[1][f]), f
     assert np.array_equal(two[2], one[2])
+
+
+@pytest.mark.parametrize("model", ["patchy", "continuous"])
+def test_whole_grid_tile_kernel_vs_single_step(c1, model):
+    """The tile kernel, which configuration 1 runs by default and tuned, over both 4001 x 4001 models from a
+    random state (state stored past the caches, tens of thousands of tiles): 21 steps on two and on three
+    steps per launch and by default equal the single-step kernel bitwise over the whole grid."""
+    from poe2d_amd.configs import config1_continuous
+    prob = c1 if model == "patchy" else config1_continuous(nt=21)
+    init = random_state(prob.nx, seed=13)
+
+    def gpu(*shape):
+        say(f"{model} 4001^2 random state: {shape or 'default'}, 21 steps")
+        with Solver(prob) as s:
+            if shape:
+                s.set_schedule(*shape)
+            for f, a in init.items():
+                s.set_field(f, a)
+            s.run(21)
+            return s.seismograms()[..., :21], {f: s.snapshot(f) for f in FIELDS}, s.checkpoint()
+
+    one = gpu(0, 256, 8)
+    for shape in ((3, 64, 36), (3, 64, 30), ()):
+        got = gpu(*shape)
+        assert np.array_equal(got[0], one[0]), f"{shape}: seismograms differ"
+        for f in FIELDS:
+            assert np.abs(got[1][f]).max() > 0 and np.array_equal(got[1][f], one[1][f]), (shape, f)
+        assert np.array_equal(got[2], one[2]), f"{shape}: checkpoints differ"

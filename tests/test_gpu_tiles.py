@@ -161,3 +161,39 @@ def test_long_traces_are_read_in_parts(precision):
             got.append(g[..., :7])
             assert not g[..., 7:].any()
     assert np.abs(got[0]).max() > 0 and np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("opts", [dict(), dict(staggered_material=1)])
+@pytest.mark.parametrize("entries", [2, 40, 0])
+@pytest.mark.parametrize("precision", [32, 64])
+def test_launches_of_more_tiles_than_compute_units(opts, entries, precision):
+    """Over 256 tiles, an FP32 launch runs two blocks to a CU: half the registers, profiles of the columns in
+    LDS, coefficients read where they are used.  46 to 92 MB of state are also stored through the caches
+    (smaller launches store past them).  Receivers stand on the edges of 46- and 52-column tiles."""
+    prob = _problem(900, 800, 20, entries, **opts)
+    ix = np.unique([0, 1, 45, 46, 47, 51, 52, 53, 91, 92, 103, 104, 459, 460, 467, 468, 850, 899, 900]).astype(np.int32)
+    iz = np.unique([0, 1, 26, 29, 30, 35, 36, 61, 62, 400, 401, 772, 799, 800]).astype(np.int32)
+    gx, gz = (a.ravel() for a in np.meshgrid(ix, iz))
+    prob.receivers = ReceiverSpec(ix=gx, iz=gz)
+    ref = _run(prob, precision, (0, 256, 14), [7])
+    for shape, steps in (((3, 64, 36), [7]), ((3, 64, 30), [5, 2]), ((3, 64, 12), [7]), ((3, 64, 6), [7]), (None, [4, 3])):
+        _same(_run(prob, precision, shape, steps), ref, f"{opts} {entries} entries shape {shape}")
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+def test_batch_of_palette_and_continuous_members_on_tiles(precision):
+    # the whole batch reads the coefficient groups; large enough for more tiles than compute units
+    probs = [_problem(520, 610, 10, 2, seed=1), _problem(430, 500, 10, 0, seed=2), _problem(61, 200, 10, 40, seed=3)]
+    alone = [_run(p, precision, (0, 256, 14), [9]) for p in probs]
+    solvers = [Solver(p, precision=precision) for p in probs]
+    for s in solvers:
+        g = np.random.default_rng(11)
+        for f in STATE:
+            s.set_field(f, g.standard_normal((s.problem.nz + 1, s.problem.nx + 1)) * (1e-9 if f[0] in "ez" else 1e-6))
+    with Batch(solvers) as b:
+        b.run(4)
+        b.run(5)
+        for s, ref in zip(solvers, alone):
+            _same((s.seismograms(), {f: s.snapshot(f) for f in STATE + ("p",)}, s.checkpoint()), ref, "batch")
+    for s in solvers:
+        s.close()
