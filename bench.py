@@ -300,7 +300,7 @@ def secondary_no_palette(prob, nt, label):
 
 def batch_bench(args):
     """Configuration 2: batch A or batch B, FP32, advanced in lock-step by one work-list launch per
-    time step (per two steps on the two-step kernel) with the loop in HIP graphs; tile shape and
+    time step (per two or three steps on schedule 3's kernels); tile shape and
     kernel autotuned.  value = sum over members of points x nt / device time of one batch run."""
     nt = args.nt if args.nt_given else 3000
     members, workload, bytes_per_point, npts = build_batch(args.workload, nt)
@@ -321,8 +321,9 @@ def batch_bench(args):
                    "tile": f"{tile[0]}x{tile[1]} ({'autotuned' if fixed is None else 'fixed'})",
                    "step": "one batch run of nt steps",
                    "schedule": SCHEDULE_NAMES[schedule],
-                   "launch": "one work-list launch per time step (per two steps with the two-step kernel), "
-                             "32-step HIP graphs", "traces_finite": finite},
+                   "launch": (f"one work-list launch per {steps_per_launch(tile, schedule)} time step(s), " +
+                              ("direct" if schedule == 3 and tile[0] == 64 else "32-step HIP graphs")),
+                   "traces_finite": finite},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
                      "per_launch": f"one time step of the batch: {bytes_per_point:.1f} B x {npts} points "

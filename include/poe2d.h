@@ -156,7 +156,8 @@ poe2d_status poe2d_set_source(poe2d_solver *s, const poe2d_source *src);
 poe2d_status poe2d_set_wavelet(poe2d_solver *s, const double *w, int n);
 
 /* Set the receivers and allocate the device trace buffer.  Replaces panj/panj2/a0_pos/a1_pos/
- * samprek (:496-502, :759-762) and the save1_kernel gather (:114-201). */
+ * samprek (:496-502, :759-762) and the save1_kernel gather (:114-201).  A call that fails for want of
+ * device memory leaves the handle without receivers. */
 poe2d_status poe2d_set_receivers(poe2d_solver *s, const poe2d_receivers *rec);
 
 /* Choose how a time step is executed on this handle (no counterpart in the reference, whose

@@ -22,7 +22,8 @@ STATUS_NAMES = {
 F32 = 32
 F64 = 64
 
-# palette entries up to which schedule 3 (two steps per launch) runs; larger palettes run schedule 0
+# palette entries up to which schedule 3's marching kernel (block widths 128 and 256) reads the palette;
+# with more it reads the coefficient groups
 MAX_PALETTE_TWO_STEP = 28
 
 STRESS_AS_WRITTEN = 0

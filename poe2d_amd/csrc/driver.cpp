@@ -37,7 +37,7 @@ struct Options {
     std::string input1 = "input1.txt", input2 = "input2.txt", outdir = ".";
     int precision = 32;
     std::string tile = "auto";
-    int schedule = -1;  // -1: the handle's default (3 for FP32, 0 for FP64)
+    int schedule = -1;  // -1: 3 in FP32, 0 in FP64
     bool quiet = false;
     int stress_law = POE2D_STRESS_AS_WRITTEN;
     int material = POE2D_MATERIAL_AS_WRITTEN;

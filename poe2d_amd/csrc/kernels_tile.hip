@@ -16,7 +16,7 @@
 // where a block marching down its rows pays one per row step (about 2 us each, 4 with C-PML records):
 // two steps of a 161^2 grid take 11 us instead of 119, 401^2 12 instead of 122, 701 x 523 FP64 28
 // instead of 127 (two single-step launches).  Large grids are bound by HBM: 4001^2 takes 231 us per
-// launch against 298 for the marching kernel, 1.17 GB (1.04 compulsory) at 5.0 TB/s (128 VGPRs, four
+// launch against 298 for the marching kernel, 1.14 GB (1.06 compulsory) at 4.95 TB/s (128 VGPRs, four
 // waves per SIMD, two blocks per CU).  Mid-sized ones by their edges' wider halo: with P = 3 and both
 // axes' code along every edge, 401^2 took 6.1 us a step instead of 5.0 (three steps per launch), 801^2
 // 12.0 instead of 8.8, 1201^2 16.7 instead of 15.1, 64 models of 401^2 127 instead of 103.

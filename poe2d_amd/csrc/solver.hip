@@ -931,9 +931,9 @@ poe2d_status build_tiles(StepList &L, const std::vector<poe2d_solver *> &members
     // Stores past the caches where a launch's state, both buffers of it, fits neither the L2s nor the
     // memory-side cache (the halos neighbours read stay in L2 instead), and where it fits the L2s with
     // room to spare (less to write back at the launch's end); between the two the next launch reads
-    // what this one left there.  us per step, cached / past: 701^2 9.0 / 8.7 (31 MB), 801^2 12.2 / 13.0,
-    // 2001^2 35.6 / 37.4 (256 MB), 2201^2 43.4 / 42.5, 4001^2 126 / 118; FP64, which HBM does not bound,
-    // 401^2 9.05 / 8.6, 1201^2 41.5 / 46.4, 2801^2 200 / 214.
+    // what this one left there.  us per step, cached / past: 701^2 8.74 / 8.54 (31 MB), 801^2 8.96 / 8.75,
+    // 1201^2 15.3 / 16.0, 2001^2 33.4 / 33.9 (256 MB), 2201^2 41.0 / 39.9, 4001^2 123 / 115; FP64, which HBM
+    // does not bound, 401^2 8.5 / 8.25, 1201^2 38.1 / 40.9, 2801^2 196 / 209.
     size_t state = 0;
     for (const poe2d_solver *s : members)
         state += (size_t)(s->grid.nx + 1) * (s->grid.nz + 1) * (palette ? 16 : 24) * sizeof(T);
@@ -1071,8 +1071,9 @@ bool single_step_faster(const std::vector<poe2d_solver *> &members)
 }
 
 // The tile shape the members advance with: the chosen one (block width 64: the tile kernel, the
-// height selecting steps per launch and tile kind), or by default the tile kernel on tall tiles
-// (never slower than short ones: 161^2 5.9 / 5.9, 401^2 6.5 / 6.6 us per step, 4001^2 127 / 172).
+// height selecting steps per launch and tile kind), or by default the tile kernel on tall tiles.  Short
+// ones are faster only on the smallest grids, by 3 %; us per step, the faster tall / short: 161^2 4.8 / 5.2
+// (averaged 5.5 / 5.4), 401^2 5.2 / 6.5, 1201^2 15.2 / 19.3, 4001^2 113 / 168.
 TileShape tile_shape(const std::vector<poe2d_solver *> &members, bool auto_shape, int bw, int th)
 {
     for (const poe2d_solver *s : members)

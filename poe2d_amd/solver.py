@@ -217,7 +217,9 @@ class Solver(HandleSolver):
         the coefficients through the material palette when the grid has one;
         1: separate stress and velocity launches;
         2: as 0, always reading the per-point coefficient arrays;
-        3: two steps per launch (block_w 64: the tile kernel, what a handle runs until this call)."""
+        3: several steps per launch: the tile kernel at block_w 64 (tile_rows 12 and from 36 on: two
+        steps, else three), the marching two-step kernel at 128 and 256.  Until this call a handle runs
+        schedule 3 by the size of its grid (see poe2d.h)."""
         self._check(self._lib.poe2d_set_schedule(self._h, schedule, block_w, tile_rows), "set_schedule")
 
     def set_graphs(self, on=True):

@@ -160,7 +160,7 @@ def receiver_points(geom=CONFIG3):
     return ix, np.full(geom["nrec"], c + geom["rec_dz"], np.int32)
 
 
-TILE = (128, 24)  # starting tile shape of the batched two-step kernel (then autotuned)
+TILE = (128, 24)  # tile shape of the handles until their batch is autotuned
 
 
 def gather_shape(geom=CONFIG3):
@@ -193,7 +193,7 @@ class SolverPool:
         try:
             for p in problems:
                 s = Solver(p)
-                s.set_schedule(3, *TILE)  # two steps per launch (bitwise equal to one)
+                s.set_schedule(3, *TILE)  # several steps per launch (bitwise equal to one)
                 self.solvers.append(s)
         except Exception:
             self.close()

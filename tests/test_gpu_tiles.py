@@ -197,3 +197,35 @@ def test_batch_of_palette_and_continuous_members_on_tiles(precision):
             _same((s.seismograms(), {f: s.snapshot(f) for f in STATE + ("p",)}, s.checkpoint()), ref, "batch")
     for s in solvers:
         s.close()
+
+
+@pytest.mark.parametrize("after", [(0, 256, 14), (1, 256, 14), (2, 256, 14), (3, 256, 24), (3, 64, 36), None])
+@pytest.mark.parametrize("before", [(0, 256, 14), (1, 256, 14), (3, 256, 24), (3, 64, 30), None])
+def test_reset_clears_what_any_kernel_reads(before, after):
+    # every field set at every point (the border's too), or infinite somewhere, whichever buffer and kernel
+    # it ran on: after a reset every kernel starts from zero
+    prob = _problem(104, 131, 10, 2)
+    rng = np.random.default_rng(1)
+    noise = {f: rng.standard_normal((132, 105)) * (1e-9 if f[0] in "ez" else 1e-6) for f in STATE}
+    with Solver(prob) as s:
+        if after:
+            s.set_schedule(*after)
+        s.run(9)
+        ref = s.seismograms(), {f: s.snapshot(f) for f in STATE}, s.checkpoint()
+    for broken in (False, True):
+        with Solver(prob) as s:
+            if before:
+                s.set_schedule(*before)
+            for f in STATE:
+                s.set_field(f, noise[f])
+            if broken:
+                s.set_field("vy", np.where(rng.random((132, 105)) < 0.01, np.inf, noise["vy"]))
+                with pytest.raises(_abi.Poe2dError):
+                    s.run(4)
+            else:
+                s.run(5)
+            s.reset()
+            if after or before:
+                s.set_schedule(*(after or (3, 64, 30)))
+            s.run(9)
+            _same((s.seismograms(), {f: s.snapshot(f) for f in STATE}, s.checkpoint()), ref, f"{before} then {after}")
