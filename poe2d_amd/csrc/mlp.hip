@@ -474,7 +474,7 @@ poe2d_status ensemble_batch(poe2d_mlp *m, int nb, float *mean, float *spread)
     for (int li = 0; li < m->L; ++li) {
         const Layer &l = m->members[0].layers[li];
         if (li == m->L - 1) {
-            if (!ensemble_in_registers(nb, l.out, l.inp)) return output_by_member(m, h, stride, nb, mean, spread);
+            if (!ensemble_in_registers(nb, l.out, l.inp, E == 1)) return output_by_member(m, h, stride, nb, mean, spread);
             HIP_TRY(ensemble_output(h, l.inp, stride, m->ens_w[li], l.inp, m->ens_b[li], E, nb, l.out, l.inp, mean, l.out,
                                     m->oscale, m->ens_part, spread, m->stream));
             break;
@@ -713,7 +713,7 @@ static poe2d_status alloc_scratch(poe2d_mlp *m, bool predict)
          (st = dmalloc(&m->acc_mean, (size_t)B * sizes[nlayers])) ||
          (st = dmalloc(&m->ens_part, ensemble_part_doubles(B, sizes[nlayers])))))
         return st;
-    if (predict && !ensemble_in_registers(1, sizes[nlayers], pad128(sizes[nlayers - 1])) &&
+    if (predict && !ensemble_in_registers(1, sizes[nlayers], pad128(sizes[nlayers - 1]), m->members.size() == 1) &&
         (st = dmalloc(&m->acc_m2, (size_t)B * sizes[nlayers])))
         return st;
     if (predict) {

@@ -41,3 +41,9 @@ def test_output_layers_of_many_inputs_and_few_tiles_run_member_by_member(tmp_pat
               (65, 4032, 8192): 1, (64, 4096, 8192): 1, (256, 300, 65536): 0, (2147483647, 64, 1 << 24): 0}
     body = "".join(f'printf("%d\\n", ensemble_in_registers({m}, {n}, {k}));' for m, n, k in shapes)
     assert [v for v, in run(tmp_path, body)] == list(shapes.values())
+
+
+def test_output_layers_of_one_member_run_split_from_2048_inputs_on(tmp_path):
+    shapes = {(1, 8, 2048): 1, (1, 8, 2176): 0, (37, 300, 3072): 0, (256, 300, 3072): 1, (1, 8, 1 << 24): 0}
+    body = "".join(f'printf("%d\\n", ensemble_in_registers({m}, {n}, {k}, true));' for m, n, k in shapes)
+    assert [v for v, in run(tmp_path, body)] == list(shapes.values())
